@@ -556,47 +556,47 @@ void phase_matrix_csr(const PhaseMatrix& pm, std::vector<int32_t>& off, std::vec
     }
 }
 
-// G+ = pinv(A^T A) of a phase matrix into d_Gp (N x N, device), from the device
-// copies of its row pairs and per-antenna rows; the components come from the host.
-void gram_pinv_device(leap_ctx* ctx, const PhaseMatrix& pm, const int2* d_pairs, const int32_t* d_off,
-                      const int32_t* d_ent, double* d_Gp) {
-    hipStream_t s = ctx->stream;
-    const int32_t N = pm.cols;
-    const GramComponents comps = gram_components(pm);
-    std::vector<int64_t> ws_off(comps.has_c.size() + 1, 0);
-    for (size_t c = 0; c < comps.has_c.size(); ++c) {
-        const int64_t n = comps.off[c + 1] - comps.off[c];
-        ws_off[c + 1] = ws_off[c] + 2 * n * n;
-    }
-    DeviceBuffer d_comp_off, d_members, d_has_c, d_ws_off, d_ws, d_G, d_status;
-    upload(s, d_comp_off, comps.off);
-    upload(s, d_members, comps.members);
-    upload(s, d_has_c, comps.has_c);
-    upload(s, d_ws_off, ws_off);
-    d_ws.reserve(std::max<size_t>(1, size_t(ws_off.back())) * sizeof(double));
-    d_G.reserve(size_t(N) * N * sizeof(double));
-    const std::vector<int32_t> zero(1, 0);
-    upload(s, d_status, zero);
-    GramPinv g{};
-    g.N = N;
-    g.constraint = pm.constraint;
-    g.csr_off = d_off;
-    g.csr_ent = d_ent;
-    g.pairs = d_pairs;
-    g.n_components = int32_t(comps.has_c.size());
-    g.comp_off = d_comp_off.as<int32_t>();
-    g.members = d_members.as<int32_t>();
-    g.has_c = d_has_c.as<uint8_t>();
-    g.ws_off = d_ws_off.as<int64_t>();
-    g.ws = d_ws.as<double>();
-    g.G = d_G.as<double>();
-    g.Gp = d_Gp;
-    g.status = d_status.as<int32_t>();
-    launch_gram_pinv(s, g);
+// What gram_pinv_device leaves running on the stream: host and device memory that has to
+// outlive the next synchronisation, and the status to look at after it.
+struct GramWork {
+    std::vector<GramComponents> comps;
+    std::vector<GramPinv> mats;
+    DeviceBuffer d_scratch, d_mats, d_status;
+    std::vector<DeviceBuffer> d_comp, d_shift;
     int32_t status = 0;
-    LEAP_HIP(hipMemcpyAsync(&status, d_status.ptr, sizeof(int32_t), hipMemcpyDeviceToHost, s));
-    LEAP_HIP(hipStreamSynchronize(s));  // before the scratch buffers go
-    require(status == 0, LEAP_ERR_INTERNAL, "phase matrix Gram block is not positive definite");
+    const std::vector<int32_t> zero{0};
+};
+
+struct GramSource {
+    const PhaseMatrix* pm;
+    const int2* d_pairs;
+    const int32_t *d_off, *d_ent;  // each antenna's rows
+    double* d_Gp;                  // N x N output
+};
+
+// G+ = pinv(A^T A) of phase matrices of one antenna count, all in the same launches,
+// from the device copies of their row pairs and per-antenna rows; the components come
+// from the host.
+void gram_pinv_device(leap_ctx* ctx, const std::vector<GramSource>& from, int32_t N, GramWork& w) {
+    hipStream_t s = ctx->stream;
+    const size_t nn = size_t(N) * N;
+    w.comps.reserve(from.size());
+    w.d_comp = std::vector<DeviceBuffer>(from.size());
+    w.d_shift = std::vector<DeviceBuffer>(from.size());
+    w.d_scratch.reserve(std::max<size_t>(1, 2 * nn * from.size()) * sizeof(double));
+    upload(s, w.d_status, w.zero);
+    for (size_t i = 0; i < from.size(); ++i) {
+        const GramSource& f = from[i];
+        w.comps.push_back(gram_components(*f.pm));
+        upload(s, w.d_comp[i], w.comps[i].comp);
+        upload(s, w.d_shift[i], w.comps[i].shift);
+        double* buf = w.d_scratch.as<double>() + 2 * nn * i;
+        w.mats.push_back(GramPinv{f.pm->constraint, f.d_off, f.d_ent, f.d_pairs, w.d_comp[i].as<int32_t>(),
+                                  w.d_shift[i].as<double>(), {buf, buf + nn}, f.d_Gp, nullptr, w.d_status.as<int32_t>()});
+    }
+    upload(s, w.d_mats, w.mats);
+    launch_gram_pinv(s, w.d_mats.as<GramPinv>(), uint32_t(w.mats.size()), N);
+    LEAP_HIP(hipMemcpyAsync(&w.status, w.d_status.ptr, sizeof(int32_t), hipMemcpyDeviceToHost, s));
 }
 
 leap_metadata* create_metadata(leap_ctx* ctx, const leap_ms_view& ms, int32_t ref_ant, double thr, int use_cache) {
@@ -650,31 +650,27 @@ leap_metadata* create_metadata(leap_ctx* ctx, const leap_ms_view& ms, int32_t re
     md->d_Gp.reserve(size_t(N) * N * sizeof(double) * 2);
     double* gp = md->d_Gp.as<double>();
     double* g1p = gp + size_t(N) * N;
-    gram_pinv_device(ctx, md->A1, md->d_pairs1.as<int2>(), d_off1.as<int32_t>(), d_ent1.as<int32_t>(), g1p);
-    if (use_cache) {
-        const uint64_t key = hash_phase_matrix(md->A);
-        auto it = ctx->gram_cache.find(key);
-        if (it == ctx->gram_cache.end()) {
-            gram_pinv_device(ctx, md->A, md->d_pairs.as<int2>(), md->d_csr_off.as<int32_t>(),
-                             md->d_csr_ent.as<int32_t>(), gp);
-            std::vector<double> host(size_t(N) * N);
-            LEAP_HIP(hipMemcpyAsync(host.data(), gp, host.size() * sizeof(double), hipMemcpyDeviceToHost, s));
-            LEAP_HIP(hipStreamSynchronize(s));
-            ctx->gram_cache.emplace(key, std::move(host));
-        } else {
-            LEAP_HIP(hipMemcpyAsync(gp, it->second.data(), it->second.size() * sizeof(double), hipMemcpyHostToDevice,
-                                    s));
-        }
-    } else {
-        gram_pinv_device(ctx, md->A, md->d_pairs.as<int2>(), md->d_csr_off.as<int32_t>(), md->d_csr_ent.as<int32_t>(),
-                         gp);
-    }
+    std::vector<GramSource> from{{&md->A1, md->d_pairs1.as<int2>(), d_off1.as<int32_t>(), d_ent1.as<int32_t>(), g1p}};
+    const uint64_t key = use_cache ? hash_phase_matrix(md->A) : 0;
+    const auto cached = use_cache ? ctx->gram_cache.find(key) : ctx->gram_cache.end();
+    if (cached == ctx->gram_cache.end())
+        from.push_back({&md->A, md->d_pairs.as<int2>(), md->d_csr_off.as<int32_t>(), md->d_csr_ent.as<int32_t>(), gp});
+    else
+        LEAP_HIP(hipMemcpyAsync(gp, cached->second.data(), cached->second.size() * sizeof(double),
+                                hipMemcpyHostToDevice, s));
+    GramWork work;
+    gram_pinv_device(ctx, from, N, work);
+    std::vector<double> keep(use_cache && from.size() > 1 ? size_t(N) * N : 0);
+    if (!keep.empty())
+        LEAP_HIP(hipMemcpyAsync(keep.data(), gp, keep.size() * sizeof(double), hipMemcpyDeviceToHost, s));
     md->d_AdT.reserve(size_t(K) * N * sizeof(double));
     md->d_Ad1T.reserve(size_t(K1) * N * sizeof(double));
     launch_assemble_ad(s, gp, N, md->d_pairs.as<int2>(), K - 1, md->A.constraint, md->d_AdT.as<double>());
     launch_assemble_ad(s, g1p, N, md->d_pairs1.as<int2>(), K1 - 1, md->A1.constraint, md->d_Ad1T.as<double>());
     LEAP_HIP(hipStreamSynchronize(s));  // the host vectors above end with this function
     md->d_AdT_planes.reserve(bf16_planes_bytes(uint32_t(N), K));
+    require(work.status == 0, LEAP_ERR_INTERNAL, "phase matrix Gram block is not positive definite");
+    if (!keep.empty()) ctx->gram_cache.emplace(key, std::move(keep));
     launch_split_b(s, md->d_AdT.as<double>(), K, N, md->d_AdT_planes.ptr);
     std::vector<double> tables32, tables64, tables16;
     if (nufft_supported(md->channels)) {

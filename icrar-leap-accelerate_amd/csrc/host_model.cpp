@@ -158,7 +158,9 @@ struct UnionFind {
 // formed exactly.  Its null space is spanned by the indicator vectors of the
 // connected components of the baseline graph that do not contain c (an unused
 // antenna is a component of its own with a zero column).  So, per component S:
-//   c in S:       G_SS is positive definite       ->  G+_SS = G_SS^-1
+//   c in S:       G_SS 1 = e_c                    ->  G+_SS = J + X, X the inverse of L_SS without row
+//                                                     and column c (zero there); G_SS itself is worse
+//                                                     conditioned by a factor of |S|
 //   c not in S:   G_SS = L_S with null vector 1   ->  G+_SS = (L_S + J/|S|)^-1 - J/|S|
 //   isolated:     G_SS = 0                        ->  G+_SS = 0
 // and G+ is zero between components.  Then pinv(A) = G+ A^T.  This is the
@@ -182,51 +184,43 @@ std::vector<double> gram_pinv(const PhaseMatrix& pm) {
         ++degree[b];
         uf.unite(a, b);
     }
-    g(pm.constraint, pm.constraint) += 1.0;
     std::vector<double> Gp(size_t(N) * N, 0.0);
     std::vector<std::vector<int32_t>> comps(static_cast<size_t>(N));
     for (int32_t a = 0; a < N; ++a) comps[uf.find(a)].push_back(a);
     for (const auto& S : comps) {
-        const int32_t n = int32_t(S.size());
-        if (n == 0) continue;
+        if (S.empty()) continue;
         const bool has_c = std::find(S.begin(), S.end(), pm.constraint) != S.end();
-        if (n == 1 && !has_c && degree[S[0]] == 0) continue;  // unused antenna
+        if (S.size() == 1 && !has_c && degree[S[0]] == 0) continue;  // unused antenna
+        std::vector<int32_t> R(S);  // the block to invert
+        if (has_c) R.erase(std::find(R.begin(), R.end(), pm.constraint));
+        const int32_t n = int32_t(R.size());
+        const double shift = has_c ? 0.0 : 1.0 / double(n);
         std::vector<double> M(size_t(n) * n);
         for (int32_t j = 0; j < n; ++j)
-            for (int32_t i = 0; i < n; ++i) M[size_t(j) * n + i] = g(S[i], S[j]);
-        const double inv_n = 1.0 / double(n);
-        if (!has_c)
-            for (auto& x : M) x += inv_n;
+            for (int32_t i = 0; i < n; ++i) M[size_t(j) * n + i] = g(R[i], R[j]) + shift;
         spd_inverse(M, n);
-        if (!has_c)
-            for (auto& x : M) x -= inv_n;
+        if (has_c)
+            for (int32_t j : S)
+                for (int32_t i : S) Gp[size_t(j) * N + i] = 1.0;
         for (int32_t j = 0; j < n; ++j)
-            for (int32_t i = 0; i < n; ++i) Gp[size_t(S[j]) * N + S[i]] = M[size_t(j) * n + i];
+            for (int32_t i = 0; i < n; ++i) Gp[size_t(R[j]) * N + R[i]] += M[size_t(j) * n + i] - shift;
     }
     return Gp;
 }
 
 GramComponents gram_components(const PhaseMatrix& pm) {
-    const int32_t N = pm.cols;
-    UnionFind uf(N);
-    std::vector<int32_t> degree(static_cast<size_t>(N), 0);
-    for (size_t k = 0; k < pm.ant1.size(); ++k) {
-        uf.unite(pm.ant1[k], pm.ant2[k]);
-        ++degree[pm.ant1[k]];
-        ++degree[pm.ant2[k]];
-    }
-    std::vector<std::vector<int32_t>> comps(static_cast<size_t>(N));
-    for (int32_t a = 0; a < N; ++a) comps[uf.find(a)].push_back(a);
+    const size_t N = size_t(pm.cols);
+    UnionFind uf(pm.cols);
+    for (size_t k = 0; k < pm.ant1.size(); ++k) uf.unite(pm.ant1[k], pm.ant2[k]);
     GramComponents out;
-    out.off.push_back(0);
-    for (const auto& S : comps) {
-        if (S.empty()) continue;
-        const bool has_c = std::find(S.begin(), S.end(), pm.constraint) != S.end();
-        if (S.size() == 1 && !has_c && degree[S[0]] == 0) continue;  // unused antenna: G+ = 0
-        out.members.insert(out.members.end(), S.begin(), S.end());
-        out.off.push_back(int32_t(out.members.size()));
-        out.has_c.push_back(has_c ? 1 : 0);
-    }
+    out.comp.resize(N);
+    out.shift.resize(N);
+    std::vector<int32_t> size(N, 0);
+    for (size_t a = 0; a < N; ++a) ++size[size_t(out.comp[a] = uf.find(int32_t(a)))];
+    // a reference antenna past the last antenna with baselines has no column (none holds it)
+    const int32_t with_c = pm.constraint < pm.cols ? out.comp[size_t(pm.constraint)] : -1;
+    for (size_t a = 0; a < N; ++a)
+        out.shift[a] = out.comp[a] == with_c ? 0.0 : 1.0 / double(size[size_t(out.comp[a])]);
     return out;
 }
 
@@ -240,7 +234,7 @@ int32_t null_components(const PhaseMatrix& pm) {
     const int32_t N = pm.cols;
     UnionFind uf(N);
     for (size_t k = 0; k < pm.ant1.size(); ++k) uf.unite(pm.ant1[k], pm.ant2[k]);
-    const int32_t c = uf.find(pm.constraint);
+    const int32_t c = pm.constraint < N ? uf.find(pm.constraint) : -1;
     int32_t k = 0;
     for (int32_t a = 0; a < N; ++a)
         if (uf.find(a) == a && a != c) ++k;

@@ -386,26 +386,23 @@ void launch_rotate_f64(hipStream_t s, const void* vis, int32_t vis_dtype, const 
                        uint32_t P, const double* lambda, double* avg);
 // G+ = pinv(A^T A) on the device (kernels_f64.hip); all pointers device memory.
 struct GramPinv {
-    int32_t N, constraint;
-    const int32_t* csr_off;   // N + 1: antenna a's rows of A
-    const int32_t* csr_ent;   // 2 k + (a is antenna2 of row k)
-    const int2* pairs;        // antenna pairs of A's rows
-    int32_t n_components;     // components to invert (unused antennas left out)
-    const int32_t* comp_off;  // n_components + 1 offsets into members
-    const int32_t* members;   // antennas of each component, ascending
-    const uint8_t* has_c;     // 1 where the component holds the constraint antenna
-    const int64_t* ws_off;    // offset (doubles) of each component's 2 n^2 workspace
-    double* ws;
-    double* G;                // N x N scratch (the Gram matrix)
-    double* Gp;               // N x N output
-    int32_t* status;          // set to 1 when a block is not positive definite
+    int32_t constraint;
+    const int32_t* csr_off;  // N + 1: antenna a's rows of A
+    const int32_t* csr_ent;  // 2 k + (a is antenna2 of row k)
+    const int2* pairs;       // antenna pairs of A's rows
+    const int32_t* comp;     // N: component of each antenna
+    const double* shift;     // N: 1 / |S| of the antenna's component S, 0 where it holds the constraint
+    double* buf[2];          // N x N scratch each
+    double* Gp;              // N x N output
+    double* Gx;              // N x N output without the ones of the constraint's component, or null
+    int32_t* status;         // set to 1 when a pivot is not positive
 };
-void launch_gram_pinv(hipStream_t s, const GramPinv& g);
-// Components of the baseline graph of A (plus the constraint) whose block of G+
-// is computed: every component but unused antennas (union-find, host).
+// The matrices d_mats[0 .. n_mats) (device memory), all N x N.
+void launch_gram_pinv(hipStream_t s, const GramPinv* d_mats, uint32_t n_mats, int32_t N);
+// Components of the baseline graph of A (union-find, host), as GramPinv takes them.
 struct GramComponents {
-    std::vector<int32_t> off, members;
-    std::vector<uint8_t> has_c;
+    std::vector<int32_t> comp;
+    std::vector<double> shift;
 };
 GramComponents gram_components(const PhaseMatrix& pm);
 void launch_assemble_ad(hipStream_t s, const double* Gp, int32_t N, const int2* pairs,

@@ -1,0 +1,50 @@
+"""The device pseudo-inverse (block sweeps of 32 antennas) around its tile edges.
+
+Against the host routine leap_phase_matrix_pinv, an unblocked Cholesky of the same
+exact integer matrix.  Both invert a diagonally dominant matrix and add the exact ones
+of the constraint's component, with N rounded steps per entry each: the tolerance is
+16 N eps of the largest entry.
+"""
+import numpy as np
+import pytest
+
+pytestmark = pytest.mark.gpu
+
+
+def _ms(a1, a2, fg):
+    nbl, n_ant = len(a1), int(max(a1.max(), a2.max())) + 1
+    return {"num_stations": n_ant, "total_antennas": n_ant, "num_baselines": nbl, "num_rows": nbl, "num_channels": 1,
+            "num_pols": 1, "freq_start_hz": 1e8, "freq_inc_hz": 1e6, "phase_centre": (0.1, -0.5), "antenna1": a1,
+            "antenna2": a2, "time": np.zeros(nbl), "flag": fg, "uvw": np.zeros((nbl, 3)),
+            "vis": np.zeros((nbl, 1, 1), dtype=np.complex128)}
+
+
+@pytest.mark.parametrize("graph", ["dense", "chain", "split"])
+@pytest.mark.parametrize("n_ant", [2, 31, 32, 33, 64, 65, 130])
+def test_pseudo_inverse_at_tile_edges(leap, ctx, n_ant, graph):
+    """dense: 3% flagged; chain: only neighbours, repeated twice (the longest paths and twice the
+    counts); split: two halves, one without the constraint, and one antenna without baselines."""
+    from test_capi import _host_phase_matrix
+
+    a1, a2 = (x.astype(np.int32) for x in np.triu_indices(n_ant))
+    rng = np.random.default_rng(n_ant)
+    fg = np.zeros(len(a1), dtype=np.uint8)
+    if graph == "dense":
+        fg[n_ant:] = rng.random(len(a1) - n_ant) < 0.03
+    elif graph == "chain":
+        fg[:] = a2 - a1 != 1
+        fg[0] = 0
+        a1, a2, fg = np.tile(a1, 2), np.tile(a2, 2), np.tile(fg, 2)
+    else:
+        half = n_ant // 2
+        fg[:] = ((a1 < half) != (a2 < half)) | ((a2 == n_ant - 1) & (n_ant > 2))
+        fg[0] = 0
+    print(f"pseudo-inverse: {n_ant} antennas, {graph}", flush=True)
+    got = ctx.metadata(leap.view_from_arrays(_ms(a1, a2, fg)), ref_ant=0).copy()
+    for name, ref in (("", None), ("1", 0)):
+        A, _, want = _host_phase_matrix(leap, a1, a2, fg, ref)
+        assert np.array_equal(got["A" + name], A)
+        scale = max(1.0, np.abs(want).max())
+        err = np.abs(got["Ad" + name] - want).max() / scale
+        print(f"Ad{name}: {err:.2e}")
+        assert err <= 16 * n_ant * np.finfo(float).eps
