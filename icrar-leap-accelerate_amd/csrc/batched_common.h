@@ -12,6 +12,13 @@
 namespace leap {
 namespace dev {
 
+// Orders a wave's LDS writes before its later reads (no workgroup barrier).
+__device__ inline void wave_fence() {
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+}
+
 template <typename T>
 struct C2 {
     T x, y;

@@ -442,12 +442,13 @@ int32_t batched_tile(leap_ctx* ctx, const leap_metadata& md, const leap_ms_view&
 // avgData of D directions for T timesteps starting at the staged rows, into
 // ctx->d_avg; returns the pols it holds per (direction, baseline).  With
 // pol0_only (calibrations: only pol 0 reaches cal, CpuLeapCalibrator.cc:161,171)
-// the NUFFT route writes pol 0 alone, a quarter of the bytes for 4 pols.
+// the NUFFT and per-direction routes write pol 0 alone, a quarter of the bytes for 4 pols.
 uint32_t rotate_directions(leap_ctx* ctx, const leap_metadata& md, const leap_ms_view& ms, const DeviceRows& rows,
                            uint32_t T, uint32_t D, const leap_options& opts, int32_t tile = 0,
                            bool pol0_only = false) {
     const bool nufft_route = opts.strategy == LEAP_STRATEGY_BATCHED && is_nufft(opts.channel_sum);
-    const uint32_t avg_pols = pol0_only && nufft_route ? 1u : md.pols;
+    const bool narrow = nufft_route || opts.strategy == LEAP_STRATEGY_PER_DIRECTION;
+    const uint32_t avg_pols = pol0_only && narrow ? 1u : md.pols;
     const size_t per_dir = size_t(md.nbl) * md.pols * 2;  // room for the full layout (autotune probes)
     ctx->d_avg.reserve(per_dir * D * sizeof(double));
     if (opts.strategy == LEAP_STRATEGY_BATCHED && packed_route(opts, tile)) {
@@ -478,13 +479,11 @@ uint32_t rotate_directions(leap_ctx* ctx, const leap_metadata& md, const leap_ms
         record_rotate_end(ctx);
         return avg_pols;
     }
-    for (uint32_t d = 0; d < D; ++d) {
-        record_rotate_begin(ctx);
-        launch_rotate_f64(ctx->stream, rows.vis, ms.vis_dtype, rows.uvw, ctx->d_dd.as<double>() + 9 * d, 0, T,
-                          md.nbl, md.channels, md.pols, md.d_lambda.as<double>(),
-                          ctx->d_avg.as<double>() + per_dir * d);
-        record_rotate_end(ctx);
-    }
+    record_rotate_begin(ctx);
+    launch_rotate_f64(ctx->stream, {rows.vis, ms.vis_dtype, rows.uvw, ctx->d_dd.as<double>(), D, T, 1, md.nbl,
+                                    md.channels, md.pols, avg_pols, md.d_lambda.as<double2>(),
+                                    ctx->d_avg.as<double>()});
+    record_rotate_end(ctx);
     return avg_pols;
 }
 
@@ -505,7 +504,7 @@ void invert_directions(leap_ctx* ctx, const leap_metadata& md, uint32_t D, const
     if (opts.strategy != LEAP_STRATEGY_BATCHED) {
         // Per-direction GEMVs, the reference's schedule (CudaLeapCalibrator.cu:256-259).
         ctx->d_partial.reserve(inversion_partial_doubles(K, N, D) * sizeof(double));
-        launch_inversion_f64(ctx->stream, md, avg, D, ctx->d_phase.as<double>(),
+        launch_inversion_f64(ctx->stream, md, avg, avg_pols, D, ctx->d_phase.as<double>(),
                              ctx->d_cal1.as<double>(), ctx->d_delta.as<double>(), ctx->d_partial.as<double>(),
                              cal);
         return;
@@ -631,9 +630,11 @@ leap_metadata* create_metadata(leap_ctx* ctx, const leap_ms_view& ms, int32_t re
     std::vector<int32_t> off, ent, off1, ent1;
     phase_matrix_csr(md->A, off, ent);
     phase_matrix_csr(md->A1, off1, ent1);
-    std::vector<double> lambda(md->channels);
-    for (uint32_t c = 0; c < md->channels; ++c)
-        lambda[c] = kSpeedOfLight / (md->freq_start_hz + int32_t(c) * md->freq_inc_hz);  // MetaData.h:95-98
+    std::vector<double2> lambda(md->channels);
+    for (uint32_t c = 0; c < md->channels; ++c) {
+        const double l = kSpeedOfLight / (md->freq_start_hz + int32_t(c) * md->freq_inc_hz);  // MetaData.h:95-98
+        lambda[c] = make_double2(l, 1.0 / l);
+    }
     hipStream_t s = ctx->stream;
     upload(s, md->d_pairs, pairs);
     upload(s, md->d_pairs1, pairs1);
@@ -668,9 +669,9 @@ leap_metadata* create_metadata(leap_ctx* ctx, const leap_ms_view& ms, int32_t re
     launch_assemble_ad(s, gp, N, md->d_pairs.as<int2>(), K - 1, md->A.constraint, md->d_AdT.as<double>());
     launch_assemble_ad(s, g1p, N, md->d_pairs1.as<int2>(), K1 - 1, md->A1.constraint, md->d_Ad1T.as<double>());
     LEAP_HIP(hipStreamSynchronize(s));  // the host vectors above end with this function
-    md->d_AdT_planes.reserve(bf16_planes_bytes(uint32_t(N), K));
     require(work.status == 0, LEAP_ERR_INTERNAL, "phase matrix Gram block is not positive definite");
     if (!keep.empty()) ctx->gram_cache.emplace(key, std::move(keep));
+    md->d_AdT_planes.reserve(bf16_planes_bytes(uint32_t(N), K));
     launch_split_b(s, md->d_AdT.as<double>(), K, N, md->d_AdT_planes.ptr);
     std::vector<double> tables32, tables64, tables16;
     if (nufft_supported(md->channels)) {

@@ -10,21 +10,16 @@
 // c64); uvw [row][3] f64; avgData [direction][baseline][pol] complex128;
 // Ad stored transposed as AdT [K][N] (row k = column k of Ad) so the GEMV
 // reads whole rows; cal [direction][N].
+#include "batched_common.h"
 #include "inversion_common.h"
 #include "leap_internal.h"
+
+#include <type_traits>
 
 namespace leap {
 namespace {
 
 constexpr int kBlock = 256;       // 4 wave64 per workgroup
-constexpr int kWaves = kBlock / 64;
-constexpr uint32_t kTChunk = 512;  // timesteps whose phase factors sit in LDS at once
-
-__device__ inline double wave_sum(double v) {
-    for (int off = 32; off > 0; off >>= 1) v += __shfl_xor(v, off, 64);
-    return v;
-}
-
 // ---------------------------------------------------------------------------
 // dd matrices, one thread per direction; dd row-major [d][3][3].
 // ---------------------------------------------------------------------------
@@ -53,108 +48,288 @@ __global__ void dd_kernel(double ra0, double dec0, const double* __restrict__ di
 }
 
 // ---------------------------------------------------------------------------
-// rotate_average_f64: one workgroup per baseline.  It streams the baseline's
-// T_interval rows (C x P complex each, contiguous) once, rotates every
-// (row, channel) by exp(i * shift) with shift = sf(row) / lambda(channel),
-// skips a (row, channel) whose rotated polarisations hold a NaN, and sums the
-// rest in registers; a wave64 butterfly plus an LDS step then reduce the
-// workgroup to avgData[baseline][pol].  No atomics and no write-back to the
-// cube.  The sum order is fixed, so results are reproducible bit for bit.
+// rotate_average_f64: every (row, channel) sample of a baseline rotated by
+// exp(i * shift), shift = sf(row) / lambda(channel), for up to ND directions at once
+// and summed per direction; a sample whose rotated polarisations hold a NaN is skipped.
+// No atomics and no write-back to the cube; the sum order depends on the set's shape
+// alone, so a direction's result has the same bits whatever ND and the number of pols
+// kept (PO: 1 for calibrations, which use pol 0 only; P otherwise).
+//
+// One pass serves ND directions because the cube is what a single direction waits for
+// (5.9 TB/s on complex64, 6.0 to 6.2 on complex128, 4.2 ms for 26 GB), while a direction's
+// own work is some 34 instructions per sample.  256 stations, 32 t, 384 ch, 4 pols: 4
+// directions of the complex64 cube (13 GB) take 2.41 ms in one pass against 8.87 in four,
+// 2 of the complex128 cube 4.36 against 8.34; 16 directions of 128 stations, 14 t, 48 ch
+// (355 MB) 0.20 ms in two passes against 1.10 in sixteen, bound by the arithmetic.
+// A wave owns its samples of one baseline and holds ND sums per pol in registers:
+//  - shift is the correctly rounded quotient: q = sf * r, r = RN(1 / lambda), then
+//    fma(fma(-q, lambda, sf), r, q) (Markstein 1990), 3 instructions against a division's 11
+//  - exp(i shift) by reduction modulo pi / 32 with a two-part constant through FMAs,
+//    a 64-entry table in LDS and the series to r^8 (cos) and r^7 (sin) on |r| <= pi / 64,
+//    whose next terms are below 2.5e-20 and 4.6e-18: 18 instructions
+//  - the rotated sample goes into the sums as four FMAs
+// Samples that are not finite and shifts that are not below kMaxShift take the plain form
+// (division, sincos, rotate every pol, look for a NaN), exactly as the reference does it.
 // ---------------------------------------------------------------------------
-template <typename T, int P>
-struct VisLoad;
+constexpr int kPhasorTable = 64;
+constexpr double kMaxShift = 67108864.0;    // 2^26 rad: 32 / pi times it stays below 2^31
+constexpr uint32_t kRowChunk = 32;          // rows whose shift factors a wave keeps in LDS
+constexpr uint32_t kLambdaLds = 1024;       // channels whose wavelengths sit in LDS
 
-template <int P>
-struct VisLoad<double, P> {
-    double v[2 * P];
-    __device__ inline void load(const double* __restrict__ p) {
+template <typename T, int P>
+struct VisLoad {
+    T v[2 * P];
+    VisLoad() = default;
+    __device__ inline explicit VisLoad(const T* __restrict__ p) { load(p); }
+    __device__ inline void load(const T* __restrict__ p) {
+        typedef T T2 __attribute__((ext_vector_type(2)));
 #pragma unroll
         for (int q = 0; q < P; ++q) {
-            const double2 x = reinterpret_cast<const double2*>(p)[q];
+            const T2 x = reinterpret_cast<const T2*>(p)[q];
             v[2 * q] = x.x;
             v[2 * q + 1] = x.y;
         }
     }
-};
-
-template <int P>
-struct VisLoad<float, P> {
-    double v[2 * P];
-    __device__ inline void load(const float* __restrict__ p) {
+    // 0 * x is NaN exactly for infinities and NaNs.
+    __device__ inline bool finite() const {
+        T z = T(0);
 #pragma unroll
-        for (int q = 0; q < P; ++q) {
-            const float2 x = reinterpret_cast<const float2*>(p)[q];
-            v[2 * q] = double(x.x);  // the reference widens complex<float> (ms/utils.h:141-142)
-            v[2 * q + 1] = double(x.y);
-        }
+        for (int q = 0; q < 2 * P; ++q) z = fma(T(0), v[q], z);
+        return z == T(0);
     }
 };
 
-template <typename T, int P>
-__global__ __launch_bounds__(kBlock) void rotate_average_f64(
-    const T* __restrict__ vis, const double* __restrict__ uvw, const double* __restrict__ dd,
-    uint32_t row_start, uint32_t T_steps, uint32_t nbl, uint32_t C,
-    const double* __restrict__ lambda, double* __restrict__ avg) {
+// exp(i th) for |th| <= kMaxShift.
+__device__ inline double2 phasor_table(const double2* __restrict__ table, double th) {
 #pragma clang fp contract(off)
-    __shared__ double s_sf[kTChunk];
-    __shared__ double s_red[kWaves][2 * P];
-    const uint32_t bl = blockIdx.x;
-    const double dz0 = dd[6], dz1 = dd[7], dz2 = dd[8];
-    double acc[2 * P];
-#pragma unroll
-    for (int q = 0; q < 2 * P; ++q) acc[q] = 0.0;
+    constexpr double kStep = 10.185916357881301489;         // 32 / pi
+    constexpr double kPiO32Hi = 0.098174770424681034875;    // double(pi / 32)
+    constexpr double kPiO32Lo = 3.8270212473354786e-18;     // pi / 32 - double(pi / 32)
+    const double k = rint(th * kStep);
+    const double2 t = table[int32_t(k) & (kPhasorTable - 1)];
+    double r = fma(-k, kPiO32Hi, th);
+    r = fma(-k, kPiO32Lo, r);
+    const double r2 = r * r;
+    double s = fma(-1.0 / 5040.0, r2, 1.0 / 120.0);
+    s = fma(s, r2, -1.0 / 6.0);
+    s = fma(r * r2, s, r);  // sin r
+    double c = fma(1.0 / 40320.0, r2, -1.0 / 720.0);
+    c = fma(c, r2, 1.0 / 24.0);
+    c = fma(c, r2, -0.5) * r2;  // cos r - 1
+    return make_double2(fma(-t.y, s, fma(t.x, c, t.x)), fma(t.x, s, fma(t.y, c, t.y)));
+}
 
-    for (uint32_t t0 = 0; t0 < T_steps; t0 += kTChunk) {
-        const uint32_t tn = min(kTChunk, T_steps - t0);
-        __syncthreads();
-        for (uint32_t t = threadIdx.x; t < tn; t += kBlock) {
-            const size_t row = size_t(row_start) + size_t(t0 + t) * nbl + bl;
-            const double u = uvw[3 * row], v = uvw[3 * row + 1], w = uvw[3 * row + 2];
-            const double wrot = dz0 * u + dz1 * v + dz2 * w;  // (dd * uvw).z, MetaData.cc:227
-            s_sf[t] = -kTwoPi * (wrot - w);                     // CpuLeapCalibrator.cc:190
-        }
-        __syncthreads();
-        // Pair (t, c) of this chunk handled by this thread: i = threadIdx.x + k * kBlock.
-        uint32_t t = 0, c = threadIdx.x;
-        while (c >= C) { c -= C; ++t; }
-        for (; t < tn;) {
-            const size_t row = size_t(row_start) + size_t(t0 + t) * nbl + bl;
-            VisLoad<T, P> x;
-            x.load(vis + (row * C + c) * (2 * P));
-            const double shift = s_sf[t] / lambda[c];  // CpuLeapCalibrator.cc:195
-            double sn, cs;
-            sincos(shift, &sn, &cs);
-            double r[2 * P];
-            bool nan = false;
+// Sums of N values over a wave: every step halves the values a lane holds while there is
+// more than one, so N + 4 exchanges do instead of 6 N.  The lane's value is number
+// wave_sum_index<N>(lane); each is summed over the lanes in the same tree whatever N.
+template <int N>
+__device__ inline double wave_sum_n(double* v, uint32_t lane) {
+    int n = N;
 #pragma unroll
-            for (int q = 0; q < P; ++q) {
-                const double a = x.v[2 * q], b = x.v[2 * q + 1];
-                r[2 * q] = a * cs - b * sn;  // (a + ib)(cs + i sn), :198
-                r[2 * q + 1] = a * sn + b * cs;
-                nan |= __builtin_isnan(r[2 * q]) || __builtin_isnan(r[2 * q + 1]);  // :201-206
-            }
-            if (!nan) {
+    for (int m = 32; m > 0; m >>= 1) {
+        if (n > 1) {
+            n /= 2;
+            const bool up = lane & m;
 #pragma unroll
-                for (int q = 0; q < 2 * P; ++q) acc[q] += r[q];  // :208-214
+            for (int j = 0; j < n; ++j) {
+                const double send = up ? v[j] : v[j + n], keep = up ? v[j + n] : v[j];
+                v[j] = keep + __shfl_xor(send, m, 64);
             }
-            c += kBlock;
-            while (c >= C) { c -= C; ++t; }
+        } else {
+            v[0] += __shfl_xor(v[0], m, 64);
         }
     }
-    // Workgroup reduction: wave butterfly, then the kWaves partials in order.
-    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-#pragma unroll
-    for (int q = 0; q < 2 * P; ++q) {
-        const double s = wave_sum(acc[q]);
-        if (lane == 0) s_red[wave][q] = s;
+    return v[0];
+}
+
+template <int N>
+__device__ inline uint32_t wave_sum_index(uint32_t lane) {
+    return lane / (64 / N);  // the upper half of the values goes to the lanes with bit 32, and so on
+}
+
+constexpr int pow2_at_least(int n) {
+    int p = 1;
+    while (p < n) p *= 2;
+    return p;
+}
+
+// Grid: (groups of directions fastest, baselines) x solution intervals; waves of a baseline:
+// wpb (1: the workgroup's waves take one baseline each).  lambda2: (lambda, RN(1 / lambda)).
+// avg[interval][direction][baseline][PO].
+template <typename T, int P, int PO, int ND, bool kWide>
+__global__ __launch_bounds__(kWide ? 256 : 1024) void rotate_average_f64(
+    const T* __restrict__ vis, const double* __restrict__ uvw, const double* __restrict__ dd, uint32_t D,
+    uint32_t groups, uint32_t wpb, uint32_t T_steps, uint32_t nbl, uint32_t C,
+    const double2* __restrict__ lambda2, double* __restrict__ avg) {
+#pragma clang fp contract(off)
+    constexpr int NV = pow2_at_least(2 * PO * ND);
+    __shared__ double2 s_lambda[kLambdaLds];
+    __shared__ double2 s_table[kPhasorTable];
+    // kWide, for 64-byte samples (4 complex128 pols) of which pol 0 is kept: a lane loading its own
+    // sample strides the wave's four loads by 64 bytes and leaves the reuse of their lines to the
+    // L1, which the waves in flight overflow.  So the wave loads its 64 samples as 256 consecutive
+    // 16-byte units, a pol a lane, and hands the pol-0 units over through LDS.
+    static_assert(!kWide || (PO == 1 && P * sizeof(T) == 32), "wide loads: four 16-byte pols, pol 0 kept");
+    __shared__ double2 s_pol0[kWide ? 4 * 64 : 1];
+    extern __shared__ double s_dyn[];  // shift factors [wave][row][ND], then partial sums [wave][NV]
+    const uint32_t lane = threadIdx.x & 63, wave = threadIdx.x >> 6, waves = blockDim.x >> 6;
+    double* s_sf = s_dyn + size_t(wave) * (kRowChunk * ND);
+    double* s_red = s_dyn + size_t(waves) * (kRowChunk * ND);
+    const bool in_lds = C <= kLambdaLds;
+    if (in_lds)
+        for (uint32_t c = threadIdx.x; c < C; c += blockDim.x) s_lambda[c] = lambda2[c];
+    for (uint32_t k = threadIdx.x; k < kPhasorTable; k += blockDim.x) {
+        double sn, cs;
+        sincospi(double(k) / 32.0, &sn, &cs);
+        s_table[k] = make_double2(cs, sn);
     }
     __syncthreads();
-    if (threadIdx.x < 2 * P) {
-        double s = 0.0;
+    const uint32_t group = blockIdx.x % groups, block = blockIdx.x / groups;
+    const uint32_t per_group = (D + groups - 1) / groups;
+    const uint32_t d0 = group * per_group;
+    const uint32_t active = min(per_group, D - d0);  // the host leaves no group empty
+    const uint32_t bl = wpb == 1 ? block * waves + wave : block;
+    const uint32_t part = wpb == 1 ? 0 : wave;  // this wave's share of the baseline's samples
+    const size_t rows0 = size_t(blockIdx.y) * T_steps * nbl;
+    double acc[NV];
 #pragma unroll
-        for (int w = 0; w < kWaves; ++w) s += s_red[w][threadIdx.x];
-        avg[size_t(bl) * (2 * P) + threadIdx.x] = s;
+    for (int q = 0; q < NV; ++q) acc[q] = 0.0;
+
+    if (bl < nbl) {
+        const uint32_t step_t = 64 * wpb / C, step_c = 64 * wpb % C;
+        for (uint32_t t0 = 0; t0 < T_steps; t0 += kRowChunk) {
+            const uint32_t tn = min(kRowChunk, T_steps - t0);
+            dev::wave_fence();  // the previous chunk's factors have been read
+            for (uint32_t i = lane; i < tn * ND; i += 64) {
+                const uint32_t t = i / ND, d = i % ND;
+                const size_t row = rows0 + size_t(t0 + t) * nbl + bl;
+                const double* dz = dd + size_t(min(d0 + d, D - 1)) * 9 + 6;
+                const double u = uvw[3 * row], v = uvw[3 * row + 1], w = uvw[3 * row + 2];
+                const double wrot = dz[0] * u + dz[1] * v + dz[2] * w;  // (dd * uvw).z, MetaData.cc:227
+                s_sf[i] = -kTwoPi * (wrot - w);                        // CpuLeapCalibrator.cc:190
+            }
+            dev::wave_fence();
+            // samples lane + 64 * (part + k * wpb) of the chunk, in (row, channel) order
+            const size_t at0 = rows0 + size_t(t0) * nbl + bl;
+            auto at = [&](uint32_t t, uint32_t c) { return vis + ((at0 + size_t(t) * nbl) * C + c) * (2 * P); };
+            auto advance = [&](uint32_t& t, uint32_t& c) {
+                t += step_t;
+                c += step_c;
+                if (c >= C) {
+                    c -= C;
+                    ++t;
+                }
+            };
+            uint32_t t = (64 * part + lane) / C, c = (64 * part + lane) % C;
+            VisLoad<T, P> next;                                  // !kWide: this lane's next sample
+            uint32_t tu[kWide ? 4 : 1], cu[kWide ? 4 : 1];       // kWide: row and channel of unit 64 j + lane's sample
+            double2 unit[kWide ? 4 : 1];
+            auto load_units = [&] {
+#pragma unroll
+                for (int j = 0; j < 4; ++j) {
+                    unit[j] = make_double2(0.0, 0.0);
+                    if (tu[j] < tn) unit[j] = reinterpret_cast<const double2*>(at(tu[j], cu[j]))[lane & 3];
+                    advance(tu[j], cu[j]);
+                }
+            };
+            if constexpr (kWide) {
+#pragma unroll
+                for (int j = 0; j < 4; ++j) {
+                    tu[j] = (64 * part + 16 * j + lane / 4) / C;
+                    cu[j] = (64 * part + 16 * j + lane / 4) % C;
+                }
+                load_units();
+            } else if (t < tn) {
+                next.load(at(t, c));
+            }
+            for (uint32_t first = 64 * part; kWide ? first < tn * C : t < tn; first += 64 * wpb) {
+                double v[2 * PO];
+                VisLoad<T, P> x;
+                bool plain = true;
+                if constexpr (kWide) {
+                    bool bad = false;
+                    dev::wave_fence();  // the batch before has been read
+#pragma unroll
+                    for (int j = 0; j < 4; ++j) {
+                        bad |= fma(0.0, unit[j].x, 0.0 * unit[j].y) != 0.0;  // also where it is NaN
+                        if ((lane & 3) == 0) s_pol0[wave * 64 + 16 * j + lane / 4] = unit[j];
+                    }
+                    dev::wave_fence();
+                    const double2 p0 = s_pol0[wave * 64 + lane];
+                    load_units();
+                    const bool look = __any(bad);  // one of the wave's 64 samples is not finite
+                    if (t >= tn) break;            // the chunk's last samples need not fill the wave
+                    v[0] = p0.x;
+                    v[1] = p0.y;
+                    if (look) plain = VisLoad<T, P>(at(t, c)).finite();
+                } else {
+                    x = next;
+                    plain = x.finite();
+#pragma unroll
+                    for (int q = 0; q < 2 * PO; ++q) v[q] = double(x.v[q]);
+                }
+                const double* sf = s_sf + t * ND;
+                const double2 l = in_lds ? s_lambda[c] : lambda2[c];
+                const uint32_t ts = t, cs0 = c;
+                advance(t, c);
+                if constexpr (!kWide)
+                    if (t < tn) next.load(at(t, c));
+                double shift[ND];
+#pragma unroll
+                for (int d = 0; d < ND; ++d) {
+                    const double q = sf[d] * l.y;
+                    shift[d] = fma(fma(-q, l.x, sf[d]), l.y, q);  // sf / lambda, :195
+                    plain = plain && fabs(shift[d]) < kMaxShift;
+                }
+                if (plain) {
+#pragma unroll
+                    for (int d = 0; d < ND; ++d) {
+                        if ((d & 1) == 0 && uint32_t(d) >= active) break;
+                        const double2 e = phasor_table(s_table, shift[d]);
+#pragma unroll
+                        for (int q = 0; q < PO; ++q) {  // (a + ib)(cs + i sn), :198, :208-214
+                            double* o = acc + 2 * (d * PO + q);
+                            o[0] = fma(-v[2 * q + 1], e.y, fma(v[2 * q], e.x, o[0]));
+                            o[1] = fma(v[2 * q + 1], e.x, fma(v[2 * q], e.y, o[1]));
+                        }
+                    }
+                } else {
+                    if constexpr (kWide) x.load(at(ts, cs0));
+#pragma unroll 1
+                    for (int d = 0; d < ND; ++d) {
+                        double sn, cs, r[2 * P];
+                        sincos(sf[d] / l.x, &sn, &cs);
+                        bool nan = false;
+#pragma unroll
+                        for (int q = 0; q < P; ++q) {
+                            const double a = double(x.v[2 * q]), b = double(x.v[2 * q + 1]);
+                            r[2 * q] = a * cs - b * sn;
+                            r[2 * q + 1] = a * sn + b * cs;
+                            nan |= __builtin_isnan(r[2 * q]) || __builtin_isnan(r[2 * q + 1]);  // :201-206
+                        }
+#pragma unroll
+                        for (int k = 0; k < ND; ++k)  // sums indexed by constants stay in registers
+                            if (k == d && !nan)
+#pragma unroll
+                                for (int q = 0; q < 2 * PO; ++q) acc[2 * k * PO + q] += r[q];
+                    }
+                }
+            }
+        }
     }
+    double s = wave_sum_n<NV>(acc, lane);
+    const uint32_t v = wave_sum_index<NV>(lane);
+    const bool first = lane % (64 / NV) == 0;
+    if (wpb != 1) {  // the baseline's waves in order
+        if (first) s_red[wave * NV + v] = s;
+        __syncthreads();
+        if (wave != 0) return;
+        s = s_red[v];
+        for (uint32_t w = 1; w < waves; ++w) s += s_red[w * NV + v];
+    }
+    const uint32_t d = v / (2 * PO);
+    if (first && bl < nbl && d < active)
+        avg[((size_t(blockIdx.y) * D + d0 + d) * nbl + bl) * (2 * PO) + v % (2 * PO)] = s;
 }
 
 // ---------------------------------------------------------------------------
@@ -449,19 +624,54 @@ __global__ __launch_bounds__(kBlock) void gram_sweep_kernel(const GramPinv* __re
     }
 }
 
+template <typename T, int P, int PO, int ND>
+void launch_rotate_nd(hipStream_t s, const RotateF64& a) {
+    const uint32_t groups = (a.D + ND - 1) / ND;
+    const uint32_t waves = a.wpb == 1 ? 4 : a.wpb;
+    const uint64_t blocks = uint64_t(groups) * (a.wpb == 1 ? (a.nbl + 3) / 4 : a.nbl);
+    require(blocks < (1ull << 31) && a.intervals < 65536, LEAP_ERR_RANGE, "too many workgroups for one launch");
+    constexpr int NV = pow2_at_least(2 * PO * ND);
+    const size_t lds = size_t(waves) * (kRowChunk * ND + NV) * sizeof(double);
+    auto launch = [&](auto wide) {
+        rotate_average_f64<T, P, PO, ND, decltype(wide)::value>
+            <<<dim3(uint32_t(blocks), a.intervals), 64 * waves, lds, s>>>(static_cast<const T*>(a.vis), a.uvw, a.dd, a.D,
+                                                                         groups, a.wpb, a.T, a.nbl, a.C, a.lambda2,
+                                                                         a.avg);
+        LEAP_HIP(hipGetLastError());
+    };
+    // Wide loads up to 4 directions, where the visibilities are the bound; with 8 their registers
+    // cost half the waves (16 directions on 355 MB: 249 us against 200).
+    if constexpr (PO == 1 && P * sizeof(T) == 32 && ND <= 4) {
+        if (waves <= 4) return launch(std::true_type{});
+    }
+    launch(std::false_type{});
+}
+
+template <typename T, int P>
+void launch_rotate_pols(hipStream_t s, const RotateF64& a, uint32_t nd) {
+    if (a.pols_out == 1) {
+        switch (nd) {
+            case 1: return launch_rotate_nd<T, P, 1, 1>(s, a);
+            case 2: return launch_rotate_nd<T, P, 1, 2>(s, a);
+            case 4: return launch_rotate_nd<T, P, 1, 4>(s, a);
+            default: return launch_rotate_nd<T, P, 1, 8>(s, a);
+        }
+    }
+    if constexpr (P > 1) {
+        if (nd == 1) return launch_rotate_nd<T, P, P, 1>(s, a);
+        return launch_rotate_nd<T, P, P, 2>(s, a);
+    }
+}
+
 template <typename T>
-void launch_rotate_typed(hipStream_t s, const T* vis, const double* uvw, const double* dd,
-                         uint32_t row_start, uint32_t T_steps, uint32_t nbl, uint32_t C, uint32_t P,
-                         const double* lambda, double* avg) {
-    const dim3 grid(nbl), block(kBlock);
-    switch (P) {
-        case 1: rotate_average_f64<T, 1><<<grid, block, 0, s>>>(vis, uvw, dd, row_start, T_steps, nbl, C, lambda, avg); break;
-        case 2: rotate_average_f64<T, 2><<<grid, block, 0, s>>>(vis, uvw, dd, row_start, T_steps, nbl, C, lambda, avg); break;
-        case 3: rotate_average_f64<T, 3><<<grid, block, 0, s>>>(vis, uvw, dd, row_start, T_steps, nbl, C, lambda, avg); break;
-        case 4: rotate_average_f64<T, 4><<<grid, block, 0, s>>>(vis, uvw, dd, row_start, T_steps, nbl, C, lambda, avg); break;
+void launch_rotate_typed(hipStream_t s, const RotateF64& a, uint32_t nd) {
+    switch (a.P) {
+        case 1: return launch_rotate_pols<T, 1>(s, a, nd);
+        case 2: return launch_rotate_pols<T, 2>(s, a, nd);
+        case 3: return launch_rotate_pols<T, 3>(s, a, nd);
+        case 4: return launch_rotate_pols<T, 4>(s, a, nd);
         default: throw Error(LEAP_ERR_NOT_IMPLEMENTED, "unsupported polarisation count");
     }
-    LEAP_HIP(hipGetLastError());
 }
 
 }  // namespace
@@ -472,14 +682,22 @@ void launch_dd(hipStream_t s, double ra0, double dec0, const double* d_dirs, uin
     LEAP_HIP(hipGetLastError());
 }
 
-void launch_rotate_f64(hipStream_t s, const void* vis, int32_t vis_dtype, const double* uvw,
-                       const double* dd, uint32_t row_start, uint32_t T_steps, uint32_t nbl,
-                       uint32_t C, uint32_t P, const double* lambda, double* avg) {
-    if (nbl == 0) return;
-    if (vis_dtype == LEAP_VIS_C64)
-        launch_rotate_typed(s, static_cast<const float*>(vis), uvw, dd, row_start, T_steps, nbl, C, P, lambda, avg);
+void launch_rotate_f64(hipStream_t s, const RotateF64& in) {
+    if (in.nbl == 0 || in.D == 0 || in.intervals == 0) return;
+    RotateF64 a = in;
+    // Waves of a baseline, from the set's shape alone: one where the baselines alone are
+    // 4 waves per SIMD, four below, sixteen where even those leave most SIMDs empty and a
+    // baseline has samples for all of them.
+    a.wpb = a.nbl >= 4096 ? 1 : a.nbl < 512 && uint64_t(a.T) * a.C >= 4096 ? 16 : 4;
+    // Directions per pass: as many as D has, up to 8, but no more than leaves 4 waves per SIMD
+    // (splitting the directions over workgroups shortens each wave's chain instead).
+    const uint64_t waves = uint64_t(a.nbl) * a.wpb * a.intervals;
+    uint32_t nd = a.pols_out == 1 ? 8 : 2;
+    while (nd > 1 && (nd / 2 >= a.D || waves * ((a.D + nd - 1) / nd) < 4096)) nd /= 2;
+    if (a.vis_dtype == LEAP_VIS_C64)
+        launch_rotate_typed<float>(s, a, nd);
     else
-        launch_rotate_typed(s, static_cast<const double*>(vis), uvw, dd, row_start, T_steps, nbl, C, P, lambda, avg);
+        launch_rotate_typed<double>(s, a, nd);
 }
 
 void launch_gram_pinv(hipStream_t s, const GramPinv* d_mats, uint32_t n_mats, int32_t N) {
@@ -500,11 +718,11 @@ void launch_assemble_ad(hipStream_t s, const double* Gp, int32_t N, const int2* 
     LEAP_HIP(hipGetLastError());
 }
 
-void launch_inversion_f64(hipStream_t s, const leap_metadata& md, const double* avg, uint32_t D,
+void launch_inversion_f64(hipStream_t s, const leap_metadata& md, const double* avg, uint32_t avg_pols, uint32_t D,
                           double* phase, double* cal1, double* delta, double* partial, double* cal) {
     if (D == 0) return;
     const int32_t K = md.A.rows, N = md.A.cols, K1 = md.A1.rows;
-    const uint32_t nbl = md.nbl, P = md.pols;
+    const uint32_t nbl = md.nbl, P = avg_pols;
     phase_i1_kernel<<<dim3((K1 + 255) / 256, D), 256, 0, s>>>(avg, nbl, P, md.d_I1.as<int32_t>(), K1, phase);
     LEAP_HIP(hipGetLastError());
     cal1_kernel<<<dim3((N + 63) / 64, (D + kCal1Dirs - 1) / kCal1Dirs), 64, 0, s>>>(md.d_Ad1T.as<double>(), K1, N,

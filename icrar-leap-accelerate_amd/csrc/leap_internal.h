@@ -165,7 +165,7 @@ struct leap_metadata {
     // the inversion's adjoint: A's baseline indices I, A1's antenna pairs, and
     // each antenna's rows of A (CSR: offsets N + 1, entries 2 row + (antenna2 ? 1 : 0))
     leap::DeviceBuffer d_I, d_pairs1, d_csr_off, d_csr_ent;
-    leap::DeviceBuffer d_lambda;   // channels doubles: wavelength of each channel
+    leap::DeviceBuffer d_lambda;   // channels double2: wavelength of each channel and its reciprocal
     leap::DeviceBuffer d_Gp;       // G+ = pinv(A^T A) then G1+ = pinv(A1^T A1), N x N each
     leap::DeviceBuffer d_AdT_planes;  // split-3 x BF16 planes of AdT in MFMA operand layout
     // NUFFT plans (N == 0 when the channel count is not supported) and their
@@ -381,10 +381,20 @@ int32_t multi_blocks_per_cu(int32_t tile);
 // Kernel launchers (kernels_f64.hip)
 void launch_dd(hipStream_t s, double ra0, double dec0, const double* d_dirs, uint32_t D,
                double* d_dd);
-void launch_rotate_f64(hipStream_t s, const void* vis, int32_t vis_dtype, const double* uvw,
-                       const double* dd, uint32_t row_start, uint32_t T, uint32_t nbl, uint32_t C,
-                       uint32_t P, const double* lambda, double* avg);
-// G+ = pinv(A^T A) on the device (kernels_f64.hip); all pointers device memory.
+// The per-direction FP64 rotate/average of D directions over consecutive solution intervals
+// of T timesteps each, from the first interval's first row.
+struct RotateF64 {
+    const void* vis;
+    int32_t vis_dtype;
+    const double* uvw;
+    const double* dd;  // [D][3][3]
+    uint32_t D, T, intervals, nbl, C, P, pols_out;  // pols_out: 1 (pol 0) or P
+    const double2* lambda2;                         // C pairs (lambda, RN(1 / lambda))
+    double* avg;                                    // [intervals][D][nbl][pols_out]
+    uint32_t wpb = 0;                               // waves per baseline, chosen by the launcher
+};
+void launch_rotate_f64(hipStream_t s, const RotateF64& a);
+// G+ = pinv(A^T A) of one phase matrix (kernels_f64.hip); all pointers device memory.
 struct GramPinv {
     int32_t constraint;
     const int32_t* csr_off;  // N + 1: antenna a's rows of A
@@ -407,7 +417,7 @@ struct GramComponents {
 GramComponents gram_components(const PhaseMatrix& pm);
 void launch_assemble_ad(hipStream_t s, const double* Gp, int32_t N, const int2* pairs,
                         int32_t n_pairs, int32_t constraint, double* AdT);
-void launch_inversion_f64(hipStream_t s, const leap_metadata& md, const double* avg, uint32_t D,
+void launch_inversion_f64(hipStream_t s, const leap_metadata& md, const double* avg, uint32_t avg_pols, uint32_t D,
                           double* phase, double* cal1, double* delta, double* partial, double* cal);
 void launch_rotate_batched(hipStream_t s, int32_t precision, int32_t direction_block, bool all_pols,
                            const void* vis, int32_t vis_dtype, const double* uvw, const double* dd, uint32_t D,

@@ -127,9 +127,9 @@ extern "C" int leap_hip_calibrate_md_noalloc(leap_ctx* ctx, const leap_metadata*
             const void* vis = static_cast<const char*>(ms->vis) + row_begin * row_bytes;
             const double* uvw = ms->uvw_device + row_begin * 3;
             for (uint32_t d = 0; d < D; ++d) {
-                launch_rotate_f64(ctx->stream, vis, ms->vis_dtype, uvw, d_dd + 9 * size_t(d), 0, interval, nbl,
-                                  md->channels, md->pols, md->d_lambda.as<double>(), d_avg);
-                launch_inversion_f64(ctx->stream, *md, d_avg, 1, d_phase, d_cal1, d_delta, d_partial,
+                launch_rotate_f64(ctx->stream, {vis, ms->vis_dtype, uvw, d_dd + 9 * size_t(d), 1, interval, 1, nbl,
+                                                md->channels, md->pols, 1, md->d_lambda.as<double2>(), d_avg});
+                launch_inversion_f64(ctx->stream, *md, d_avg, 1, 1, d_phase, d_cal1, d_delta, d_partial,
                                      cal_out + (size_t(s) * D + d) * size_t(N));
             }
         }

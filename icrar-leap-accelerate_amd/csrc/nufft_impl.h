@@ -220,12 +220,7 @@ __device__ inline void idft(C2<F>* x) {
     }
 }
 
-// Orders the wave's LDS accesses across lanes (the workgroup is one wave).
-__device__ inline void wave_fence() {
-    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-    __builtin_amdgcn_wave_barrier();
-    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
-}
+using dev::wave_fence;
 
 __device__ inline uint32_t padded(uint32_t e) { return e + (e >> 4); }
 
