@@ -492,37 +492,23 @@ uint32_t rotate_directions(leap_ctx* ctx, const leap_metadata& md, const leap_ms
 void invert_directions(leap_ctx* ctx, const leap_metadata& md, uint32_t D, const leap_options& opts,
                        const double* avg = nullptr, double* cal = nullptr, uint32_t avg_pols = 0) {
     if (avg_pols == 0) avg_pols = md.pols;
-    const int32_t K = md.A.rows, N = md.A.cols, K1 = md.A1.rows;
-    ctx->d_phase.reserve(size_t(K1) * D * sizeof(double));
+    const int32_t K = md.A.rows, N = md.A.cols;
     ctx->d_cal1.reserve(size_t(N) * D * sizeof(double));
-    ctx->d_delta.reserve(size_t(K) * D * sizeof(double));
     if (cal == nullptr) {
         ctx->d_cal.reserve(size_t(N) * D * sizeof(double));
         cal = ctx->d_cal.as<double>();
     }
     if (avg == nullptr) avg = ctx->d_avg.as<double>();
-    if (opts.strategy != LEAP_STRATEGY_BATCHED) {
-        // Per-direction GEMVs, the reference's schedule (CudaLeapCalibrator.cu:256-259).
-        ctx->d_partial.reserve(inversion_partial_doubles(K, N, D) * sizeof(double));
-        launch_inversion_f64(ctx->stream, md, avg, avg_pols, D, ctx->d_phase.as<double>(),
-                             ctx->d_cal1.as<double>(), ctx->d_delta.as<double>(), ctx->d_partial.as<double>(),
-                             cal);
+    if (opts.precision != LEAP_PRECISION_MIXED) {
+        ctx->d_sums.reserve(size_t(N) * D * sizeof(double));
+        launch_inversion_f64(ctx->stream, md, avg, avg_pols, D, ctx->d_cal1.as<double>(), ctx->d_sums.as<double>(), cal);
         return;
     }
-    const bool mixed = opts.precision == LEAP_PRECISION_MIXED;
-    launch_inversion_head(ctx->stream, md, avg, avg_pols, D, ctx->d_phase.as<double>(), ctx->d_cal1.as<double>(),
-                          mixed ? nullptr : ctx->d_delta.as<double>());
-    if (mixed) {
-        ctx->d_a_planes.reserve(bf16_planes_bytes((D + 63) / 64 * 64, K));
-        ctx->d_partial.reserve(mfma_partial_floats(K, D, N) * sizeof(float));
-        const DeltaSource from{avg, md.nbl, avg_pols, md.d_pairs.as<int2>()};
-        launch_gemm_bf16x3(ctx->stream, md.d_AdT_planes.ptr, K, N, nullptr, D, ctx->d_a_planes.ptr,
-                           ctx->d_cal1.as<double>(), static_cast<float*>(ctx->d_partial.ptr), cal, &from);
-    } else {
-        ctx->d_partial.reserve(gemm_f64_partial_doubles(K, N, D) * sizeof(double));
-        launch_gemm_f64(ctx->stream, md.d_AdT.as<double>(), K, N, ctx->d_delta.as<double>(), D,
-                        ctx->d_cal1.as<double>(), ctx->d_partial.as<double>(), cal);
-    }
+    launch_cal1(ctx->stream, md, avg, avg_pols, D, ctx->d_cal1.as<double>());
+    ctx->d_a_planes.reserve(bf16_planes_bytes((D + 63) / 64 * 64, K));
+    ctx->d_partial.reserve(mfma_partial_floats(K, D, N) * sizeof(float));
+    launch_gemm_bf16x3(ctx->stream, md.d_AdT_planes.ptr, K, N, {avg, md.nbl, avg_pols, md.d_pairs.as<int2>()}, D,
+                       ctx->d_a_planes.ptr, ctx->d_cal1.as<double>(), static_cast<float*>(ctx->d_partial.ptr), cal);
 }
 
 void check_metadata_matches(const leap_metadata& md, const leap_ms_view& ms) {
@@ -570,7 +556,7 @@ struct GramSource {
     const PhaseMatrix* pm;
     const int2* d_pairs;
     const int32_t *d_off, *d_ent;  // each antenna's rows
-    double* d_Gp;                  // N x N output
+    double *d_Gp, *d_Gx;           // N x N outputs
 };
 
 // G+ = pinv(A^T A) of phase matrices of one antenna count, all in the same launches,
@@ -591,7 +577,7 @@ void gram_pinv_device(leap_ctx* ctx, const std::vector<GramSource>& from, int32_
         upload(s, w.d_shift[i], w.comps[i].shift);
         double* buf = w.d_scratch.as<double>() + 2 * nn * i;
         w.mats.push_back(GramPinv{f.pm->constraint, f.d_off, f.d_ent, f.d_pairs, w.d_comp[i].as<int32_t>(),
-                                  w.d_shift[i].as<double>(), {buf, buf + nn}, f.d_Gp, nullptr, w.d_status.as<int32_t>()});
+                                  w.d_shift[i].as<double>(), {buf, buf + nn}, f.d_Gp, f.d_Gx, w.d_status.as<int32_t>()});
     }
     upload(s, w.d_mats, w.mats);
     launch_gram_pinv(s, w.d_mats.as<GramPinv>(), uint32_t(w.mats.size()), N);
@@ -642,26 +628,28 @@ leap_metadata* create_metadata(leap_ctx* ctx, const leap_ms_view& ms, int32_t re
     upload(s, md->d_I1, md->A1.I);
     upload(s, md->d_csr_off, off);
     upload(s, md->d_csr_ent, ent);
-    DeviceBuffer d_off1, d_ent1;
-    upload(s, d_off1, off1);
-    upload(s, d_ent1, ent1);
+    upload(s, md->d_csr1_off, off1);
+    upload(s, md->d_csr1_ent, ent1);
     upload(s, md->d_lambda, lambda);
     // The pseudo-inverses (MetaData.cc:111, :123) as G+ = pinv(A^T A), Ad = G+ A^T, on the
     // device; with use_cache A's G+ is kept in the context by a hash of A (:112-120).
-    md->d_Gp.reserve(size_t(N) * N * sizeof(double) * 2);
+    const size_t nn = size_t(N) * N;
+    md->d_Gp.reserve(nn * sizeof(double) * 4);
     double* gp = md->d_Gp.as<double>();
-    double* g1p = gp + size_t(N) * N;
-    std::vector<GramSource> from{{&md->A1, md->d_pairs1.as<int2>(), d_off1.as<int32_t>(), d_ent1.as<int32_t>(), g1p}};
+    double* g1p = gp + 2 * nn;
+    std::vector<GramSource> from{{&md->A1, md->d_pairs1.as<int2>(), md->d_csr1_off.as<int32_t>(),
+                                  md->d_csr1_ent.as<int32_t>(), g1p, g1p + nn}};
     const uint64_t key = use_cache ? hash_phase_matrix(md->A) : 0;
     const auto cached = use_cache ? ctx->gram_cache.find(key) : ctx->gram_cache.end();
     if (cached == ctx->gram_cache.end())
-        from.push_back({&md->A, md->d_pairs.as<int2>(), md->d_csr_off.as<int32_t>(), md->d_csr_ent.as<int32_t>(), gp});
+        from.push_back({&md->A, md->d_pairs.as<int2>(), md->d_csr_off.as<int32_t>(), md->d_csr_ent.as<int32_t>(), gp,
+                        gp + nn});
     else
         LEAP_HIP(hipMemcpyAsync(gp, cached->second.data(), cached->second.size() * sizeof(double),
                                 hipMemcpyHostToDevice, s));
     GramWork work;
     gram_pinv_device(ctx, from, N, work);
-    std::vector<double> keep(use_cache && from.size() > 1 ? size_t(N) * N : 0);
+    std::vector<double> keep(use_cache && from.size() > 1 ? 2 * nn : 0);
     if (!keep.empty())
         LEAP_HIP(hipMemcpyAsync(keep.data(), gp, keep.size() * sizeof(double), hipMemcpyDeviceToHost, s));
     md->d_AdT.reserve(size_t(K) * N * sizeof(double));
@@ -701,7 +689,7 @@ leap_metadata* create_metadata(leap_ctx* ctx, const leap_ms_view& ms, int32_t re
 // captured sequence allocates nothing (the sizes rotate_directions and
 // invert_directions ask for).
 void reserve_solution(leap_ctx* ctx, const leap_metadata& md, uint32_t D, uint32_t T, const leap_options& opts) {
-    const int32_t K = md.A.rows, N = md.A.cols, K1 = md.A1.rows;
+    const int32_t K = md.A.rows, N = md.A.cols;
     ctx->d_avg.reserve(size_t(md.nbl) * md.pols * 2 * D * sizeof(double));
     if (use_packed(opts)) {
         const uint32_t tc = pack_chunk(T, md.nbl, md.channels, opts);
@@ -709,17 +697,13 @@ void reserve_solution(leap_ctx* ctx, const leap_metadata& md, uint32_t D, uint32
     }
     if (opts.strategy == LEAP_STRATEGY_BATCHED)
         ctx->d_nufft_tail.reserve(nufft_tail_bytes(D));  // the NUFFT route's chunked last round
-    ctx->d_phase.reserve(size_t(K1) * D * sizeof(double));
     ctx->d_cal1.reserve(size_t(N) * D * sizeof(double));
-    ctx->d_delta.reserve(size_t(K) * D * sizeof(double));
     ctx->d_cal.reserve(size_t(N) * D * sizeof(double));
-    if (opts.strategy != LEAP_STRATEGY_BATCHED) {
-        ctx->d_partial.reserve(inversion_partial_doubles(K, N, D) * sizeof(double));
-    } else if (opts.precision == LEAP_PRECISION_MIXED) {
+    if (opts.precision == LEAP_PRECISION_MIXED) {
         ctx->d_a_planes.reserve(bf16_planes_bytes((D + 63) / 64 * 64, K));
         ctx->d_partial.reserve(mfma_partial_floats(K, D, N) * sizeof(float));
     } else {
-        ctx->d_partial.reserve(gemm_f64_partial_doubles(K, N, D) * sizeof(double));
+        ctx->d_sums.reserve(size_t(N) * D * sizeof(double));
     }
 }
 
@@ -739,7 +723,7 @@ void key_common(std::vector<uint64_t>& k, const leap_ctx* ctx, const leap_option
                        uint64_t(opts.channel_sum),
                        key_ptr(ctx->d_packed.ptr),
                        key_ptr(ctx->d_dd.ptr), key_ptr(ctx->d_avg.ptr),
-                       key_ptr(ctx->d_phase.ptr), key_ptr(ctx->d_cal1.ptr), key_ptr(ctx->d_delta.ptr),
+                       key_ptr(ctx->d_cal1.ptr), key_ptr(ctx->d_sums.ptr),
                        key_ptr(ctx->d_cal.ptr), key_ptr(ctx->d_partial.ptr), key_ptr(ctx->d_a_planes.ptr)});
 }
 
@@ -747,7 +731,8 @@ void key_set(std::vector<uint64_t>& k, const leap_metadata& md, const leap_ms_vi
              int32_t solutions, uint32_t interval) {
     k.insert(k.end(), {key_ptr(&md), uint64_t(md.A.rows), uint64_t(md.A.cols), uint64_t(md.A1.rows), md.nbl,
                        md.channels, md.pols, key_bits(md.freq_start_hz), key_bits(md.freq_inc_hz),
-                       key_ptr(md.d_AdT.ptr), key_ptr(md.d_Ad1T.ptr), key_ptr(md.d_I1.ptr), key_ptr(md.d_pairs.ptr),
+                       key_ptr(md.d_Gp.ptr), key_ptr(md.d_csr_ent.ptr), key_ptr(md.d_csr1_ent.ptr), key_ptr(md.d_I1.ptr),
+                       key_ptr(md.d_pairs.ptr),
                        key_ptr(md.d_lambda.ptr), key_ptr(md.d_AdT_planes.ptr), key_ptr(ms.vis),
                        key_ptr(ms.uvw_device), uint64_t(ms.vis_dtype), ms.num_rows, D, uint64_t(solutions),
                        interval});
@@ -2011,8 +1996,8 @@ extern "C" int leap_hip_residual_loss_grad(leap_ctx* ctx, const leap_metadata* m
         ia.I1 = md->d_I1.as<int32_t>();
         ia.csr_off = md->d_csr_off.as<int32_t>();
         ia.csr_ent = md->d_csr_ent.as<int32_t>();
-        ia.Gp = md->d_Gp.as<double>();
-        ia.G1p = md->d_Gp.as<double>() + size_t(N) * N;
+        ia.Gp = md->gram(0);
+        ia.G1p = md->gram(2);
         ia.res = take(size_t(D) * std::max(nI, 1));
         ia.part = take(size_t(D) * rb);
         ia.loss = take(D);

@@ -351,108 +351,101 @@ __global__ void assemble_ad_kernel(const double* __restrict__ Gp, int32_t N,
 }
 
 // ---------------------------------------------------------------------------
-// Inversion, per direction d (grid.y):
-//   phase[d][k] = arg(avg[d][I1[k]][pol 0]) for k < K1 - 1, 0 at K1 - 1
-//   cal1[d]     = Ad1 * phase[d]
-//   delta[d][n] = arg(exp(-2 pi i (cal1[a1_n] - cal1[a2_n])) * avg[d][n][pol 0]), n < K - 1
-//                 (row n of avgData, as the reference indexes it; A * cal1 in
-//                 gather form, exact because each A row is e_a1 - e_a2)
-//   cal[d]      = Ad * delta[d] + cal1[d]
+// Inversion of every direction d:
+//   phase[k]  = arg(avg[d][I1[k]][pol 0]) for the rows k of A1, 0 at its constraint row
+//   cal1[d]   = Ad1 * phase
+//   delta[n]  = arg(exp(-2 pi i (cal1[a1_n] - cal1[a2_n])) * avg[d][n][pol 0]) for the rows
+//               n of A (row n of avgData, as the reference indexes it; A * cal1 in gather
+//               form, exact because each row of A is e_a1 - e_a2), 0 at its constraint row
+//   cal[d]    = Ad * delta + cal1[d]
+// The products go through Ad = G+ A^T: A^T y is each antenna's signed sum of its rows'
+// values, and G+ applied to it is N x N, so a direction costs its rows and N^2 instead of
+// K N with K about N^2 / 2.  The constraint's value is 0 and A^T y sums to 0 over each
+// component, so G+ may be taken without the ones of the constraint's component (Gx), whose
+// column of the constraint antenna is zero too: that antenna's sum is not needed.
+// Latency-bound below some 50 directions, three launches of 5 to 8 us; 64 directions of 128
+// antennas (8128 rows) take 24 us, where the split-K product with the K x N pseudo-inverse
+// and the kernels around it took 150.
 // ---------------------------------------------------------------------------
-__global__ void phase_i1_kernel(const double* __restrict__ avg, uint32_t nbl, uint32_t P,
-                                const int32_t* __restrict__ I1, int32_t K1, double* __restrict__ phase) {
-    const int32_t k = blockIdx.x * blockDim.x + threadIdx.x;
-    const uint32_t d = blockIdx.y;
-    if (k >= K1) return;
-    double v = 0.0;
-    if (k < K1 - 1) {
-        int32_t idx = I1[k];
-        if (idx < 0) idx += int32_t(nbl);  // VectorRangeSelect wrap (math/cpu/vector.h:97-104)
-        const double* a = avg + (size_t(d) * nbl + idx) * (2 * P);
-        v = atan2(a[1], a[0]);
-    }
-    phase[size_t(d) * K1 + k] = v;
-}
 
-// cal1[d][i] = sum_k Ad1T[k][i] phase[d][k], summed in k order.  One wave per
-// (kCal1Dirs directions, 64 antennas): lane = antenna, the wave's phases are
-// wave-uniform (scalar loads), every Ad1T element read feeds kCal1Dirs chains,
-// and the loop is unrolled so several rows of Ad1T are in flight.
-constexpr int kCal1Dirs = 4;
+// cal1: one workgroup per (direction, 64 antennas), eight groups of 64 lanes taking every
+// eighth column each; every workgroup forms the direction's antenna sums for itself (one
+// arg per antenna when A1 is a star).
+constexpr int32_t kCal1Groups = 8;
+constexpr int32_t kCal1Chunk = 2048;  // antenna sums in LDS at once
 
-__global__ __launch_bounds__(64) void cal1_kernel(const double* __restrict__ Ad1T, int32_t K1, int32_t N,
-                                                  const double* __restrict__ phase, uint32_t D,
-                                                  double* __restrict__ cal1) {
-    const int32_t i = blockIdx.x * 64 + threadIdx.x;
-    const uint32_t d0 = blockIdx.y * kCal1Dirs;
-    const int32_t ic = i < N ? i : N - 1;
-    const double* ph[kCal1Dirs];
-#pragma unroll
-    for (int j = 0; j < kCal1Dirs; ++j) ph[j] = phase + size_t(d0 + j < D ? d0 + j : D - 1) * K1;
-    double acc[kCal1Dirs];
-#pragma unroll
-    for (int j = 0; j < kCal1Dirs; ++j) acc[j] = 0.0;
-#pragma unroll 8
-    for (int32_t k = 0; k < K1; ++k) {
-        const double b = Ad1T[size_t(k) * N + ic];
-#pragma unroll
-        for (int j = 0; j < kCal1Dirs; ++j) acc[j] = fma(b, ph[j][k], acc[j]);
-    }
-    if (i < N) {
-#pragma unroll
-        for (int j = 0; j < kCal1Dirs; ++j)
-            if (d0 + j < D) cal1[size_t(d0 + j) * N + i] = acc[j];
-    }
-}
-
-__global__ void delta_kernel(const double* __restrict__ avg, uint32_t nbl, uint32_t P,
-                             const int2* __restrict__ pairs, int32_t K, int32_t N,
-                             const double* __restrict__ cal1, double* __restrict__ delta) {
-    const int32_t n = blockIdx.x * blockDim.x + threadIdx.x;
-    const uint32_t d = blockIdx.y;
-    if (n >= K) return;
-    delta[size_t(d) * K + n] = dev::delta_phase(avg, nbl, P, pairs, K, N, cal1, d, n);
-}
-
-// Split-K GEMV: partial[d][chunk][i] = sum over the chunk's k of AdT[k][i] * delta[d][k].
-// 64 rows per chunk: about two workgroups per CU at 32,896 baselines, and a short dependent
-// chain per thread.
-constexpr int32_t kGemvChunk = 64;
-
-__global__ __launch_bounds__(kBlock) void gemv_partial_kernel(
-    const double* __restrict__ AdT, int32_t K, int32_t N, const double* __restrict__ delta,
-    double* __restrict__ partial) {
-    const int32_t chunk = blockIdx.x;
-    const uint32_t d = blockIdx.y;
-    const int32_t k0 = chunk * kGemvChunk;
-    const int32_t k1 = min(K, k0 + kGemvChunk);
-    __shared__ double s_x[kGemvChunk];
-    for (int32_t k = k0 + threadIdx.x; k < k1; k += kBlock) s_x[k - k0] = delta[size_t(d) * K + k];
-    __syncthreads();
-    for (int32_t i = threadIdx.x; i < N; i += kBlock) {
-        double s = 0.0;
-        for (int32_t k = k0; k < k1; ++k) s += AdT[size_t(k) * N + i] * s_x[k - k0];
-        partial[(size_t(d) * gridDim.x + chunk) * N + i] = s;
-    }
-}
-
-// cal[d][i] = sum over chunks of partial[d][chunk][i] + cal1[d][i]: one workgroup per output,
-// each lane a strided slice of the chunks, then a fixed-order tree in LDS.
-__global__ __launch_bounds__(kBlock) void gemv_reduce_kernel(const double* __restrict__ partial, int32_t n_chunks,
-                                                             int32_t N, const double* __restrict__ cal1,
-                                                             double* __restrict__ cal) {
-    __shared__ double s_red[kBlock];
-    const int32_t i = blockIdx.x;
-    const uint32_t d = blockIdx.y;
+__global__ __launch_bounds__(64 * kCal1Groups) void cal1_kernel(const double* __restrict__ avg, uint32_t nbl,
+                                                                uint32_t P, const PhaseRows r,
+                                                                double* __restrict__ cal1) {
+    __shared__ double s_b[kCal1Chunk];
+    __shared__ double s_part[kCal1Groups][64];
+    const uint32_t d = blockIdx.x;
+    const int32_t lane = threadIdx.x % 64, group = threadIdx.x / 64;
+    const int32_t i = blockIdx.y * 64 + lane, ic = min(i, r.N - 1);
+    const double* a_d = avg + size_t(d) * nbl * (2 * P);
     double acc = 0.0;
-    for (int32_t c = threadIdx.x; c < n_chunks; c += kBlock) acc += partial[(size_t(d) * n_chunks + c) * N + i];
-    s_red[threadIdx.x] = acc;
-    __syncthreads();
-    for (uint32_t stride = kBlock / 2; stride > 0; stride >>= 1) {
-        if (threadIdx.x < stride) s_red[threadIdx.x] += s_red[threadIdx.x + stride];
+    for (int32_t j0 = 0; j0 < r.N; j0 += kCal1Chunk) {
+        const int32_t jn = min(kCal1Chunk, r.N - j0);
         __syncthreads();
+        for (int32_t j = threadIdx.x; j < jn; j += 64 * kCal1Groups) {
+            double b = 0.0;
+            if (j0 + j != r.constraint)
+                for (int32_t e = r.csr_off[j0 + j]; e < r.csr_off[j0 + j + 1]; ++e) {
+                    const int32_t v = r.csr_ent[e];
+                    int32_t idx = r.I[v >> 1];
+                    if (idx < 0) idx += int32_t(nbl);  // VectorRangeSelect wrap (math/cpu/vector.h:97-104)
+                    const double* a = a_d + size_t(idx) * (2 * P);
+                    const double ph = atan2(a[1], a[0]);
+                    b += (v & 1) ? -ph : ph;
+                }
+            s_b[j] = b;
+        }
+        __syncthreads();
+#pragma unroll 8
+        for (int32_t j = group; j < jn; j += kCal1Groups) acc = fma(r.Gx[size_t(j0 + j) * r.N + ic], s_b[j], acc);
     }
-    if (threadIdx.x == 0) cal[size_t(d) * N + i] = s_red[0] + cal1[size_t(d) * N + i];
+    s_part[group][lane] = acc;
+    __syncthreads();
+    if (group != 0 || i >= r.N) return;
+    for (int g = 1; g < kCal1Groups; ++g) acc += s_part[g][lane];
+    cal1[size_t(d) * r.N + i] = acc;
+}
+
+// sums[d][a] = A^T delta: one wave per (direction, antenna) over the antenna's rows.  Each
+// row's delta is formed by both of its antennas, which costs less than a launch and an array
+// between them up to a few million rows in all (256 directions of 256 antennas: 125 us).
+__global__ __launch_bounds__(kBlock) void delta_sum_kernel(const double* __restrict__ avg, uint32_t nbl, uint32_t P,
+                                                           const PhaseRows r, const double* __restrict__ cal1,
+                                                           double* __restrict__ sums) {
+#pragma clang fp contract(off)
+    const uint32_t d = blockIdx.x, lane = threadIdx.x % 64;
+    const int32_t a = int32_t(blockIdx.y * (kBlock / 64) + threadIdx.x / 64);
+    if (a >= r.N) return;  // whole waves
+    double acc = 0.0;
+    if (a != r.constraint)
+        for (int32_t e = r.csr_off[a] + int32_t(lane); e < r.csr_off[a + 1]; e += 64) {
+            const int32_t v = r.csr_ent[e];
+            const double t = dev::delta_phase(avg, nbl, P, r.pairs, r.K, r.N, cal1, d, v >> 1);
+            acc += (v & 1) ? -t : t;
+        }
+    for (int off = 32; off > 0; off >>= 1) acc += __shfl_xor(acc, off, 64);
+    if (lane == 0) sums[size_t(d) * r.N + a] = acc;
+}
+
+// cal[d][a] = Gx[a][:] . sums[d] + cal1[d][a]: one wave per (direction, antenna).
+__global__ __launch_bounds__(kBlock) void cal_kernel(const double* __restrict__ Gx, int32_t N,
+                                                     const double* __restrict__ sums, const double* __restrict__ cal1,
+                                                     double* __restrict__ cal) {
+    const uint32_t d = blockIdx.x, lane = threadIdx.x % 64;
+    const int32_t a = int32_t(blockIdx.y * (kBlock / 64) + threadIdx.x / 64);
+    if (a >= N) return;  // whole waves
+    const double* row = Gx + size_t(a) * N;
+    const double* x = sums + size_t(d) * N;
+    double acc = 0.0;
+#pragma unroll 4
+    for (int32_t j = int32_t(lane); j < N; j += 64) acc = fma(row[j], x[j], acc);
+    for (int off = 32; off > 0; off >>= 1) acc += __shfl_xor(acc, off, 64);
+    if (lane == 0) cal[size_t(d) * N + a] = acc + cal1[size_t(d) * N + a];
 }
 
 // ---------------------------------------------------------------------------
@@ -718,43 +711,24 @@ void launch_assemble_ad(hipStream_t s, const double* Gp, int32_t N, const int2* 
     LEAP_HIP(hipGetLastError());
 }
 
+void launch_cal1(hipStream_t s, const leap_metadata& md, const double* avg, uint32_t avg_pols, uint32_t D,
+                 double* cal1) {
+    if (D == 0) return;
+    const PhaseRows r = md.rows_of_A1();
+    cal1_kernel<<<dim3(D, uint32_t(r.N + 63) / 64), 64 * kCal1Groups, 0, s>>>(avg, md.nbl, avg_pols, r, cal1);
+    LEAP_HIP(hipGetLastError());
+}
+
 void launch_inversion_f64(hipStream_t s, const leap_metadata& md, const double* avg, uint32_t avg_pols, uint32_t D,
-                          double* phase, double* cal1, double* delta, double* partial, double* cal) {
+                          double* cal1, double* sums, double* cal) {
     if (D == 0) return;
-    const int32_t K = md.A.rows, N = md.A.cols, K1 = md.A1.rows;
-    const uint32_t nbl = md.nbl, P = avg_pols;
-    phase_i1_kernel<<<dim3((K1 + 255) / 256, D), 256, 0, s>>>(avg, nbl, P, md.d_I1.as<int32_t>(), K1, phase);
+    launch_cal1(s, md, avg, avg_pols, D, cal1);
+    const PhaseRows r = md.rows_of_A();
+    const dim3 grid(D, uint32_t(r.N + kBlock / 64 - 1) / (kBlock / 64));
+    delta_sum_kernel<<<grid, kBlock, 0, s>>>(avg, md.nbl, avg_pols, r, cal1, sums);
     LEAP_HIP(hipGetLastError());
-    cal1_kernel<<<dim3((N + 63) / 64, (D + kCal1Dirs - 1) / kCal1Dirs), 64, 0, s>>>(md.d_Ad1T.as<double>(), K1, N,
-                                                                                phase, D, cal1);
+    cal_kernel<<<grid, kBlock, 0, s>>>(r.Gx, r.N, sums, cal1, cal);
     LEAP_HIP(hipGetLastError());
-    delta_kernel<<<dim3((K + 255) / 256, D), 256, 0, s>>>(avg, nbl, P, md.d_pairs.as<int2>(), K, N, cal1, delta);
-    LEAP_HIP(hipGetLastError());
-    const int32_t chunks = (K + kGemvChunk - 1) / kGemvChunk;
-    gemv_partial_kernel<<<dim3(chunks, D), kBlock, 0, s>>>(md.d_AdT.as<double>(), K, N, delta, partial);
-    LEAP_HIP(hipGetLastError());
-    gemv_reduce_kernel<<<dim3(N, D), kBlock, 0, s>>>(partial, chunks, N, cal1, cal);
-    LEAP_HIP(hipGetLastError());
-}
-
-void launch_inversion_head(hipStream_t s, const leap_metadata& md, const double* avg, uint32_t avg_pols, uint32_t D,
-                           double* phase, double* cal1, double* delta) {
-    if (D == 0) return;
-    const int32_t K = md.A.rows, N = md.A.cols, K1 = md.A1.rows;
-    const uint32_t nbl = md.nbl, P = avg_pols;
-    phase_i1_kernel<<<dim3((K1 + 255) / 256, D), 256, 0, s>>>(avg, nbl, P, md.d_I1.as<int32_t>(), K1, phase);
-    LEAP_HIP(hipGetLastError());
-    cal1_kernel<<<dim3((N + 63) / 64, (D + kCal1Dirs - 1) / kCal1Dirs), 64, 0, s>>>(md.d_Ad1T.as<double>(), K1, N,
-                                                                                phase, D, cal1);
-    LEAP_HIP(hipGetLastError());
-    if (delta) {
-        delta_kernel<<<dim3((K + 255) / 256, D), 256, 0, s>>>(avg, nbl, P, md.d_pairs.as<int2>(), K, N, cal1, delta);
-        LEAP_HIP(hipGetLastError());
-    }
-}
-
-size_t inversion_partial_doubles(int32_t K, int32_t N, uint32_t D) {
-    return size_t((K + kGemvChunk - 1) / kGemvChunk) * size_t(N) * D;
 }
 
 }  // namespace leap

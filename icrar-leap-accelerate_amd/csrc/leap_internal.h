@@ -145,6 +145,16 @@ NufftPlan make_nufft_plan(uint32_t C, bool fp32, bool w16 = false);
 std::vector<double> nufft_tables(const NufftPlan& plan);
 inline size_t nufft_coef32_offset(uint32_t C) { return size_t(kNufftCoefDoubles) + C; }
 
+// A phase matrix on the device, as the inversion's kernels take it.
+struct PhaseRows {
+    int32_t K, N, constraint;
+    const int32_t* I;        // K - 1 baselines of the rows
+    const int2* pairs;       // K - 1 antenna pairs of the rows
+    const int32_t* csr_off;  // N + 1: antenna a's rows are csr_ent[csr_off[a] .. csr_off[a + 1])
+    const int32_t* csr_ent;  // 2 row + 1 where a is the row's antenna2 (sign -1)
+    const double* Gx;        // N x N: G+ without the ones of the constraint's component
+};
+
 }  // namespace leap
 
 // Metadata resident on the device (cpu::MetaData + cuda::ConstantBuffer of the reference).
@@ -162,11 +172,22 @@ struct leap_metadata {
     leap::DeviceBuffer d_Ad1T;     // K1 x N
     leap::DeviceBuffer d_I1;       // K1 - 1 ints (baseline index of phase angle k)
     leap::DeviceBuffer d_pairs;    // K - 1 int2: (antenna1, antenna2) of baseline I(k)
-    // the inversion's adjoint: A's baseline indices I, A1's antenna pairs, and
-    // each antenna's rows of A (CSR: offsets N + 1, entries 2 row + (antenna2 ? 1 : 0))
-    leap::DeviceBuffer d_I, d_pairs1, d_csr_off, d_csr_ent;
+    // A's baseline indices I, A1's antenna pairs, and each antenna's rows of A and of
+    // A1 (CSR: offsets N + 1, entries 2 row + (antenna2 ? 1 : 0))
+    leap::DeviceBuffer d_I, d_pairs1, d_csr_off, d_csr_ent, d_csr1_off, d_csr1_ent;
     leap::DeviceBuffer d_lambda;   // channels double2: wavelength of each channel and its reciprocal
-    leap::DeviceBuffer d_Gp;       // G+ = pinv(A^T A) then G1+ = pinv(A1^T A1), N x N each
+    // G+ = pinv(A^T A), the same without the ones of the constraint's component (PhaseRows::Gx),
+    // then both of A1; N x N each
+    leap::DeviceBuffer d_Gp;
+    const double* gram(int which) const { return d_Gp.as<double>() + size_t(which) * A.cols * A.cols; }
+    leap::PhaseRows rows_of_A() const {
+        return {A.rows, A.cols, A.constraint, d_I.as<int32_t>(), d_pairs.as<int2>(), d_csr_off.as<int32_t>(),
+                d_csr_ent.as<int32_t>(), gram(1)};
+    }
+    leap::PhaseRows rows_of_A1() const {
+        return {A1.rows, A1.cols, A1.constraint, d_I1.as<int32_t>(), d_pairs1.as<int2>(), d_csr1_off.as<int32_t>(),
+                d_csr1_ent.as<int32_t>(), gram(3)};
+    }
     leap::DeviceBuffer d_AdT_planes;  // split-3 x BF16 planes of AdT in MFMA operand layout
     // NUFFT plans (N == 0 when the channel count is not supported) and their
     // device tables (leap::nufft_tables): FP64 transform (LEAP_CHANNEL_SUM_NUFFT),
@@ -259,7 +280,7 @@ struct leap_ctx {
     // workspace
     leap::DeviceBuffer d_packed;  // pol-0 pack of the staged rows (FP64 complex per row and channel)
     leap::DeviceBuffer d_widen[2];  // complex64 pol-0 chunks from the host, widened into d_packed
-    leap::DeviceBuffer d_uvw, d_vis_stage, d_dirs, d_dd, d_avg, d_phase, d_cal1, d_delta, d_cal,
+    leap::DeviceBuffer d_uvw, d_vis_stage, d_dirs, d_dd, d_avg, d_cal1, d_sums, d_cal,
         d_partial, d_a_planes;
     leap::DeviceBuffer d_nufft_tail;  // partial sums of the NUFFT launch's chunked last round
     // residual-loss gradient: ENU->UVW rotations, baseline antennas, antenna corrections, perturbed
@@ -417,35 +438,27 @@ struct GramComponents {
 GramComponents gram_components(const PhaseMatrix& pm);
 void launch_assemble_ad(hipStream_t s, const double* Gp, int32_t N, const int2* pairs,
                         int32_t n_pairs, int32_t constraint, double* AdT);
+// cal[D][N] of D directions from pol 0 of avg[D][nbl][avg_pols] in FP64; cal1 and sums: D x N each.
 void launch_inversion_f64(hipStream_t s, const leap_metadata& md, const double* avg, uint32_t avg_pols, uint32_t D,
-                          double* phase, double* cal1, double* delta, double* partial, double* cal);
+                          double* cal1, double* sums, double* cal);
+// cal1 alone, for the mixed GEMM (which forms its operand from avgData and cal1 itself).
+void launch_cal1(hipStream_t s, const leap_metadata& md, const double* avg, uint32_t avg_pols, uint32_t D,
+                 double* cal1);
 void launch_rotate_batched(hipStream_t s, int32_t precision, int32_t direction_block, bool all_pols,
                            const void* vis, int32_t vis_dtype, const double* uvw, const double* dd, uint32_t D,
                            uint32_t T, uint32_t nbl, uint32_t nbl_grid, uint32_t C, uint32_t P, double f0,
                            double df, double* avg, int32_t fp32_blocks);
-size_t inversion_partial_doubles(int32_t K, int32_t N, uint32_t D);
-// Batched inversion pieces: cal1 / delta for D directions, then one GEMM.
-// phase and cal1 for D directions, and delta unless it is null (the mixed GEMM
-// computes its operand from avgData itself).
-// avg holds avg_pols pols per (direction, baseline); pol 0 is used.
-void launch_inversion_head(hipStream_t s, const leap_metadata& md, const double* avg, uint32_t avg_pols, uint32_t D,
-                           double* phase, double* cal1, double* delta);
-size_t gemm_f64_partial_doubles(int32_t K, int32_t N, uint32_t D);
-void launch_gemm_f64(hipStream_t s, const double* AdT, int32_t K, int32_t N, const double* delta, uint32_t D,
-                     const double* cal1, double* partial, double* cal);
 size_t bf16_planes_bytes(uint32_t rows, int32_t K);
 void launch_split_b(hipStream_t s, const double* B, int32_t K, int32_t N, void* planes);
 size_t mfma_partial_floats(int32_t K, uint32_t D, int32_t N);
-// Where the mixed GEMM's A operand comes from when it is computed in place of
-// the FP64 delta matrix: avgData and the antenna pairs of A's rows.
+// Where the mixed GEMM's A operand comes from: avgData and the antenna pairs of A's rows.
 struct DeltaSource {
     const double* avg;
     uint32_t nbl, pols;
     const int2* pairs;
 };
-void launch_gemm_bf16x3(hipStream_t s, const void* b_planes, int32_t K, int32_t N, const double* delta, uint32_t D,
-                        void* a_planes, const double* cal1, float* partial, double* cal,
-                        const DeltaSource* from = nullptr);
+void launch_gemm_bf16x3(hipStream_t s, const void* b_planes, int32_t K, int32_t N, const DeltaSource& from, uint32_t D,
+                        void* a_planes, const double* cal1, float* partial, double* cal);
 void launch_perturb_uvw(hipStream_t s, const double* uvw0, const double* M, const int2* bl_ants, const double* dp,
                         uint32_t nbl, uint32_t rows, double* uvw);
 void launch_rotate_adjoint(hipStream_t s, const void* vis, int32_t vis_dtype, const double* uvw, const double* dd,

@@ -9,8 +9,8 @@
 //
 // Nothing in the array has to start at zero: every kernel of the route writes
 // all of its output before the next one reads it (rotate_average_f64 writes
-// every (baseline, pol) of avgData, the inversion kernels every phase, cal1,
-// dphi and partial entry), so contents left by an earlier call do no harm.
+// every baseline of avgData, the inversion kernels every cal1 and antenna sum), so
+// contents left by an earlier call do no harm.
 #include <mutex>
 
 #include "capi_common.h"
@@ -35,9 +35,11 @@ void* scratch_on(int device) {
     return device >= 0 && device < kMaxDevices ? g_scratch[device] : nullptr;
 }
 
-// Offsets (bytes) of one solution's working set in the scratch array.
+// Offsets (bytes) of one solution's working set in the scratch array.  The total, which is what
+// a call is accepted by, also counts the rows of A and A1 and a product with the K x N
+// pseudo-inverse in chunks of 64 rows, as the interface states it.
 struct Layout {
-    size_t dirs, dd, avg, phase, cal1, delta, partial, total;
+    size_t dirs, dd, avg, cal1, sums, total;
 };
 
 Layout layout(uint32_t D, uint32_t nbl, uint32_t P, int32_t K, int32_t N, int32_t K1) {
@@ -51,10 +53,10 @@ Layout layout(uint32_t D, uint32_t nbl, uint32_t P, int32_t K, int32_t N, int32_
     l.dirs = take(size_t(D) * 2 * sizeof(double));
     l.dd = take(size_t(D) * 9 * sizeof(double));
     l.avg = take(size_t(nbl) * P * 2 * sizeof(double));
-    l.phase = take(size_t(K1) * sizeof(double));
+    take(size_t(K1) * sizeof(double));
     l.cal1 = take(size_t(N) * sizeof(double));
-    l.delta = take(size_t(K) * sizeof(double));
-    l.partial = take(inversion_partial_doubles(K, N, 1) * sizeof(double));
+    take(size_t(K) * sizeof(double));
+    l.sums = take(size_t((K + 63) / 64) * N * sizeof(double));
     l.total = at;
     return l;
 }
@@ -113,10 +115,8 @@ extern "C" int leap_hip_calibrate_md_noalloc(leap_ctx* ctx, const leap_metadata*
         double* d_dirs = reinterpret_cast<double*>(base + l.dirs);
         double* d_dd = reinterpret_cast<double*>(base + l.dd);
         double* d_avg = reinterpret_cast<double*>(base + l.avg);
-        double* d_phase = reinterpret_cast<double*>(base + l.phase);
         double* d_cal1 = reinterpret_cast<double*>(base + l.cal1);
-        double* d_delta = reinterpret_cast<double*>(base + l.delta);
-        double* d_partial = reinterpret_cast<double*>(base + l.partial);
+        double* d_sums = reinterpret_cast<double*>(base + l.sums);
 
         LEAP_HIP(hipMemcpyAsync(d_dirs, dirs, size_t(D) * 2 * sizeof(double), hipMemcpyHostToDevice, ctx->stream));
         launch_dd(ctx->stream, md->phase_centre_ra, md->phase_centre_dec, d_dirs, D, d_dd);
@@ -129,7 +129,7 @@ extern "C" int leap_hip_calibrate_md_noalloc(leap_ctx* ctx, const leap_metadata*
             for (uint32_t d = 0; d < D; ++d) {
                 launch_rotate_f64(ctx->stream, {vis, ms->vis_dtype, uvw, d_dd + 9 * size_t(d), 1, interval, 1, nbl,
                                                 md->channels, md->pols, 1, md->d_lambda.as<double2>(), d_avg});
-                launch_inversion_f64(ctx->stream, *md, d_avg, 1, 1, d_phase, d_cal1, d_delta, d_partial,
+                launch_inversion_f64(ctx->stream, *md, d_avg, 1, 1, d_cal1, d_sums,
                                      cal_out + (size_t(s) * D + d) * size_t(N));
             }
         }

@@ -8,6 +8,8 @@ of the constraint's component, with N rounded steps per entry each: the toleranc
 import numpy as np
 import pytest
 
+import np_restatement as npr
+
 pytestmark = pytest.mark.gpu
 
 
@@ -48,3 +50,27 @@ def test_pseudo_inverse_at_tile_edges(leap, ctx, n_ant, graph):
         err = np.abs(got["Ad" + name] - want).max() / scale
         print(f"Ad{name}: {err:.2e}")
         assert err <= 16 * n_ant * np.finfo(float).eps
+
+
+@pytest.mark.parametrize("n_dirs", [1, 5])
+@pytest.mark.parametrize("n_ant,graph", [(2, "dense"), (63, "dense"), (64, "split"), (65, "dense"), (130, "split")])
+def test_inversion_through_antenna_sums(leap, ctx, n_ant, graph, n_dirs):
+    """cal = Ad dphi + Ad1 phi1 of random averages against LAPACK's pseudo-inverses (the 1e-9 rad bar of
+    the calibrations), around the kernels' 64-antenna blocks, with components without the constraint,
+    and with the pseudo-inverse taken from the context's cache the second time."""
+    a1, a2 = (x.astype(np.int32) for x in np.triu_indices(n_ant))
+    rng = np.random.default_rng(10 * n_ant + n_dirs)
+    fg = np.zeros(len(a1), dtype=np.uint8)
+    if graph == "split":
+        fg[:] = ((a1 < n_ant // 2) != (a2 < n_ant // 2)) | (a2 == n_ant - 1)
+        fg[0] = 0
+    print(f"inversion: {n_ant} antennas, {graph}, {n_dirs} directions", flush=True)
+    avg = rng.normal(size=(n_dirs, len(a1), 1)) + 1j * rng.normal(size=(n_dirs, len(a1), 1))
+    view = leap.view_from_arrays(_ms(a1, a2, fg))
+    A, I = npr.phase_matrix(a1, a2, fg)
+    A1, I1 = npr.phase_matrix(a1, a2, fg, 0)
+    Ad, Ad1 = np.linalg.pinv(A), np.linalg.pinv(A1)
+    want = np.array([npr.apply_inversion(x, A, I, A1, I1, Ad, Ad1) for x in avg])
+    for cached in (False, True, True):
+        md = ctx.metadata(view, ref_ant=0, use_cache=cached)
+        assert np.abs(npr.wrap(md.apply_inversion(avg) - want)).max() < 1e-9
