@@ -196,18 +196,14 @@ bool use_packed(const leap_options& opts) {
            !(opts.precision == LEAP_PRECISION_MIXED && opts.fp32_blocks) && !opts.direct_cube;
 }
 
-// The batched pol-0 route for a tuned call on a device-resident cube: the pack
-// pass (every pol read, pol 0 written as FP64) pays only when the FP64 work is
-// large enough.  Rates measured on MI355X at the 256-station set (32,896
-// baselines, 128 t, 384 ch): pack 5.2 TB/s; packed Horner 32 / 50 / 55 TFLOP/s
-// with 1 / 2 / 4 directions per lane (up to 64, 128, more directions); the
-// Horner kernel straight from the cube reads at most 6.4 TB/s and computes
-// 30 TFLOP/s up to 128 directions, 51 (complex64) or 45 (complex128) above.
-// E.g. 256 directions: from the cube for complex64 (65 vs 72 ms) and
-// complex128 (74 vs 82 ms); 64 directions on complex128: from the cube (27 vs
-// 50 ms); the pack pays from about 800 (complex64) or 480 (complex128)
-// directions.  Host-resident cubes always take the packed route (pol 0 only
-// crosses the bus).
+// The batched pol-0 Horner route for a tuned call on a device-resident cube: the pack pass (every
+// pol read, pol 0 written as FP64) pays only when the FP64 work is large enough.  Rates measured on
+// MI355X: pack 5.2 TB/s; packed Horner 32 / 50 / 55 TFLOP/s with 1 / 2 / 4 directions per lane (up
+// to 64, 128, more directions); the wave kernel straight from the cube 5.7 TB/s and 50 TFLOP/s
+// (complex64) or 47 (complex128), both less by the phasors of a row (20 channels' worth: 48
+// channels, 256 directions 37 TFLOP/s, 384 channels 49).  So the pack pays from about 800
+// directions on complex64.  Host-resident cubes always take the packed route (pol 0 only crosses
+// the bus).
 leap_options routed(const leap_options& o, const leap_ms_view& ms, uint32_t T, uint32_t D) {
     leap_options r = o;
     if (r.channel_sum == LEAP_CHANNEL_SUM_AUTO) {
@@ -235,9 +231,11 @@ leap_options routed(const leap_options& o, const leap_ms_view& ms, uint32_t T, u
     const double rc = double(T) * ms.num_baselines * ms.num_channels;  // (row, channel)s
     const double s = ms.vis_dtype == LEAP_VIS_C64 ? 8.0 : 16.0;
     const double flops = 8.0 * rc * D;
-    const double packed = rc * (ms.num_pols * s + 16.0) / 5.2e12 + flops / (D > 128 ? 55e12 : D > 64 ? 50e12 : 32e12);
-    const double direct_rate = D > 128 ? (ms.vis_dtype == LEAP_VIS_C64 ? 51e12 : 45e12) : 30e12;
-    const double direct = std::max(rc * ms.num_pols * s / 6.4e12, flops / direct_rate);
+    const double rows = double(ms.num_channels) / (ms.num_channels + 20.0);
+    const double packed =
+        rc * (ms.num_pols * s + 16.0) / 5.2e12 + flops / (rows * (D > 128 ? 55e12 : D > 64 ? 50e12 : 32e12));
+    const double direct = std::max(rc * ms.num_pols * s / 5.7e12,
+                                   flops / (rows * (ms.vis_dtype == LEAP_VIS_C64 ? 50e12 : 47e12)));
     if (packed > direct) r.direct_cube = 1;
     return r;
 }
@@ -251,6 +249,26 @@ bool packed_route(const leap_options& opts, int32_t tile) {
     return packed_tile_supported(opts.direction_block * 10 + (opts.lane_directions ? opts.lane_directions : 1));
 }
 
+// The autotuner's key of a batched call's shape and route.
+TuneKey tune_key(const leap_metadata& md, const leap_ms_view& ms, uint32_t T, uint32_t D, const leap_options& opts) {
+    return {opts.precision * 4 + (opts.fp32_blocks ? 2 : 0) + (opts.lane_directions ? 1 : 0) +
+                16 * opts.lane_directions + (use_packed(opts) ? kTunePackedBit : 0) +
+                (is_nufft(opts.channel_sum) ? kTuneNufftBit : 0) +
+                (opts.channel_sum == LEAP_CHANNEL_SUM_NUFFT_FP32 ? kTuneNufft32Bit : 0) +
+                (opts.channel_sum == LEAP_CHANNEL_SUM_NUFFT_W16 ? kTuneNufftW16Bit : 0),
+            ms.vis_dtype, opts.all_pols, D, T, md.channels, md.pols};
+}
+
+// Whether a routed batched call takes the wave-at-a-time Horner kernel: pol 0 straight from the
+// cube, no tile named by the caller or by loaded tuning.
+bool wave_route(const leap_ctx* ctx, const leap_metadata& md, const leap_ms_view& ms, uint32_t T, uint32_t D,
+                const leap_options& opts) {
+    return opts.strategy == LEAP_STRATEGY_BATCHED && opts.channel_sum == LEAP_CHANNEL_SUM_HORNER &&
+           opts.direct_cube && !opts.all_pols && !(opts.precision == LEAP_PRECISION_MIXED && opts.fp32_blocks) &&
+           opts.direction_block == 0 && opts.lane_directions == 0 &&
+           ctx->tuned.find(tune_key(md, ms, T, D, opts)) == ctx->tuned.end();
+}
+
 // Direction block for the batched kernel: the fastest of the candidates on a
 // slice of the baselines, timed once per shape and kept in the context.
 int32_t tuned_direction_block(leap_ctx* ctx, const leap_metadata& md, const leap_ms_view& ms, const DeviceRows& rows,
@@ -262,11 +280,7 @@ int32_t tuned_direction_block(leap_ctx* ctx, const leap_metadata& md, const leap
     if (opts.direction_block != 0 && opts.lane_directions == 0) return opts.direction_block * 10 + 1;
     const bool packed = use_packed(opts);
     const bool nufft = is_nufft(opts.channel_sum);
-    const TuneKey key{opts.precision * 4 + (opts.fp32_blocks ? 2 : 0) + (opts.lane_directions ? 1 : 0) +
-                          16 * opts.lane_directions + (packed ? kTunePackedBit : 0) + (nufft ? kTuneNufftBit : 0) +
-                          (opts.channel_sum == LEAP_CHANNEL_SUM_NUFFT_FP32 ? kTuneNufft32Bit : 0) +
-                          (opts.channel_sum == LEAP_CHANNEL_SUM_NUFFT_W16 ? kTuneNufftW16Bit : 0),
-                      ms.vis_dtype, opts.all_pols, D, T, md.channels, md.pols};
+    const TuneKey key = tune_key(md, ms, T, D, opts);
     auto it = ctx->tuned.find(key);
     if (it != ctx->tuned.end()) return it->second;
     // Candidate tiles (directions per workgroup * 10 + directions per lane).
@@ -423,11 +437,15 @@ void rotate_packed_pipeline(leap_ctx* ctx, const leap_metadata& md, const leap_m
     }
 }
 
+// Stands for the wave-at-a-time Horner kernel where a tile is asked for.
+constexpr int32_t kWaveTile = -1;
+
 // Tile of the batched kernel for this shape: the caller's, the cached one, or
 // tuned now.  The packed path is tuned on its first chunk, packed into the
 // first buffer just before the probe launches.
 int32_t batched_tile(leap_ctx* ctx, const leap_metadata& md, const leap_ms_view& ms, const DeviceRows& rows,
                      uint32_t T, uint32_t D, const leap_options& opts) {
+    if (wave_route(ctx, md, ms, T, D, opts)) return kWaveTile;
     if (!use_packed(opts)) return tuned_direction_block(ctx, md, ms, rows, T, D, opts);
     const uint32_t tc = std::min(T, pack_chunk(T, md.nbl, md.channels, opts));
     const size_t n = size_t(tc) * md.nbl * md.channels;
@@ -442,15 +460,26 @@ int32_t batched_tile(leap_ctx* ctx, const leap_metadata& md, const leap_ms_view&
 // avgData of D directions for T timesteps starting at the staged rows, into
 // ctx->d_avg; returns the pols it holds per (direction, baseline).  With
 // pol0_only (calibrations: only pol 0 reaches cal, CpuLeapCalibrator.cc:161,171)
-// the NUFFT and per-direction routes write pol 0 alone, a quarter of the bytes for 4 pols.
+// the NUFFT, wave and per-direction routes write pol 0 alone, a quarter of the bytes for 4 pols.
 uint32_t rotate_directions(leap_ctx* ctx, const leap_metadata& md, const leap_ms_view& ms, const DeviceRows& rows,
                            uint32_t T, uint32_t D, const leap_options& opts, int32_t tile = 0,
                            bool pol0_only = false) {
     const bool nufft_route = opts.strategy == LEAP_STRATEGY_BATCHED && is_nufft(opts.channel_sum);
-    const bool narrow = nufft_route || opts.strategy == LEAP_STRATEGY_PER_DIRECTION;
+    const bool wave = tile == kWaveTile || (tile == 0 && wave_route(ctx, md, ms, T, D, opts));
+    const bool narrow = nufft_route || wave || opts.strategy == LEAP_STRATEGY_PER_DIRECTION;
     const uint32_t avg_pols = pol0_only && narrow ? 1u : md.pols;
     const size_t per_dir = size_t(md.nbl) * md.pols * 2;  // room for the full layout (autotune probes)
     ctx->d_avg.reserve(per_dir * D * sizeof(double));
+    if (wave) {
+        require(rows.vis != nullptr, LEAP_ERR_INTERNAL, "visibilities were not staged");
+        ctx->last_direction_block = horner_wave_tile(D, md.nbl, md.channels, 1);
+        record_rotate_begin(ctx);
+        launch_horner_wave(ctx->stream, {rows.vis, ms.vis_dtype, rows.uvw, ctx->d_dd.as<double>(), D, T, 1, md.nbl,
+                                         md.channels, md.pols, avg_pols, md.freq_start_hz, md.freq_inc_hz,
+                                         ctx->d_avg.as<double>()});
+        record_rotate_end(ctx);
+        return avg_pols;
+    }
     if (opts.strategy == LEAP_STRATEGY_BATCHED && packed_route(opts, tile)) {
         rotate_packed_pipeline(ctx, md, ms, rows, T, D, opts, tile, avg_pols);
         return avg_pols;
@@ -781,9 +810,9 @@ void calibrate_loop_graph(leap_ctx* ctx, const leap_metadata& md, const leap_ms_
         if (opts.strategy == LEAP_STRATEGY_BATCHED) {
             const DeviceRows rows0 = stage_rows(ctx, ms, 0, interval * nbl);
             tile = batched_tile(ctx, md, ms, rows0, interval, D, opts);
-            ctx->last_direction_block = tile;
+            ctx->last_direction_block = tile == kWaveTile ? horner_wave_tile(D, md.nbl, md.channels, 1) : tile;
         }
-        std::vector<uint64_t> key{uint64_t(tile)};
+        std::vector<uint64_t> key{uint64_t(uint32_t(tile))};
         key_common(key, ctx, opts);
         key_set(key, md, ms, D, solutions, interval);
         if (!ctx->seq_single || ctx->seq_single->key != key) {

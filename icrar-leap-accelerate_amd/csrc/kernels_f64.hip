@@ -68,11 +68,10 @@ __global__ void dd_kernel(double ra0, double dec0, const double* __restrict__ di
 //    a 64-entry table in LDS and the series to r^8 (cos) and r^7 (sin) on |r| <= pi / 64,
 //    whose next terms are below 2.5e-20 and 4.6e-18: 18 instructions
 //  - the rotated sample goes into the sums as four FMAs
-// Samples that are not finite and shifts that are not below kMaxShift take the plain form
+// Samples that are not finite and shifts that are not below 2^26 rad take the plain form
 // (division, sincos, rotate every pol, look for a NaN), exactly as the reference does it.
 // ---------------------------------------------------------------------------
-constexpr int kPhasorTable = 64;
-constexpr double kMaxShift = 67108864.0;    // 2^26 rad: 32 / pi times it stays below 2^31
+constexpr double kMaxShift = 67108864.0;  // 2^26 rad, far inside the phasor table's range
 constexpr uint32_t kRowChunk = 32;          // rows whose shift factors a wave keeps in LDS
 constexpr uint32_t kLambdaLds = 1024;       // channels whose wavelengths sit in LDS
 
@@ -98,26 +97,6 @@ struct VisLoad {
         return z == T(0);
     }
 };
-
-// exp(i th) for |th| <= kMaxShift.
-__device__ inline double2 phasor_table(const double2* __restrict__ table, double th) {
-#pragma clang fp contract(off)
-    constexpr double kStep = 10.185916357881301489;         // 32 / pi
-    constexpr double kPiO32Hi = 0.098174770424681034875;    // double(pi / 32)
-    constexpr double kPiO32Lo = 3.8270212473354786e-18;     // pi / 32 - double(pi / 32)
-    const double k = rint(th * kStep);
-    const double2 t = table[int32_t(k) & (kPhasorTable - 1)];
-    double r = fma(-k, kPiO32Hi, th);
-    r = fma(-k, kPiO32Lo, r);
-    const double r2 = r * r;
-    double s = fma(-1.0 / 5040.0, r2, 1.0 / 120.0);
-    s = fma(s, r2, -1.0 / 6.0);
-    s = fma(r * r2, s, r);  // sin r
-    double c = fma(1.0 / 40320.0, r2, -1.0 / 720.0);
-    c = fma(c, r2, 1.0 / 24.0);
-    c = fma(c, r2, -0.5) * r2;  // cos r - 1
-    return make_double2(fma(-t.y, s, fma(t.x, c, t.x)), fma(t.x, s, fma(t.y, c, t.y)));
-}
 
 // Sums of N values over a wave: every step halves the values a lane holds while there is
 // more than one, so N + 4 exchanges do instead of 6 N.  The lane's value is number
@@ -164,7 +143,7 @@ __global__ __launch_bounds__(kWide ? 256 : 1024) void rotate_average_f64(
 #pragma clang fp contract(off)
     constexpr int NV = pow2_at_least(2 * PO * ND);
     __shared__ double2 s_lambda[kLambdaLds];
-    __shared__ double2 s_table[kPhasorTable];
+    __shared__ double2 s_table[dev::kPhasorTable];
     // kWide, for 64-byte samples (4 complex128 pols) of which pol 0 is kept: a lane loading its own
     // sample strides the wave's four loads by 64 bytes and leaves the reuse of their lines to the
     // L1, which the waves in flight overflow.  So the wave loads its 64 samples as 256 consecutive
@@ -178,11 +157,7 @@ __global__ __launch_bounds__(kWide ? 256 : 1024) void rotate_average_f64(
     const bool in_lds = C <= kLambdaLds;
     if (in_lds)
         for (uint32_t c = threadIdx.x; c < C; c += blockDim.x) s_lambda[c] = lambda2[c];
-    for (uint32_t k = threadIdx.x; k < kPhasorTable; k += blockDim.x) {
-        double sn, cs;
-        sincospi(double(k) / 32.0, &sn, &cs);
-        s_table[k] = make_double2(cs, sn);
-    }
+    dev::phasor_table_init(s_table);
     __syncthreads();
     const uint32_t group = blockIdx.x % groups, block = blockIdx.x / groups;
     const uint32_t per_group = (D + groups - 1) / groups;
@@ -285,7 +260,7 @@ __global__ __launch_bounds__(kWide ? 256 : 1024) void rotate_average_f64(
 #pragma unroll
                     for (int d = 0; d < ND; ++d) {
                         if ((d & 1) == 0 && uint32_t(d) >= active) break;
-                        const double2 e = phasor_table(s_table, shift[d]);
+                        const double2 e = dev::phasor_table(s_table, shift[d]);
 #pragma unroll
                         for (int q = 0; q < PO; ++q) {  // (a + ib)(cs + i sn), :198, :208-214
                             double* o = acc + 2 * (d * PO + q);

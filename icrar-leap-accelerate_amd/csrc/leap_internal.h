@@ -402,6 +402,20 @@ int32_t multi_blocks_per_cu(int32_t tile);
 // Kernel launchers (kernels_f64.hip)
 void launch_dd(hipStream_t s, double ra0, double dec0, const double* d_dirs, uint32_t D,
                double* d_dd);
+// Pol 0 of avgData of D directions over consecutive solution intervals of T timesteps each
+// by FP64 Horner channel sums straight from the cube (kernels_wave.hip).
+struct HornerWave {
+    const void* vis;
+    int32_t vis_dtype;
+    const double* uvw;
+    const double* dd;  // [D][3][3]
+    uint32_t D, T, intervals, nbl, C, P, pols_out;
+    double f0, df;
+    double* avg;  // [intervals][D][nbl][pols_out]
+};
+// Directions of a wave * 10 + directions of a lane.
+int32_t horner_wave_tile(uint32_t D, uint32_t nbl, uint32_t C, uint32_t intervals);
+void launch_horner_wave(hipStream_t s, const HornerWave& h);
 // The per-direction FP64 rotate/average of D directions over consecutive solution intervals
 // of T timesteps each, from the first interval's first row.
 struct RotateF64 {
