@@ -300,6 +300,10 @@ int32_t tuned_direction_block(leap_ctx* ctx, const leap_metadata& md, const leap
         for (int32_t t : all64)
             if (opts.lane_directions == 0 || t % 10 == opts.lane_directions) candidates.push_back(t);
     }
+    if (candidates.size() == 1) {  // nothing to choose
+        ctx->tuned.emplace(key, candidates.front());
+        return candidates.front();
+    }
     // Enough baselines for several rounds of workgroups on every CU.
     const uint32_t probe_bl = std::min<uint32_t>(md.nbl, 8192);
     if (before_probe) before_probe();
@@ -323,7 +327,7 @@ int32_t tuned_direction_block(leap_ctx* ctx, const leap_metadata& md, const leap
                                     md.freq_inc_hz, ctx->d_avg.as<double>(), 0);
             else if (packed)
                 launch_rotate_packed(ctx->stream, tile, ctx->d_packed.as<double>(), rows.uvw, ctx->d_dd.as<double>(),
-                                     D, T, md.nbl, probe_bl, md.channels, md.pols, md.freq_start_hz, md.freq_inc_hz,
+                                     D, T, md.nbl, probe_bl, md.channels, md.pols, md.pols, md.freq_start_hz, md.freq_inc_hz,
                                      ctx->d_avg.as<double>(), 0);
             else
                 launch_rotate_batched(ctx->stream, opts.precision, tile, opts.all_pols != 0, rows.vis, ms.vis_dtype,
@@ -367,10 +371,12 @@ uint32_t pack_chunk(uint32_t T, uint32_t nbl, uint32_t C, const leap_options& op
 // packed by the host staging instead (pol 0 only crosses the bus), which
 // orders itself on the context stream.
 void rotate_packed_pipeline(leap_ctx* ctx, const leap_metadata& md, const leap_ms_view& ms, const DeviceRows& rows,
-                            uint32_t T, uint32_t D, const leap_options& opts, int32_t tile, uint32_t avg_pols) {
-    const uint32_t tc = pack_chunk(T, md.nbl, md.channels, opts);
+                            uint32_t T, uint32_t D, const leap_options& opts, int32_t tile, uint32_t avg_pols,
+                            uint32_t intervals) {
+    // several solution intervals are packed as one chunk (interval_group sees to their size)
+    const uint32_t tc = intervals > 1 ? T : pack_chunk(T, md.nbl, md.channels, opts);
     const uint32_t n_chunks = (T + tc - 1) / tc;
-    const size_t per_t = size_t(md.nbl) * md.channels;  // (row, channel)s per timestep
+    const size_t per_t = size_t(md.nbl) * md.channels * intervals;  // (row, channel)s per timestep
     const size_t buf_elems = size_t(tc) * per_t;
     ctx->d_packed.reserve(buf_elems * (n_chunks > 1 ? 2 : 1) * 2 * sizeof(double));
     const size_t vis_row_bytes = vis_elem_bytes(ms) * md.channels;
@@ -402,11 +408,11 @@ void rotate_packed_pipeline(leap_ctx* ctx, const leap_metadata& md, const leap_m
                                 rows.uvw + size_t(t0) * md.nbl * 3, ctx->d_dd.as<double>(), D, nt, md.nbl, md.nbl,
                                 md.channels, md.pols, avg_pols, md.freq_start_hz, md.freq_inc_hz,
                                 ctx->d_avg.as<double>(), k > 0 ? 1 : 0, ctx->d_nufft_tail.as<double>(),
-                                nufft_tail_bytes(D));
+                                nufft_tail_bytes(D), intervals);
         else
             launch_rotate_packed(ctx->stream, tile, buf[k % 2], rows.uvw + size_t(t0) * md.nbl * 3,
-                                 ctx->d_dd.as<double>(), D, nt, md.nbl, md.nbl, md.channels, md.pols,
-                                 md.freq_start_hz, md.freq_inc_hz, ctx->d_avg.as<double>(), k > 0 ? 1 : 0);
+                                 ctx->d_dd.as<double>(), D, nt, md.nbl, md.nbl, md.channels, md.pols, avg_pols,
+                                 md.freq_start_hz, md.freq_inc_hz, ctx->d_avg.as<double>(), k > 0 ? 1 : 0, intervals);
         record_rotate_end(ctx);
     };
     pack(0, ctx->stream);
@@ -457,31 +463,33 @@ int32_t batched_tile(leap_ctx* ctx, const leap_metadata& md, const leap_ms_view&
     });
 }
 
-// avgData of D directions for T timesteps starting at the staged rows, into
-// ctx->d_avg; returns the pols it holds per (direction, baseline).  With
+// avgData of D directions for consecutive solution intervals of T timesteps each, starting at
+// the staged rows, into ctx->d_avg [interval][direction][baseline][pols]; returns the pols it
+// holds.  Several intervals only where interval_group gives them.  With
 // pol0_only (calibrations: only pol 0 reaches cal, CpuLeapCalibrator.cc:161,171)
 // the NUFFT, wave and per-direction routes write pol 0 alone, a quarter of the bytes for 4 pols.
 uint32_t rotate_directions(leap_ctx* ctx, const leap_metadata& md, const leap_ms_view& ms, const DeviceRows& rows,
                            uint32_t T, uint32_t D, const leap_options& opts, int32_t tile = 0,
-                           bool pol0_only = false) {
+                           bool pol0_only = false, uint32_t intervals = 1) {
     const bool nufft_route = opts.strategy == LEAP_STRATEGY_BATCHED && is_nufft(opts.channel_sum);
     const bool wave = tile == kWaveTile || (tile == 0 && wave_route(ctx, md, ms, T, D, opts));
-    const bool narrow = nufft_route || wave || opts.strategy == LEAP_STRATEGY_PER_DIRECTION;
+    const bool packed = !wave && opts.strategy == LEAP_STRATEGY_BATCHED && packed_route(opts, tile);
+    const bool narrow = nufft_route || wave || packed || opts.strategy == LEAP_STRATEGY_PER_DIRECTION;
     const uint32_t avg_pols = pol0_only && narrow ? 1u : md.pols;
     const size_t per_dir = size_t(md.nbl) * md.pols * 2;  // room for the full layout (autotune probes)
-    ctx->d_avg.reserve(per_dir * D * sizeof(double));
+    ctx->d_avg.reserve(per_dir * D * intervals * sizeof(double));
     if (wave) {
         require(rows.vis != nullptr, LEAP_ERR_INTERNAL, "visibilities were not staged");
-        ctx->last_direction_block = horner_wave_tile(D, md.nbl, md.channels, 1);
+        ctx->last_direction_block = horner_wave_tile(D, md.nbl, md.channels, intervals);
         record_rotate_begin(ctx);
-        launch_horner_wave(ctx->stream, {rows.vis, ms.vis_dtype, rows.uvw, ctx->d_dd.as<double>(), D, T, 1, md.nbl,
-                                         md.channels, md.pols, avg_pols, md.freq_start_hz, md.freq_inc_hz,
+        launch_horner_wave(ctx->stream, {rows.vis, ms.vis_dtype, rows.uvw, ctx->d_dd.as<double>(), D, T, intervals,
+                                         md.nbl, md.channels, md.pols, avg_pols, md.freq_start_hz, md.freq_inc_hz,
                                          ctx->d_avg.as<double>()});
         record_rotate_end(ctx);
         return avg_pols;
     }
-    if (opts.strategy == LEAP_STRATEGY_BATCHED && packed_route(opts, tile)) {
-        rotate_packed_pipeline(ctx, md, ms, rows, T, D, opts, tile, avg_pols);
+    if (packed) {
+        rotate_packed_pipeline(ctx, md, ms, rows, T, D, opts, tile, avg_pols, intervals);
         return avg_pols;
     }
     require(rows.vis != nullptr, LEAP_ERR_INTERNAL, "visibilities were not staged");
@@ -494,7 +502,7 @@ uint32_t rotate_directions(leap_ctx* ctx, const leap_metadata& md, const leap_ms
                             rows.vis, true, ms.vis_dtype, rows.uvw,
                             ctx->d_dd.as<double>(), D, T, md.nbl, md.nbl, md.channels, md.pols, avg_pols,
                             md.freq_start_hz, md.freq_inc_hz, ctx->d_avg.as<double>(), 0,
-                            ctx->d_nufft_tail.as<double>(), nufft_tail_bytes(D));
+                            ctx->d_nufft_tail.as<double>(), nufft_tail_bytes(D), intervals);
         record_rotate_end(ctx);
         return avg_pols;
     }
@@ -509,7 +517,7 @@ uint32_t rotate_directions(leap_ctx* ctx, const leap_metadata& md, const leap_ms
         return avg_pols;
     }
     record_rotate_begin(ctx);
-    launch_rotate_f64(ctx->stream, {rows.vis, ms.vis_dtype, rows.uvw, ctx->d_dd.as<double>(), D, T, 1, md.nbl,
+    launch_rotate_f64(ctx->stream, {rows.vis, ms.vis_dtype, rows.uvw, ctx->d_dd.as<double>(), D, T, intervals, md.nbl,
                                     md.channels, md.pols, avg_pols, md.d_lambda.as<double2>(),
                                     ctx->d_avg.as<double>()});
     record_rotate_end(ctx);
@@ -538,6 +546,49 @@ void invert_directions(leap_ctx* ctx, const leap_metadata& md, uint32_t D, const
     ctx->d_partial.reserve(mfma_partial_floats(K, D, N) * sizeof(float));
     launch_gemm_bf16x3(ctx->stream, md.d_AdT_planes.ptr, K, N, {avg, md.nbl, avg_pols, md.d_pairs.as<int2>()}, D,
                        ctx->d_a_planes.ptr, ctx->d_cal1.as<double>(), static_cast<float*>(ctx->d_partial.ptr), cal);
+}
+
+// The inversion of several solution intervals' averages [interval][direction]: all at once in
+// FP64; in mixed precision as many as the GEMM takes in one K-split of its whole output, whose
+// sums do not depend on how many directions it is given.
+void invert_intervals(leap_ctx* ctx, const leap_metadata& md, uint32_t D, uint32_t intervals, const leap_options& opts,
+                      uint32_t avg_pols, double* cal = nullptr) {
+    const int32_t N = md.A.cols;
+    uint32_t step = intervals;
+    if (opts.precision == LEAP_PRECISION_MIXED) {
+        step = 1;
+        while (step < intervals && mfma_full_output(D, N) && mfma_full_output((step + 1) * D, N)) ++step;
+    }
+    if (cal == nullptr) {
+        ctx->d_cal.reserve(size_t(N) * D * intervals * sizeof(double));
+        cal = ctx->d_cal.as<double>();
+    }
+    for (uint32_t i = 0; i < intervals; i += step) {
+        const uint32_t n = std::min(step, intervals - i);
+        invert_directions(ctx, md, D * n, opts, ctx->d_avg.as<double>() + size_t(i) * D * md.nbl * avg_pols * 2,
+                          cal + size_t(i) * D * N, avg_pols);
+    }
+}
+
+// Solution intervals run as one rotate and one inversion.  An interval of a few integrations leaves
+// most of the GPU idle for the length of seven launches, a copy and a synchronisation (14
+// one-timestep intervals of 128 antennas, 48 channels, 16 directions: 0.59 ms one by one, 0.21
+// together), so intervals are grouped up to 1 GiB of cube, about 0.2 ms of reading, and 256 MiB of
+// averages.  Routes whose kernels take one interval (tiles named by the caller, every pol, FP32
+// blocks, pack chunks) run them one by one.
+uint32_t interval_group(leap_ctx* ctx, const leap_metadata& md, const leap_ms_view& ms, uint32_t T, uint32_t D,
+                        uint32_t solutions, const leap_options& opts) {
+    if (solutions <= 1 || D == 0) return 1;
+    const bool packed = packed_route(opts, 0);
+    if (opts.strategy == LEAP_STRATEGY_BATCHED && !packed && !is_nufft(opts.channel_sum) &&
+        !wave_route(ctx, md, ms, T, D, opts))
+        return 1;
+    if (packed && opts.pack_timesteps > 0) return 1;
+    const size_t rows = size_t(md.nbl) * T, samples = rows * md.channels;
+    const size_t cube = samples * std::max(vis_elem_bytes(ms), packed ? size_t(16) : size_t(0));
+    const size_t avg = size_t(md.nbl) * md.pols * 16 * D;
+    const size_t fit = std::min((size_t(1) << 30) / std::max<size_t>(1, cube), (size_t(256) << 20) / avg);
+    return uint32_t(std::max<size_t>(1, std::min<size_t>({fit, solutions, 4096})));
 }
 
 void check_metadata_matches(const leap_metadata& md, const leap_ms_view& ms) {
@@ -717,15 +768,17 @@ leap_metadata* create_metadata(leap_ctx* ctx, const leap_ms_view& ms, int32_t re
 // Device buffers one solution interval uses, reserved before a capture so the
 // captured sequence allocates nothing (the sizes rotate_directions and
 // invert_directions ask for).
-void reserve_solution(leap_ctx* ctx, const leap_metadata& md, uint32_t D, uint32_t T, const leap_options& opts) {
+void reserve_solution(leap_ctx* ctx, const leap_metadata& md, uint32_t D, uint32_t T, const leap_options& opts,
+                      uint32_t intervals = 1) {
     const int32_t K = md.A.rows, N = md.A.cols;
-    ctx->d_avg.reserve(size_t(md.nbl) * md.pols * 2 * D * sizeof(double));
+    ctx->d_avg.reserve(size_t(md.nbl) * md.pols * 2 * D * intervals * sizeof(double));
     if (use_packed(opts)) {
-        const uint32_t tc = pack_chunk(T, md.nbl, md.channels, opts);
-        ctx->d_packed.reserve(size_t(tc) * md.nbl * md.channels * (T > tc ? 2 : 1) * 2 * sizeof(double));
+        const uint32_t tc = intervals > 1 ? T : pack_chunk(T, md.nbl, md.channels, opts);
+        ctx->d_packed.reserve(size_t(tc) * intervals * md.nbl * md.channels * (T > tc ? 2 : 1) * 2 * sizeof(double));
     }
     if (opts.strategy == LEAP_STRATEGY_BATCHED)
         ctx->d_nufft_tail.reserve(nufft_tail_bytes(D));  // the NUFFT route's chunked last round
+    D *= intervals;  // the inversion takes every interval's directions alike
     ctx->d_cal1.reserve(size_t(N) * D * sizeof(double));
     ctx->d_cal.reserve(size_t(N) * D * sizeof(double));
     if (opts.precision == LEAP_PRECISION_MIXED) {
@@ -805,12 +858,13 @@ void calibrate_loop_graph(leap_ctx* ctx, const leap_metadata& md, const leap_ms_
     CapturedSequence* seq = nullptr;
     if (D > 0 && solutions > 0) {
         upload_directions(ctx, md, dirs, D);
-        reserve_solution(ctx, md, D, interval, opts);
+        const uint32_t group = interval_group(ctx, md, ms, interval, D, uint32_t(solutions), opts);
+        reserve_solution(ctx, md, D, interval, opts, group);
         int32_t tile = 0;
         if (opts.strategy == LEAP_STRATEGY_BATCHED) {
             const DeviceRows rows0 = stage_rows(ctx, ms, 0, interval * nbl);
             tile = batched_tile(ctx, md, ms, rows0, interval, D, opts);
-            ctx->last_direction_block = tile == kWaveTile ? horner_wave_tile(D, md.nbl, md.channels, 1) : tile;
+            ctx->last_direction_block = tile == kWaveTile ? horner_wave_tile(D, md.nbl, md.channels, group) : tile;
         }
         std::vector<uint64_t> key{uint64_t(uint32_t(tile))};
         key_common(key, ctx, opts);
@@ -821,11 +875,12 @@ void calibrate_loop_graph(leap_ctx* ctx, const leap_metadata& md, const leap_ms_
             seq->key = key;
             seq->d_cal.reserve(per_sol * size_t(solutions) * sizeof(double));
             capture(ctx, *seq, [&] {
-                for (int32_t s = 0; s < solutions; ++s) {
-                    const DeviceRows rows = stage_rows(ctx, ms, uint32_t(size_t(s) * interval * nbl),
-                                                       uint32_t(size_t(s + 1) * interval * nbl));
-                    const uint32_t ap = rotate_directions(ctx, md, ms, rows, interval, D, opts, tile, true);
-                    invert_directions(ctx, md, D, opts, nullptr, seq->d_cal.as<double>() + per_sol * size_t(s), ap);
+                for (uint32_t i = 0; i < uint32_t(solutions); i += group) {
+                    const uint32_t n = std::min(group, uint32_t(solutions) - i);
+                    const DeviceRows rows = stage_rows(ctx, ms, uint32_t(size_t(i) * interval * nbl),
+                                                       uint32_t(size_t(i + n) * interval * nbl));
+                    const uint32_t ap = rotate_directions(ctx, md, ms, rows, interval, D, opts, tile, true, n);
+                    invert_intervals(ctx, md, D, n, opts, ap, seq->d_cal.as<double>() + per_sol * size_t(i));
                 }
             });
             ctx->last_graph = 1;
@@ -877,12 +932,23 @@ void calibrate_loop(leap_ctx* ctx, const leap_metadata& md, const leap_ms_view& 
     ctx->last_graph = 0;
     begin_timing(ctx);
     if (D > 0) upload_directions(ctx, md, dirs, D);
-    ctx->h_cal.reserve(std::max<size_t>(1, size_t(N) * D) * sizeof(double));
+    const uint32_t group = interval_group(ctx, md, ms, interval, D, uint32_t(std::max(solutions, 0)), opts);
+    const size_t per_sol = size_t(N) * D;
+    ctx->h_cal.reserve(std::max<size_t>(1, per_sol * group) * sizeof(double));
     double* h_cal = ctx->h_cal.as<double>();
     for (int32_t s = 0; s < solutions; ++s) {  // :104
-        // :113-119 — rows [s * interval * nbl, +interval * nbl); the slice start is not added.
-        const uint32_t row_begin = uint32_t(size_t(s) * interval * nbl);
-        const uint32_t row_end = uint32_t(size_t(s + 1) * interval * nbl);
+        const uint32_t at = uint32_t(s) % group;
+        if (D > 0 && at == 0) {
+            // :113-119 — rows [s * interval * nbl, +interval * nbl); the slice start is not added.
+            const uint32_t n = std::min(group, uint32_t(solutions - s));
+            const DeviceRows rows = stage_rows(ctx, ms, uint32_t(size_t(s) * interval * nbl),
+                                               uint32_t(size_t(s + n) * interval * nbl), !packed_route(opts, 0));
+            const uint32_t ap = rotate_directions(ctx, md, ms, rows, interval, D, opts, 0, true, n);
+            invert_intervals(ctx, md, D, n, opts, ap);
+            LEAP_HIP(hipMemcpyAsync(h_cal, ctx->d_cal.ptr, per_sol * n * sizeof(double), hipMemcpyDeviceToHost,
+                                    ctx->stream));
+            LEAP_HIP(hipStreamSynchronize(ctx->stream));
+        }
         leap_solution sol{};
         sol.index = uint32_t(s);
         sol.start_epoch = ms.time[size_t(s) * interval * nbl];               // :107-109
@@ -890,15 +956,7 @@ void calibrate_loop(leap_ctx* ctx, const leap_metadata& md, const leap_ms_view& 
         sol.n_directions = D;
         sol.directions = dirs;
         sol.n_antennas = uint32_t(N);
-        sol.calibrations = h_cal;
-        if (D > 0) {
-            const DeviceRows rows = stage_rows(ctx, ms, row_begin, row_end, !packed_route(opts, 0));
-            const uint32_t ap = rotate_directions(ctx, md, ms, rows, interval, D, opts, 0, true);
-            invert_directions(ctx, md, D, opts, nullptr, nullptr, ap);
-            LEAP_HIP(hipMemcpyAsync(h_cal, ctx->d_cal.ptr, size_t(N) * D * sizeof(double),
-                                    hipMemcpyDeviceToHost, ctx->stream));
-            LEAP_HIP(hipStreamSynchronize(ctx->stream));
-        }
+        sol.calibrations = h_cal + per_sol * at;
         if (cb && cb(user, &sol) != 0) throw Error(LEAP_ERR_CALLBACK, "output callback requested a stop");
     }
     LEAP_HIP(hipStreamSynchronize(ctx->stream));

@@ -726,7 +726,7 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(ND == 
     volatile double* vacc = &s_red[wave][lane][0][0];
     const uint32_t npairs = C / 2;
     for (uint32_t t = wave; t < T; t += RP) {
-        const size_t row = size_t(t) * nbl + bl;
+        const size_t row = size_t(blockIdx.z) * T * nbl + size_t(t) * nbl + bl;  // z: solution interval
         const double u = uvw[3 * row], v = uvw[3 * row + 1], ww = uvw[3 * row + 2];
         const C2<double>* wr = w + row * C;
         double sf[ND];
@@ -809,7 +809,7 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(ND == 
                 re += s_red[r][lane][j][0];
                 im += s_red[r][lane][j][1];
             }
-            double* o = avg + (size_t(dj) * nbl + bl) * P * 2;
+            double* o = avg + ((size_t(blockIdx.z) * D + dj) * nbl + bl) * P * 2;
             if (accumulate) {
                 o[0] += re;
                 o[1] += im;
@@ -950,14 +950,17 @@ void launch_widen_c64(hipStream_t s, const void* in, size_t n, double* out) {
 bool packed_tile_supported(int32_t tile) { return tile == 641 || tile == 1282 || tile == 2564; }
 
 void launch_rotate_packed(hipStream_t s, int32_t tile, const double* w, const double* uvw, const double* dd,
-                          uint32_t D, uint32_t T, uint32_t nbl, uint32_t nbl_grid, uint32_t C, uint32_t P, double f0,
-                          double df, double* avg, int32_t accumulate) {
+                          uint32_t D, uint32_t T, uint32_t nbl, uint32_t nbl_grid, uint32_t C, uint32_t P,
+                          uint32_t pols_out, double f0, double df, double* avg, int32_t accumulate,
+                          uint32_t intervals) {
     if (nbl_grid == 0 || D == 0) return;
+    require(intervals == 1 || !accumulate, LEAP_ERR_INTERNAL, "several intervals are not accumulated");
+    P = pols_out;  // the packed rows hold pol 0; the kernel's P is the output's
     const double kappa0 = f0 / kSpeedOfLight;
     const double dkappa = df / kSpeedOfLight;
     const C2<double>* wp = reinterpret_cast<const C2<double>*>(w);
     const uint32_t db = uint32_t(tile / 10);
-    const dim3 grid(nbl_grid, (D + db - 1) / db);
+    const dim3 grid(nbl_grid, (D + db - 1) / db, intervals);
     switch (tile) {
         case 641: rotate_average_packed<1><<<grid, kThreads, 0, s>>>(wp, uvw, dd, D, T, nbl, C, P, kappa0, dkappa, avg, accumulate); break;
         case 1282: rotate_average_packed<2><<<grid, kThreads, 0, s>>>(wp, uvw, dd, D, T, nbl, C, P, kappa0, dkappa, avg, accumulate); break;

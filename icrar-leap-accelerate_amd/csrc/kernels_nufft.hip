@@ -10,7 +10,7 @@ void launch_rotate_nufft_f64(hipStream_t s, const nufft::NufftLaunch& l) {
     if (plan.N == N_ && plan.W == W_) {                                                                      \
         nufft::launch_nw<N_, W_, double>(s, l.tile, l.nbl_grid, l.src, l.src_pols, l.scale, l.uvw, l.dd, l.D, \
                                          l.T, l.nbl, l.C, l.P_out, l.args, l.avg, l.accumulate, l.tail,      \
-                                         l.tail_doubles);                                                    \
+                                         l.tail_doubles, l.intervals);                                                    \
         return;                                                                                              \
     }
     LEAP_NUFFT(256, 10)
@@ -73,7 +73,7 @@ bool nufft_cube_supported(int32_t vis_dtype, uint32_t P, bool w16) {
 void launch_rotate_nufft(hipStream_t s, int32_t tile, const NufftPlan& plan, const double* tables, const void* src,
                          bool cube, int32_t vis_dtype, const double* uvw, const double* dd, uint32_t D, uint32_t T,
                          uint32_t nbl, uint32_t nbl_grid, uint32_t C, uint32_t P, uint32_t P_out, double f0,
-                         double df, double* avg, int32_t accumulate, double* tail, size_t tail_bytes) {
+                         double df, double* avg, int32_t accumulate, double* tail, size_t tail_bytes, uint32_t intervals) {
     if (nbl_grid == 0 || D == 0) return;
     require(P_out >= 1, LEAP_ERR_INTERNAL, "NUFFT output needs at least pol 0");
     require(plan.N != 0 && plan.scale.size() == C, LEAP_ERR_INTERNAL, "NUFFT plan does not match the channel count");
@@ -90,7 +90,10 @@ void launch_rotate_nufft(hipStream_t s, int32_t tile, const NufftPlan& plan, con
     l.D = D;
     l.T = T;
     l.nbl = nbl;
+    require(intervals == 1 || (nbl_grid == nbl && !accumulate), LEAP_ERR_INTERNAL,
+            "several intervals are whole and not accumulated");
     l.nbl_grid = nbl_grid;
+    l.intervals = intervals;
     l.C = C;
     l.P_out = P_out;
     l.args.coef = tables;

@@ -10,7 +10,7 @@ void launch_rotate_nufft_f32(hipStream_t s, const nufft::NufftLaunch& l) {
     if (plan.N == N_ && plan.W == W_) {                                                                      \
         nufft::launch_nw<N_, W_, float>(s, l.tile, l.nbl_grid, l.src, l.src_pols, l.scale, l.uvw, l.dd, l.D,  \
                                         l.T, l.nbl, l.C, l.P_out, l.args, l.avg, l.accumulate, l.tail,       \
-                                        l.tail_doubles);                                                     \
+                                        l.tail_doubles, l.intervals);                                                     \
         return;                                                                                              \
     }
     LEAP_NUFFT(256, 8)

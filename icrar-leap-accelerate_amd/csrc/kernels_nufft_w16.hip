@@ -11,7 +11,7 @@ void launch_rotate_nufft_w16(hipStream_t s, const nufft::NufftLaunch& l) {
     if (plan.N == N_ && plan.W == 16) {                                                                        \
         nufft::launch_nw<N_, 16, double>(s, l.tile, l.nbl_grid, l.src, l.src_pols, l.scale, l.uvw, l.dd, l.D, \
                                          l.T, l.nbl, l.C, l.P_out, l.args, l.avg, l.accumulate, l.tail,        \
-                                         l.tail_doubles);                                                      \
+                                         l.tail_doubles, l.intervals);                                                      \
         return;                                                                                                \
     }
     LEAP_NUFFT(256)

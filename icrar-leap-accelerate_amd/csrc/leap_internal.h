@@ -361,13 +361,14 @@ void launch_scale_channels(hipStream_t s, double* x, size_t n, const double* sca
 // tables: the plan on the device, kNufftCoefDoubles coefficients (coef[j][m])
 // then the C precorrection factors.
 bool nufft_cube_supported(int32_t vis_dtype, uint32_t P, bool w16);
-// avg holds P_out pols per (direction, baseline) (pol 0 summed, the others
+// avg holds P_out pols per (interval, direction, baseline) (pol 0 summed, the others
 // set to zero unless accumulating); P is the cube's pol count.
 void launch_rotate_nufft(hipStream_t s, int32_t tile, const NufftPlan& plan, const double* tables, const void* src,
                          bool cube, int32_t vis_dtype, const double* uvw, const double* dd, uint32_t D, uint32_t T,
                          uint32_t nbl,
                          uint32_t nbl_grid, uint32_t C, uint32_t P, uint32_t P_out, double f0, double df,
-                         double* avg, int32_t accumulate, double* tail = nullptr, size_t tail_bytes = 0);
+                         double* avg, int32_t accumulate, double* tail = nullptr, size_t tail_bytes = 0,
+                         uint32_t intervals = 1);
 // Scratch for launch_rotate_nufft's chunked last round (D directions, a single
 // direction block): at most twice the resident workgroups x D complex sums.
 size_t nufft_tail_bytes(uint32_t D);
@@ -396,8 +397,9 @@ void launch_rotate_nufft_sets(hipStream_t s, int32_t tile, const NufftPlan& plan
                               const NufftSetDesc* sets, const uint32_t* items, uint32_t n_items);
 bool packed_tile_supported(int32_t tile);
 void launch_rotate_packed(hipStream_t s, int32_t tile, const double* w, const double* uvw, const double* dd,
-                          uint32_t D, uint32_t T, uint32_t nbl, uint32_t nbl_grid, uint32_t C, uint32_t P, double f0,
-                          double df, double* avg, int32_t accumulate);
+                          uint32_t D, uint32_t T, uint32_t nbl, uint32_t nbl_grid, uint32_t C, uint32_t P,
+                          uint32_t pols_out, double f0, double df, double* avg, int32_t accumulate,
+                          uint32_t intervals = 1);
 int32_t multi_blocks_per_cu(int32_t tile);
 // Kernel launchers (kernels_f64.hip)
 void launch_dd(hipStream_t s, double ra0, double dec0, const double* d_dirs, uint32_t D,
@@ -465,6 +467,8 @@ void launch_rotate_batched(hipStream_t s, int32_t precision, int32_t direction_b
 size_t bf16_planes_bytes(uint32_t rows, int32_t K);
 void launch_split_b(hipStream_t s, const double* B, int32_t K, int32_t N, void* planes);
 size_t mfma_partial_floats(int32_t K, uint32_t D, int32_t N);
+// Whether D directions run as one K-split of the whole output, whose sums do not depend on D.
+bool mfma_full_output(uint32_t D, int32_t N);
 // Where the mixed GEMM's A operand comes from: avgData and the antenna pairs of A's rows.
 struct DeltaSource {
     const double* avg;

@@ -917,8 +917,9 @@ __device__ __forceinline__ void nufft_rows(const void* wr, const LEAP_GLOBAL dou
     }
 }
 
-// One launch over a set's baselines (blockIdx.x, resolved through the span)
-// and direction blocks of 64 NDL (blockIdx.y).
+// One launch over a set's baselines (blockIdx.x, resolved through the span),
+// direction blocks of 64 NDL (blockIdx.y) and consecutive solution intervals of
+// T timesteps (blockIdx.z).  avg[interval][direction][baseline][Pout].
 template <int N, int W, int NDL, int SP, int CPL, typename F>
 __global__ __launch_bounds__(kWave) void rotate_average_nufft(const void* __restrict__ w,
                                                               const LEAP_GLOBAL double* __restrict__ scale,
@@ -939,9 +940,13 @@ __global__ __launch_bounds__(kWave) void rotate_average_nufft(const void* __rest
     const uint32_t bl = span.bl_base + (span.chunks > 1 ? item / span.chunks : item);
     const uint32_t t_begin = uint32_t(uint64_t(chunk) * T / max(span.chunks, 1u));
     const uint32_t t_count = uint32_t(uint64_t(chunk + 1) * T / max(span.chunks, 1u)) - t_begin;
-    const void* wr = Source<N, SP, CPL>::advance(w, size_t(t_begin) * nbl, C);
-    const LEAP_GLOBAL double* uvr = uvw + size_t(t_begin) * nbl * 3;
-    LEAP_GLOBAL double* out = mode == kNufftPartial ? avg + size_t(item) * D * 2 : avg + size_t(bl) * Pout * 2;
+    const size_t row0 = (size_t(blockIdx.z) * T + t_begin) * nbl;
+    const void* wr = Source<N, SP, CPL>::advance(w, row0, C);
+    const LEAP_GLOBAL double* uvr = uvw + row0 * 3;
+    LEAP_GLOBAL double* out = mode == kNufftPartial ? avg + size_t(item) * D * 2
+                                                    : avg + (size_t(blockIdx.z) * D * nbl + bl) * Pout * 2;
+    // Opaque, so that the row loop keeps the resolved pointers instead of their parts.
+    asm volatile("" : "+s"(wr), "+s"(uvr), "+s"(out));
     const uint32_t dstride = mode == kNufftPartial ? 2u : nbl * Pout * 2;  // doubles between directions
     nufft_rows<N, W, NDL, SP, CPL, F>(wr, scale, uvr, dd, D, t_count, nbl, bl, C, args, blockIdx.y * (kWave * NDL),
                                       out, dstride, mode, Pout, s_g, s_turn, lane);
@@ -981,15 +986,15 @@ uint32_t resident_workgroups(K kernel) {
 // rounds of resident workgroups, the whole rounds run as usual and the
 // remaining baselines' rows are split into chunks so that the last round is
 // full (and short): their partial sums go to the tail scratch and are added by
-// nufft_tail_sum.  Not for accumulating launches.
+// nufft_tail_sum.  Not for accumulating launches or several intervals.
 template <int N, int W, int NDL, int SP, int CPL, typename F>
 void launch_nufft_tile(hipStream_t s, uint32_t nbl_grid, const void* w, const LEAP_GLOBAL double* gs,
                        const LEAP_GLOBAL double* gu, const LEAP_GLOBAL double* gd, uint32_t D, uint32_t T, uint32_t nbl,
                        uint32_t C, uint32_t Pout, const NufftArgs& a, LEAP_GLOBAL double* ga, int32_t accumulate,
-                       double* tail, size_t tail_doubles) {
+                       double* tail, size_t tail_doubles, uint32_t intervals) {
     auto* kernel = rotate_average_nufft<N, W, NDL, SP, CPL, F>;
     const uint32_t ny = (D + kWave * NDL - 1) / (kWave * NDL);
-    if (tail && !accumulate && ny == 1 && T >= 2) {
+    if (tail && !accumulate && intervals == 1 && ny == 1 && T >= 2) {
         static const uint32_t slots = resident_workgroups(kernel);
         const uint32_t full = nbl_grid / slots * slots, rem = nbl_grid - full;
         const uint32_t chunks = rem ? std::min(T, (slots + rem - 1) / rem) : 0;
@@ -1011,7 +1016,7 @@ void launch_nufft_tile(hipStream_t s, uint32_t nbl_grid, const void* w, const LE
             return;
         }
     }
-    kernel<<<dim3(nbl_grid, ny), kWave, 0, s>>>(w, gs, gu, gd, D, T, nbl, C, Pout, a, ga,
+    kernel<<<dim3(nbl_grid, ny, intervals), kWave, 0, s>>>(w, gs, gu, gd, D, T, nbl, C, Pout, a, ga,
                                                accumulate ? kNufftAccumulate : kNufftSet, NufftSpan{0, 1});
 }
 
@@ -1076,12 +1081,13 @@ void dispatch_nufft(int32_t tile, int32_t src_pols, uint32_t C, Fn&& fn) {
 template <int N, int W, typename F>
 void launch_nw(hipStream_t s, int32_t tile, uint32_t nbl_grid, const void* w, int32_t src_pols, const double* scale,
                const double* uvw, const double* dd, uint32_t D, uint32_t T, uint32_t nbl, uint32_t C, uint32_t Pout,
-               const NufftArgs& a, double* avg, int32_t accumulate, double* tail, size_t tail_doubles) {
+               const NufftArgs& a, double* avg, int32_t accumulate, double* tail, size_t tail_doubles,
+               uint32_t intervals) {
     dispatch_nufft<N, W, F>(tile, src_pols, C, [&](auto ndl, auto sp, auto cpl) {
         launch_nufft_tile<N, W, decltype(ndl)::value, decltype(sp)::value, decltype(cpl)::value, F>(
             s, nbl_grid, w, (const LEAP_GLOBAL double*)scale, (const LEAP_GLOBAL double*)uvw,
             (const LEAP_GLOBAL double*)dd, D, T, nbl, C, Pout, a, (LEAP_GLOBAL double*)avg, accumulate, tail,
-            tail_doubles);
+            tail_doubles, intervals);
     });
 }
 
@@ -1139,6 +1145,7 @@ struct NufftLaunch {
     int32_t accumulate;
     double* tail;
     size_t tail_doubles;
+    uint32_t intervals;
 };
 
 }  // namespace nufft
