@@ -480,7 +480,7 @@ uint32_t rotate_directions(leap_ctx* ctx, const leap_metadata& md, const leap_ms
     ctx->d_avg.reserve(per_dir * D * intervals * sizeof(double));
     if (wave) {
         require(rows.vis != nullptr, LEAP_ERR_INTERNAL, "visibilities were not staged");
-        ctx->last_direction_block = horner_wave_tile(D, md.nbl, md.channels, intervals);
+        ctx->last_direction_block = horner_wave_tile(D, md.nbl, intervals);
         record_rotate_begin(ctx);
         launch_horner_wave(ctx->stream, {rows.vis, ms.vis_dtype, rows.uvw, ctx->d_dd.as<double>(), D, T, intervals,
                                          md.nbl, md.channels, md.pols, avg_pols, md.freq_start_hz, md.freq_inc_hz,
@@ -864,7 +864,7 @@ void calibrate_loop_graph(leap_ctx* ctx, const leap_metadata& md, const leap_ms_
         if (opts.strategy == LEAP_STRATEGY_BATCHED) {
             const DeviceRows rows0 = stage_rows(ctx, ms, 0, interval * nbl);
             tile = batched_tile(ctx, md, ms, rows0, interval, D, opts);
-            ctx->last_direction_block = tile == kWaveTile ? horner_wave_tile(D, md.nbl, md.channels, group) : tile;
+            ctx->last_direction_block = tile == kWaveTile ? horner_wave_tile(D, md.nbl, group) : tile;
         }
         std::vector<uint64_t> key{uint64_t(uint32_t(tile))};
         key_common(key, ctx, opts);
@@ -2034,28 +2034,21 @@ extern "C" int leap_hip_residual_loss_grad(leap_ctx* ctx, const leap_metadata* m
             uvw = d_uvwp.as<double>();
         }
         // forward avgData (pol 0), FP64
-        const size_t per_dir = size_t(nbl) * md->pols * 2;
-        ctx->d_avg.reserve(per_dir * D * sizeof(double));
-        const int32_t tile = D <= 16 ? 162 : D <= 32 ? 321 : D <= 64 ? 641 : D <= 128 ? 1282 : 2562;
+        ctx->d_avg.reserve(size_t(D) * nbl * 2 * sizeof(double));
         if (row_sums) ctx->d_adj_q.reserve(size_t(R) * D * 4 * sizeof(double));
         LEAP_HIP(hipEventRecord(ctx->ev_grad[0], s));
-        if (row_sums)
-            launch_rotate_forward_q(s, tile, rows.vis, ms->vis_dtype, uvw, ctx->d_dd.as<double>(), D, T, nbl,
-                                    md->channels, md->pols, md->freq_start_hz, md->freq_inc_hz,
-                                    ctx->d_avg.as<double>(), ctx->d_adj_q.as<double>());
-        else
-            launch_rotate_batched(s, LEAP_PRECISION_FP64, tile, false, rows.vis, ms->vis_dtype, uvw,
-                                  ctx->d_dd.as<double>(), D, T, nbl, nbl, md->channels, md->pols, md->freq_start_hz,
-                                  md->freq_inc_hz, ctx->d_avg.as<double>(), 0);
+        launch_horner_wave(s, {rows.vis, ms->vis_dtype, uvw, ctx->d_dd.as<double>(), D, T, 1, nbl, md->channels,
+                               md->pols, 1, md->freq_start_hz, md->freq_inc_hz, ctx->d_avg.as<double>(),
+                               row_sums ? ctx->d_adj_q.as<double>() : nullptr});
         LEAP_HIP(hipEventRecord(ctx->ev_grad[1], s));
         ctx->last_grad_adjoint_ms = 0.0;
         // the inversion (CpuLeapCalibrator.cc:159-178) by the calibration's own kernels
         leap_options inv{};
-        invert_directions(ctx, *md, D, inv);
+        invert_directions(ctx, *md, D, inv, nullptr, nullptr, 1);
         // pol 0 of avgData and its arguments
         DeviceBuffer& d_avg0 = ctx->d_adj_avg0;
         d_avg0.reserve(size_t(D) * nbl * 3 * sizeof(double));
-        launch_gather_pol0(s, ctx->d_avg.as<double>(), D * nbl, md->pols, d_avg0.as<double>());
+        launch_gather_pol0(s, ctx->d_avg.as<double>(), D * nbl, 1, d_avg0.as<double>());
         // loss and the adjoint of the inversion, on the device
         const int32_t K = md->A.rows, K1 = md->A1.rows, nI = K - 1;
         const size_t rb = size_t(std::max(1, (nI + 255) / 256));

@@ -8,7 +8,7 @@
 //                = Re(conj(abar) * i * e0 * (kappa0 P(z) + dkappa z P'(z)))
 // with e0 = exp(i sf kappa0), z = exp(i sf dkappa), P(z) = sum_c v_c z^c.  When
 // the forward pass has kept each row's sums e0 P(z) and e0 z P'(z) (32 bytes per
-// row and direction, rotate_average_horner64_q), adjoint_q_kernel reads them
+// row and direction, horner_wave_kernel), adjoint_q_kernel reads them
 // and the cube is not read again; otherwise rotate_adjoint_kernel evaluates P
 // and P' together by Horner's rule (p' <- p' z + p; p <- p z + v) from the
 // cube.  Then
@@ -213,7 +213,7 @@ __global__ __launch_bounds__(kThreads) void rotate_adjoint_kernel(
 }
 
 // The same outputs from the forward pass's per-row sums q[row][d] = (e0 P(z),
-// e0 z P'(z)) (rotate_average_horner64 with row sums), so the cube is not read
+// e0 z P'(z)) (horner_wave_kernel's q), so the cube is not read
 // again: s1 = kappa0 q0 + dkappa q1 is the sum above.  Lanes, rows and the
 // reductions as in rotate_adjoint_kernel.
 template <int DL, int ND>

@@ -413,10 +413,11 @@ struct HornerWave {
     const double* dd;  // [D][3][3]
     uint32_t D, T, intervals, nbl, C, P, pols_out;
     double f0, df;
-    double* avg;  // [intervals][D][nbl][pols_out]
+    double* avg;          // [intervals][D][nbl][pols_out]
+    double* q = nullptr;  // each row's sums [row][D] = (e0 P(z), e0 z P'(z)), or null
 };
 // Directions of a wave * 10 + directions of a lane.
-int32_t horner_wave_tile(uint32_t D, uint32_t nbl, uint32_t C, uint32_t intervals);
+int32_t horner_wave_tile(uint32_t D, uint32_t nbl, uint32_t intervals);
 void launch_horner_wave(hipStream_t s, const HornerWave& h);
 // The per-direction FP64 rotate/average of D directions over consecutive solution intervals
 // of T timesteps each, from the first interval's first row.
@@ -482,13 +483,7 @@ void launch_perturb_uvw(hipStream_t s, const double* uvw0, const double* M, cons
 void launch_rotate_adjoint(hipStream_t s, const void* vis, int32_t vis_dtype, const double* uvw, const double* dd,
                            const double* abar, uint32_t D, uint32_t T, uint32_t nbl, uint32_t C, uint32_t P, double f0,
                            double df, double* g_uvw, double* g_dz_partial);
-// The residual-loss forward pass that also keeps each row's sums
-// q[row][d] = (e0 P(z), e0 z P'(z)) (4 doubles; kernels_batched.hip), pol 0 of
-// avgData as launch_rotate_batched in FP64; tiles 162, 321, 641, 1282, 2562.
-void launch_rotate_forward_q(hipStream_t s, int32_t tile, const void* vis, int32_t vis_dtype, const double* uvw,
-                             const double* dd, uint32_t D, uint32_t T, uint32_t nbl, uint32_t C, uint32_t P, double f0,
-                             double df, double* avg, double* q);
-// launch_rotate_adjoint's outputs from those row sums (no pass over the cube).
+// launch_rotate_adjoint's outputs from the row sums of HornerWave::q (no pass over the cube).
 void launch_adjoint_q(hipStream_t s, const double* q, const double* uvw, const double* dd, const double* abar,
                       uint32_t D, uint32_t T, uint32_t nbl, double f0, double df, double* g_uvw,
                       double* g_dz_partial);

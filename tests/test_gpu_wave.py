@@ -1,5 +1,5 @@
-"""The wave-at-a-time Horner rotate/average: its tiles (8 to 256 directions a wave, direction blocks
-that are not full), rows of several baselines and of several timesteps, channel chunks that are
+"""The wave-at-a-time rotate/average: its tiles (one to four directions a lane, direction blocks
+that are not full), rows of several baselines and of several timesteps, channel blocks that are
 partial, odd or single, and every cube type, against the oracle (avgData within 1e-12 of its
 largest magnitude, the bar of the other FP64 batched routes)."""
 import numpy as np
@@ -30,15 +30,15 @@ def on_device(leap, ctx):
 @pytest.mark.parametrize("dtype", [np.complex64, np.complex128])
 @pytest.mark.parametrize("n_ant,T,C,P,D", [
     (4, 1, 1, 1, 1),       # one sample per baseline
-    (7, 3, 33, 2, 8),      # 16 rows a wave, several baselines and timesteps, chunks of 8 and 16 channels
-    (40, 17, 9, 3, 9),     # a direction past a full block
-    (91, 1, 31, 4, 16),    # 4186 baselines of one timestep: eight baselines a wave
-    (91, 2, 70, 1, 30),    # four rows a wave, two chunks
-    (91, 3, 65, 4, 64),    # two rows a wave, a chunk and one channel
-    (65, 2, 150, 2, 130),  # narrow tiles (2145 baselines), 17 blocks
-    (91, 2, 40, 4, 100),   # 128 directions a wave
-    (91, 1, 24, 2, 250),   # four directions a lane
-    (91, 1, 20, 1, 300),   # two blocks of 150
+    (7, 3, 33, 2, 8),      # several timesteps of a baseline, a channel past two blocks
+    (40, 17, 9, 3, 9),     # a baseline's timesteps over four waves
+    (91, 1, 31, 4, 16),    # 4186 baselines of one timestep: four baselines a wave
+    (91, 2, 70, 1, 30),    # two directions a lane, two chunks
+    (91, 3, 65, 4, 64),    # four directions a lane, a block and one channel
+    (65, 2, 150, 2, 130),  # three blocks of three directions a lane
+    (91, 2, 40, 4, 100),   # two blocks of 50
+    (91, 1, 24, 2, 250),   # four blocks
+    (91, 1, 20, 1, 300),   # five blocks of 60
 ])
 def test_wave_horner_edges(leap, ctx, oracle, on_device, dtype, n_ant, T, C, P, D):
     print(f"wave Horner: {n_ant} antennas, {T} t, {C} ch, {P} pols, {D} directions, {np.dtype(dtype).name}", flush=True)
@@ -55,3 +55,36 @@ def test_wave_horner_edges(leap, ctx, oracle, on_device, dtype, n_ant, T, C, P, 
         want = omd.rotate(dirs[d])
         assert np.abs(got[d, :, 0] - want[:, 0]).max() <= 1e-12 * np.abs(want[:, 0]).max(), d
     assert not got[:, :, 1:].any()
+
+
+@pytest.mark.parametrize("dtype", [np.complex64, np.complex128])
+@pytest.mark.parametrize("n_ant,T,C,P,D", [
+    (5, 1, 1, 1, 1),     # one channel: the derivative is zero
+    (7, 3, 33, 2, 9),    # a channel past two blocks
+    (9, 5, 70, 3, 16),   # timesteps past the four waves' rows
+    (12, 2, 130, 4, 17), # direction blocks that are not full
+    (12, 1, 9, 4, 256),  # the most directions
+])
+def test_wave_row_sums_edges(leap, ctx, oracle, on_device, dtype, n_ant, T, C, P, D):
+    """The residual loss and its gradient from the row sums, and the loss alone, against the oracle
+    at the bars of the other gradient tests (loss 1e-11 relative, gradients 1e-7 of the largest)."""
+    print(f"row sums: {n_ant} antennas, {T} t, {C} ch, {P} pols, {D} directions, {np.dtype(dtype).name}", flush=True)
+    s = leap.SynthMS(n_antennas=n_ant, n_timesteps=T, n_channels=C, n_pols=P, nan_fraction=0.003, seed=C + D)
+    s.fill_host(dtype)
+    ms = s.host_dict()
+    view = on_device(ms)
+    md = ctx.metadata(view)
+    rng = np.random.default_rng(D)
+    dirs = np.asarray(ms["phase_centre"]) + rng.uniform(-0.02, 0.02, (D, 2))
+    off, dp = rng.normal(0, 1e-4, (D, 2)), rng.normal(0, 0.01, (n_ant, 3))
+    want, want_off, want_ant = oracle.loss_grad(ms, dirs, s.enu_to_uvw, off, dp)
+    ctx.set_adjoint_mode(2)
+    try:
+        loss, g_off, g_ant = md.loss_grad(view, dirs, s.enu_to_uvw, off, dp)
+    finally:
+        ctx.set_adjoint_mode(0)
+    alone, _, _ = md.loss_grad(view, dirs, s.enu_to_uvw, off, dp, want_grad=False)
+    assert abs(loss - want) <= 1e-11 * abs(want)
+    assert abs(alone - want) <= 1e-11 * abs(want)
+    assert np.abs(g_off - want_off).max() <= 1e-7 * np.abs(want_off).max()
+    assert np.abs(g_ant - want_ant).max() <= 1e-7 * np.abs(want_ant).max()
