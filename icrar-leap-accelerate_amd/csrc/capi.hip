@@ -196,20 +196,35 @@ bool use_packed(const leap_options& opts) {
            !(opts.precision == LEAP_PRECISION_MIXED && opts.fp32_blocks) && !opts.direct_cube;
 }
 
-// The batched pol-0 Horner route for a tuned call on a device-resident cube: the pack pass (every
-// pol read, pol 0 written as FP64) pays only when the FP64 work is large enough.  Rates measured on
-// MI355X: pack 5.2 TB/s; packed Horner 32 / 50 / 55 TFLOP/s with 1 / 2 / 4 directions per lane (up
-// to 64, 128, more directions); the wave kernel straight from the cube 5.7 TB/s and 50 TFLOP/s
-// (complex64) or 47 (complex128), both less by the phasors of a row (20 channels' worth: 48
-// channels, 256 directions 37 TFLOP/s, 384 channels 49).  So the pack pays from about 800
-// directions on complex64.  Host-resident cubes always take the packed route (pol 0 only crosses
-// the bus).
+// Whether an automatic FP64 call on a device cube takes the folded Horner kernel (kernels_wave.hip)
+// where the width-16 NUFFT is the other choice.  Both read the cube once; up to three directions a
+// lane the folded sums run at the cube's bytes and beside the NUFFT's transform a row costs less.
+// 256 stations, 6 t, FP64, folded against NUFFT: 96 channels of complex64 137 against 290 us with 32
+// directions, 160 against 294 with 48, 195 against 284 with 64; 384 channels 472 against 615, 520
+// against 635, 625 against 634; complex128 911 against 999, 886 against 1027.  Sets of few rows
+// leave it without waves where the NUFFT splits a baseline's rows (30 antennas, 10 t, 384 channels of
+// complex128, 48 directions: 52 against 44 us; 32 directions 38 against 44), and below 2,048 rows
+// both take about ten microseconds.  The mixed-precision NUFFT (width 10) keeps its calls: another
+// route would move its results by up to 2e-9 of themselves.
+bool folded_beats_nufft(uint32_t rows, uint32_t D) {
+    return (D <= 32 && rows >= 2048) || (D <= 48 && rows >= 16384);
+}
+
+// The route of a batched call.  Horner calls on a device-resident cube that name no tile go straight
+// from the cube: the folded kernel costs less than the packed kernel alone from 48 channels and 256
+// directions (45 against 39 TFLOP/s of direct sums) to 384 channels (70 against 55), so the pack
+// pass never pays.  With a lane_directions named (tiles of kernels_batched.hip and the packed kernel)
+// it pays from the rates measured on those: pack 5.2 TB/s, packed Horner 32 / 50 / 55 TFLOP/s up to
+// 64, 128, more directions, from the cube 6.4 TB/s and 30 or 51 (45 on complex128).  Host-resident
+// cubes always take the packed route (pol 0 only crosses the bus).
 leap_options routed(const leap_options& o, const leap_ms_view& ms, uint32_t T, uint32_t D) {
     leap_options r = o;
     if (r.channel_sum == LEAP_CHANNEL_SUM_AUTO) {
         const bool fp64 = r.precision == LEAP_PRECISION_FP64;
+        const bool folded = fp64 && ms.vis_on_device && r.direction_block == 0 && r.lane_directions == 0 &&
+                            r.pack_timesteps == 0 && folded_beats_nufft(T * ms.num_baselines, D);
         const bool nufft = use_packed(r) && nufft_supported(ms.num_channels) &&
-                           ms.num_channels >= kNufftMinChannels && D >= kNufftMinDirections;
+                           ms.num_channels >= kNufftMinChannels && D >= kNufftMinDirections && !folded;
         r.channel_sum = !nufft ? LEAP_CHANNEL_SUM_HORNER : fp64 ? LEAP_CHANNEL_SUM_NUFFT_W16 : LEAP_CHANNEL_SUM_NUFFT;
     }
     if (is_nufft(r.channel_sum)) {
@@ -228,14 +243,16 @@ leap_options routed(const leap_options& o, const leap_ms_view& ms, uint32_t T, u
         return r;
     }
     if (!use_packed(o) || o.direction_block != 0 || !ms.vis_on_device) return r;
+    if (o.lane_directions == 0) {
+        r.direct_cube = 1;
+        return r;
+    }
     const double rc = double(T) * ms.num_baselines * ms.num_channels;  // (row, channel)s
     const double s = ms.vis_dtype == LEAP_VIS_C64 ? 8.0 : 16.0;
     const double flops = 8.0 * rc * D;
-    const double rows = double(ms.num_channels) / (ms.num_channels + 20.0);
-    const double packed =
-        rc * (ms.num_pols * s + 16.0) / 5.2e12 + flops / (rows * (D > 128 ? 55e12 : D > 64 ? 50e12 : 32e12));
-    const double direct = std::max(rc * ms.num_pols * s / 5.7e12,
-                                   flops / (rows * (ms.vis_dtype == LEAP_VIS_C64 ? 50e12 : 47e12)));
+    const double packed = rc * (ms.num_pols * s + 16.0) / 5.2e12 + flops / (D > 128 ? 55e12 : D > 64 ? 50e12 : 32e12);
+    const double direct_rate = D > 128 ? (ms.vis_dtype == LEAP_VIS_C64 ? 51e12 : 45e12) : 30e12;
+    const double direct = std::max(rc * ms.num_pols * s / 6.4e12, flops / direct_rate);
     if (packed > direct) r.direct_cube = 1;
     return r;
 }
@@ -804,6 +821,7 @@ void key_common(std::vector<uint64_t>& k, const leap_ctx* ctx, const leap_option
                        uint64_t(opts.fp32_blocks), uint64_t(opts.direct_cube), uint64_t(opts.pack_timesteps),
                        uint64_t(opts.channel_sum),
                        key_ptr(ctx->d_packed.ptr),
+                       key_ptr(ctx->d_nufft_tail.ptr),
                        key_ptr(ctx->d_dd.ptr), key_ptr(ctx->d_avg.ptr),
                        key_ptr(ctx->d_cal1.ptr), key_ptr(ctx->d_sums.ptr),
                        key_ptr(ctx->d_cal.ptr), key_ptr(ctx->d_partial.ptr), key_ptr(ctx->d_a_planes.ptr)});

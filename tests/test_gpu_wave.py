@@ -88,3 +88,31 @@ def test_wave_row_sums_edges(leap, ctx, oracle, on_device, dtype, n_ant, T, C, P
     assert abs(alone - want) <= 1e-11 * abs(want)
     assert np.abs(g_off - want_off).max() <= 1e-7 * np.abs(want_off).max()
     assert np.abs(g_ant - want_ant).max() <= 1e-7 * np.abs(want_ant).max()
+
+
+@pytest.mark.parametrize("n_ant,T,P,D,precision,route", [
+    (64, 1, 4, 32, 0, 1),    # 2080 rows
+    (64, 1, 4, 33, 0, 4),
+    (63, 1, 4, 32, 0, 4),    # 2016 rows
+    (130, 2, 2, 48, 0, 1),   # 17030 rows
+    (130, 2, 2, 49, 0, 4),
+    (90, 4, 1, 48, 0, 4),    # 16380 rows
+    (64, 1, 3, 16, 0, 1),    # a pol count the NUFFT packs
+    (64, 1, 4, 32, 1, 2),    # mixed precision keeps its NUFFT
+])
+def test_automatic_route_of_device_cubes(leap, ctx, on_device, n_ant, T, P, D, precision, route):
+    """The automatic channel sums at the borders of the rule, as close to the other route's as the
+    routes of forced calls are (1e-12 of the largest magnitude in FP64, 1e-5 mixed)."""
+    print(f"automatic route: {n_ant} antennas, {T} t, {P} pols, {D} directions", flush=True)
+    s = leap.SynthMS(n_antennas=n_ant, n_timesteps=T, n_channels=96, n_pols=P, nan_fraction=0.003, seed=D)
+    s.fill_host(np.complex64)
+    ms = s.host_dict()
+    view = on_device(ms)
+    md = ctx.metadata(view)
+    dirs = np.asarray(ms["phase_centre"]) + np.random.default_rng(D).uniform(-0.03, 0.03, (D, 2))
+    got = md.rotate(view, dirs, opts=leap.options(strategy=1, precision=precision))
+    assert ctx.last_route()[0] == route
+    other = md.rotate(view, dirs, opts=leap.options(strategy=1, precision=precision,
+                                                    channel_sum=1 if route != 1 else 4))
+    bar = 1e-5 if precision else 1e-12
+    assert np.abs(got[:, :, 0] - other[:, :, 0]).max() <= bar * np.abs(other[:, :, 0]).max()
