@@ -210,6 +210,8 @@ bool folded_beats_nufft(uint32_t rows, uint32_t D) {
     return (D <= 32 && rows >= 2048) || (D <= 48 && rows >= 16384);
 }
 
+bool names_no_tile(const leap_options& opts) { return opts.direction_block == 0 && opts.lane_directions == 0; }
+
 // The route of a batched call.  Horner calls on a device-resident cube that name no tile go straight
 // from the cube: the folded kernel costs less than the packed kernel alone from 48 channels and 256
 // directions (45 against 39 TFLOP/s of direct sums) to 384 channels (70 against 55), so the pack
@@ -221,8 +223,8 @@ leap_options routed(const leap_options& o, const leap_ms_view& ms, uint32_t T, u
     leap_options r = o;
     if (r.channel_sum == LEAP_CHANNEL_SUM_AUTO) {
         const bool fp64 = r.precision == LEAP_PRECISION_FP64;
-        const bool folded = fp64 && ms.vis_on_device && r.direction_block == 0 && r.lane_directions == 0 &&
-                            r.pack_timesteps == 0 && folded_beats_nufft(T * ms.num_baselines, D);
+        const bool folded = fp64 && ms.vis_on_device && names_no_tile(r) && r.pack_timesteps == 0 &&
+                            folded_beats_nufft(T * ms.num_baselines, D);
         const bool nufft = use_packed(r) && nufft_supported(ms.num_channels) &&
                            ms.num_channels >= kNufftMinChannels && D >= kNufftMinDirections && !folded;
         r.channel_sum = !nufft ? LEAP_CHANNEL_SUM_HORNER : fp64 ? LEAP_CHANNEL_SUM_NUFFT_W16 : LEAP_CHANNEL_SUM_NUFFT;
@@ -282,8 +284,7 @@ bool wave_route(const leap_ctx* ctx, const leap_metadata& md, const leap_ms_view
                 const leap_options& opts) {
     return opts.strategy == LEAP_STRATEGY_BATCHED && opts.channel_sum == LEAP_CHANNEL_SUM_HORNER &&
            opts.direct_cube && !opts.all_pols && !(opts.precision == LEAP_PRECISION_MIXED && opts.fp32_blocks) &&
-           opts.direction_block == 0 && opts.lane_directions == 0 &&
-           ctx->tuned.find(tune_key(md, ms, T, D, opts)) == ctx->tuned.end();
+           names_no_tile(opts) && ctx->tuned.find(tune_key(md, ms, T, D, opts)) == ctx->tuned.end();
 }
 
 // Direction block for the batched kernel: the fastest of the candidates on a
@@ -820,7 +821,8 @@ void key_common(std::vector<uint64_t>& k, const leap_ctx* ctx, const leap_option
     k.insert(k.end(), {uint64_t(opts.precision), uint64_t(opts.strategy), uint64_t(opts.all_pols),
                        uint64_t(opts.fp32_blocks), uint64_t(opts.direct_cube), uint64_t(opts.pack_timesteps),
                        uint64_t(opts.channel_sum),
-                       key_ptr(ctx->d_packed.ptr),
+                       uint64_t(uint32_t(opts.direction_block)), uint64_t(uint32_t(opts.lane_directions)),
+                       uint64_t(uint32_t(opts.workgroups_per_cu)), key_ptr(ctx->d_packed.ptr),
                        key_ptr(ctx->d_nufft_tail.ptr),
                        key_ptr(ctx->d_dd.ptr), key_ptr(ctx->d_avg.ptr),
                        key_ptr(ctx->d_cal1.ptr), key_ptr(ctx->d_sums.ptr),
@@ -1035,6 +1037,8 @@ struct NufftGroup {
     int32_t tile = 0;
     std::vector<NufftSetDesc> sets;
     std::vector<uint32_t> items;
+    const leap_metadata* md = nullptr;  // of the first set
+    int32_t vis_dtype = 0;
 };
 
 // The channel sums a set of a multi-set call takes: 0 (Horner) or the NUFFT
@@ -1043,7 +1047,8 @@ struct NufftGroup {
 // complex128 for the width-16 kernel, with 1, 2 or 4 pols), by the single-set
 // automatic rule (96..512 channels, 16 or more directions) unless the NUFFT is
 // asked for.
-int32_t set_nufft_route(const leap_options& opts, const leap_metadata& md, const leap_ms_view& ms, uint32_t D) {
+int32_t set_nufft_route(const leap_options& opts, const leap_metadata& md, const leap_ms_view& ms, uint32_t D,
+                        uint32_t interval) {
     if (D == 0) return 0;
     int32_t cs = opts.channel_sum;
     if (cs == LEAP_CHANNEL_SUM_AUTO)
@@ -1058,7 +1063,17 @@ int32_t set_nufft_route(const leap_options& opts, const leap_metadata& md, const
                     "pols at an aligned address");
         return cs;
     }
+    if (opts.precision == LEAP_PRECISION_FP64 && names_no_tile(opts) && folded_beats_nufft(interval * md.nbl, D))
+        return 0;
     return cube_ok && md.channels >= kNufftMinChannels && D >= kNufftMinDirections ? cs : 0;
+}
+
+// Whether a Horner set of a multi-set call gets a launch of the folded kernel of its own instead of a
+// place in the shared launch of Horner tiles: where no tile is named and the set's rows give the chip
+// two waves per SIMD.  128 antennas, 14 t, 48 channels of complex64, 64 directions: 81 us against 151,
+// and the host plans no schedule of the set's 8,256 work items (0.4 ms).
+bool own_launch(const leap_options& opts, uint32_t rows) {
+    return names_no_tile(opts) && opts.workgroups_per_cu == 0 && rows >= 8192;
 }
 
 // NUFFT tile of a multi-set launch: the caller's when it is a NUFFT tile,
@@ -1076,12 +1091,13 @@ void plan_nufft_group(NufftGroup& g, const leap_options& opts) {
     uint32_t max_d = 0;
     for (const NufftSetDesc& d : g.sets) max_d = std::max(max_d, d.D);
     g.tile = nufft_group_tile(opts, max_d);
+    g.items.clear();
+    if (g.sets.size() == 1) return;  // launched as a single set
     const uint32_t per_block = 64u * uint32_t(g.tile % 10);
     require(g.sets.size() <= 0xffff, LEAP_ERR_RANGE, "too many sets for one NUFFT launch");
     std::vector<uint32_t> order(g.sets.size());
     for (uint32_t i = 0; i < order.size(); ++i) order[i] = i;
     std::stable_sort(order.begin(), order.end(), [&](uint32_t a, uint32_t b) { return g.sets[a].T > g.sets[b].T; });
-    g.items.clear();
     for (uint32_t s : order) {
         const NufftSetDesc& d = g.sets[s];
         const uint32_t blocks = (d.D + per_block - 1) / per_block;
@@ -1096,7 +1112,10 @@ void plan_nufft_group(NufftGroup& g, const leap_options& opts) {
 }
 
 // A round of a multi-set call: the Horner launch's tables and each NUFFT
-// group's descriptors and items, at byte offsets of one uploaded block.
+// group's descriptors and items, at byte offsets of one uploaded block, and the
+// sets launched by themselves.  A NUFFT group of one set takes the single-set launch, which also
+// splits its last round's rows (36 antennas, 32 t, 300 channels, 64 directions: 84 us against 173; 256
+// antennas, 64 t, 96 channels: the same 2.2 ms) and needs no list of items from the host.
 struct RoundTables {
     MultiTables horner;
     struct Nufft {
@@ -1106,14 +1125,27 @@ struct RoundTables {
         const NufftPlan* plan = nullptr;
     };
     std::vector<Nufft> nufft;
+    struct SingleNufft {
+        NufftSetDesc set;
+        const leap_metadata* md;
+        const NufftPlan* plan;
+        int32_t tile, vis_dtype;
+    };
+    std::vector<SingleNufft> single;
+    std::vector<HornerWave> waves;
 };
 
 RoundTables append_round(leap_ctx* ctx, std::vector<uint8_t>& bytes, const std::vector<MultiSetDesc>& descs,
                          const std::vector<MultiShape>& shapes, int32_t tile, int32_t per_cu,
-                         const std::vector<NufftGroup>& groups) {
+                         const std::vector<NufftGroup>& groups, const std::vector<HornerWave>& waves) {
     RoundTables t;
+    t.waves = waves;
     if (!descs.empty()) t.horner = append_tables(ctx, bytes, descs, shapes, tile, per_cu);
     for (const NufftGroup& g : groups) {
+        if (g.sets.size() == 1) {
+            t.single.push_back({g.sets[0], g.md, g.plan, g.tile, g.vis_dtype});
+            continue;
+        }
         RoundTables::Nufft n;
         n.descs = put_bytes(bytes, g.sets.data(), g.sets.size() * sizeof(NufftSetDesc));
         n.items = put_bytes(bytes, g.items.data(), g.items.size() * sizeof(uint32_t));
@@ -1143,6 +1175,14 @@ void launch_round(leap_ctx* ctx, const void* block, const RoundTables& t, int32_
         launch_rotate_nufft_sets(ctx->stream, n.tile, *n.plan, n.C, n.P,
                                  reinterpret_cast<const NufftSetDesc*>(b + n.descs),
                                  reinterpret_cast<const uint32_t*>(b + n.items), n.n_items);
+    for (const RoundTables::SingleNufft& n : t.single) {
+        const NufftSetDesc& d = n.set;
+        ctx->d_nufft_tail.reserve(nufft_tail_bytes(d.D));
+        launch_rotate_nufft(ctx->stream, n.tile, *n.plan, d.coef, d.vis, true, n.vis_dtype, d.uvw, d.dd, d.D, d.T, d.nbl,
+                            d.nbl, d.C, n.md->pols, 1, n.md->freq_start_hz, n.md->freq_inc_hz, d.avg, 0,
+                            ctx->d_nufft_tail.as<double>(), nufft_tail_bytes(d.D));
+    }
+    for (const HornerWave& w : t.waves) launch_horner_wave(ctx->stream, w);
 }
 
 // Plans, uploads and launches one multi-set rotate/average.  The host copy of
@@ -1165,13 +1205,19 @@ void run_multi(leap_ctx* ctx, const std::vector<MultiSetDesc>& descs, const std:
 // Plans, uploads and launches one round of a multi-set call (the Horner
 // tables and the NUFFT groups in one block), timed as one rotate.
 void run_round(leap_ctx* ctx, const std::vector<MultiSetDesc>& descs, const std::vector<MultiShape>& shapes,
-               int32_t tile, int32_t per_cu, const std::vector<NufftGroup>& groups) {
-    LEAP_HIP(hipStreamSynchronize(ctx->stream));  // the previous upload has left h_tables
+               int32_t tile, int32_t per_cu, const std::vector<NufftGroup>& groups,
+               const std::vector<HornerWave>& waves) {
+    const bool tables = !descs.empty() || std::any_of(groups.begin(), groups.end(), [](const NufftGroup& g) {
+        return g.sets.size() > 1;
+    });
+    if (tables) LEAP_HIP(hipStreamSynchronize(ctx->stream));  // the previous upload has left h_tables
     ctx->h_tables.clear();
-    const RoundTables t = append_round(ctx, ctx->h_tables, descs, shapes, tile, per_cu, groups);
-    ctx->d_tables.reserve(ctx->h_tables.size());
-    LEAP_HIP(hipMemcpyAsync(ctx->d_tables.ptr, ctx->h_tables.data(), ctx->h_tables.size(), hipMemcpyHostToDevice,
-                            ctx->stream));
+    const RoundTables t = append_round(ctx, ctx->h_tables, descs, shapes, tile, per_cu, groups, waves);
+    if (tables) {
+        ctx->d_tables.reserve(ctx->h_tables.size());
+        LEAP_HIP(hipMemcpyAsync(ctx->d_tables.ptr, ctx->h_tables.data(), ctx->h_tables.size(), hipMemcpyHostToDevice,
+                                ctx->stream));
+    }
     record_rotate_begin(ctx);
     launch_round(ctx, ctx->d_tables.ptr, t, tile);
     record_rotate_end(ctx);
@@ -1258,7 +1304,8 @@ struct BatchState {
     int32_t solutions;
     uint32_t interval;
     std::vector<double> h_cal;
-    int32_t nufft = 0;  // NUFFT route of the channel sums, 0 for Horner (avgData holds pol 0 alone)
+    int32_t nufft = 0;  // NUFFT route of the channel sums, 0 for Horner
+    bool own = false;   // Horner sums in a launch of their own
 };
 
 void calibrate_batch(leap_ctx* ctx, const leap_batch_set* sets, uint32_t n_sets, const leap_options& opts,
@@ -1286,7 +1333,8 @@ void calibrate_batch(leap_ctx* ctx, const leap_batch_set* sets, uint32_t n_sets,
         evaluate_slice(in.slice_start, in.slice_interval, in.slice_end, T, range);
         st[i] = BatchState{in.metadata, in.ms, in.directions, in.n_directions,
                            (range[2] - range[0]) / range[1], uint32_t(range[1]), {},
-                           set_nufft_route(opts, *in.metadata, *in.ms, in.n_directions)};
+                           set_nufft_route(opts, *in.metadata, *in.ms, in.n_directions, uint32_t(range[1]))};
+        st[i].own = !st[i].nufft && own_launch(opts, uint32_t(range[1]) * in.metadata->nbl);
         rounds = std::max(rounds, st[i].solutions);
     }
     while (ctx->batch_sets.size() < n_sets) ctx->batch_sets.push_back(std::make_unique<SetBuffers>());
@@ -1295,25 +1343,29 @@ void calibrate_batch(leap_ctx* ctx, const leap_batch_set* sets, uint32_t n_sets,
         if (b.nufft) ctx->last_channel_sum = b.nufft;  // one NUFFT route per call (set by the precision)
     ctx->last_direct_cube = 1;
     begin_timing(ctx);
+    // every set's directions in one upload
+    std::vector<double> dirs;
+    for (const BatchState& b : st) dirs.insert(dirs.end(), b.dirs, b.dirs + size_t(b.D) * 2);
+    ctx->d_dirs.reserve(std::max<size_t>(1, dirs.size()) * sizeof(double));
+    if (!dirs.empty())
+        LEAP_HIP(hipMemcpyAsync(ctx->d_dirs.ptr, dirs.data(), dirs.size() * sizeof(double), hipMemcpyHostToDevice,
+                                ctx->stream));
+    const double* d_dirs = ctx->d_dirs.as<double>();
     for (uint32_t i = 0; i < n_sets; ++i) {
         BatchState& b = st[i];
         SetBuffers& buf = *ctx->batch_sets[i];
-        const uint32_t N = uint32_t(b.md->A.cols);
-        b.h_cal.assign(size_t(N) * b.D, 0.0);
+        b.h_cal.assign(size_t(b.md->A.cols) * b.D, 0.0);
         if (b.D == 0) continue;
-        buf.d_dirs.reserve(size_t(b.D) * 2 * sizeof(double));
         buf.d_dd.reserve(size_t(b.D) * 9 * sizeof(double));
         buf.d_avg.reserve(size_t(b.D) * b.md->nbl * b.md->pols * 2 * sizeof(double));
-        buf.d_cal.reserve(size_t(N) * b.D * sizeof(double));
-        LEAP_HIP(hipMemcpyAsync(buf.d_dirs.ptr, b.dirs, size_t(b.D) * 2 * sizeof(double), hipMemcpyHostToDevice,
-                                ctx->stream));
-        launch_dd(ctx->stream, b.md->phase_centre_ra, b.md->phase_centre_dec, buf.d_dirs.as<double>(), b.D,
-                  buf.d_dd.as<double>());
+        launch_dd(ctx->stream, b.md->phase_centre_ra, b.md->phase_centre_dec, d_dirs, b.D, buf.d_dd.as<double>());
+        d_dirs += size_t(b.D) * 2;
     }
     // Descriptors of round r: solution interval r of every set that has one,
     // Horner sets into descs / shapes, NUFFT sets into groups of one launch.
     auto round_descs = [&](int32_t r, std::vector<MultiSetDesc>& descs, std::vector<MultiShape>& shapes,
-                           std::vector<NufftGroup>& groups, std::vector<uint32_t>& active) {
+                           std::vector<NufftGroup>& groups, std::vector<HornerWave>& waves,
+                           std::vector<uint32_t>& active) {
         for (uint32_t i = 0; i < n_sets; ++i) {
             BatchState& b = st[i];
             if (r >= b.solutions || b.D == 0) continue;
@@ -1334,6 +1386,8 @@ void calibrate_batch(leap_ctx* ctx, const leap_batch_set* sets, uint32_t n_sets,
                     groups.emplace_back();
                     g = groups.end() - 1;
                     g->plan = &plan;
+                    g->md = b.md;
+                    g->vis_dtype = b.ms->vis_dtype;
                     g->key = key;
                     g->C = C;
                     g->P = src;
@@ -1347,6 +1401,12 @@ void calibrate_batch(leap_ctx* ctx, const leap_batch_set* sets, uint32_t n_sets,
                                                df / kSpeedOfLight, int32_t(plan.h), nbl, b.interval, C, b.D});
                 continue;
             }
+            if (b.own) {
+                waves.push_back(HornerWave{rows.vis, b.ms->vis_dtype, rows.uvw, buf.d_dd.as<double>(), b.D, b.interval,
+                                           1, nbl, b.md->channels, b.md->pols, 1, b.md->freq_start_hz,
+                                           b.md->freq_inc_hz, buf.d_avg.as<double>()});
+                continue;
+            }
             descs.push_back(MultiSetDesc{rows.vis, rows.uvw, buf.d_dd.as<double>(), buf.d_avg.as<double>(), nbl,
                                          b.interval, b.md->channels, b.md->pols, b.D,
                                          b.ms->vis_dtype == LEAP_VIS_C64 ? 1 : 0,
@@ -1355,7 +1415,7 @@ void calibrate_batch(leap_ctx* ctx, const leap_batch_set* sets, uint32_t n_sets,
         }
         for (NufftGroup& g : groups) plan_nufft_group(g, opts);
     };
-    auto avg_pols = [&](uint32_t i) { return st[i].nufft ? 1u : st[i].md->pols; };
+    auto avg_pols = [&](uint32_t i) { return st[i].nufft || st[i].own ? 1u : st[i].md->pols; };
     auto deliver = [&](int32_t r, auto&& cal_of) {
         for (uint32_t i = 0; i < n_sets; ++i) {
             const BatchState& b = st[i];
@@ -1379,6 +1439,7 @@ void calibrate_batch(leap_ctx* ctx, const leap_batch_set* sets, uint32_t n_sets,
         std::vector<std::vector<MultiSetDesc>> rdescs(n_rounds);
         std::vector<std::vector<MultiShape>> rshapes(n_rounds);
         std::vector<std::vector<NufftGroup>> rgroups(n_rounds);
+        std::vector<std::vector<HornerWave>> rwaves(n_rounds);
         std::vector<std::vector<uint32_t>> ractive(n_rounds);
         std::vector<size_t> cal_at(n_sets, 0);
         size_t cal_total = 0;
@@ -1392,7 +1453,7 @@ void calibrate_batch(leap_ctx* ctx, const leap_batch_set* sets, uint32_t n_sets,
             reserve_solution(ctx, *b.md, b.D, b.interval, ro);
             cal_total += size_t(b.md->A.cols) * b.D * size_t(b.solutions);
         }
-        for (int32_t r = 0; r < rounds; ++r) round_descs(r, rdescs[r], rshapes[r], rgroups[r], ractive[r]);
+        for (int32_t r = 0; r < rounds; ++r) round_descs(r, rdescs[r], rshapes[r], rgroups[r], rwaves[r], ractive[r]);
         for (int32_t r = 0; r < rounds && launch.first == 0; ++r)
             if (!rdescs[r].empty()) launch = multi_tile(ctx, rdescs[r], rshapes[r], opts);
         ctx->last_direction_block = launch.first;
@@ -1412,10 +1473,12 @@ void calibrate_batch(leap_ctx* ctx, const leap_batch_set* sets, uint32_t n_sets,
             std::vector<uint8_t> bytes;
             std::vector<RoundTables> tables(n_rounds);
             for (int32_t r = 0; r < rounds; ++r)
-                tables[r] = append_round(ctx, bytes, rdescs[r], rshapes[r], launch.first, launch.second, rgroups[r]);
+                tables[r] = append_round(ctx, bytes, rdescs[r], rshapes[r], launch.first, launch.second, rgroups[r],
+                                         rwaves[r]);
             seq->d_tables.reserve(bytes.size());
-            LEAP_HIP(hipMemcpyAsync(seq->d_tables.ptr, bytes.data(), bytes.size(), hipMemcpyHostToDevice,
-                                    ctx->stream));
+            if (!bytes.empty())
+                LEAP_HIP(hipMemcpyAsync(seq->d_tables.ptr, bytes.data(), bytes.size(), hipMemcpyHostToDevice,
+                                        ctx->stream));
             LEAP_HIP(hipStreamSynchronize(ctx->stream));
             seq->d_cal.reserve(cal_total * sizeof(double));
             capture(ctx, *seq, [&] {
@@ -1454,21 +1517,34 @@ void calibrate_batch(leap_ctx* ctx, const leap_batch_set* sets, uint32_t n_sets,
         std::vector<MultiSetDesc> descs;
         std::vector<MultiShape> shapes;
         std::vector<NufftGroup> groups;
+        std::vector<HornerWave> waves;
         std::vector<uint32_t> active;
-        round_descs(r, descs, shapes, groups, active);
+        round_descs(r, descs, shapes, groups, waves, active);
         if (!active.empty()) {
             if (launch.first == 0 && !descs.empty()) launch = multi_tile(ctx, descs, shapes, opts);
             ctx->last_direction_block = launch.first;
             ctx->last_workgroups_per_cu = launch.second;
-            run_round(ctx, descs, shapes, launch.first, launch.second, groups);
+            run_round(ctx, descs, shapes, launch.first, launch.second, groups, waves);
+            // every set's calibrations side by side, copied back together
+            size_t total = 0;
+            for (uint32_t i : active) total += st[i].h_cal.size();
+            ctx->d_cal.reserve(total * sizeof(double));
+            ctx->h_cal.reserve(total * sizeof(double));
+            size_t at = 0;
             for (uint32_t i : active) {
                 BatchState& b = st[i];
-                SetBuffers& buf = *ctx->batch_sets[i];
-                invert_directions(ctx, *b.md, b.D, opts, buf.d_avg.as<double>(), buf.d_cal.as<double>(), avg_pols(i));
-                LEAP_HIP(hipMemcpyAsync(b.h_cal.data(), buf.d_cal.ptr, b.h_cal.size() * sizeof(double),
-                                        hipMemcpyDeviceToHost, ctx->stream));
+                invert_directions(ctx, *b.md, b.D, opts, ctx->batch_sets[i]->d_avg.as<double>(),
+                                  ctx->d_cal.as<double>() + at, avg_pols(i));
+                at += b.h_cal.size();
             }
+            LEAP_HIP(hipMemcpyAsync(ctx->h_cal.ptr, ctx->d_cal.ptr, total * sizeof(double), hipMemcpyDeviceToHost,
+                                    ctx->stream));
             LEAP_HIP(hipStreamSynchronize(ctx->stream));
+            const double* from = ctx->h_cal.as<double>();
+            for (uint32_t i : active) {
+                std::copy(from, from + st[i].h_cal.size(), st[i].h_cal.begin());
+                from += st[i].h_cal.size();
+            }
         }
         deliver(r, [&](uint32_t i) -> const double* { return st[i].h_cal.data(); });
     }

@@ -233,7 +233,7 @@ struct TuneKey {
 namespace leap {
 // Per-set device buffers of leap_hip_calibrate_batch.
 struct SetBuffers {
-    DeviceBuffer d_dirs, d_dd, d_avg, d_cal, d_vis, d_uvw;
+    DeviceBuffer d_dd, d_avg, d_vis, d_uvw;
 };
 
 // A calibration sequence captured as a HIP graph, with the key of shapes,

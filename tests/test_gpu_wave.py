@@ -116,3 +116,31 @@ def test_automatic_route_of_device_cubes(leap, ctx, on_device, n_ant, T, P, D, p
                                                     channel_sum=1 if route != 1 else 4))
     bar = 1e-5 if precision else 1e-12
     assert np.abs(got[:, :, 0] - other[:, :, 0]).max() <= bar * np.abs(other[:, :, 0]).max()
+
+
+@pytest.mark.parametrize("precision", [0, 1], ids=["fp64", "mixed"])
+def test_multi_set_launches_of_their_own(leap, ctx, on_device, precision):
+    """A multi-set call whose sets take every kind of launch (folded sums of their own, the shared Horner
+    tiles, a NUFFT group of one set) over uneven numbers of solutions: as the sets' own calls give
+    (1e-9 rad in FP64, 1e-6 mixed), and the captured call and its replay equal to the eager one."""
+    print(f"multi-set launches, precision {precision}", flush=True)
+    sets = []
+    for n_ant, T, C, D, slice_ in ((130, 3, 20, 9, (0, 1, -1)), (9, 4, 30, 5, (0, 2, -1)),
+                                   (20, 4, 128, 40, (0, -1, -1)), (95, 2, 33, 70, (0, -1, -1))):
+        s = leap.SynthMS(n_antennas=n_ant, n_timesteps=T, n_channels=C, nan_fraction=0.003, seed=C)
+        s.fill_host(np.complex64)
+        ms = s.host_dict()
+        view = on_device(ms)
+        dirs = np.asarray(ms["phase_centre"]) + np.random.default_rng(D).uniform(-0.02, 0.02, (D, 2))
+        sets.append((ctx.metadata(view), view, dirs, slice_))
+    opts = dict(strategy=1, precision=precision)
+    eager = ctx.calibrate_batch(sets, leap.options(**opts))
+    for (md, view, dirs, slice_), (got, epochs) in zip(sets, eager):
+        want, want_epochs = ctx.calibrate(view, dirs, slice_, opts=leap.options(**opts), md=md)
+        assert np.array_equal(epochs, want_epochs)
+        diff = np.angle(np.exp(1j * (got - want)))
+        assert np.abs(diff).max() <= (1e-6 if precision else 1e-9)
+    for _ in range(3):
+        again = ctx.calibrate_batch(sets, leap.options(graph=1, **opts))
+        for (got, _), (want, _) in zip(again, eager):
+            assert np.array_equal(got, want)
