@@ -58,9 +58,11 @@ __global__ void dd_kernel(double ra0, double dec0, const double* __restrict__ di
 // One pass serves ND directions because the cube is what a single direction waits for
 // (5.9 TB/s on complex64, 6.0 to 6.2 on complex128, 4.2 ms for 26 GB), while a direction's
 // own work is some 34 instructions per sample.  256 stations, 32 t, 384 ch, 4 pols: 4
-// directions of the complex64 cube (13 GB) take 2.41 ms in one pass against 8.87 in four,
+// directions of the complex64 cube (13 GB) take 2.35 ms in one pass against 8.87 in four,
 // 2 of the complex128 cube 4.36 against 8.34; 16 directions of 128 stations, 14 t, 48 ch
-// (355 MB) 0.20 ms in two passes against 1.10 in sixteen, bound by the arithmetic.
+// (355 MB) 0.13 ms in two passes against 1.10 in sixteen, bound by the arithmetic.  There a wave
+// has some ten samples a lane, and its sums over the lanes took 0.04 ms while their step sizes were
+// variables and every value was picked by comparisons.
 // A wave owns its samples of one baseline and holds ND sums per pol in registers:
 //  - shift is the correctly rounded quotient: q = sf * r, r = RN(1 / lambda), then
 //    fma(fma(-q, lambda, sf), r, q) (Markstein 1990), 3 instructions against a division's 11
@@ -68,10 +70,12 @@ __global__ void dd_kernel(double ra0, double dec0, const double* __restrict__ di
 //    a 64-entry table in LDS and the series to r^8 (cos) and r^7 (sin) on |r| <= pi / 64,
 //    whose next terms are below 2.5e-20 and 4.6e-18: 18 instructions
 //  - the rotated sample goes into the sums as four FMAs
-// Samples that are not finite and shifts that are not below 2^26 rad take the plain form
-// (division, sincos, rotate every pol, look for a NaN), exactly as the reference does it.
+// Samples that are not finite, a baseline's chunk of rows where a shift is not below 2^25 rad
+// (looked at once a row and direction) and channels without a finite wavelength take the plain
+// form (division, sincos, rotate every pol, look for a NaN), exactly as the reference does it.
 // ---------------------------------------------------------------------------
 constexpr double kMaxShift = 67108864.0;  // 2^26 rad, far inside the phasor table's range
+constexpr double kMaxLambda = 0x1p900;    // longer ones (a channel at 0 Hz) are divided by
 constexpr uint32_t kRowChunk = 32;          // rows whose shift factors a wave keeps in LDS
 constexpr uint32_t kLambdaLds = 1024;       // channels whose wavelengths sit in LDS
 
@@ -101,24 +105,22 @@ struct VisLoad {
 // Sums of N values over a wave: every step halves the values a lane holds while there is
 // more than one, so N + 4 exchanges do instead of 6 N.  The lane's value is number
 // wave_sum_index<N>(lane); each is summed over the lanes in the same tree whatever N.
-template <int N>
-__device__ inline double wave_sum_n(double* v, uint32_t lane) {
-    int n = N;
+template <int N, int M = 32>
+__device__ inline double wave_sum_n(const double (&v)[N], uint32_t lane) {
+    constexpr int H = N > 1 ? N / 2 : 1;  // the step's sizes are constants, so v stays in registers
+    double s[H];
+    if constexpr (N > 1) {
+        const bool up = lane & M;
 #pragma unroll
-    for (int m = 32; m > 0; m >>= 1) {
-        if (n > 1) {
-            n /= 2;
-            const bool up = lane & m;
-#pragma unroll
-            for (int j = 0; j < n; ++j) {
-                const double send = up ? v[j] : v[j + n], keep = up ? v[j + n] : v[j];
-                v[j] = keep + __shfl_xor(send, m, 64);
-            }
-        } else {
-            v[0] += __shfl_xor(v[0], m, 64);
+        for (int j = 0; j < H; ++j) {
+            const double send = up ? v[j] : v[j + H], keep = up ? v[j + H] : v[j];
+            s[j] = keep + __shfl_xor(send, M, 64);
         }
+    } else {
+        s[0] = v[0] + __shfl_xor(v[0], M, 64);
     }
-    return v[0];
+    if constexpr (M > 1) return wave_sum_n<H, M / 2>(s, lane);
+    return s[0];
 }
 
 template <int N>
@@ -135,8 +137,11 @@ constexpr int pow2_at_least(int n) {
 // Grid: (groups of directions fastest, baselines) x solution intervals; waves of a baseline:
 // wpb (1: the workgroup's waves take one baseline each).  lambda2: (lambda, RN(1 / lambda)).
 // avg[interval][direction][baseline][PO].
+// Sixteen waves of a baseline (1,024 threads, 128 registers) with up to four directions a pass.
+constexpr int max_threads(bool wide, int nd) { return wide || nd > 4 ? 256 : 1024; }
+
 template <typename T, int P, int PO, int ND, bool kWide>
-__global__ __launch_bounds__(kWide ? 256 : 1024) void rotate_average_f64(
+__global__ __launch_bounds__(max_threads(kWide, ND)) void rotate_average_f64(
     const T* __restrict__ vis, const double* __restrict__ uvw, const double* __restrict__ dd, uint32_t D,
     uint32_t groups, uint32_t wpb, uint32_t T_steps, uint32_t nbl, uint32_t C,
     const double2* __restrict__ lambda2, double* __restrict__ avg) {
@@ -171,10 +176,14 @@ __global__ __launch_bounds__(kWide ? 256 : 1024) void rotate_average_f64(
     for (int q = 0; q < NV; ++q) acc[q] = 0.0;
 
     if (bl < nbl) {
+        // the largest |1 / lambda|, at an end of the band: one look at a row's shift factors stands for
+        // its samples' shifts
+        const double r_max = fmax(fabs(lambda2[0].y), fabs(lambda2[C - 1].y));
         const uint32_t step_t = 64 * wpb / C, step_c = 64 * wpb % C;
         for (uint32_t t0 = 0; t0 < T_steps; t0 += kRowChunk) {
             const uint32_t tn = min(kRowChunk, T_steps - t0);
             dev::wave_fence();  // the previous chunk's factors have been read
+            bool far = false;
             for (uint32_t i = lane; i < tn * ND; i += 64) {
                 const uint32_t t = i / ND, d = i % ND;
                 const size_t row = rows0 + size_t(t0 + t) * nbl + bl;
@@ -182,8 +191,10 @@ __global__ __launch_bounds__(kWide ? 256 : 1024) void rotate_average_f64(
                 const double u = uvw[3 * row], v = uvw[3 * row + 1], w = uvw[3 * row + 2];
                 const double wrot = dz[0] * u + dz[1] * v + dz[2] * w;  // (dd * uvw).z, MetaData.cc:227
                 s_sf[i] = -kTwoPi * (wrot - w);                        // CpuLeapCalibrator.cc:190
+                far |= !(fabs(s_sf[i]) * r_max < 0.5 * kMaxShift);
             }
             dev::wave_fence();
+            const bool near = !__any(far);
             // samples lane + 64 * (part + k * wpb) of the chunk, in (row, channel) order
             const size_t at0 = rows0 + size_t(t0) * nbl + bl;
             auto at = [&](uint32_t t, uint32_t c) { return vis + ((at0 + size_t(t) * nbl) * C + c) * (2 * P); };
@@ -249,18 +260,14 @@ __global__ __launch_bounds__(kWide ? 256 : 1024) void rotate_average_f64(
                 advance(t, c);
                 if constexpr (!kWide)
                     if (t < tn) next.load(at(t, c));
-                double shift[ND];
-#pragma unroll
-                for (int d = 0; d < ND; ++d) {
-                    const double q = sf[d] * l.y;
-                    shift[d] = fma(fma(-q, l.x, sf[d]), l.y, q);  // sf / lambda, :195
-                    plain = plain && fabs(shift[d]) < kMaxShift;
-                }
+                plain = plain && near && fabs(l.x) < kMaxLambda;
                 if (plain) {
 #pragma unroll
                     for (int d = 0; d < ND; ++d) {
                         if ((d & 1) == 0 && uint32_t(d) >= active) break;
-                        const double2 e = dev::phasor_table(s_table, shift[d]);
+                        const double q = sf[d] * l.y;
+                        const double shift = fma(fma(-q, l.x, sf[d]), l.y, q);  // sf / lambda, :195
+                        const double2 e = dev::phasor_table(s_table, shift);
 #pragma unroll
                         for (int q = 0; q < PO; ++q) {  // (a + ib)(cs + i sn), :198, :208-214
                             double* o = acc + 2 * (d * PO + q);
@@ -608,7 +615,7 @@ void launch_rotate_nd(hipStream_t s, const RotateF64& a) {
         LEAP_HIP(hipGetLastError());
     };
     // Wide loads up to 4 directions, where the visibilities are the bound; with 8 their registers
-    // cost half the waves (16 directions on 355 MB: 249 us against 200).
+    // cost half the waves (16 directions on 355 MB: 220 us against 130).
     if constexpr (PO == 1 && P * sizeof(T) == 32 && ND <= 4) {
         if (waves <= 4) return launch(std::true_type{});
     }
@@ -660,7 +667,7 @@ void launch_rotate_f64(hipStream_t s, const RotateF64& in) {
     // Directions per pass: as many as D has, up to 8, but no more than leaves 4 waves per SIMD
     // (splitting the directions over workgroups shortens each wave's chain instead).
     const uint64_t waves = uint64_t(a.nbl) * a.wpb * a.intervals;
-    uint32_t nd = a.pols_out == 1 ? 8 : 2;
+    uint32_t nd = a.pols_out != 1 ? 2 : a.wpb > 4 ? 4 : 8;
     while (nd > 1 && (nd / 2 >= a.D || waves * ((a.D + nd - 1) / nd) < 4096)) nd /= 2;
     if (a.vis_dtype == LEAP_VIS_C64)
         launch_rotate_typed<float>(s, a, nd);

@@ -75,3 +75,11 @@ def test_plain_rotate_extreme_rows(leap, ctx, oracle):
         err = np.abs(got[d, :, 0] - want[:, 0])
         print(f"direction {d}: error over bar {(err / (bar + 1e-12 * np.abs(want).max())).max():.2e}")
         assert (err <= bar + 1e-12 * np.abs(want).max()).all()
+
+
+@pytest.mark.parametrize("dtype", [np.complex64, np.complex128])
+def test_plain_rotate_channel_at_zero_hz(leap, ctx, oracle, dtype):
+    """A band through 0 Hz: that channel's wavelength is infinite and its phase zero."""
+    s = leap.SynthMS(n_antennas=9, n_timesteps=2, n_channels=9, freq_start_hz=-8e6, freq_inc_hz=2e6, seed=9)
+    s.fill_host(dtype)
+    _check(leap, ctx, oracle, s.host_dict(), 5, 9, calibrate=False)
