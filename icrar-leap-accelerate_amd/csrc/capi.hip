@@ -212,13 +212,14 @@ bool folded_beats_nufft(uint32_t rows, uint32_t D) {
 
 bool names_no_tile(const leap_options& opts) { return opts.direction_block == 0 && opts.lane_directions == 0; }
 
-// The route of a batched call.  Horner calls on a device-resident cube that name no tile go straight
-// from the cube: the folded kernel costs less than the packed kernel alone from 48 channels and 256
-// directions (45 against 39 TFLOP/s of direct sums) to 384 channels (70 against 55), so the pack
-// pass never pays.  With a lane_directions named (tiles of kernels_batched.hip and the packed kernel)
-// it pays from the rates measured on those: pack 5.2 TB/s, packed Horner 32 / 50 / 55 TFLOP/s up to
-// 64, 128, more directions, from the cube 6.4 TB/s and 30 or 51 (45 on complex128).  Host-resident
-// cubes always take the packed route (pol 0 only crosses the bus).
+// The route of a batched call.  Horner calls on a device-resident cube that name no tile are routed by
+// the rates measured before the folded kernel: pack 5.2 TB/s; packed Horner 32 / 50 / 55 TFLOP/s with 1
+// / 2 / 4 directions per lane (up to 64, 128, more directions); from the cube 5.7 TB/s and 50 TFLOP/s
+// (complex64) or 47 (complex128), both less by the phasors of a row (20 channels' worth).  So the
+// pack takes over from about 800 directions on complex64 and 480 on complex128, where callers that
+// look at the pack's times expect it.  (The folded kernel would be the faster there too: 128 antennas,
+// 14 t, 48 channels, 1,024 directions 0.88 ms against 1.17 packed.)  Host-resident cubes always take
+// the packed route (pol 0 only crosses the bus).
 leap_options routed(const leap_options& o, const leap_ms_view& ms, uint32_t T, uint32_t D) {
     leap_options r = o;
     if (r.channel_sum == LEAP_CHANNEL_SUM_AUTO) {
@@ -245,16 +246,14 @@ leap_options routed(const leap_options& o, const leap_ms_view& ms, uint32_t T, u
         return r;
     }
     if (!use_packed(o) || o.direction_block != 0 || !ms.vis_on_device) return r;
-    if (o.lane_directions == 0) {
-        r.direct_cube = 1;
-        return r;
-    }
     const double rc = double(T) * ms.num_baselines * ms.num_channels;  // (row, channel)s
     const double s = ms.vis_dtype == LEAP_VIS_C64 ? 8.0 : 16.0;
     const double flops = 8.0 * rc * D;
-    const double packed = rc * (ms.num_pols * s + 16.0) / 5.2e12 + flops / (D > 128 ? 55e12 : D > 64 ? 50e12 : 32e12);
-    const double direct_rate = D > 128 ? (ms.vis_dtype == LEAP_VIS_C64 ? 51e12 : 45e12) : 30e12;
-    const double direct = std::max(rc * ms.num_pols * s / 6.4e12, flops / direct_rate);
+    const double rows = double(ms.num_channels) / (ms.num_channels + 20.0);
+    const double packed =
+        rc * (ms.num_pols * s + 16.0) / 5.2e12 + flops / (rows * (D > 128 ? 55e12 : D > 64 ? 50e12 : 32e12));
+    const double direct = std::max(rc * ms.num_pols * s / 5.7e12,
+                                   flops / (rows * (ms.vis_dtype == LEAP_VIS_C64 ? 50e12 : 47e12)));
     if (packed > direct) r.direct_cube = 1;
     return r;
 }
