@@ -12,6 +12,11 @@
 namespace leap {
 namespace dev {
 
+// The device clock at the launch's first workgroup.
+__device__ inline void stamp(uint64_t* at) {
+    if (at && blockIdx.x == 0 && blockIdx.y == 0 && threadIdx.x == 0) *at = uint64_t(wall_clock64());
+}
+
 // Orders a wave's LDS writes before its later reads (no workgroup barrier).
 __device__ inline void wave_fence() {
     __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");

@@ -59,6 +59,22 @@ size_t vis_elem_bytes(const leap_ms_view& ms) {
     return (ms.vis_dtype == LEAP_VIS_C64 ? 8 : 16) * size_t(ms.num_pols);
 }
 
+// The rotate kernel of a calibration stamps the device clock where it starts and the inversion's first
+// kernel where that starts, instead of events around the kernel: recording events between kernels, or
+// with a kernel's dispatch, costs a call 20 us (46 against 67 us for six stations).
+uint64_t* stamp_rotate(leap_ctx* ctx) {
+    if (ctx->capturing || !ctx->stamps) return nullptr;
+    ctx->stamped = true;
+    return ctx->stamps;
+}
+
+// For the kernel that follows a stamped rotate.
+uint64_t* stamp_next(leap_ctx* ctx) {
+    if (!ctx->stamped || ctx->stamps[1] != 0) return nullptr;
+    ctx->stamps[1] = 1;  // taken; the kernel writes it later
+    return ctx->stamps + 1;
+}
+
 void record_rotate_begin(leap_ctx* ctx) {
     if (ctx->capturing) return;  // a captured sequence is timed as a whole
     if (ctx->rotate_events_used == ctx->rotate_events.size()) {
@@ -97,16 +113,43 @@ void begin_timing(leap_ctx* ctx) {
     ctx->last_stage_bytes = 0;
     ctx->pack_events_used = 0;
     ctx->rotate_events_used = 0;
+    ctx->stamps = nullptr;
+    ctx->stamped = false;
+    ctx->stamp_ms = 0.0;
+    ctx->stamp_launches = 0;
     LEAP_HIP(hipEventRecord(ctx->ev_start, ctx->stream));
 }
 
-// Call after the stream has been synchronised.
-void end_timing(leap_ctx* ctx) {
+// Stamps from here on, until the call ends.
+void begin_stamps(leap_ctx* ctx) {
+    if (ctx->clock_khz == 0.0) {
+        int khz = 0;
+        LEAP_HIP(hipDeviceGetAttribute(&khz, hipDeviceAttributeWallClockRate, ctx->device));
+        ctx->clock_khz = double(std::max(khz, 1));
+    }
+    ctx->h_stamps.reserve(2 * sizeof(uint64_t));
+    ctx->stamps = ctx->h_stamps.as<uint64_t>();
+    ctx->stamps[1] = 0;
+}
+
+// Waits for the call's device work, whose end is the end of the call's device time.
+void finish_stream(leap_ctx* ctx) {
     LEAP_HIP(hipEventRecord(ctx->ev_stop, ctx->stream));
-    LEAP_HIP(hipEventSynchronize(ctx->ev_stop));
+    LEAP_HIP(hipStreamSynchronize(ctx->stream));
+    ctx->dirs_in_use = false;
+    if (!ctx->stamped) return;
+    ctx->stamp_ms += double(ctx->stamps[1] - ctx->stamps[0]) / ctx->clock_khz;
+    ++ctx->stamp_launches;
+    ctx->stamped = false;
+    ctx->stamps[1] = 0;
+}
+
+// Call after finish_stream.
+void end_timing(leap_ctx* ctx) {
     float total = 0.f;
     LEAP_HIP(hipEventElapsedTime(&total, ctx->ev_start, ctx->ev_stop));
-    double sum = 0.0;
+    ctx->stamps = nullptr;
+    double sum = ctx->stamp_ms;
     for (size_t i = 0; i < ctx->rotate_events_used; ++i) {
         float ms = 0.f;
         LEAP_HIP(hipEventElapsedTime(&ms, ctx->rotate_events[i].first, ctx->rotate_events[i].second));
@@ -121,8 +164,8 @@ void end_timing(leap_ctx* ctx) {
     ctx->last_pack_launches = int32_t(ctx->pack_events_used);
     ctx->last_pack_ms_avg = ctx->pack_events_used ? pack_sum / double(ctx->pack_events_used) : 0.0;
     ctx->last_total_ms = total;
-    ctx->last_rotate_launches = int32_t(ctx->rotate_events_used);
-    ctx->last_rotate_ms_avg = ctx->rotate_events_used ? sum / double(ctx->rotate_events_used) : 0.0;
+    ctx->last_rotate_launches = int32_t(ctx->rotate_events_used) + ctx->stamp_launches;
+    ctx->last_rotate_ms_avg = ctx->last_rotate_launches ? sum / double(ctx->last_rotate_launches) : 0.0;
 }
 
 // Device pointers of visibilities and uvw covering rows [row_begin, row_end);
@@ -171,13 +214,24 @@ DeviceRows stage_rows(leap_ctx* ctx, const leap_ms_view& ms, uint32_t row_begin,
     return stage_rows_into(ctx, ms, row_begin, row_end, ctx->d_vis_stage, ctx->d_uvw, with_vis);
 }
 
-void upload_directions(leap_ctx* ctx, const leap_metadata& md, const double* dirs, uint32_t D) {
-    ctx->d_dirs.reserve(size_t(D) * 2 * sizeof(double));
+// Room for n directions in the context's pinned memory, which the kernels read themselves: a few
+// kilobytes read once cost less than a copy in the queue (5 us of a call of 70).
+double* directions_room(leap_ctx* ctx, size_t n) {
+    if (ctx->dirs_in_use) LEAP_HIP(hipStreamSynchronize(ctx->stream));  // a call that ended early
+    ctx->h_dirs.reserve(std::max<size_t>(1, n * 2) * sizeof(double));
+    ctx->dirs_in_use = true;
+    return ctx->h_dirs.as<double>();
+}
+
+void upload_directions(leap_ctx* ctx, double ra0, double dec0, const double* dirs, uint32_t D) {
     ctx->d_dd.reserve(size_t(D) * 9 * sizeof(double));
-    LEAP_HIP(hipMemcpyAsync(ctx->d_dirs.ptr, dirs, size_t(D) * 2 * sizeof(double), hipMemcpyHostToDevice,
-                            ctx->stream));
-    launch_dd(ctx->stream, md.phase_centre_ra, md.phase_centre_dec, ctx->d_dirs.as<double>(), D,
-              ctx->d_dd.as<double>());
+    double* h_dirs = directions_room(ctx, D);
+    std::copy(dirs, dirs + size_t(D) * 2, h_dirs);
+    launch_dd(ctx->stream, ra0, dec0, h_dirs, D, ctx->d_dd.as<double>());
+}
+
+void upload_directions(leap_ctx* ctx, const leap_metadata& md, const double* dirs, uint32_t D) {
+    upload_directions(ctx, md.phase_centre_ra, md.phase_centre_dec, dirs, D);
 }
 
 // Whether the NUFFT kernel can read the cube itself: a supported type and pol
@@ -498,11 +552,12 @@ uint32_t rotate_directions(leap_ctx* ctx, const leap_metadata& md, const leap_ms
     if (wave) {
         require(rows.vis != nullptr, LEAP_ERR_INTERNAL, "visibilities were not staged");
         ctx->last_direction_block = horner_wave_tile(D, md.nbl, intervals);
-        record_rotate_begin(ctx);
+        uint64_t* started = stamp_rotate(ctx);
+        if (!started) record_rotate_begin(ctx);
         launch_horner_wave(ctx->stream, {rows.vis, ms.vis_dtype, rows.uvw, ctx->d_dd.as<double>(), D, T, intervals,
                                          md.nbl, md.channels, md.pols, avg_pols, md.freq_start_hz, md.freq_inc_hz,
-                                         ctx->d_avg.as<double>()});
-        record_rotate_end(ctx);
+                                         ctx->d_avg.as<double>(), nullptr, started});
+        if (!started) record_rotate_end(ctx);
         return avg_pols;
     }
     if (packed) {
@@ -533,11 +588,12 @@ uint32_t rotate_directions(leap_ctx* ctx, const leap_metadata& md, const leap_ms
         record_rotate_end(ctx);
         return avg_pols;
     }
-    record_rotate_begin(ctx);
+    uint64_t* started = stamp_rotate(ctx);
+    if (!started) record_rotate_begin(ctx);
     launch_rotate_f64(ctx->stream, {rows.vis, ms.vis_dtype, rows.uvw, ctx->d_dd.as<double>(), D, T, intervals, md.nbl,
                                     md.channels, md.pols, avg_pols, md.d_lambda.as<double2>(),
-                                    ctx->d_avg.as<double>()});
-    record_rotate_end(ctx);
+                                    ctx->d_avg.as<double>(), started});
+    if (!started) record_rotate_end(ctx);
     return avg_pols;
 }
 
@@ -555,10 +611,11 @@ void invert_directions(leap_ctx* ctx, const leap_metadata& md, uint32_t D, const
     if (avg == nullptr) avg = ctx->d_avg.as<double>();
     if (opts.precision != LEAP_PRECISION_MIXED) {
         ctx->d_sums.reserve(size_t(N) * D * sizeof(double));
-        launch_inversion_f64(ctx->stream, md, avg, avg_pols, D, ctx->d_cal1.as<double>(), ctx->d_sums.as<double>(), cal);
+        launch_inversion_f64(ctx->stream, md, avg, avg_pols, D, ctx->d_cal1.as<double>(), ctx->d_sums.as<double>(), cal,
+                             stamp_next(ctx));
         return;
     }
-    launch_cal1(ctx->stream, md, avg, avg_pols, D, ctx->d_cal1.as<double>());
+    launch_cal1(ctx->stream, md, avg, avg_pols, D, ctx->d_cal1.as<double>(), stamp_next(ctx));
     ctx->d_a_planes.reserve(bf16_planes_bytes((D + 63) / 64 * 64, K));
     ctx->d_partial.reserve(mfma_partial_floats(K, D, N) * sizeof(float));
     launch_gemm_bf16x3(ctx->stream, md.d_AdT_planes.ptr, K, N, {avg, md.nbl, avg_pols, md.d_pairs.as<int2>()}, D,
@@ -912,7 +969,7 @@ void calibrate_loop_graph(leap_ctx* ctx, const leap_metadata& md, const leap_ms_
         LEAP_HIP(hipMemcpyAsync(seq->h_cal.data(), seq->d_cal.ptr, seq->h_cal.size() * sizeof(double),
                                 hipMemcpyDeviceToHost, ctx->stream));
     }
-    LEAP_HIP(hipStreamSynchronize(ctx->stream));
+    finish_stream(ctx);
     end_timing(ctx);
     for (int32_t s = 0; s < solutions; ++s) {
         leap_solution sol{};
@@ -926,6 +983,10 @@ void calibrate_loop_graph(leap_ctx* ctx, const leap_metadata& md, const leap_ms_
         if (cb && cb(user, &sol) != 0) throw Error(LEAP_ERR_CALLBACK, "output callback requested a stop");
     }
 }
+
+// Calibrations a kernel writes to pinned memory itself: 14 solutions of 16 directions of 128 antennas
+// (229 kB) cost a call 194 us so and 208 with a copy, 64 directions (66 kB) 187 and 205.
+constexpr size_t kDirectResults = 32768;
 
 // The Calibrate loop (CpuLeapCalibrator.cc:61-145) over prepared metadata.
 void calibrate_loop(leap_ctx* ctx, const leap_metadata& md, const leap_ms_view& ms, const double* dirs, uint32_t D,
@@ -955,6 +1016,8 @@ void calibrate_loop(leap_ctx* ctx, const leap_metadata& md, const leap_ms_view& 
     const size_t per_sol = size_t(N) * D;
     ctx->h_cal.reserve(std::max<size_t>(1, per_sol * group) * sizeof(double));
     double* h_cal = ctx->h_cal.as<double>();
+    const bool direct = per_sol * group <= kDirectResults;
+    begin_stamps(ctx);
     for (int32_t s = 0; s < solutions; ++s) {  // :104
         const uint32_t at = uint32_t(s) % group;
         if (D > 0 && at == 0) {
@@ -963,10 +1026,11 @@ void calibrate_loop(leap_ctx* ctx, const leap_metadata& md, const leap_ms_view& 
             const DeviceRows rows = stage_rows(ctx, ms, uint32_t(size_t(s) * interval * nbl),
                                                uint32_t(size_t(s + n) * interval * nbl), !packed_route(opts, 0));
             const uint32_t ap = rotate_directions(ctx, md, ms, rows, interval, D, opts, 0, true, n);
-            invert_intervals(ctx, md, D, n, opts, ap);
-            LEAP_HIP(hipMemcpyAsync(h_cal, ctx->d_cal.ptr, per_sol * n * sizeof(double), hipMemcpyDeviceToHost,
-                                    ctx->stream));
-            LEAP_HIP(hipStreamSynchronize(ctx->stream));
+            invert_intervals(ctx, md, D, n, opts, ap, direct ? h_cal : nullptr);
+            if (!direct)
+                LEAP_HIP(hipMemcpyAsync(h_cal, ctx->d_cal.ptr, per_sol * n * sizeof(double), hipMemcpyDeviceToHost,
+                                        ctx->stream));
+            finish_stream(ctx);
         }
         leap_solution sol{};
         sol.index = uint32_t(s);
@@ -978,7 +1042,7 @@ void calibrate_loop(leap_ctx* ctx, const leap_metadata& md, const leap_ms_view& 
         sol.calibrations = h_cal + per_sol * at;
         if (cb && cb(user, &sol) != 0) throw Error(LEAP_ERR_CALLBACK, "output callback requested a stop");
     }
-    LEAP_HIP(hipStreamSynchronize(ctx->stream));
+    if (D == 0 || solutions <= 0) finish_stream(ctx);
     end_timing(ctx);
 }
 
@@ -1342,14 +1406,9 @@ void calibrate_batch(leap_ctx* ctx, const leap_batch_set* sets, uint32_t n_sets,
         if (b.nufft) ctx->last_channel_sum = b.nufft;  // one NUFFT route per call (set by the precision)
     ctx->last_direct_cube = 1;
     begin_timing(ctx);
-    // every set's directions in one upload
-    std::vector<double> dirs;
-    for (const BatchState& b : st) dirs.insert(dirs.end(), b.dirs, b.dirs + size_t(b.D) * 2);
-    ctx->d_dirs.reserve(std::max<size_t>(1, dirs.size()) * sizeof(double));
-    if (!dirs.empty())
-        LEAP_HIP(hipMemcpyAsync(ctx->d_dirs.ptr, dirs.data(), dirs.size() * sizeof(double), hipMemcpyHostToDevice,
-                                ctx->stream));
-    const double* d_dirs = ctx->d_dirs.as<double>();
+    size_t n_dirs = 0;
+    for (const BatchState& b : st) n_dirs += b.D;
+    double* h_dirs = directions_room(ctx, n_dirs);
     for (uint32_t i = 0; i < n_sets; ++i) {
         BatchState& b = st[i];
         SetBuffers& buf = *ctx->batch_sets[i];
@@ -1357,8 +1416,9 @@ void calibrate_batch(leap_ctx* ctx, const leap_batch_set* sets, uint32_t n_sets,
         if (b.D == 0) continue;
         buf.d_dd.reserve(size_t(b.D) * 9 * sizeof(double));
         buf.d_avg.reserve(size_t(b.D) * b.md->nbl * b.md->pols * 2 * sizeof(double));
-        launch_dd(ctx->stream, b.md->phase_centre_ra, b.md->phase_centre_dec, d_dirs, b.D, buf.d_dd.as<double>());
-        d_dirs += size_t(b.D) * 2;
+        std::copy(b.dirs, b.dirs + size_t(b.D) * 2, h_dirs);
+        launch_dd(ctx->stream, b.md->phase_centre_ra, b.md->phase_centre_dec, h_dirs, b.D, buf.d_dd.as<double>());
+        h_dirs += size_t(b.D) * 2;
     }
     // Descriptors of round r: solution interval r of every set that has one,
     // Horner sets into descs / shapes, NUFFT sets into groups of one launch.
@@ -1501,7 +1561,7 @@ void calibrate_batch(leap_ctx* ctx, const leap_batch_set* sets, uint32_t n_sets,
             LEAP_HIP(hipMemcpyAsync(seq->h_cal.data(), seq->d_cal.ptr, cal_total * sizeof(double),
                                     hipMemcpyDeviceToHost, ctx->stream));
         }
-        LEAP_HIP(hipStreamSynchronize(ctx->stream));
+        finish_stream(ctx);
         end_timing(ctx);
         for (int32_t r = 0; r < rounds; ++r)
             deliver(r, [&](uint32_t i) -> const double* {
@@ -1538,7 +1598,7 @@ void calibrate_batch(leap_ctx* ctx, const leap_batch_set* sets, uint32_t n_sets,
             }
             LEAP_HIP(hipMemcpyAsync(ctx->h_cal.ptr, ctx->d_cal.ptr, total * sizeof(double), hipMemcpyDeviceToHost,
                                     ctx->stream));
-            LEAP_HIP(hipStreamSynchronize(ctx->stream));
+            finish_stream(ctx);
             const double* from = ctx->h_cal.as<double>();
             for (uint32_t i : active) {
                 std::copy(from, from + st[i].h_cal.size(), st[i].h_cal.begin());
@@ -1547,7 +1607,7 @@ void calibrate_batch(leap_ctx* ctx, const leap_batch_set* sets, uint32_t n_sets,
         }
         deliver(r, [&](uint32_t i) -> const double* { return st[i].h_cal.data(); });
     }
-    LEAP_HIP(hipStreamSynchronize(ctx->stream));
+    if (n_dirs == 0 || rounds == 0) finish_stream(ctx);
     end_timing(ctx);
 }
 
@@ -1720,7 +1780,7 @@ int leap_hip_rotate_visibilities(leap_ctx* ctx, const leap_metadata* md, const l
         rotate_directions(ctx, *md, *ms, rows, n_rows / ms->num_baselines, D, o);
         const size_t n = size_t(md->nbl) * md->pols * 2 * D;
         if (n) LEAP_HIP(hipMemcpyAsync(avg_out, ctx->d_avg.ptr, n * sizeof(double), hipMemcpyDeviceToHost, ctx->stream));
-        LEAP_HIP(hipStreamSynchronize(ctx->stream));
+        finish_stream(ctx);
         end_timing(ctx);
     });
 }
@@ -1745,11 +1805,7 @@ int leap_hip_dd_matrix(leap_ctx* ctx, double ra0, double dec0, const double* dir
     return guarded(ctx, [&] {
         require(ctx && dirs && dd_out, LEAP_ERR_INVALID_ARGUMENT, "null argument");
         DeviceScope scope(ctx->device);
-        ctx->d_dirs.reserve(size_t(D) * 2 * sizeof(double));
-        ctx->d_dd.reserve(size_t(D) * 9 * sizeof(double));
-        LEAP_HIP(hipMemcpyAsync(ctx->d_dirs.ptr, dirs, size_t(D) * 2 * sizeof(double), hipMemcpyHostToDevice,
-                                ctx->stream));
-        launch_dd(ctx->stream, ra0, dec0, ctx->d_dirs.as<double>(), D, ctx->d_dd.as<double>());
+        upload_directions(ctx, ra0, dec0, dirs, D);
         LEAP_HIP(hipMemcpyAsync(dd_out, ctx->d_dd.ptr, size_t(D) * 9 * sizeof(double), hipMemcpyDeviceToHost,
                                 ctx->stream));
         LEAP_HIP(hipStreamSynchronize(ctx->stream));
@@ -2218,7 +2274,7 @@ extern "C" int leap_hip_residual_loss_grad(leap_ctx* ctx, const leap_metadata* m
         // dL/d(dz row of dd) reduced over baselines and mapped to dL/d(ra, dec) (MetaData.cc:166-203
         // differentiated) on the device
         launch_reduce_gdz_offsets(s, d_gdzp.as<double>(), nbl, D, md->phase_centre_ra, md->phase_centre_dec,
-                                  ctx->d_dirs.as<double>(), d_gdz.as<double>());
+                                  ctx->h_dirs.as<double>(), d_gdz.as<double>());
         if (grad_offsets)
             LEAP_HIP(hipMemcpyAsync(h_out + D, d_gdz.as<double>() + 3 * size_t(D), size_t(D) * 2 * sizeof(double),
                                     hipMemcpyDeviceToHost, s));

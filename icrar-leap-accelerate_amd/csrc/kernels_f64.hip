@@ -144,8 +144,9 @@ template <typename T, int P, int PO, int ND, bool kWide>
 __global__ __launch_bounds__(max_threads(kWide, ND)) void rotate_average_f64(
     const T* __restrict__ vis, const double* __restrict__ uvw, const double* __restrict__ dd, uint32_t D,
     uint32_t groups, uint32_t wpb, uint32_t T_steps, uint32_t nbl, uint32_t C,
-    const double2* __restrict__ lambda2, double* __restrict__ avg) {
+    const double2* __restrict__ lambda2, double* __restrict__ avg, uint64_t* __restrict__ started) {
 #pragma clang fp contract(off)
+    dev::stamp(started);
     constexpr int NV = pow2_at_least(2 * PO * ND);
     __shared__ double2 s_lambda[kLambdaLds];
     __shared__ double2 s_table[dev::kPhasorTable];
@@ -358,7 +359,9 @@ constexpr int32_t kCal1Chunk = 2048;  // antenna sums in LDS at once
 
 __global__ __launch_bounds__(64 * kCal1Groups) void cal1_kernel(const double* __restrict__ avg, uint32_t nbl,
                                                                 uint32_t P, const PhaseRows r,
-                                                                double* __restrict__ cal1) {
+                                                                double* __restrict__ cal1,
+                                                                uint64_t* __restrict__ started) {
+    dev::stamp(started);
     __shared__ double s_b[kCal1Chunk];
     __shared__ double s_part[kCal1Groups][64];
     const uint32_t d = blockIdx.x;
@@ -611,7 +614,7 @@ void launch_rotate_nd(hipStream_t s, const RotateF64& a) {
         rotate_average_f64<T, P, PO, ND, decltype(wide)::value>
             <<<dim3(uint32_t(blocks), a.intervals), 64 * waves, lds, s>>>(static_cast<const T*>(a.vis), a.uvw, a.dd, a.D,
                                                                          groups, a.wpb, a.T, a.nbl, a.C, a.lambda2,
-                                                                         a.avg);
+                                                                         a.avg, a.started);
         LEAP_HIP(hipGetLastError());
     };
     // Wide loads up to 4 directions, where the visibilities are the bound; with 8 their registers
@@ -694,17 +697,17 @@ void launch_assemble_ad(hipStream_t s, const double* Gp, int32_t N, const int2* 
 }
 
 void launch_cal1(hipStream_t s, const leap_metadata& md, const double* avg, uint32_t avg_pols, uint32_t D,
-                 double* cal1) {
+                 double* cal1, uint64_t* started) {
     if (D == 0) return;
     const PhaseRows r = md.rows_of_A1();
-    cal1_kernel<<<dim3(D, uint32_t(r.N + 63) / 64), 64 * kCal1Groups, 0, s>>>(avg, md.nbl, avg_pols, r, cal1);
+    cal1_kernel<<<dim3(D, uint32_t(r.N + 63) / 64), 64 * kCal1Groups, 0, s>>>(avg, md.nbl, avg_pols, r, cal1, started);
     LEAP_HIP(hipGetLastError());
 }
 
 void launch_inversion_f64(hipStream_t s, const leap_metadata& md, const double* avg, uint32_t avg_pols, uint32_t D,
-                          double* cal1, double* sums, double* cal) {
+                          double* cal1, double* sums, double* cal, uint64_t* started) {
     if (D == 0) return;
-    launch_cal1(s, md, avg, avg_pols, D, cal1);
+    launch_cal1(s, md, avg, avg_pols, D, cal1, started);
     const PhaseRows r = md.rows_of_A();
     const dim3 grid(D, uint32_t(r.N + kBlock / 64 - 1) / (kBlock / 64));
     delta_sum_kernel<<<grid, kBlock, 0, s>>>(avg, md.nbl, avg_pols, r, cal1, sums);

@@ -62,12 +62,8 @@ struct WaveArgs {
     double kappa0, dkappa;
     double* avg;  // [interval][D][nbl][pols_out]
     double* q;    // [row][D][4]
+    uint64_t* started;
 };
-
-// a b with fused operations.
-__device__ inline C2<double> cmul_fused(C2<double> a, C2<double> b) {
-    return {fma(a.x, b.x, -(a.y * b.y)), fma(a.x, b.y, a.y * b.x)};
-}
 
 // x of lane 7 - n in lane n of every eight lanes.
 __device__ inline float half_mirror(float x) {
@@ -110,6 +106,7 @@ __attribute__((amdgpu_waves_per_eu(waves_per_simd(sizeof(VT) == 8, ND, Q), 8))) 
 #pragma clang fp contract(off)
     constexpr int K = samples_ahead(2 * P * int(sizeof(VT)));
     constexpr uint32_t CC = kLanes * K;  // channels of a chunk
+    stamp(a.started);
     __shared__ double2 s_table[kPhasorTable];
     __shared__ C2<double> s_part[kWaves][ND][64];
     phasor_table_init(s_table);
@@ -206,9 +203,9 @@ __attribute__((amdgpu_waves_per_eu(waves_per_simd(sizeof(VT) == 8, ND, Q), 8))) 
             const double2 half = phasor_table(s_table, 0.5 * theta), eight = phasor_table(s_table, 8.0 * theta);
             zb[j] = {eight.x, eight.y};
             e[j][0] = {half.x, half.y};
-            const C2<double> z = cmul_fused(e[j][0], e[j][0]);
+            const C2<double> z = cmul(e[j][0], e[j][0]);
 #pragma unroll
-            for (int s = 1; s < 4; ++s) e[j][s] = cmul_fused(e[j][s - 1], z);
+            for (int s = 1; s < 4; ++s) e[j][s] = cmul(e[j][s - 1], z);
             h[j] = {0.0, 0.0};
             if constexpr (Q) g[j] = {0.0, 0.0};
         }
@@ -242,13 +239,13 @@ __attribute__((amdgpu_waves_per_eu(waves_per_simd(sizeof(VT) == 8, ND, Q), 8))) 
 #pragma unroll
             for (int j = 0; j < ND; ++j) {
                 const double2 e0 = phasor_table(s_table, sf[j] * a.kappa0);
-                const C2<double> mid = cmul_fused(C2<double>{e0.x, e0.y}, e[j][3]);  // e0 z^(7/2)
-                const C2<double> r = cmul_fused(mid, h[j]);
+                const C2<double> mid = cmul(C2<double>{e0.x, e0.y}, e[j][3]);  // e0 z^(7/2)
+                const C2<double> r = cmul(mid, h[j]);
                 acc[j].x += r.x;
                 acc[j].y += r.y;
                 if constexpr (Q) {
                     if (direction(j) < d_end) {
-                        const C2<double> r1 = cmul_fused(mid, C2<double>{fma(3.5, h[j].x, g[j].x), fma(3.5, h[j].y, g[j].y)});
+                        const C2<double> r1 = cmul(mid, C2<double>{fma(3.5, h[j].x, g[j].x), fma(3.5, h[j].y, g[j].y)});
                         f64x2* o = reinterpret_cast<f64x2*>(a.q) +
                                    ((rows0 + size_t(t0 + my_t) * a.nbl + my_bl) * a.D + direction(j)) * 2;
                         o[0] = f64x2{r.x, r.y};
@@ -357,7 +354,7 @@ void launch_horner_wave(hipStream_t s, const HornerWave& h) {
     const uint32_t nd = directions_per_lane(h.D, h.nbl, h.intervals, h.q ? kMaxNDQ : kMaxND);
     const uint32_t blocks = (h.D + kLanes * nd - 1) / (kLanes * nd);
     const WaveArgs a{h.uvw, h.dd, h.D, (h.D + blocks - 1) / blocks, h.T, h.nbl, h.C, 0, 0, h.pols_out,
-                     h.f0 / kSpeedOfLight, h.df / kSpeedOfLight, h.avg, h.q};
+                     h.f0 / kSpeedOfLight, h.df / kSpeedOfLight, h.avg, h.q, h.started};
     const bool c64 = h.vis_dtype == LEAP_VIS_C64;
     if (h.q)
         (c64 ? launch_pols<float, true> : launch_pols<double, true>)(s, nd, h.vis, h.P, h.intervals, blocks, a);

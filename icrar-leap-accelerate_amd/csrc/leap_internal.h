@@ -269,6 +269,14 @@ struct leap_ctx {
     hipEvent_t ev_fork = nullptr, ev_packed[2] = {nullptr, nullptr}, ev_consumed[2] = {nullptr, nullptr};
     std::string error;
     hipEvent_t ev_start = nullptr, ev_stop = nullptr;
+    // device clock at the rotate kernel's and the following kernel's start (pinned pair); null where
+    // the call's rotate launches are timed by events.  stamped: the launch took the first
+    leap::PinnedBuffer h_stamps;
+    uint64_t* stamps = nullptr;
+    bool stamped = false;
+    double stamp_ms = 0.0;
+    int32_t stamp_launches = 0;
+    double clock_khz = 0.0;
     std::vector<std::pair<hipEvent_t, hipEvent_t>> rotate_events;
     size_t rotate_events_used = 0;
     std::vector<std::pair<hipEvent_t, hipEvent_t>> pack_events;
@@ -280,7 +288,7 @@ struct leap_ctx {
     // workspace
     leap::DeviceBuffer d_packed;  // pol-0 pack of the staged rows (FP64 complex per row and channel)
     leap::DeviceBuffer d_widen[2];  // complex64 pol-0 chunks from the host, widened into d_packed
-    leap::DeviceBuffer d_uvw, d_vis_stage, d_dirs, d_dd, d_avg, d_cal1, d_sums, d_cal,
+    leap::DeviceBuffer d_uvw, d_vis_stage, d_dd, d_avg, d_cal1, d_sums, d_cal,
         d_partial, d_a_planes;
     leap::DeviceBuffer d_nufft_tail;  // partial sums of the NUFFT launch's chunked last round
     // residual-loss gradient: ENU->UVW rotations, baseline antennas, antenna corrections, perturbed
@@ -299,8 +307,11 @@ struct leap_ctx {
     hipEvent_t ev_grad[4] = {nullptr, nullptr, nullptr, nullptr};  // around the forward and adjoint kernels
     double last_grad_forward_ms = 0.0, last_grad_adjoint_ms = 0.0;
     std::vector<double> h_avg;
-    // calibrations of the last solution interval copied back (pinned, so the copy is a direct DMA)
+    // calibrations of the last group of solution intervals (pinned: written by a kernel or a direct DMA)
     leap::PinnedBuffer h_cal;
+    // directions of the last call (pinned, read by kernels); in use until the stream is waited for
+    leap::PinnedBuffer h_dirs;
+    bool dirs_in_use = false;
     // pseudo-inverse cache keyed by a hash of A (use_cache)
     std::map<uint64_t, std::vector<double>> gram_cache;
     // autotuned direction blocks of the batched kernel
@@ -415,6 +426,7 @@ struct HornerWave {
     double f0, df;
     double* avg;          // [intervals][D][nbl][pols_out]
     double* q = nullptr;  // each row's sums [row][D] = (e0 P(z), e0 z P'(z)), or null
+    uint64_t* started = nullptr;  // set to the device clock by the first workgroup
 };
 // Directions of a wave * 10 + directions of a lane.
 int32_t horner_wave_tile(uint32_t D, uint32_t nbl, uint32_t intervals);
@@ -429,6 +441,7 @@ struct RotateF64 {
     uint32_t D, T, intervals, nbl, C, P, pols_out;  // pols_out: 1 (pol 0) or P
     const double2* lambda2;                         // C pairs (lambda, RN(1 / lambda))
     double* avg;                                    // [intervals][D][nbl][pols_out]
+    uint64_t* started = nullptr;  // set to the device clock by the first workgroup
     uint32_t wpb = 0;                               // waves per baseline, chosen by the launcher
 };
 void launch_rotate_f64(hipStream_t s, const RotateF64& a);
@@ -457,10 +470,11 @@ void launch_assemble_ad(hipStream_t s, const double* Gp, int32_t N, const int2* 
                         int32_t n_pairs, int32_t constraint, double* AdT);
 // cal[D][N] of D directions from pol 0 of avg[D][nbl][avg_pols] in FP64; cal1 and sums: D x N each.
 void launch_inversion_f64(hipStream_t s, const leap_metadata& md, const double* avg, uint32_t avg_pols, uint32_t D,
-                          double* cal1, double* sums, double* cal);
+                          double* cal1, double* sums, double* cal, uint64_t* started = nullptr);
 // cal1 alone, for the mixed GEMM (which forms its operand from avgData and cal1 itself).
+// started: set to the device clock by the first workgroup, where not null.
 void launch_cal1(hipStream_t s, const leap_metadata& md, const double* avg, uint32_t avg_pols, uint32_t D,
-                 double* cal1);
+                 double* cal1, uint64_t* started = nullptr);
 void launch_rotate_batched(hipStream_t s, int32_t precision, int32_t direction_block, bool all_pols,
                            const void* vis, int32_t vis_dtype, const double* uvw, const double* dd, uint32_t D,
                            uint32_t T, uint32_t nbl, uint32_t nbl_grid, uint32_t C, uint32_t P, double f0,

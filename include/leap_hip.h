@@ -460,7 +460,10 @@ int leap_hip_memcpy_h2d(leap_ctx* ctx, void* dst, const void* src, uint64_t byte
 
 /* ---- timing of the last calibrate / rotate call --------------------------- */
 /* Average device time per launch (ms) of the rotate/average kernel and number of
- * launches in the last call, measured with HIP events on the context's stream. */
+ * launches in the last call: from the kernel's first workgroup to the start of the
+ * inversion on the device's clock where a calibration takes one plain or folded Horner
+ * kernel, else by HIP events on the context's stream.  total_ms: HIP events from the
+ * start of the call to the end of its last device work. */
 int leap_hip_last_kernel_times(const leap_ctx* ctx, double* rotate_ms_avg, int32_t* rotate_launches,
                                double* total_ms);
 /* Tile the batched kernel used in the last call: directions per workgroup * 10

@@ -83,3 +83,33 @@ def test_plain_rotate_channel_at_zero_hz(leap, ctx, oracle, dtype):
     s = leap.SynthMS(n_antennas=9, n_timesteps=2, n_channels=9, freq_start_hz=-8e6, freq_inc_hz=2e6, seed=9)
     s.fill_host(dtype)
     _check(leap, ctx, oracle, s.host_dict(), 5, 9, calibrate=False)
+
+
+@pytest.mark.parametrize("opts_kw", [dict(), dict(strategy=1, channel_sum=1)], ids=["plain", "folded"])
+def test_calibrations_and_times_of_small_and_large_results(leap, ctx, opts_kw):
+    """Results up to 32,768 calibrations are written to pinned memory by the inversion, larger ones are
+    copied: a direction's calibrations are the same (1e-9 rad) either way.  The rotate's time is that
+    of one launch and lies inside the call's."""
+    s = leap.SynthMS(n_antennas=20, n_timesteps=2, n_channels=3, seed=20)
+    s.fill_host(np.complex64)
+    ms = s.host_dict()
+    vis = np.ascontiguousarray(ms["vis"])
+    vp, up = ctx.malloc(vis.nbytes), ctx.malloc(ms["uvw"].nbytes)
+    try:
+        ctx.h2d(vp, vis)
+        ctx.h2d(up, np.ascontiguousarray(ms["uvw"]))
+        view = leap.view_from_arrays(ms, vis_device=vp, uvw_device=up, vis_dtype=leap.LEAP_VIS_C64)
+        md = ctx.metadata(view)
+        dirs = np.asarray(ms["phase_centre"]) + np.random.default_rng(20).uniform(-0.02, 0.02, (1639, 2))
+        got = []
+        for n in (1638, 1639):
+            cal, _ = ctx.calibrate(view, dirs[:n], opts=leap.options(**opts_kw), md=md)
+            got.append(cal)
+            ms_rotate, launches, ms_total = ctx.last_kernel_times()
+            assert launches == 1 and 0 < ms_rotate < ms_total
+        assert np.abs(npr.wrap(got[0] - got[1][:, :1638])).max() < 1e-9
+        ctx.calibrate(view, dirs[:3], (0, 1, -1), opts=leap.options(**opts_kw), md=md)  # two solutions, one launch
+        assert ctx.last_kernel_times()[1] == 1
+    finally:
+        ctx.free(vp)
+        ctx.free(up)
