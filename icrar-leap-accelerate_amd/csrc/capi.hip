@@ -127,7 +127,7 @@ void begin_stamps(leap_ctx* ctx) {
         LEAP_HIP(hipDeviceGetAttribute(&khz, hipDeviceAttributeWallClockRate, ctx->device));
         ctx->clock_khz = double(std::max(khz, 1));
     }
-    ctx->h_stamps.reserve(2 * sizeof(uint64_t));
+    ctx->h_stamps.reserve(4 * sizeof(uint64_t));
     ctx->stamps = ctx->h_stamps.as<uint64_t>();
     ctx->stamps[1] = 0;
 }
@@ -1641,7 +1641,6 @@ int leap_hip_create(leap_ctx** out, int32_t device) {
         LEAP_HIP(hipEventCreate(&ctx->ev_start));
         LEAP_HIP(hipEventCreate(&ctx->ev_stop));
         LEAP_HIP(hipEventCreateWithFlags(&ctx->ev_fork, hipEventDisableTiming));
-        for (auto& e : ctx->ev_grad) LEAP_HIP(hipEventCreate(&e));
         for (int b = 0; b < 2; ++b) {
             LEAP_HIP(hipEventCreateWithFlags(&ctx->ev_packed[b], hipEventDisableTiming));
             LEAP_HIP(hipEventCreateWithFlags(&ctx->ev_consumed[b], hipEventDisableTiming));
@@ -1678,8 +1677,6 @@ void leap_hip_destroy(leap_ctx* ctx) {
     if (ctx->ev_start) (void)hipEventDestroy(ctx->ev_start);
     if (ctx->ev_stop) (void)hipEventDestroy(ctx->ev_stop);
     if (ctx->ev_fork) (void)hipEventDestroy(ctx->ev_fork);
-    for (auto& e : ctx->ev_grad)
-        if (e) (void)hipEventDestroy(e);
     for (int b = 0; b < 2; ++b) {
         if (ctx->ev_packed[b]) (void)hipEventDestroy(ctx->ev_packed[b]);
         if (ctx->ev_consumed[b]) (void)hipEventDestroy(ctx->ev_consumed[b]);
@@ -2169,41 +2166,43 @@ extern "C" int leap_hip_residual_loss_grad(leap_ctx* ctx, const leap_metadata* m
         for (uint32_t d = 0; d < 2 * D; ++d) dirs[d] = directions[d] + (offsets ? offsets[d] : 0.0);
         upload_directions(ctx, *md, dirs.data(), D);
         const DeviceRows rows = stage_rows(ctx, *ms, 0, R);
-        // perturbed uvw
-        DeviceBuffer &d_M = ctx->d_adj_M, &d_ants = ctx->d_adj_ants, &d_dp = ctx->d_adj_dp, &d_uvwp = ctx->d_adj_uvw;
-        d_M.reserve(size_t(T) * 9 * sizeof(double));
-        LEAP_HIP(hipMemcpyAsync(d_M.ptr, enu_to_uvw, size_t(T) * 9 * sizeof(double), hipMemcpyHostToDevice, s));
+        // rotations and corrections in one copy; perturbed uvw.  (upload_directions has seen to it that
+        // no earlier call still reads the pinned memory.)
+        DeviceBuffer &d_M = ctx->d_adj_M, &d_ants = ctx->d_adj_ants, &d_uvwp = ctx->d_adj_uvw;
+        const size_t n_M = size_t(T) * 9, n_dp = antenna_delta ? size_t(N) * 3 : 0;
+        d_M.reserve((n_M + n_dp) * sizeof(double));
+        ctx->h_adj_in.reserve((n_M + n_dp) * sizeof(double));
+        double* h_in = ctx->h_adj_in.as<double>();
+        std::copy(enu_to_uvw, enu_to_uvw + n_M, h_in);
+        if (antenna_delta) std::copy(antenna_delta, antenna_delta + n_dp, h_in + n_M);
+        LEAP_HIP(hipMemcpyAsync(d_M.ptr, h_in, (n_M + n_dp) * sizeof(double), hipMemcpyHostToDevice, s));
         const double* uvw = rows.uvw;
         if (antenna_delta) {
-            d_dp.reserve(size_t(N) * 3 * sizeof(double));
             d_uvwp.reserve(size_t(R) * 3 * sizeof(double));
-            LEAP_HIP(hipMemcpyAsync(d_dp.ptr, antenna_delta, size_t(N) * 3 * sizeof(double), hipMemcpyHostToDevice, s));
-            launch_perturb_uvw(s, rows.uvw, d_M.as<double>(), d_ants.as<int2>(), d_dp.as<double>(), nbl, R,
+            launch_perturb_uvw(s, rows.uvw, d_M.as<double>(), d_ants.as<int2>(), d_M.as<double>() + n_M, nbl, R,
                                d_uvwp.as<double>());
             uvw = d_uvwp.as<double>();
         }
         // forward avgData (pol 0), FP64
         ctx->d_avg.reserve(size_t(D) * nbl * 2 * sizeof(double));
         if (row_sums) ctx->d_adj_q.reserve(size_t(R) * D * 4 * sizeof(double));
-        LEAP_HIP(hipEventRecord(ctx->ev_grad[0], s));
+        begin_stamps(ctx);
+        uint64_t* stamps = ctx->stamps;
         launch_horner_wave(s, {rows.vis, ms->vis_dtype, uvw, ctx->d_dd.as<double>(), D, T, 1, nbl, md->channels,
                                md->pols, 1, md->freq_start_hz, md->freq_inc_hz, ctx->d_avg.as<double>(),
-                               row_sums ? ctx->d_adj_q.as<double>() : nullptr});
-        LEAP_HIP(hipEventRecord(ctx->ev_grad[1], s));
+                               row_sums ? ctx->d_adj_q.as<double>() : nullptr, stamp_rotate(ctx)});
         ctx->last_grad_adjoint_ms = 0.0;
         // the inversion (CpuLeapCalibrator.cc:159-178) by the calibration's own kernels
         leap_options inv{};
         invert_directions(ctx, *md, D, inv, nullptr, nullptr, 1);
-        // pol 0 of avgData and its arguments
-        DeviceBuffer& d_avg0 = ctx->d_adj_avg0;
-        d_avg0.reserve(size_t(D) * nbl * 3 * sizeof(double));
-        launch_gather_pol0(s, ctx->d_avg.as<double>(), D * nbl, 1, d_avg0.as<double>());
+        ctx->stamped = false;
         // loss and the adjoint of the inversion, on the device
         const int32_t K = md->A.rows, K1 = md->A1.rows, nI = K - 1;
         const size_t rb = size_t(std::max(1, (nI + 255) / 256));
-        const size_t n_inv = size_t(D) * (size_t(std::max(nI, 1)) * 2 + rb + 1 + size_t(nbl) + 4 * size_t(N));
+        const size_t n_inv = size_t(D) * (size_t(std::max(nI, 1)) + rb + size_t(nbl) + 4 * size_t(N));
         ctx->d_adj_inv.reserve(n_inv * sizeof(double));
-        ctx->d_adj_abar.reserve(size_t(D) * nbl * 2 * sizeof(double));
+        ctx->h_adj_out.reserve((size_t(D) * 3 + size_t(N) * 3) * sizeof(double));
+        double* h_out = ctx->h_adj_out.as<double>();  // losses, dL/d(ra, dec), antenna gradients
         double* w = ctx->d_adj_inv.as<double>();
         auto take = [&](size_t n) {
             double* p = w;
@@ -2217,8 +2216,7 @@ extern "C" int leap_hip_residual_loss_grad(leap_ctx* ctx, const leap_metadata* m
         ia.N = N;
         ia.K1 = K1;
         ia.cal = ctx->d_cal.as<double>();
-        ia.avg0 = d_avg0.as<double>();
-        ia.ph = d_avg0.as<double>() + 2 * size_t(D) * nbl;
+        ia.avg = ctx->d_avg.as<double>();
         ia.pairs = md->d_pairs.as<int2>();
         ia.I = md->d_I.as<int32_t>();
         ia.pairs1 = md->d_pairs1.as<int2>();
@@ -2229,70 +2227,48 @@ extern "C" int leap_hip_residual_loss_grad(leap_ctx* ctx, const leap_metadata* m
         ia.G1p = md->gram(2);
         ia.res = take(size_t(D) * std::max(nI, 1));
         ia.part = take(size_t(D) * rb);
-        ia.loss = take(D);
-        ia.g_arg = take(size_t(D) * nbl);
+        ia.loss = h_out;
+        ia.g_arg = want_grad ? take(size_t(D) * nbl) : nullptr;
         ia.g_cal = take(size_t(D) * N);
         ia.y = take(size_t(D) * N);
-        ia.gacal1 = take(size_t(D) * std::max(nI, 1));
         ia.g_cal1 = take(size_t(D) * N);
         ia.y1 = take(size_t(D) * N);
-        ia.abar = want_grad ? ctx->d_adj_abar.as<double>() : nullptr;
         launch_inversion_adjoint(s, ia);
-        ctx->h_adj_out.reserve((size_t(D) * 3 + size_t(N) * 3) * sizeof(double));
-        double* h_out = ctx->h_adj_out.as<double>();
-        LEAP_HIP(hipMemcpyAsync(h_out, ia.loss, size_t(D) * sizeof(double), hipMemcpyDeviceToHost, s));
-        // The losses are read after the last synchronisation (the gradient's
-        // work is queued behind their copy).
-        auto finish_loss = [&] {
-            float fwd_ms = 0.f;
-            LEAP_HIP(hipEventElapsedTime(&fwd_ms, ctx->ev_grad[0], ctx->ev_grad[1]));
-            ctx->last_grad_forward_ms = fwd_ms;
+        auto finish = [&] {
+            LEAP_HIP(hipStreamSynchronize(s));
+            ctx->dirs_in_use = false;
+            ctx->stamps = nullptr;
+            ctx->last_grad_forward_ms = double(stamps[1] - stamps[0]) / ctx->clock_khz;
             double loss = 0.0;
             for (uint32_t d = 0; d < D; ++d) loss += h_out[d];  // directions in order
             *loss_out = loss;
         };
         if (!want_grad) {
-            LEAP_HIP(hipStreamSynchronize(s));
-            finish_loss();
+            finish();
             return;
         }
         // adjoint of rotate -> average on the device
-        DeviceBuffer &d_abar = ctx->d_adj_abar, &d_guvw = ctx->d_adj_guvw, &d_gdzp = ctx->d_adj_gdzp,
-                     &d_gdz = ctx->d_adj_gdz;
+        DeviceBuffer &d_guvw = ctx->d_adj_guvw, &d_gdzp = ctx->d_adj_gdzp;
         d_guvw.reserve(size_t(R) * 3 * sizeof(double));
         d_gdzp.reserve(size_t(nbl) * D * 3 * sizeof(double));
-        d_gdz.reserve(size_t(D) * 5 * sizeof(double));  // g_dz (3 D), then dL/d(ra, dec) (2 D)
-        LEAP_HIP(hipEventRecord(ctx->ev_grad[2], s));
         if (row_sums)
-            launch_adjoint_q(s, ctx->d_adj_q.as<double>(), uvw, ctx->d_dd.as<double>(), d_abar.as<double>(), D, T, nbl,
-                             md->freq_start_hz, md->freq_inc_hz, d_guvw.as<double>(), d_gdzp.as<double>());
+            launch_adjoint_q(s, ctx->d_adj_q.as<double>(), uvw, ctx->d_dd.as<double>(), ia.avg, ia.g_arg, D, T, nbl,
+                             md->freq_start_hz, md->freq_inc_hz, d_guvw.as<double>(), d_gdzp.as<double>(), stamps + 2);
         else
-            launch_rotate_adjoint(s, rows.vis, ms->vis_dtype, uvw, ctx->d_dd.as<double>(), d_abar.as<double>(), D, T,
-                                  nbl, md->channels, md->pols, md->freq_start_hz, md->freq_inc_hz,
-                                  d_guvw.as<double>(), d_gdzp.as<double>());
-        LEAP_HIP(hipEventRecord(ctx->ev_grad[3], s));
+            launch_rotate_adjoint(s, rows.vis, ms->vis_dtype, uvw, ctx->d_dd.as<double>(), ia.avg, ia.g_arg, D, T, nbl,
+                                  md->channels, md->pols, md->freq_start_hz, md->freq_inc_hz, d_guvw.as<double>(),
+                                  d_gdzp.as<double>(), stamps + 2);
         // dL/d(dz row of dd) reduced over baselines and mapped to dL/d(ra, dec) (MetaData.cc:166-203
         // differentiated) on the device
         launch_reduce_gdz_offsets(s, d_gdzp.as<double>(), nbl, D, md->phase_centre_ra, md->phase_centre_dec,
-                                  ctx->h_dirs.as<double>(), d_gdz.as<double>());
-        if (grad_offsets)
-            LEAP_HIP(hipMemcpyAsync(h_out + D, d_gdz.as<double>() + 3 * size_t(D), size_t(D) * 2 * sizeof(double),
-                                    hipMemcpyDeviceToHost, s));
-        if (grad_antenna) {
-            DeviceBuffer& d_gant = ctx->d_adj_gant;
-            d_gant.reserve(size_t(N) * 3 * sizeof(double));
+                                  ctx->h_dirs.as<double>(), h_out + D, stamps + 3);
+        if (grad_antenna)
             launch_antenna_grad(s, d_guvw.as<double>(), d_M.as<double>(), ctx->d_adj_off.as<int32_t>(),
                                 ctx->d_adj_bls.as<int32_t>(), ctx->d_adj_sgn.as<int32_t>(), N, nbl, T,
-                                d_gant.as<double>());
-            LEAP_HIP(hipMemcpyAsync(h_out + 3 * size_t(D), d_gant.ptr, size_t(N) * 3 * sizeof(double),
-                                    hipMemcpyDeviceToHost, s));
-        }
-        LEAP_HIP(hipStreamSynchronize(s));
-        finish_loss();
+                                h_out + 3 * size_t(D));
+        finish();
+        ctx->last_grad_adjoint_ms = double(stamps[3] - stamps[2]) / ctx->clock_khz;
         if (grad_antenna) std::copy(h_out + 3 * size_t(D), h_out + 3 * size_t(D) + size_t(N) * 3, grad_antenna);
-        float adj_ms = 0.f;
-        LEAP_HIP(hipEventElapsedTime(&adj_ms, ctx->ev_grad[2], ctx->ev_grad[3]));
-        ctx->last_grad_adjoint_ms = adj_ms;
         if (grad_offsets) std::copy(h_out + D, h_out + 3 * size_t(D), grad_offsets);
     });
 }

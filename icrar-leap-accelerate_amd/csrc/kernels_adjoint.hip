@@ -33,6 +33,22 @@ __device__ inline Cx cmulx(Cx a, Cx b) { return {a.x * b.x - a.y * b.y, a.x * b.
 __device__ inline Cx hstep(Cx a, Cx z, Cx v) {
     return {fma(a.x, z.x, fma(-a.y, z.y, v.x)), fma(a.x, z.y, fma(a.y, z.x, v.y))};
 }
+// Sum of the 64 lanes' values of a wave by a butterfly of xor shuffles: a fixed
+// order, so every lane gets the same bits on every run.
+__device__ inline double wave_sum(double v) {
+#pragma unroll
+    for (int m = 32; m >= 1; m >>= 1) v += __shfl_xor(v, m, 64);
+    return v;
+}
+
+// dL/dRe avg + i dL/dIm avg = i g / conj(z) = (-g y / |z|^2, g x / |z|^2) from g = dL/d arg z, 0 where
+// z = avg is 0.
+__device__ inline Cx abar_of(const double* __restrict__ avg, const double* __restrict__ g_arg, size_t i) {
+#pragma clang fp contract(off)
+    const double x = avg[2 * i], y = avg[2 * i + 1], m = x * x + y * y, g = g_arg[i];
+    return m == 0.0 ? Cx{0.0, 0.0} : Cx{-g * y / m, g * x / m};
+}
+
 __device__ inline Cx expi(double t) {
     double s, c;
     sincos(t, &s, &c);
@@ -65,8 +81,10 @@ __global__ void perturb_uvw_kernel(const double* __restrict__ uvw0, const double
 template <typename VT, int DL, int ND>
 __global__ __launch_bounds__(kThreads) void rotate_adjoint_kernel(
     const VT* __restrict__ vis, const double* __restrict__ uvw, const double* __restrict__ dd,
-    const double* __restrict__ abar, uint32_t D, uint32_t T, uint32_t nbl, uint32_t C, uint32_t P, double kappa0,
-    double dkappa, double* __restrict__ g_uvw, double* __restrict__ g_dz_partial) {
+    const double* __restrict__ avg, const double* __restrict__ g_arg, uint32_t D, uint32_t T, uint32_t nbl, uint32_t C,
+    uint32_t P, double kappa0, double dkappa, double* __restrict__ g_uvw, double* __restrict__ g_dz_partial,
+    uint64_t* __restrict__ started) {
+    dev::stamp(started);
     constexpr int RP = kThreads / DL;
     constexpr int kCC = 256 / RP > 16 ? 256 / RP : 16;  // channels per chunk
     constexpr int DW = DL * ND;                          // directions of the workgroup
@@ -93,7 +111,7 @@ __global__ __launch_bounds__(kThreads) void rotate_adjoint_kernel(
         dz[j][1] = dd[9 * dc + 7];
         dz[j][2] = dd[9 * dc + 8];
         ab[j] = Cx{0.0, 0.0};
-        if (dir_ok[j]) ab[j] = {abar[2 * (size_t(dc) * nbl + bl)], abar[2 * (size_t(dc) * nbl + bl) + 1]};
+        if (dir_ok[j]) ab[j] = abar_of(avg, g_arg, size_t(dc) * nbl + bl);
         gdz[j][0] = gdz[j][1] = gdz[j][2] = 0.0;
     }
     const uint32_t n_chunks = (C + kCC - 1) / kCC;
@@ -206,7 +224,7 @@ __global__ __launch_bounds__(kThreads) void rotate_adjoint_kernel(
             for (int k = 0; k < 3; ++k) {
                 double s = 0.0;
                 for (int r = 0; r < RP; ++r) s += s_g[r][dj][k];
-                g_dz_partial[(size_t(bl) * D + dj) * 3 + k] = s;
+                g_dz_partial[size_t(3 * dj + k) * nbl + bl] = s;
             }
         }
     }
@@ -214,22 +232,31 @@ __global__ __launch_bounds__(kThreads) void rotate_adjoint_kernel(
 
 // The same outputs from the forward pass's per-row sums q[row][d] = (e0 P(z),
 // e0 z P'(z)) (horner_wave_kernel's q), so the cube is not read
-// again: s1 = kappa0 q0 + dkappa q1 is the sum above.  Lanes, rows and the
-// reductions as in rotate_adjoint_kernel.
+// again: s1 = kappa0 q0 + dkappa q1 is the sum above.  A row's
+// directions lie in one wave (DL lanes with ND directions each), so its sums over
+// the directions are exchanged between lanes and the rows need no barrier.  A wave takes 64 / DL
+// baselines side by side, whose rows lie side by side in q, uvw and g_uvw, and the workgroup's four
+// waves their timesteps in turn.  Bound by reading q: 128 stations, 64 t, 16 directions
+// (266 MB) 69 us (4.2 TB/s with the gradients written) against 81 with a
+// baseline a workgroup and the sums in LDS behind two barriers a row.
 template <int DL, int ND>
 __global__ __launch_bounds__(kThreads) void adjoint_q_kernel(const double* __restrict__ q,
                                                              const double* __restrict__ uvw,
                                                              const double* __restrict__ dd,
-                                                             const double* __restrict__ abar, uint32_t D, uint32_t T,
+                                                             const double* __restrict__ avg,
+                                                             const double* __restrict__ g_arg, uint32_t D, uint32_t T,
                                                              uint32_t nbl, double kappa0, double dkappa,
                                                              double* __restrict__ g_uvw,
-                                                             double* __restrict__ g_dz_partial) {
-    constexpr int RP = kThreads / DL;
+                                                             double* __restrict__ g_dz_partial,
+                                                             uint64_t* __restrict__ started) {
+    dev::stamp(started);
+    static_assert(DL <= 64, "a row's directions in one wave");
+    constexpr int BB = 64 / DL, kW = kThreads / 64;
     constexpr int DW = DL * ND;
-    __shared__ double s_g[RP][DW][3];
-    const uint32_t bl = blockIdx.x;
-    const uint32_t lane_d = threadIdx.x % DL;
-    const uint32_t rsub = threadIdx.x / DL;
+    __shared__ double s_g[kW][BB][DW][3];
+    const uint32_t lane_d = threadIdx.x % DL, sub = threadIdx.x % 64 / DL, wave = threadIdx.x / 64;
+    const bool bl_ok = blockIdx.x * BB + sub < nbl;
+    const uint32_t bl = min(blockIdx.x * BB + sub, nbl - 1);
     bool dir_ok[ND];
     double dz[ND][3], gdz[ND][3];
     Cx ab[ND];
@@ -242,136 +269,117 @@ __global__ __launch_bounds__(kThreads) void adjoint_q_kernel(const double* __res
         dz[j][1] = dd[9 * dc + 7];
         dz[j][2] = dd[9 * dc + 8];
         ab[j] = Cx{0.0, 0.0};
-        if (dir_ok[j]) ab[j] = {abar[2 * (size_t(dc) * nbl + bl)], abar[2 * (size_t(dc) * nbl + bl) + 1]};
+        if (dir_ok[j]) ab[j] = abar_of(avg, g_arg, size_t(dc) * nbl + bl);
         gdz[j][0] = gdz[j][1] = gdz[j][2] = 0.0;
     }
-    for (uint32_t tb = 0; tb < T; tb += RP) {
-        const uint32_t t = tb + rsub;
-        const bool row_ok = t < T;
+    for (uint32_t t = wave; t < T; t += kW) {
         const size_t row = size_t(t) * nbl + bl;
-        double u = 0.0, v = 0.0, w = 0.0;
-        if (row_ok) {
-            u = uvw[3 * row];
-            v = uvw[3 * row + 1];
-            w = uvw[3 * row + 2];
-        }
+        const double u = uvw[3 * row], v = uvw[3 * row + 1], w = uvw[3 * row + 2];
+        double g[3] = {0.0, 0.0, 0.0};
 #pragma unroll
         for (int j = 0; j < ND; ++j) {
+            const double2* qp = reinterpret_cast<const double2*>(q) + (row * D + min(lane_d + DL * j, D - 1)) * 2;
+            const double2 q0 = qp[0], q1 = qp[1];
             double gsf = 0.0;
-            if (row_ok && dir_ok[j]) {
-                const double* qp = q + (row * D + lane_d + DL * j) * 4;
-                const Cx s1 = {kappa0 * qp[0] + dkappa * qp[2], kappa0 * qp[1] + dkappa * qp[3]};
+            if (dir_ok[j]) {
+                const Cx s1 = {kappa0 * q0.x + dkappa * q1.x, kappa0 * q0.y + dkappa * q1.y};
                 gsf = -ab[j].x * s1.y + ab[j].y * s1.x;
                 gdz[j][0] += -kTwoPi * gsf * u;
                 gdz[j][1] += -kTwoPi * gsf * v;
                 gdz[j][2] += -kTwoPi * gsf * w;
             }
-            s_g[rsub][lane_d + DL * j][0] = -kTwoPi * gsf * dz[j][0];
-            s_g[rsub][lane_d + DL * j][1] = -kTwoPi * gsf * dz[j][1];
-            s_g[rsub][lane_d + DL * j][2] = -kTwoPi * gsf * (dz[j][2] - 1.0);
+            g[0] += -kTwoPi * gsf * dz[j][0];
+            g[1] += -kTwoPi * gsf * dz[j][1];
+            g[2] += -kTwoPi * gsf * (dz[j][2] - 1.0);
         }
-        __syncthreads();
-        if (lane_d < 3 && row_ok) {
-            double s = 0.0;
-            for (int j = 0; j < DW; ++j) s += s_g[rsub][j][lane_d];  // direction order
-            g_uvw[3 * row + lane_d] = s;
-        }
-        __syncthreads();
+#pragma unroll
+        for (int m = DL / 2; m > 0; m /= 2)
+#pragma unroll
+            for (int k = 0; k < 3; ++k) g[k] += __shfl_xor(g[k], m, 64);
+        if (lane_d < 3 && bl_ok) g_uvw[3 * row + lane_d] = lane_d == 0 ? g[0] : lane_d == 1 ? g[1] : g[2];
     }
 #pragma unroll
     for (int j = 0; j < ND; ++j)
-        for (int k = 0; k < 3; ++k) s_g[rsub][lane_d + DL * j][k] = dir_ok[j] ? gdz[j][k] : 0.0;
+        for (int k = 0; k < 3; ++k) s_g[wave][sub][lane_d + DL * j][k] = dir_ok[j] ? gdz[j][k] : 0.0;
     __syncthreads();
-    if (rsub == 0) {
-#pragma unroll
-        for (int j = 0; j < ND; ++j) {
-            if (!dir_ok[j]) continue;
-            const uint32_t dj = lane_d + DL * j;
-            for (int k = 0; k < 3; ++k) {
-                double s = 0.0;
-                for (int r = 0; r < RP; ++r) s += s_g[r][dj][k];
-                g_dz_partial[(size_t(bl) * D + dj) * 3 + k] = s;
-            }
-        }
+    for (uint32_t i = threadIdx.x; i < 3 * D * BB; i += kThreads) {
+        const uint32_t b = i % BB, o = i / BB;  // baselines fastest
+        if (blockIdx.x * BB + b >= nbl) continue;
+        double s = 0.0;
+        for (int w = 0; w < kW; ++w) s += s_g[w][b][o / 3][o % 3];
+        g_dz_partial[size_t(o) * nbl + blockIdx.x * BB + b] = s;
     }
 }
 
-// g_dz[d][k] = sum over baselines of g_dz_partial[b][d][k]: one workgroup per output
-// i = 3 d + k, each lane a strided slice of the baselines, then a fixed-order tree in LDS.
-__global__ __launch_bounds__(256) void reduce_gdz_kernel(const double* __restrict__ part, uint32_t nbl, uint32_t D,
-                                                         double* __restrict__ out) {
-    __shared__ double s_red[256];
-    const uint32_t i = blockIdx.x, n_out = 3 * D;
-    double acc = 0.0;
-    for (uint32_t b = threadIdx.x; b < nbl; b += 256) acc += part[size_t(b) * n_out + i];
-    s_red[threadIdx.x] = acc;
-    __syncthreads();
-    for (uint32_t stride = 128; stride > 0; stride >>= 1) {
-        if (threadIdx.x < stride) s_red[threadIdx.x] += s_red[threadIdx.x + stride];
-        __syncthreads();
-    }
-    if (threadIdx.x == 0) out[i] = s_red[0];
-}
-
-// dL/d(ra, dec) of direction d from g_dz[d] = dL/d(row 2 of its DD matrix): the
-// derivatives of dd row 2 = R_x(-pi/2 + dec) R_z(ra - ra0) R_x(pi/2 - dec0) row 2
-// (MetaData.cc:166-203) in ra and dec; dirs[d] = (ra, dec).  One thread per direction.
-__global__ void gdz_offsets_kernel(const double* __restrict__ g_dz, uint32_t D, double ra0, double dec0,
-                                   const double* __restrict__ dirs, double* __restrict__ out) {
+// g_dz[k] = sum over the baselines of g_dz_partial[3 d + k][b] = dL/d(row 2 of direction d's DD matrix),
+// then dL/d(ra, dec) = out[2 d], out[2 d + 1] by the derivatives of dd row 2 = R_x(-pi/2 + dec)
+// R_z(ra - ra0) R_x(pi/2 - dec0) row 2 (MetaData.cc:166-203) in ra and dec; dirs[d] = (ra, dec).
+// One workgroup per direction: strided slices of the baselines, then lanes and waves in order.
+constexpr int kReduceWaves = 16;
+__global__ __launch_bounds__(64 * kReduceWaves) void reduce_gdz_kernel(const double* __restrict__ part, uint32_t nbl,
+                                                                      double ra0, double dec0,
+                                                                      const double* __restrict__ dirs,
+                                                                      double* __restrict__ out,
+                                                                      uint64_t* __restrict__ started) {
 #pragma clang fp contract(off)
-    const uint32_t d = blockIdx.x * blockDim.x + threadIdx.x;
-    if (d >= D) return;
+    dev::stamp(started);
+    __shared__ double s_red[kReduceWaves][3];
+    const uint32_t d = blockIdx.x;
+    double acc[3] = {0.0, 0.0, 0.0};
+    for (uint32_t b = threadIdx.x; b < nbl; b += 64 * kReduceWaves)
+        for (int k = 0; k < 3; ++k) acc[k] += part[size_t(3 * d + k) * nbl + b];
+    for (int k = 0; k < 3; ++k) {
+        const double w = wave_sum(acc[k]);
+        if (threadIdx.x % 64 == 0) s_red[threadIdx.x / 64][k] = w;
+    }
+    __syncthreads();
+    if (threadIdx.x != 0) return;
+    double g[3] = {0.0, 0.0, 0.0};
+    for (int w = 0; w < kReduceWaves; ++w)
+        for (int k = 0; k < 3; ++k) g[k] += s_red[w][k];
     double s1, c1, s2, c2, s3, c3;
     sincos(kPi / 2.0 - dec0, &s1, &c1);
     sincos(dirs[2 * d] - ra0, &s2, &c2);
     sincos(-kPi / 2.0 + dirs[2 * d + 1], &s3, &c3);
     const double dra[3] = {-s3 * c2, -s3 * s2 * c1, s3 * s2 * s1};
     const double ddec[3] = {-c3 * s2, c3 * c2 * c1 - s3 * s1, -c3 * c2 * s1 - s3 * c1};
-    const double* g = g_dz + 3 * size_t(d);
     out[2 * size_t(d)] = g[0] * dra[0] + g[1] * dra[1] + g[2] * dra[2];
     out[2 * size_t(d) + 1] = g[0] * ddec[0] + g[1] * ddec[1] + g[2] * ddec[2];
 }
 
-// For the n = D nbl (direction, baseline) entries of P pols each: out[2 i], out[2 i + 1] = pol 0
-// of avg[i], and out[2 n + i] = its argument atan2(im, re).
-__global__ void gather_pol0_kernel(const double* __restrict__ avg, uint32_t n, uint32_t P, double* __restrict__ out) {
-    const uint32_t i = blockIdx.x * blockDim.x + threadIdx.x;
-    if (i >= n) return;
-    const double re = avg[size_t(i) * P * 2], im = avg[size_t(i) * P * 2 + 1];
-    out[2 * size_t(i)] = re;
-    out[2 * size_t(i) + 1] = im;
-    out[2 * size_t(n) + i] = atan2(im, re);
-}
-
 // One workgroup per antenna: sum over its baselines (sign +1 as antenna2, -1 as
-// antenna1) and timesteps of M_t^T g_uvw(t, b).
-__global__ __launch_bounds__(256) void antenna_grad_kernel(const double* __restrict__ g_uvw,
-                                                           const double* __restrict__ M,
-                                                           const int32_t* __restrict__ csr_off,
-                                                           const int32_t* __restrict__ csr_bl,
-                                                           const int32_t* __restrict__ csr_sign, uint32_t nbl,
-                                                           uint32_t T, double* __restrict__ out) {
-    __shared__ double s_red[256][3];
+// antenna1) and timesteps of M_t^T g_uvw(t, b); a wave takes whole timesteps.
+__global__ __launch_bounds__(64 * kReduceWaves) void antenna_grad_kernel(const double* __restrict__ g_uvw,
+                                                                        const double* __restrict__ M,
+                                                                        const int32_t* __restrict__ csr_off,
+                                                                        const int32_t* __restrict__ csr_bl,
+                                                                        const int32_t* __restrict__ csr_sign,
+                                                                        uint32_t nbl, uint32_t T,
+                                                                        double* __restrict__ out) {
+    __shared__ double s_red[kReduceWaves][3];
     const int32_t a = blockIdx.x;
     const int32_t j0 = csr_off[a], j1 = csr_off[a + 1];
-    const uint32_t nj = uint32_t(j1 - j0);
+    const uint32_t lane = threadIdx.x % 64, wave = threadIdx.x / 64;
     double acc[3] = {0.0, 0.0, 0.0};
-    for (uint32_t i = threadIdx.x; i < nj * T; i += 256) {
-        const uint32_t t = i / nj, j = i - t * nj;
-        const int32_t b = csr_bl[j0 + j];
-        const double sgn = double(csr_sign[j0 + j]);
-        const double* g = g_uvw + 3 * (size_t(t) * nbl + b);
-        const double* m = M + 9 * size_t(t);
-        for (int k = 0; k < 3; ++k) acc[k] += sgn * (m[k] * g[0] + m[3 + k] * g[1] + m[6 + k] * g[2]);
+    for (int32_t j = j0 + int32_t(lane); j < j1; j += 64) {
+        const double sgn = double(csr_sign[j]);
+        const double* g_b = g_uvw + 3 * size_t(csr_bl[j]);
+#pragma unroll 4
+        for (uint32_t t = wave; t < T; t += kReduceWaves) {
+            const double* m = M + 9 * size_t(t);
+            const double* g = g_b + 3 * size_t(t) * nbl;
+            for (int k = 0; k < 3; ++k) acc[k] += sgn * (m[k] * g[0] + m[3 + k] * g[1] + m[6 + k] * g[2]);
+        }
     }
-    for (int k = 0; k < 3; ++k) s_red[threadIdx.x][k] = acc[k];
+    for (int k = 0; k < 3; ++k) {
+        const double w = wave_sum(acc[k]);
+        if (lane == 0) s_red[wave][k] = w;
+    }
     __syncthreads();
-    for (int stride = 128; stride > 0; stride >>= 1) {
-        if (int(threadIdx.x) < stride)
-            for (int k = 0; k < 3; ++k) s_red[threadIdx.x][k] += s_red[threadIdx.x + stride][k];
-        __syncthreads();
-    }
-    if (threadIdx.x < 3) out[3 * a + threadIdx.x] = s_red[0][threadIdx.x];
+    if (threadIdx.x >= 3) return;
+    double s = 0.0;
+    for (int w = 0; w < kReduceWaves; ++w) s += s_red[w][threadIdx.x];
+    out[3 * a + threadIdx.x] = s;
 }
 
 // ---------------------------------------------------------------------------
@@ -388,27 +396,35 @@ __global__ __launch_bounds__(256) void antenna_grad_kernel(const double* __restr
 //   y1 = G1+ g_cal1;  g_arg[I1(k)] += y1[a1'(k)] - y1[a2'(k)]
 //   abar[b] = i g_arg[b] / conj(avg[b])   (d arg z = Im(dz / z))
 // The antenna sums A^T v are gathers over each antenna's rows (CSR, in row
-// order), so every sum has a fixed order and no atomics are used.
+// order), so every sum has a fixed order and no atomics are used.  Each step waits for
+// the one before and takes a launch's 5 us, so what a step needs of a row is formed where it is
+// used, by each antenna's wave again, and independent work shares a launch (blocks by role):
+// six launches, where one per line above took twelve.
 // ---------------------------------------------------------------------------
 __device__ inline double wrap_pi(double x) {
 #pragma clang fp contract(off)
     return x - kTwoPi * floor((x + kPi) / kTwoPi);
 }
 
-// res[d][n] and per-workgroup sums of res^2 (fixed-order tree) into part[d][block].
+// res[d][n], per-workgroup sums of res^2 (fixed-order tree) into part[d][block], and
+// g_arg[d][b] = 0 for every baseline.
 __global__ __launch_bounds__(256) void inv_residual_kernel(const double* __restrict__ cal, int32_t N,
                                                            const int2* __restrict__ pairs, const int32_t* __restrict__ I,
-                                                           int32_t nI, const double* __restrict__ ph, uint32_t nbl,
-                                                           double* __restrict__ res, double* __restrict__ part) {
+                                                           int32_t nI, const double* __restrict__ avg, uint32_t nbl,
+                                                           double* __restrict__ res, double* __restrict__ part,
+                                                           double* __restrict__ g_arg) {
 #pragma clang fp contract(off)
     __shared__ double s_red[256];
     const int32_t n = blockIdx.x * 256 + threadIdx.x;
     const uint32_t d = blockIdx.y;
+    if (g_arg)
+        for (uint32_t b = blockIdx.x * 256 + threadIdx.x; b < nbl; b += gridDim.x * 256) g_arg[size_t(d) * nbl + b] = 0.0;
     double r2 = 0.0;
     if (n < nI) {
         const int2 p = pairs[n];
         const double* c = cal + size_t(d) * N;
-        const double r = wrap_pi(c[p.x] - c[p.y] - ph[size_t(d) * nbl + I[n]]);
+        const double* z = avg + 2 * (size_t(d) * nbl + I[n]);
+        const double r = wrap_pi(c[p.x] - c[p.y] - atan2(z[1], z[0]));
         res[size_t(d) * nI + n] = r;
         r2 = r * r;
     }
@@ -421,65 +437,51 @@ __global__ __launch_bounds__(256) void inv_residual_kernel(const double* __restr
     if (threadIdx.x == 0) part[size_t(d) * gridDim.x + blockIdx.x] = s_red[0];
 }
 
-// loss[d] = sum of the workgroup sums in block order.
-__global__ void inv_loss_kernel(const double* __restrict__ part, uint32_t blocks, uint32_t D,
-                                double* __restrict__ loss) {
-    const uint32_t d = blockIdx.x * blockDim.x + threadIdx.x;
-    if (d >= D) return;
-    double s = 0.0;
-    for (uint32_t k = 0; k < blocks; ++k) s += part[size_t(d) * blocks + k];
-    loss[d] = s;
-}
-
-// g_arg[d][b] = 0 for every baseline, then -2 res[n] at b = I(n) (I is one-to-one).
-__global__ void inv_garg_init_kernel(double* __restrict__ g_arg, uint32_t nbl) {
-    const uint32_t b = blockIdx.x * blockDim.x + threadIdx.x;
-    if (b < nbl) g_arg[size_t(blockIdx.y) * nbl + b] = 0.0;
-}
-
-__global__ void inv_garg_res_kernel(const double* __restrict__ res, const int32_t* __restrict__ I, int32_t nI,
-                                    uint32_t nbl, double* __restrict__ g_arg) {
+// The sum over antenna a's rows e of sign_e value(row_e), on every lane of a wave; csr_ent[e] =
+// 2 row + (sign < 0).  Lane l sums entries l, l + 64, ... in order, then wave_sum.
+template <typename F>
+__device__ inline double antenna_sum(const int32_t* __restrict__ csr_off, const int32_t* __restrict__ csr_ent, int32_t a,
+                                     F&& value) {
 #pragma clang fp contract(off)
-    const int32_t n = blockIdx.x * blockDim.x + threadIdx.x;
-    const uint32_t d = blockIdx.y;
-    if (n >= nI) return;
-    double& g = g_arg[size_t(d) * nbl + I[n]];
-    g -= 2.0 * res[size_t(d) * nI + n];
-}
-
-// Sum of the 64 lanes' values of a wave by a butterfly of xor shuffles: a fixed
-// order, so every lane gets the same bits on every run.
-__device__ inline double wave_sum(double v) {
-#pragma unroll
-    for (int m = 32; m >= 1; m >>= 1) v += __shfl_xor(v, m, 64);
-    return v;
-}
-
-// out[d][a] = (base ? base[d][a] : 0) + sum over antenna a's rows e of
-// sign_e * scale * src[d][row_e]; csr_ent[e] = 2 row + (sign < 0).  One wave
-// per (a, d) (four per workgroup): lane l sums entries l, l + 64, ... in order,
-// then the lanes are summed by wave_sum.
-__global__ __launch_bounds__(256) void inv_antenna_sum_kernel(const double* __restrict__ src, int32_t nI,
-                                                              double scale, const int32_t* __restrict__ csr_off,
-                                                              const int32_t* __restrict__ csr_ent, int32_t N,
-                                                              const double* __restrict__ base,
-                                                              double* __restrict__ out) {
-#pragma clang fp contract(off)
-    const int32_t a = int32_t(blockIdx.x * 4 + threadIdx.x / 64);
-    const uint32_t lane = threadIdx.x % 64, d = blockIdx.y;
-    if (a >= N) return;  // whole waves
-    const double* x = src + size_t(d) * nI;
     double acc = 0.0;
-    for (int32_t e = csr_off[a] + int32_t(lane); e < csr_off[a + 1]; e += 64) {
+    for (int32_t e = csr_off[a] + int32_t(threadIdx.x % 64); e < csr_off[a + 1]; e += 64) {
         const int32_t v = csr_ent[e];
-        const double t = scale * x[v >> 1];
+        const double t = value(v >> 1);
         if (v & 1)
             acc -= t;
         else
             acc += t;
     }
-    acc = wave_sum(acc);
-    if (lane == 0) out[size_t(d) * N + a] = (base ? base[size_t(d) * N + a] : 0.0) + acc;
+    return wave_sum(acc);
+}
+
+// Blocks of direction blockIdx.y by role: the first ga take four antennas each (a wave an antenna),
+// g_cal[d][a] = the antenna's sum of 2 res; the next gn take 256 rows each, g_arg[d][I(n)] -= 2 res[n]
+// (I is one-to-one); the last one adds the residual's workgroup sums in block order, loss[d].
+__global__ __launch_bounds__(256) void inv_residual_grad_kernel(const double* __restrict__ res, int32_t nI,
+                                                                const int32_t* __restrict__ I,
+                                                                const int32_t* __restrict__ csr_off,
+                                                                const int32_t* __restrict__ csr_ent, int32_t N,
+                                                                uint32_t ga, uint32_t gn, uint32_t nbl,
+                                                                const double* __restrict__ part, uint32_t parts,
+                                                                double* __restrict__ g_cal, double* __restrict__ g_arg,
+                                                                double* __restrict__ loss) {
+#pragma clang fp contract(off)
+    const uint32_t d = blockIdx.y, role = blockIdx.x;
+    const double* x = res + size_t(d) * nI;
+    if (role < ga) {
+        const int32_t a = int32_t(role * 4 + threadIdx.x / 64);
+        if (a >= N) return;  // whole waves
+        const double s = antenna_sum(csr_off, csr_ent, a, [&](int32_t n) { return 2.0 * x[n]; });
+        if (threadIdx.x % 64 == 0) g_cal[size_t(d) * N + a] = s;
+    } else if (role < ga + gn) {
+        const int32_t n = int32_t((role - ga) * 256 + threadIdx.x);
+        if (n < nI) g_arg[size_t(d) * nbl + I[n]] -= 2.0 * x[n];
+    } else if (threadIdx.x == 0) {
+        double s = 0.0;
+        for (uint32_t k = 0; k < parts; ++k) s += part[size_t(d) * parts + k];
+        loss[d] = s;
+    }
 }
 
 // y[d][a] = sum_i Gp[a N + i] g[d][i] (Gp is symmetric, so column a is row a):
@@ -498,17 +500,30 @@ __global__ __launch_bounds__(256) void inv_gram_gemv_kernel(const double* __rest
     if (lane == 0) y[size_t(d) * N + a] = t;
 }
 
-// g = y[a1(n)] - y[a2(n)]: g_arg[d][n] += g (row n of avgData), gacal1[d][n] = -2 pi g.
-__global__ void inv_rows_kernel(const double* __restrict__ y, int32_t N, const int2* __restrict__ pairs, int32_t nI,
-                                uint32_t nbl, double* __restrict__ g_arg, double* __restrict__ gacal1) {
+// With g(n) = y[a1(n)] - y[a2(n)], blocks by role as above: g_cal1[d][a] = g_cal[d][a] + the antenna's
+// sum of -2 pi g; g_arg[d][n] += g (row n of avgData).
+__global__ __launch_bounds__(256) void inv_rows_kernel(const double* __restrict__ y, int32_t N,
+                                                       const int2* __restrict__ pairs, int32_t nI,
+                                                       const int32_t* __restrict__ csr_off,
+                                                       const int32_t* __restrict__ csr_ent, uint32_t ga, uint32_t nbl,
+                                                       const double* __restrict__ g_cal, double* __restrict__ g_cal1,
+                                                       double* __restrict__ g_arg) {
 #pragma clang fp contract(off)
-    const int32_t n = blockIdx.x * blockDim.x + threadIdx.x;
-    const uint32_t d = blockIdx.y;
-    if (n >= nI) return;
-    const int2 p = pairs[n];
-    const double g = y[size_t(d) * N + p.x] - y[size_t(d) * N + p.y];
-    g_arg[size_t(d) * nbl + n] += g;
-    gacal1[size_t(d) * nI + n] = -kTwoPi * g;
+    const uint32_t d = blockIdx.y, role = blockIdx.x;
+    const double* yd = y + size_t(d) * N;
+    auto g = [&](int32_t n) {
+        const int2 p = pairs[n];
+        return yd[p.x] - yd[p.y];
+    };
+    if (role < ga) {
+        const int32_t a = int32_t(role * 4 + threadIdx.x / 64);
+        if (a >= N) return;  // whole waves
+        const double s = antenna_sum(csr_off, csr_ent, a, [&](int32_t n) { return -kTwoPi * g(n); });
+        if (threadIdx.x % 64 == 0) g_cal1[size_t(d) * N + a] = g_cal[size_t(d) * N + a] + s;
+    } else {
+        const int32_t n = int32_t((role - ga) * 256 + threadIdx.x);
+        if (n < nI) g_arg[size_t(d) * nbl + n] += g(n);
+    }
 }
 
 // g_arg[d][I1(k)] += y1[a1'(k)] - y1[a2'(k)] (I1 is one-to-one).
@@ -525,55 +540,31 @@ __global__ void inv_rows1_kernel(const double* __restrict__ y1, int32_t N, const
     g_arg[size_t(d) * nbl + b] += y1[size_t(d) * N + p.x] - y1[size_t(d) * N + p.y];
 }
 
-// abar[d][b] = i g / conj(z) = (-g y / |z|^2, g x / |z|^2), 0 where z = 0; z = avg0[d][b].
-__global__ void inv_abar_kernel(const double* __restrict__ avg0, const double* __restrict__ g_arg, uint32_t n,
-                                double* __restrict__ abar) {
-#pragma clang fp contract(off)
-    const uint32_t i = blockIdx.x * blockDim.x + threadIdx.x;
-    if (i >= n) return;
-    const double x = avg0[2 * size_t(i)], y = avg0[2 * size_t(i) + 1], m = x * x + y * y;
-    const double g = g_arg[i];
-    abar[2 * size_t(i)] = m == 0.0 ? 0.0 : -g * y / m;
-    abar[2 * size_t(i) + 1] = m == 0.0 ? 0.0 : g * x / m;
-}
-
 }  // namespace
 
 void launch_inversion_adjoint(hipStream_t s, const InversionAdjoint& a) {
     const int32_t nI = a.K - 1, nI1 = a.K1 - 1;
     const uint32_t D = a.D, nbl = a.nbl;
-    const uint32_t rb = uint32_t(std::max(1, (nI + 255) / 256));
-    inv_residual_kernel<<<dim3(rb, D), 256, 0, s>>>(a.cal, a.N, a.pairs, a.I, nI, a.ph, nbl, a.res, a.part);
+    const uint32_t gn = uint32_t(std::max(1, (nI + 255) / 256)), ga = uint32_t(a.N + 3) / 4;
+    inv_residual_kernel<<<dim3(gn, D), 256, 0, s>>>(a.cal, a.N, a.pairs, a.I, nI, a.avg, nbl, a.res, a.part, a.g_arg);
     LEAP_HIP(hipGetLastError());
-    inv_loss_kernel<<<(D + 63) / 64, 64, 0, s>>>(a.part, rb, D, a.loss);
+    // without a gradient only the last role is left
+    const uint32_t ra = a.g_arg ? ga : 0, rn = a.g_arg ? gn : 0;
+    inv_residual_grad_kernel<<<dim3(ra + rn + 1, D), 256, 0, s>>>(a.res, nI, a.I, a.csr_off, a.csr_ent, a.N, ra, rn, nbl,
+                                                                 a.part, gn, a.g_cal, a.g_arg, a.loss);
     LEAP_HIP(hipGetLastError());
-    if (!a.abar) return;
-    inv_garg_init_kernel<<<dim3((nbl + 255) / 256, D), 256, 0, s>>>(a.g_arg, nbl);
+    if (!a.g_arg) return;
+    inv_gram_gemv_kernel<<<dim3(ga, D), 256, 0, s>>>(a.Gp, a.N, a.g_cal, a.y);
     LEAP_HIP(hipGetLastError());
-    const dim3 gn((std::max(1, nI) + 255) / 256, D), ga((a.N + 3) / 4, D);
-    if (nI > 0) {
-        inv_garg_res_kernel<<<gn, 256, 0, s>>>(a.res, a.I, nI, nbl, a.g_arg);
-        LEAP_HIP(hipGetLastError());
-    }
-    inv_antenna_sum_kernel<<<ga, 256, 0, s>>>(a.res, nI, 2.0, a.csr_off, a.csr_ent, a.N, nullptr, a.g_cal);
+    inv_rows_kernel<<<dim3(ga + gn, D), 256, 0, s>>>(a.y, a.N, a.pairs, nI, a.csr_off, a.csr_ent, ga, nbl, a.g_cal,
+                                                    a.g_cal1, a.g_arg);
     LEAP_HIP(hipGetLastError());
-    inv_gram_gemv_kernel<<<ga, 256, 0, s>>>(a.Gp, a.N, a.g_cal, a.y);
-    LEAP_HIP(hipGetLastError());
-    if (nI > 0) {
-        inv_rows_kernel<<<gn, 256, 0, s>>>(a.y, a.N, a.pairs, nI, nbl, a.g_arg, a.gacal1);
-        LEAP_HIP(hipGetLastError());
-    }
-    inv_antenna_sum_kernel<<<ga, 256, 0, s>>>(a.gacal1, nI, 1.0, a.csr_off, a.csr_ent, a.N, a.g_cal, a.g_cal1);
-    LEAP_HIP(hipGetLastError());
-    inv_gram_gemv_kernel<<<ga, 256, 0, s>>>(a.G1p, a.N, a.g_cal1, a.y1);
+    inv_gram_gemv_kernel<<<dim3(ga, D), 256, 0, s>>>(a.G1p, a.N, a.g_cal1, a.y1);
     LEAP_HIP(hipGetLastError());
     if (nI1 > 0) {
         inv_rows1_kernel<<<dim3((nI1 + 255) / 256, D), 256, 0, s>>>(a.y1, a.N, a.pairs1, a.I1, nI1, nbl, a.g_arg);
         LEAP_HIP(hipGetLastError());
     }
-    const uint32_t n = D * nbl;
-    inv_abar_kernel<<<(n + 255) / 256, 256, 0, s>>>(a.avg0, a.g_arg, n, a.abar);
-    LEAP_HIP(hipGetLastError());
 }
 
 void launch_perturb_uvw(hipStream_t s, const double* uvw0, const double* M, const int2* bl_ants, const double* dp,
@@ -583,8 +574,8 @@ void launch_perturb_uvw(hipStream_t s, const double* uvw0, const double* M, cons
 }
 
 void launch_rotate_adjoint(hipStream_t s, const void* vis, int32_t vis_dtype, const double* uvw, const double* dd,
-                           const double* abar, uint32_t D, uint32_t T, uint32_t nbl, uint32_t C, uint32_t P, double f0,
-                           double df, double* g_uvw, double* g_dz_partial) {
+                           const double* avg, const double* g_arg, uint32_t D, uint32_t T, uint32_t nbl, uint32_t C,
+                           uint32_t P, double f0, double df, double* g_uvw, double* g_dz_partial, uint64_t* started) {
     const double kappa0 = f0 / kSpeedOfLight, dkappa = df / kSpeedOfLight;
     const bool c64 = vis_dtype == LEAP_VIS_C64;
     require(D >= 1 && D <= 256, LEAP_ERR_NOT_IMPLEMENTED, "the adjoint handles 1 to 256 directions per call");
@@ -592,12 +583,12 @@ void launch_rotate_adjoint(hipStream_t s, const void* vis, int32_t vis_dtype, co
 #define LEAP_ADJ(DL_, ND_)                                                                                     \
     if (c64)                                                                                                   \
         rotate_adjoint_kernel<float, DL_, ND_><<<grid, kThreads, 0, s>>>(static_cast<const float*>(vis), uvw, dd, \
-                                                                         abar, D, T, nbl, C, P, kappa0, dkappa,   \
-                                                                         g_uvw, g_dz_partial);                    \
+                                                                         avg, g_arg, D, T, nbl, C, P, kappa0,     \
+                                                                         dkappa, g_uvw, g_dz_partial, started);   \
     else                                                                                                       \
         rotate_adjoint_kernel<double, DL_, ND_><<<grid, kThreads, 0, s>>>(static_cast<const double*>(vis), uvw,   \
-                                                                          dd, abar, D, T, nbl, C, P, kappa0,       \
-                                                                          dkappa, g_uvw, g_dz_partial)
+                                                                          dd, avg, g_arg, D, T, nbl, C, P, kappa0, \
+                                                                          dkappa, g_uvw, g_dz_partial, started)
     if (D <= 16)
         LEAP_ADJ(8, 2);
     else if (D <= 32)
@@ -612,15 +603,14 @@ void launch_rotate_adjoint(hipStream_t s, const void* vis, int32_t vis_dtype, co
     LEAP_HIP(hipGetLastError());
 }
 
-void launch_adjoint_q(hipStream_t s, const double* q, const double* uvw, const double* dd, const double* abar,
-                      uint32_t D, uint32_t T, uint32_t nbl, double f0, double df, double* g_uvw,
-                      double* g_dz_partial) {
+void launch_adjoint_q(hipStream_t s, const double* q, const double* uvw, const double* dd, const double* avg,
+                      const double* g_arg, uint32_t D, uint32_t T, uint32_t nbl, double f0, double df, double* g_uvw,
+                      double* g_dz_partial, uint64_t* started) {
     const double kappa0 = f0 / kSpeedOfLight, dkappa = df / kSpeedOfLight;
     require(D >= 1 && D <= 256, LEAP_ERR_NOT_IMPLEMENTED, "the adjoint handles 1 to 256 directions per call");
-    const dim3 grid(nbl);
-#define LEAP_ADJ(DL_, ND_)                                                                                         \
-    adjoint_q_kernel<DL_, ND_><<<grid, kThreads, 0, s>>>(q, uvw, dd, abar, D, T, nbl, kappa0, dkappa, g_uvw, \
-                                                         g_dz_partial)
+#define LEAP_ADJ(DL_, ND_)                                                                                           \
+    adjoint_q_kernel<DL_, ND_><<<(nbl + 64 / DL_ - 1) / (64 / DL_), kThreads, 0, s>>>(                               \
+        q, uvw, dd, avg, g_arg, D, T, nbl, kappa0, dkappa, g_uvw, g_dz_partial, started)
     if (D <= 16)
         LEAP_ADJ(16, 1);
     else if (D <= 32)
@@ -628,31 +618,23 @@ void launch_adjoint_q(hipStream_t s, const double* q, const double* uvw, const d
     else if (D <= 64)
         LEAP_ADJ(64, 1);
     else if (D <= 128)
-        LEAP_ADJ(128, 1);
+        LEAP_ADJ(64, 2);
     else
-        LEAP_ADJ(256, 1);
+        LEAP_ADJ(64, 4);
 #undef LEAP_ADJ
     LEAP_HIP(hipGetLastError());
 }
 
-void launch_gather_pol0(hipStream_t s, const double* avg, uint32_t n, uint32_t P, double* out) {
-    if (n == 0) return;
-    gather_pol0_kernel<<<(n + 255) / 256, 256, 0, s>>>(avg, n, P, out);
-    LEAP_HIP(hipGetLastError());
-}
-
 void launch_reduce_gdz_offsets(hipStream_t s, const double* part, uint32_t nbl, uint32_t D, double ra0, double dec0,
-                               const double* dirs, double* out) {
-    reduce_gdz_kernel<<<D * 3, 256, 0, s>>>(part, nbl, D, out);
-    LEAP_HIP(hipGetLastError());
-    gdz_offsets_kernel<<<(D + 63) / 64, 64, 0, s>>>(out, D, ra0, dec0, dirs, out + 3 * size_t(D));
+                               const double* dirs, double* out, uint64_t* started) {
+    reduce_gdz_kernel<<<D, 64 * kReduceWaves, 0, s>>>(part, nbl, ra0, dec0, dirs, out, started);
     LEAP_HIP(hipGetLastError());
 }
 
 void launch_antenna_grad(hipStream_t s, const double* g_uvw, const double* M, const int32_t* csr_off,
                          const int32_t* csr_bl, const int32_t* csr_sign, int32_t n_ant, uint32_t nbl, uint32_t T,
                          double* out) {
-    antenna_grad_kernel<<<n_ant, 256, 0, s>>>(g_uvw, M, csr_off, csr_bl, csr_sign, nbl, T, out);
+    antenna_grad_kernel<<<n_ant, 64 * kReduceWaves, 0, s>>>(g_uvw, M, csr_off, csr_bl, csr_sign, nbl, T, out);
     LEAP_HIP(hipGetLastError());
 }
 

@@ -269,8 +269,9 @@ struct leap_ctx {
     hipEvent_t ev_fork = nullptr, ev_packed[2] = {nullptr, nullptr}, ev_consumed[2] = {nullptr, nullptr};
     std::string error;
     hipEvent_t ev_start = nullptr, ev_stop = nullptr;
-    // device clock at the rotate kernel's and the following kernel's start (pinned pair); null where
-    // the call's rotate launches are timed by events.  stamped: the launch took the first
+    // device clock at the rotate kernel's and the following kernel's start (pinned; and at the adjoint's
+    // and the following kernel's); null where the call's launches are timed by events.  stamped: the
+    // launch took the first
     leap::PinnedBuffer h_stamps;
     uint64_t* stamps = nullptr;
     bool stamped = false;
@@ -291,20 +292,19 @@ struct leap_ctx {
     leap::DeviceBuffer d_uvw, d_vis_stage, d_dd, d_avg, d_cal1, d_sums, d_cal,
         d_partial, d_a_planes;
     leap::DeviceBuffer d_nufft_tail;  // partial sums of the NUFFT launch's chunked last round
-    // residual-loss gradient: ENU->UVW rotations, baseline antennas, antenna corrections, perturbed
-    // uvw, avgData adjoint, uvw / dz gradients, the antennas' baseline lists and their gradient
-    leap::DeviceBuffer d_adj_M, d_adj_ants, d_adj_dp, d_adj_uvw, d_adj_abar, d_adj_guvw, d_adj_gdzp, d_adj_gdz,
-        d_adj_off, d_adj_bls, d_adj_sgn, d_adj_gant;
-    // pol 0 of avgData with its arguments; the inversion adjoint's intermediates; the
-    // per-direction losses and offset gradients copied back (pinned)
-    leap::DeviceBuffer d_adj_avg0, d_adj_inv;
+    // residual-loss gradient: ENU->UVW rotations and antenna corrections, baseline antennas, perturbed
+    // uvw, uvw / dz gradients, the antennas' baseline lists
+    leap::DeviceBuffer d_adj_M, d_adj_ants, d_adj_uvw, d_adj_guvw, d_adj_gdzp, d_adj_off, d_adj_bls, d_adj_sgn;
+    // the inversion adjoint's intermediates
+    leap::DeviceBuffer d_adj_inv;
     // the forward pass's per-row sums (e0 P, e0 z P') for the adjoint, and the key
     // (antennas of every baseline, antenna count) the baseline tables were built for
     leap::DeviceBuffer d_adj_q;
     uint64_t adj_ants_key = 0;
     int32_t adjoint_mode = LEAP_ADJOINT_AUTO;
-    leap::PinnedBuffer h_adj_out;
-    hipEvent_t ev_grad[4] = {nullptr, nullptr, nullptr, nullptr};  // around the forward and adjoint kernels
+    // the call's rotations and corrections, copied up together; its losses and gradients, written by
+    // the kernels (pinned)
+    leap::PinnedBuffer h_adj_in, h_adj_out;
     double last_grad_forward_ms = 0.0, last_grad_adjoint_ms = 0.0;
     std::vector<double> h_avg;
     // calibrations of the last group of solution intervals (pinned: written by a kernel or a direct DMA)
@@ -494,26 +494,26 @@ void launch_gemm_bf16x3(hipStream_t s, const void* b_planes, int32_t K, int32_t 
                         void* a_planes, const double* cal1, float* partial, double* cal);
 void launch_perturb_uvw(hipStream_t s, const double* uvw0, const double* M, const int2* bl_ants, const double* dp,
                         uint32_t nbl, uint32_t rows, double* uvw);
+// From g_arg = dL/d arg avg and avg (pol 0): dL/d uvw of every row, and dL/d(row 2 of each direction's
+// DD matrix) of every baseline's rows, g_dz_partial[3 D][nbl].
 void launch_rotate_adjoint(hipStream_t s, const void* vis, int32_t vis_dtype, const double* uvw, const double* dd,
-                           const double* abar, uint32_t D, uint32_t T, uint32_t nbl, uint32_t C, uint32_t P, double f0,
-                           double df, double* g_uvw, double* g_dz_partial);
+                           const double* avg, const double* g_arg, uint32_t D, uint32_t T, uint32_t nbl, uint32_t C,
+                           uint32_t P, double f0, double df, double* g_uvw, double* g_dz_partial,
+                           uint64_t* started = nullptr);
 // launch_rotate_adjoint's outputs from the row sums of HornerWave::q (no pass over the cube).
-void launch_adjoint_q(hipStream_t s, const double* q, const double* uvw, const double* dd, const double* abar,
-                      uint32_t D, uint32_t T, uint32_t nbl, double f0, double df, double* g_uvw,
-                      double* g_dz_partial);
-// g_dz[d][k] (3 D doubles at out) reduced over baselines, then dL/d(ra, dec) of each
-// direction (2 D doubles at out + 3 D); dirs = the directions (ra, dec) on the device.
+void launch_adjoint_q(hipStream_t s, const double* q, const double* uvw, const double* dd, const double* avg,
+                      const double* g_arg, uint32_t D, uint32_t T, uint32_t nbl, double f0, double df, double* g_uvw,
+                      double* g_dz_partial, uint64_t* started = nullptr);
+// dL/d(ra, dec) of each direction (2 D doubles at out) from g_dz_partial; dirs = the directions (ra, dec).
 void launch_reduce_gdz_offsets(hipStream_t s, const double* part, uint32_t nbl, uint32_t D, double ra0, double dec0,
-                               const double* dirs, double* out);
-void launch_gather_pol0(hipStream_t s, const double* avg, uint32_t n, uint32_t P, double* out);
+                               const double* dirs, double* out, uint64_t* started = nullptr);
 // The residual loss of D calibrations and the adjoint of the inversion
 // (kernels_adjoint.hip); every array [d][...] on the device.
 struct InversionAdjoint {
     uint32_t D, nbl;
     int32_t K, N, K1;
     const double* cal;       // D x N calibrations (forward inversion)
-    const double* avg0;      // D x nbl complex pol 0 of avgData
-    const double* ph;        // D x nbl arguments of avg0
+    const double* avg;       // D x nbl complex pol 0 of avgData
     const int2* pairs;       // K - 1 antenna pairs of A's rows
     const int32_t* I;        // K - 1 baselines of A's rows
     const int2* pairs1;      // K1 - 1 antenna pairs of A1's rows
@@ -525,14 +525,12 @@ struct InversionAdjoint {
     double* res;             // D x (K - 1) residuals
     double* part;            // D x ceil((K - 1) / 256) partial loss sums
     double* loss;            // D per-direction losses
-    // backward (skipped when abar is null)
-    double* g_arg;           // D x nbl
+    // backward (skipped when g_arg is null)
+    double* g_arg;           // D x nbl: dL/d arg avg
     double* g_cal;           // D x N
     double* y;               // D x N
-    double* gacal1;          // D x (K - 1)
     double* g_cal1;          // D x N
     double* y1;              // D x N
-    double* abar;            // D x nbl complex: dL/dRe avg + i dL/dIm avg
 };
 void launch_inversion_adjoint(hipStream_t s, const InversionAdjoint& a);
 void launch_antenna_grad(hipStream_t s, const double* g_uvw, const double* M, const int32_t* csr_off,
