@@ -671,12 +671,6 @@ void check_metadata_matches(const leap_metadata& md, const leap_ms_view& ms) {
 }
 
 // Copies a host vector into a device buffer (at least one element is reserved).
-template <typename T>
-void upload(hipStream_t s, DeviceBuffer& buf, const std::vector<T>& v) {
-    buf.reserve(std::max<size_t>(1, v.size()) * sizeof(T));
-    if (!v.empty()) LEAP_HIP(hipMemcpyAsync(buf.ptr, v.data(), v.size() * sizeof(T), hipMemcpyHostToDevice, s));
-}
-
 // Each antenna's rows of a phase matrix (baseline rows only, in row order):
 // entries 2 k + 1 where the antenna is antenna2 of row k, 2 k where antenna1.
 void phase_matrix_csr(const PhaseMatrix& pm, std::vector<int32_t>& off, std::vector<int32_t>& ent) {
@@ -695,48 +689,15 @@ void phase_matrix_csr(const PhaseMatrix& pm, std::vector<int32_t>& off, std::vec
     }
 }
 
-// What gram_pinv_device leaves running on the stream: host and device memory that has to
-// outlive the next synchronisation, and the status to look at after it.
-struct GramWork {
-    std::vector<GramComponents> comps;
-    std::vector<GramPinv> mats;
-    DeviceBuffer d_scratch, d_mats, d_status;
-    std::vector<DeviceBuffer> d_comp, d_shift;
-    int32_t status = 0;
-    const std::vector<int32_t> zero{0};
-};
-
-struct GramSource {
-    const PhaseMatrix* pm;
-    const int2* d_pairs;
-    const int32_t *d_off, *d_ent;  // each antenna's rows
-    double *d_Gp, *d_Gx;           // N x N outputs
-};
-
-// G+ = pinv(A^T A) of phase matrices of one antenna count, all in the same launches,
-// from the device copies of their row pairs and per-antenna rows; the components come
-// from the host.
-void gram_pinv_device(leap_ctx* ctx, const std::vector<GramSource>& from, int32_t N, GramWork& w) {
-    hipStream_t s = ctx->stream;
-    const size_t nn = size_t(N) * N;
-    w.comps.reserve(from.size());
-    w.d_comp = std::vector<DeviceBuffer>(from.size());
-    w.d_shift = std::vector<DeviceBuffer>(from.size());
-    w.d_scratch.reserve(std::max<size_t>(1, 2 * nn * from.size()) * sizeof(double));
-    upload(s, w.d_status, w.zero);
-    for (size_t i = 0; i < from.size(); ++i) {
-        const GramSource& f = from[i];
-        w.comps.push_back(gram_components(*f.pm));
-        upload(s, w.d_comp[i], w.comps[i].comp);
-        upload(s, w.d_shift[i], w.comps[i].shift);
-        double* buf = w.d_scratch.as<double>() + 2 * nn * i;
-        w.mats.push_back(GramPinv{f.pm->constraint, f.d_off, f.d_ent, f.d_pairs, w.d_comp[i].as<int32_t>(),
-                                  w.d_shift[i].as<double>(), {buf, buf + nn}, f.d_Gp, f.d_Gx, w.d_status.as<int32_t>()});
+// Offsets of the parts of one allocation, 256 bytes apart at least.
+struct Layout {
+    size_t bytes = 0;
+    size_t add(size_t n) {
+        const size_t at = bytes;
+        bytes += (std::max<size_t>(n, 1) + 255) & ~size_t(255);
+        return at;
     }
-    upload(s, w.d_mats, w.mats);
-    launch_gram_pinv(s, w.d_mats.as<GramPinv>(), uint32_t(w.mats.size()), N);
-    LEAP_HIP(hipMemcpyAsync(&w.status, w.d_status.ptr, sizeof(int32_t), hipMemcpyDeviceToHost, s));
-}
+};
 
 leap_metadata* create_metadata(leap_ctx* ctx, const leap_ms_view& ms, int32_t ref_ant, double thr, int use_cache) {
     validate_view(ms);
@@ -775,66 +736,90 @@ leap_metadata* create_metadata(leap_ctx* ctx, const leap_ms_view& ms, int32_t re
         const double l = kSpeedOfLight / (md->freq_start_hz + int32_t(c) * md->freq_inc_hz);  // MetaData.h:95-98
         lambda[c] = make_double2(l, 1.0 / l);
     }
-    hipStream_t s = ctx->stream;
-    upload(s, md->d_pairs, pairs);
-    upload(s, md->d_pairs1, pairs1);
-    upload(s, md->d_I, md->A.I);
-    upload(s, md->d_I1, md->A1.I);
-    upload(s, md->d_csr_off, off);
-    upload(s, md->d_csr_ent, ent);
-    upload(s, md->d_csr1_off, off1);
-    upload(s, md->d_csr1_ent, ent1);
-    upload(s, md->d_lambda, lambda);
     // The pseudo-inverses (MetaData.cc:111, :123) as G+ = pinv(A^T A), Ad = G+ A^T, on the
     // device; with use_cache A's G+ is kept in the context by a hash of A (:112-120).
     const size_t nn = size_t(N) * N;
-    md->d_Gp.reserve(nn * sizeof(double) * 4);
-    double* gp = md->d_Gp.as<double>();
-    double* g1p = gp + 2 * nn;
-    std::vector<GramSource> from{{&md->A1, md->d_pairs1.as<int2>(), md->d_csr1_off.as<int32_t>(),
-                                  md->d_csr1_ent.as<int32_t>(), g1p, g1p + nn}};
     const uint64_t key = use_cache ? hash_phase_matrix(md->A) : 0;
     const auto cached = use_cache ? ctx->gram_cache.find(key) : ctx->gram_cache.end();
-    if (cached == ctx->gram_cache.end())
-        from.push_back({&md->A, md->d_pairs.as<int2>(), md->d_csr_off.as<int32_t>(), md->d_csr_ent.as<int32_t>(), gp,
-                        gp + nn});
-    else
+    const bool both = cached == ctx->gram_cache.end();
+    std::vector<GramComponents> comps{gram_components(md->A1)};
+    if (both) comps.push_back(gram_components(md->A));
+    // One allocation, whose first part goes up in one copy from pinned memory: a copy and an allocation a
+    // table took half of the time (128 antennas: 0.2 of 0.4 ms).
+    Layout l;
+    struct Part {
+        DevicePart* part;
+        const void* from;
+        size_t bytes, at;
+    };
+    std::vector<Part> parts;
+    auto table = [&](DevicePart& part, const auto& v) {
+        parts.push_back({&part, v.data(), v.size() * sizeof(v[0]), l.add(v.size() * sizeof(v[0]))});
+    };
+    DevicePart d_comp[2], d_shift[2], d_mats, d_status;
+    table(md->d_pairs, pairs);
+    table(md->d_pairs1, pairs1);
+    table(md->d_I, md->A.I);
+    table(md->d_I1, md->A1.I);
+    table(md->d_csr_off, off);
+    table(md->d_csr_ent, ent);
+    table(md->d_csr1_off, off1);
+    table(md->d_csr1_ent, ent1);
+    table(md->d_lambda, lambda);
+    for (size_t i = 0; i < comps.size(); ++i) {
+        table(d_comp[i], comps[i].comp);
+        table(d_shift[i], comps[i].shift);
+    }
+    std::vector<GramPinv> mats(comps.size());
+    std::vector<int32_t> status{0};
+    table(d_mats, mats);
+    table(d_status, status);
+    const size_t up = l.bytes;
+    const size_t at_gp = l.add(4 * nn * sizeof(double)), at_scratch = l.add(2 * nn * sizeof(double) * mats.size());
+    md->d_all.reserve(l.bytes);
+    char* base = md->d_all.as<char>();
+    for (const Part& p : parts) p.part->ptr = base + p.at;
+    md->d_Gp.ptr = base + at_gp;
+    double* gp = md->d_Gp.as<double>();
+    double* g1p = gp + 2 * nn;
+    double* scratch = reinterpret_cast<double*>(base + at_scratch);
+    auto gram = [&](size_t i, const PhaseMatrix& pm, const DevicePart& csr_off, const DevicePart& csr_ent,
+                    const DevicePart& ant_pairs, double* out) {
+        double* buf = scratch + 2 * nn * i;
+        mats[i] = GramPinv{pm.constraint, csr_off.as<int32_t>(), csr_ent.as<int32_t>(), ant_pairs.as<int2>(),
+                           d_comp[i].as<int32_t>(), d_shift[i].as<double>(), {buf, buf + nn}, out, out + nn,
+                           d_status.as<int32_t>()};
+    };
+    gram(0, md->A1, md->d_csr1_off, md->d_csr1_ent, md->d_pairs1, g1p);
+    if (both) gram(1, md->A, md->d_csr_off, md->d_csr_ent, md->d_pairs, gp);
+    hipStream_t s = ctx->stream;
+    if (ctx->md_in_use) LEAP_HIP(hipStreamSynchronize(s));  // a call that ended early
+    ctx->h_md.reserve(up);
+    char* h = ctx->h_md.as<char>();
+    for (const Part& p : parts)
+        if (p.bytes) std::memcpy(h + p.at, p.from, p.bytes);
+    ctx->md_in_use = true;
+    LEAP_HIP(hipMemcpyAsync(base, h, up, hipMemcpyHostToDevice, s));
+    if (!both)
         LEAP_HIP(hipMemcpyAsync(gp, cached->second.data(), cached->second.size() * sizeof(double),
                                 hipMemcpyHostToDevice, s));
-    GramWork work;
-    gram_pinv_device(ctx, from, N, work);
-    std::vector<double> keep(use_cache && from.size() > 1 ? 2 * nn : 0);
+    launch_gram_pinv(s, d_mats.as<GramPinv>(), uint32_t(mats.size()), N);
+    int32_t* h_status = reinterpret_cast<int32_t*>(h);  // the tables have gone up by then
+    LEAP_HIP(hipMemcpyAsync(h_status, d_status.ptr, sizeof(int32_t), hipMemcpyDeviceToHost, s));
+    std::vector<double> keep(use_cache && both ? 2 * nn : 0);
     if (!keep.empty())
         LEAP_HIP(hipMemcpyAsync(keep.data(), gp, keep.size() * sizeof(double), hipMemcpyDeviceToHost, s));
-    md->d_AdT.reserve(size_t(K) * N * sizeof(double));
-    md->d_Ad1T.reserve(size_t(K1) * N * sizeof(double));
-    launch_assemble_ad(s, gp, N, md->d_pairs.as<int2>(), K - 1, md->A.constraint, md->d_AdT.as<double>());
-    launch_assemble_ad(s, g1p, N, md->d_pairs1.as<int2>(), K1 - 1, md->A1.constraint, md->d_Ad1T.as<double>());
-    LEAP_HIP(hipStreamSynchronize(s));  // the host vectors above end with this function
-    require(work.status == 0, LEAP_ERR_INTERNAL, "phase matrix Gram block is not positive definite");
-    if (!keep.empty()) ctx->gram_cache.emplace(key, std::move(keep));
-    md->d_AdT_planes.reserve(bf16_planes_bytes(uint32_t(N), K));
-    launch_split_b(s, md->d_AdT.as<double>(), K, N, md->d_AdT_planes.ptr);
-    std::vector<double> tables32, tables64, tables16;
-    if (nufft_supported(md->channels)) {
-        md->nufft32 = make_nufft_plan(md->channels, true);
-        md->nufft64 = make_nufft_plan(md->channels, false);
-        md->nufft16 = make_nufft_plan(md->channels, false, true);
-        tables32 = nufft_tables(md->nufft32);
-        tables64 = nufft_tables(md->nufft64);
-        tables16 = nufft_tables(md->nufft16);
-        md->d_nufft32.reserve(tables32.size() * sizeof(double));
-        md->d_nufft64.reserve(tables64.size() * sizeof(double));
-        md->d_nufft16.reserve(tables16.size() * sizeof(double));
-        LEAP_HIP(hipMemcpyAsync(md->d_nufft32.ptr, tables32.data(), tables32.size() * sizeof(double),
-                                hipMemcpyHostToDevice, s));
-        LEAP_HIP(hipMemcpyAsync(md->d_nufft64.ptr, tables64.data(), tables64.size() * sizeof(double),
-                                hipMemcpyHostToDevice, s));
-        LEAP_HIP(hipMemcpyAsync(md->d_nufft16.ptr, tables16.data(), tables16.size() * sizeof(double),
-                                hipMemcpyHostToDevice, s));
-    }
     LEAP_HIP(hipStreamSynchronize(s));
+    ctx->md_in_use = false;
+    require(*h_status == 0, LEAP_ERR_INTERNAL, "phase matrix Gram block is not positive definite");
+    if (!keep.empty()) ctx->gram_cache.emplace(key, std::move(keep));
     return md.release();
+}
+
+// What a call with these options reads of the metadata beyond its tables, made now if no call has yet.
+void need_metadata(const leap_ctx* ctx, const leap_metadata& md, const leap_options& opts, int32_t channel_sum) {
+    if (opts.precision == LEAP_PRECISION_MIXED) md.need_ad(ctx->stream);
+    if (opts.strategy == LEAP_STRATEGY_BATCHED && is_nufft(channel_sum)) md.need_nufft(ctx->stream, channel_sum);
 }
 
 // ---- HIP graphs ---------------------------------------------------------------
@@ -1003,6 +988,7 @@ void calibrate_loop(leap_ctx* ctx, const leap_metadata& md, const leap_ms_view& 
     const uint32_t nbl = ms.num_baselines;
     const int32_t N = md.A.cols;
     const leap_options opts = routed(opts_in, ms, interval, D);
+    if (D > 0) need_metadata(ctx, md, opts, opts.channel_sum);
     ctx->last_channel_sum = opts.channel_sum;
     ctx->last_direct_cube = opts.direct_cube;
     if (opts.graph) {
@@ -1118,7 +1104,7 @@ int32_t set_nufft_route(const leap_options& opts, const leap_metadata& md, const
         cs = opts.precision == LEAP_PRECISION_FP64 ? LEAP_CHANNEL_SUM_NUFFT_W16 : LEAP_CHANNEL_SUM_NUFFT;
     else if (cs != LEAP_CHANNEL_SUM_NUFFT && cs != LEAP_CHANNEL_SUM_NUFFT_W16)
         return 0;
-    const bool cube_ok = nufft_cube_ok(ms, cs == LEAP_CHANNEL_SUM_NUFFT_W16) && md.nufft_plan(cs).N != 0;
+    const bool cube_ok = nufft_cube_ok(ms, cs == LEAP_CHANNEL_SUM_NUFFT_W16) && nufft_supported(md.channels);
     if (opts.channel_sum != LEAP_CHANNEL_SUM_AUTO) {
         require(cube_ok, LEAP_ERR_INVALID_ARGUMENT,
                 "the multi-set NUFFT route needs 1.." + std::to_string(kNufftMaxChannels) +
@@ -1414,6 +1400,7 @@ void calibrate_batch(leap_ctx* ctx, const leap_batch_set* sets, uint32_t n_sets,
         SetBuffers& buf = *ctx->batch_sets[i];
         b.h_cal.assign(size_t(b.md->A.cols) * b.D, 0.0);
         if (b.D == 0) continue;
+        need_metadata(ctx, *b.md, opts, b.nufft);
         buf.d_dd.reserve(size_t(b.D) * 9 * sizeof(double));
         buf.d_avg.reserve(size_t(b.D) * b.md->nbl * b.md->pols * 2 * sizeof(double));
         std::copy(b.dirs, b.dirs + size_t(b.D) * 2, h_dirs);
@@ -1613,6 +1600,34 @@ void calibrate_batch(leap_ctx* ctx, const leap_batch_set* sets, uint32_t n_sets,
 
 }  // namespace
 
+void leap_metadata::need_ad(hipStream_t s) const {
+    std::lock_guard<std::mutex> lock(making);
+    if (has_ad) return;
+    const int32_t K = A.rows, N = A.cols, K1 = A1.rows;
+    d_AdT.reserve(size_t(K) * N * sizeof(double));
+    d_Ad1T.reserve(size_t(K1) * N * sizeof(double));
+    d_AdT_planes.reserve(bf16_planes_bytes(uint32_t(N), K));
+    launch_assemble_ad(s, gram(0), N, d_pairs.as<int2>(), K - 1, A.constraint, d_AdT.as<double>());
+    launch_assemble_ad(s, gram(2), N, d_pairs1.as<int2>(), K1 - 1, A1.constraint, d_Ad1T.as<double>());
+    launch_split_b(s, d_AdT.as<double>(), K, N, d_AdT_planes.ptr);
+    LEAP_HIP(hipStreamSynchronize(s));  // for every stream
+    has_ad = true;
+}
+
+void leap_metadata::need_nufft(hipStream_t s, int32_t channel_sum) const {
+    std::lock_guard<std::mutex> lock(making);
+    const bool fp32 = channel_sum == LEAP_CHANNEL_SUM_NUFFT_FP32, w16 = channel_sum == LEAP_CHANNEL_SUM_NUFFT_W16;
+    NufftPlan& plan = fp32 ? nufft32 : w16 ? nufft16 : nufft64;
+    DeviceBuffer& tables = fp32 ? d_nufft32 : w16 ? d_nufft16 : d_nufft64;
+    if (plan.N != 0) return;
+    NufftPlan made = make_nufft_plan(channels, fp32, w16);
+    const std::vector<double> t = leap::nufft_tables(made);
+    tables.reserve(t.size() * sizeof(double));
+    LEAP_HIP(hipMemcpyAsync(tables.ptr, t.data(), t.size() * sizeof(double), hipMemcpyHostToDevice, s));
+    LEAP_HIP(hipStreamSynchronize(s));  // for every stream
+    plan = std::move(made);
+}
+
 extern "C" {
 
 const char* leap_hip_version(void) { return "leap-hip 0.1.0 (gfx950)"; }
@@ -1749,6 +1764,7 @@ int leap_hip_metadata_copy(const leap_metadata* md, double* A, int32_t* I, doubl
         }
         if (I1) std::copy(md->A1.I.begin(), md->A1.I.end(), I1);
         // AdT [K][N] row-major is Ad (N x K) column-major.
+        if (Ad || Ad1) md->need_ad(nullptr);
         if (Ad)
             LEAP_HIP(hipMemcpy(Ad, md->d_AdT.ptr, size_t(md->A.rows) * md->A.cols * sizeof(double),
                                hipMemcpyDeviceToHost));
@@ -1771,6 +1787,7 @@ int leap_hip_rotate_visibilities(leap_ctx* ctx, const leap_metadata* md, const l
         ctx->last_channel_sum = o.channel_sum;
         ctx->last_direct_cube = o.direct_cube;
         DeviceScope scope(ctx->device);
+        if (D > 0) need_metadata(ctx, *md, o, o.channel_sum);
         begin_timing(ctx);
         const DeviceRows rows = stage_rows(ctx, *ms, row_start, row_start + n_rows, !packed_route(o, 0));
         upload_directions(ctx, *md, dirs, D);
@@ -1788,6 +1805,7 @@ int leap_hip_apply_inversion(leap_ctx* ctx, const leap_metadata* md, const doubl
         require(ctx && md && avg && cal_out, LEAP_ERR_INVALID_ARGUMENT, "null argument");
         const leap_options o = resolve(opts);
         DeviceScope scope(ctx->device);
+        need_metadata(ctx, *md, o, 0);
         const size_t n = size_t(md->nbl) * md->pols * 2 * D;
         ctx->d_avg.reserve(n * sizeof(double));
         LEAP_HIP(hipMemcpyAsync(ctx->d_avg.ptr, avg, n * sizeof(double), hipMemcpyHostToDevice, ctx->stream));
@@ -2083,17 +2101,11 @@ namespace {
 // whose uvw is 0, left out) as offsets, baselines and signs.
 void adjoint_antenna_tables(leap_ctx* ctx, const leap_ms_view& ms, int32_t N) {
     const uint32_t nbl = ms.num_baselines;
-    uint64_t key = 1469598103934665603ull;  // FNV-1a over the antenna columns
-    auto mix = [&](uint64_t v) {
-        for (int k = 0; k < 8; ++k) {
-            key ^= (v >> (8 * k)) & 0xffu;
-            key *= 1099511628211ull;
-        }
+    auto same = [&](const std::vector<int32_t>& kept, const int32_t* now) {
+        return kept.size() == nbl && std::memcmp(kept.data(), now, nbl * sizeof(int32_t)) == 0;
     };
-    mix(nbl);
-    mix(uint64_t(uint32_t(N)));
-    for (uint32_t b = 0; b < nbl; ++b) mix((uint64_t(uint32_t(ms.antenna1[b])) << 32) | uint32_t(ms.antenna2[b]));
-    if (key == ctx->adj_ants_key && ctx->d_adj_ants.ptr && ctx->d_adj_off.ptr) return;
+    if (N == ctx->adj_N && same(ctx->adj_a1, ms.antenna1) && same(ctx->adj_a2, ms.antenna2)) return;
+    ctx->adj_N = 0;  // no tables until these are up
     hipStream_t s = ctx->stream;
     std::vector<int2> ants(nbl);
     std::vector<int32_t> off(size_t(N) + 1, 0), bls, sgn;
@@ -2122,7 +2134,9 @@ void adjoint_antenna_tables(leap_ctx* ctx, const leap_ms_view& ms, int32_t N) {
         LEAP_HIP(hipMemcpyAsync(ctx->d_adj_sgn.ptr, sgn.data(), sgn.size() * sizeof(int32_t), hipMemcpyHostToDevice, s));
     }
     LEAP_HIP(hipStreamSynchronize(s));  // the host vectors go out of scope
-    ctx->adj_ants_key = key;
+    ctx->adj_a1.assign(ms.antenna1, ms.antenna1 + nbl);
+    ctx->adj_a2.assign(ms.antenna2, ms.antenna2 + nbl);
+    ctx->adj_N = N;
 }
 
 }  // namespace

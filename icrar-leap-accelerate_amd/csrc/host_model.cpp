@@ -79,10 +79,14 @@ PhaseMatrix phase_matrix(const int32_t* a1, const int32_t* a2, const uint8_t* fg
     PhaseMatrix pm;
     int32_t maxa = 0;
     for (int32_t i = 0; i < n; ++i) {
-        require(a1[i] >= 0 && a2[i] >= 0, LEAP_ERR_INVALID_ARGUMENT, "negative antenna index");
+        if (a1[i] < 0 || a2[i] < 0) throw Error(LEAP_ERR_INVALID_ARGUMENT, "negative antenna index");
         maxa = std::max(maxa, std::max(a1[i], a2[i]));
     }
     pm.cols = maxa + 1;  // :59
+    const size_t most = ref_ant < 0 ? size_t(n) : size_t(pm.cols);
+    pm.I.reserve(most);
+    pm.ant1.reserve(most);
+    pm.ant2.reserve(most);
     for (int32_t i = 0; i < n; ++i) {  // :65-79
         if (a1[i] == a2[i] || fg[i]) continue;
         if (ref_ant >= 0 && a1[i] != ref_ant && a2[i] != ref_ant) continue;

@@ -6,6 +6,7 @@
 #include <cstdint>
 #include <map>
 #include <memory>
+#include <mutex>
 #include <stdexcept>
 #include <string>
 #include <vector>
@@ -41,6 +42,13 @@ struct DeviceBuffer {
     ~DeviceBuffer();
     // Grows (never shrinks) to at least n bytes; contents are not kept.
     void reserve(size_t n);
+    template <typename T>
+    T* as() const { return static_cast<T*>(ptr); }
+};
+
+// A part of a device buffer.
+struct DevicePart {
+    void* ptr = nullptr;
     template <typename T>
     T* as() const { return static_cast<T*>(ptr); }
 };
@@ -167,18 +175,17 @@ struct leap_metadata {
     leap::PhaseMatrix A, A1;
     // The reference's degeneracy warnings (MetaData.cc:129-136): Ad A != I, Ad1 A1 != I.
     bool ad_degenerate = false, ad1_degenerate = false;
-    // device
-    leap::DeviceBuffer d_AdT;      // K x N row-major == Ad column-major (N x K) transposed
-    leap::DeviceBuffer d_Ad1T;     // K1 x N
-    leap::DeviceBuffer d_I1;       // K1 - 1 ints (baseline index of phase angle k)
-    leap::DeviceBuffer d_pairs;    // K - 1 int2: (antenna1, antenna2) of baseline I(k)
+    // device: one allocation for all of these
+    leap::DeviceBuffer d_all;
+    leap::DevicePart d_I1;       // K1 - 1 ints (baseline index of phase angle k)
+    leap::DevicePart d_pairs;    // K - 1 int2: (antenna1, antenna2) of baseline I(k)
     // A's baseline indices I, A1's antenna pairs, and each antenna's rows of A and of
     // A1 (CSR: offsets N + 1, entries 2 row + (antenna2 ? 1 : 0))
-    leap::DeviceBuffer d_I, d_pairs1, d_csr_off, d_csr_ent, d_csr1_off, d_csr1_ent;
-    leap::DeviceBuffer d_lambda;   // channels double2: wavelength of each channel and its reciprocal
+    leap::DevicePart d_I, d_pairs1, d_csr_off, d_csr_ent, d_csr1_off, d_csr1_ent;
+    leap::DevicePart d_lambda;   // channels double2: wavelength of each channel and its reciprocal
     // G+ = pinv(A^T A), the same without the ones of the constraint's component (PhaseRows::Gx),
     // then both of A1; N x N each
-    leap::DeviceBuffer d_Gp;
+    leap::DevicePart d_Gp;
     const double* gram(int which) const { return d_Gp.as<double>() + size_t(which) * A.cols * A.cols; }
     leap::PhaseRows rows_of_A() const {
         return {A.rows, A.cols, A.constraint, d_I.as<int32_t>(), d_pairs.as<int2>(), d_csr_off.as<int32_t>(),
@@ -188,13 +195,21 @@ struct leap_metadata {
         return {A1.rows, A1.cols, A1.constraint, d_I1.as<int32_t>(), d_pairs1.as<int2>(), d_csr1_off.as<int32_t>(),
                 d_csr1_ent.as<int32_t>(), gram(3)};
     }
-    leap::DeviceBuffer d_AdT_planes;  // split-3 x BF16 planes of AdT in MFMA operand layout
-    // NUFFT plans (N == 0 when the channel count is not supported) and their
+    // Made by the first call that needs them (need_ad, need_nufft): a metadata may be shared by contexts
+    // and threads.
+    mutable std::mutex making;
+    mutable leap::DeviceBuffer d_AdT;         // K x N row-major == Ad column-major (N x K) transposed
+    mutable leap::DeviceBuffer d_Ad1T;        // K1 x N
+    mutable leap::DeviceBuffer d_AdT_planes;  // split-3 x BF16 planes of AdT in MFMA operand layout
+    mutable bool has_ad = false;
+    // NUFFT plans (N == 0 until made) and their
     // device tables (leap::nufft_tables): FP64 transform (LEAP_CHANNEL_SUM_NUFFT),
     // FP32 transform (LEAP_CHANNEL_SUM_NUFFT_FP32) and FP64 transform with the
     // width-16 kernel (LEAP_CHANNEL_SUM_NUFFT_W16).
-    leap::NufftPlan nufft32, nufft64, nufft16;
-    leap::DeviceBuffer d_nufft32, d_nufft64, d_nufft16;
+    mutable leap::NufftPlan nufft32, nufft64, nufft16;
+    mutable leap::DeviceBuffer d_nufft32, d_nufft64, d_nufft16;
+    void need_ad(hipStream_t s) const;
+    void need_nufft(hipStream_t s, int32_t channel_sum) const;
     const leap::NufftPlan& nufft_plan(int32_t channel_sum) const {
         return channel_sum == LEAP_CHANNEL_SUM_NUFFT_FP32 ? nufft32
                : channel_sum == LEAP_CHANNEL_SUM_NUFFT_W16 ? nufft16
@@ -297,10 +312,11 @@ struct leap_ctx {
     leap::DeviceBuffer d_adj_M, d_adj_ants, d_adj_uvw, d_adj_guvw, d_adj_gdzp, d_adj_off, d_adj_bls, d_adj_sgn;
     // the inversion adjoint's intermediates
     leap::DeviceBuffer d_adj_inv;
-    // the forward pass's per-row sums (e0 P, e0 z P') for the adjoint, and the key
-    // (antennas of every baseline, antenna count) the baseline tables were built for
+    // the forward pass's per-row sums (e0 P, e0 z P') for the adjoint, and the
+    // antennas of every baseline and the antenna count that the baseline tables were built for
     leap::DeviceBuffer d_adj_q;
-    uint64_t adj_ants_key = 0;
+    std::vector<int32_t> adj_a1, adj_a2;
+    int32_t adj_N = 0;
     int32_t adjoint_mode = LEAP_ADJOINT_AUTO;
     // the call's rotations and corrections, copied up together; its losses and gradients, written by
     // the kernels (pinned)
@@ -309,6 +325,9 @@ struct leap_ctx {
     std::vector<double> h_avg;
     // calibrations of the last group of solution intervals (pinned: written by a kernel or a direct DMA)
     leap::PinnedBuffer h_cal;
+    // a metadata's tables on their way up (pinned); in use until the stream is waited for
+    leap::PinnedBuffer h_md;
+    bool md_in_use = false;
     // directions of the last call (pinned, read by kernels); in use until the stream is waited for
     leap::PinnedBuffer h_dirs;
     bool dirs_in_use = false;

@@ -1,14 +1,18 @@
 // Host -> device staging of host-resident visibilities.
 //
 // Pageable host memory is copied in chunks through two pinned buffers: worker
-// threads fill one buffer while the DMA engine drains the other on the
-// context's copy stream.  For the packed pol-0 path the workers apply the
+// threads fill a buffer in pieces, in order, and each piece is sent on the
+// context's copy stream while the next ones are filled.  (Sent buffer by buffer, a cube that
+// fits one was first copied whole and then sent: 180 MB in 4.8 ms; 3.3 ms in pieces.)
+// For the packed pol-0 path the workers apply the
 // reference's skip rule (CpuLeapCalibrator.cc:201-214: a (row, channel) with a
 // non-finite polarisation is left out, here written as 0) and keep pol 0
 // only, so a quarter of a 4-pol cube crosses the bus.
 #include <algorithm>
+#include <atomic>
 #include <cmath>
 #include <cstring>
+#include <system_error>
 #include <thread>
 #include <vector>
 
@@ -25,22 +29,47 @@ unsigned worker_count() {
     return std::max(1u, std::min(16u, hc ? hc : 1u));
 }
 
-// Runs f(begin, end) over [0, n) split across the workers.
-template <typename F>
-void parallel_ranges(size_t n, F&& f) {
-    const unsigned w = unsigned(std::min<size_t>(worker_count(), std::max<size_t>(1, n / 4096)));
-    if (w <= 1) {
-        f(size_t(0), n);
-        return;
+constexpr size_t kPieceBytes = size_t(8) << 20;    // a copy on the bus: 0.15 ms
+constexpr size_t kBlockBytes = size_t(512) << 10;  // taken by a worker at a time
+
+// fill(begin, end) over the units [0, n) of unit_bytes each, in blocks that the workers and the calling
+// thread take in order; ready(begin, end) on the calling thread for each piece, in order, once filled.
+template <typename Fill, typename Ready>
+void fill_in_pieces(size_t n, size_t unit_bytes, Fill&& fill, Ready&& ready) {
+    const size_t block = std::max<size_t>(1, kBlockBytes / unit_bytes), per_piece = kPieceBytes / kBlockBytes;
+    const size_t blocks = (n + block - 1) / block, pieces = (blocks + per_piece - 1) / per_piece;
+    std::atomic<size_t> next{0};
+    std::vector<std::atomic<size_t>> filled(pieces);
+    for (auto& f : filled) f.store(0, std::memory_order_relaxed);
+    auto work = [&] {  // one block; false when none is left
+        const size_t b = next.fetch_add(1, std::memory_order_relaxed);
+        if (b >= blocks) return false;
+        fill(b * block, std::min(n, (b + 1) * block));
+        filled[b / per_piece].fetch_add(1, std::memory_order_release);
+        return true;
+    };
+    struct Pool {  // joined also when ready throws
+        std::vector<std::thread> threads;
+        ~Pool() {
+            for (auto& t : threads) t.join();
+        }
+    } pool;
+    const size_t helpers = std::min<size_t>(worker_count(), blocks) - 1;
+    pool.threads.reserve(helpers);
+    try {
+        for (size_t i = 0; i < helpers; ++i)
+            pool.threads.emplace_back([&work] {
+                while (work()) {
+                }
+            });
+    } catch (const std::system_error&) {  // fewer helpers, or none
     }
-    std::vector<std::thread> pool;
-    pool.reserve(w);
-    const size_t step = (n + w - 1) / w;
-    for (unsigned i = 0; i < w; ++i) {
-        const size_t b = std::min(n, size_t(i) * step), e = std::min(n, b + step);
-        if (b < e) pool.emplace_back([&f, b, e] { f(b, e); });
+    for (size_t p = 0; p < pieces; ++p) {
+        const size_t b0 = p * per_piece, b1 = std::min(blocks, b0 + per_piece);
+        while (filled[p].load(std::memory_order_acquire) < b1 - b0)
+            if (!work()) std::this_thread::yield();
+        ready(b0 * block, std::min(n, b1 * block));
     }
-    for (auto& t : pool) t.join();
 }
 
 void ensure_staging(leap_ctx* ctx) {
@@ -76,12 +105,15 @@ void acquire(leap_ctx* ctx, int b) {
     }
 }
 
-void send(leap_ctx* ctx, int b, void* device_dst, size_t bytes) {
-    LEAP_HIP(hipMemcpyAsync(device_dst, ctx->h_pinned[b], bytes, hipMemcpyHostToDevice, ctx->copy_stream));
-    LEAP_HIP(hipEventRecord(ctx->ev_h2d[b], ctx->copy_stream));
-    ctx->h2d_pending[b] = true;
+// Part of the pinned buffer b to the device; sent(b) after its last one.
+void send(leap_ctx* ctx, int b, size_t offset, void* device_dst, size_t bytes) {
+    LEAP_HIP(hipMemcpyAsync(device_dst, static_cast<const char*>(ctx->h_pinned[b]) + offset, bytes,
+                            hipMemcpyHostToDevice, ctx->copy_stream));
     ctx->last_stage_bytes += bytes;
+    ctx->h2d_pending[b] = true;
 }
+
+void sent(leap_ctx* ctx, int b) { LEAP_HIP(hipEventRecord(ctx->ev_h2d[b], ctx->copy_stream)); }
 
 template <typename VT>
 void pack_pol0_host(const VT* src, uint32_t P, size_t begin, size_t end, VT* out) {
@@ -107,8 +139,10 @@ void stage_copy(leap_ctx* ctx, const void* host_src, size_t bytes, void* device_
         const size_t len = std::min(kChunkBytes, bytes - off);
         acquire(ctx, b);
         char* pin = static_cast<char*>(ctx->h_pinned[b]);
-        parallel_ranges(len, [&](size_t lo, size_t hi) { std::memcpy(pin + lo, src + off + lo, hi - lo); });
-        send(ctx, b, dst + off, len);
+        fill_in_pieces(
+            len, 1, [&](size_t lo, size_t hi) { std::memcpy(pin + lo, src + off + lo, hi - lo); },
+            [&](size_t lo, size_t hi) { send(ctx, b, lo, dst + off + lo, hi - lo); });
+        sent(ctx, b);
     }
     join_copy_stream(ctx);
 }
@@ -129,10 +163,14 @@ void stage_pol0(leap_ctx* ctx, const void* host_vis, int32_t vis_dtype, uint32_t
         if (c64) {
             const float* src = static_cast<const float*>(host_vis) + e0 * 2 * P;
             float* pin = static_cast<float*>(ctx->h_pinned[b]);
-            parallel_ranges(m, [&](size_t lo, size_t hi) { pack_pol0_host(src, P, lo, hi, pin); });
             // the device staging buffer b is free once its previous widen kernel has run
             if (ctx->widen_pending[b]) LEAP_HIP(hipStreamWaitEvent(ctx->copy_stream, ctx->ev_widened[b], 0));
-            send(ctx, b, ctx->d_widen[b].ptr, m * out_elem);
+            fill_in_pieces(
+                m, out_elem, [&](size_t lo, size_t hi) { pack_pol0_host(src, P, lo, hi, pin); },
+                [&](size_t lo, size_t hi) {
+                    send(ctx, b, lo * out_elem, ctx->d_widen[b].as<char>() + lo * out_elem, (hi - lo) * out_elem);
+                });
+            sent(ctx, b);
             LEAP_HIP(hipStreamWaitEvent(ctx->stream, ctx->ev_h2d[b], 0));
             launch_widen_c64(ctx->stream, ctx->d_widen[b].ptr, m, device_dst + 2 * e0);
             LEAP_HIP(hipEventRecord(ctx->ev_widened[b], ctx->stream));
@@ -140,8 +178,12 @@ void stage_pol0(leap_ctx* ctx, const void* host_vis, int32_t vis_dtype, uint32_t
         } else {
             const double* src = static_cast<const double*>(host_vis) + e0 * 2 * P;
             double* pin = static_cast<double*>(ctx->h_pinned[b]);
-            parallel_ranges(m, [&](size_t lo, size_t hi) { pack_pol0_host(src, P, lo, hi, pin); });
-            send(ctx, b, device_dst + 2 * e0, m * out_elem);
+            fill_in_pieces(
+                m, out_elem, [&](size_t lo, size_t hi) { pack_pol0_host(src, P, lo, hi, pin); },
+                [&](size_t lo, size_t hi) {
+                    send(ctx, b, lo * out_elem, device_dst + 2 * (e0 + lo), (hi - lo) * out_elem);
+                });
+            sent(ctx, b);
         }
     }
     join_copy_stream(ctx);

@@ -63,3 +63,34 @@ def test_host_cube_equals_device_cube(leap, ctx, big, opts_kw):
         assert staged == rc * 2 * (elem // 2)  # pol 0 only, in the source precision
     else:
         assert staged == rc * s.num_pols * elem  # whole rows
+
+
+@pytest.mark.parametrize("strategy", [0, 1])
+@pytest.mark.parametrize("dtype", [np.complex64, np.complex128])
+@pytest.mark.parametrize("n_ant,T,C,P", [(3, 1, 1, 1), (16, 15, 125, 4), (16, 15, 129, 4), (33, 30, 70, 3), (40, 41, 64, 2)])
+def test_staged_pieces(leap, ctx, dtype, strategy, n_ant, T, C, P):
+    """Host cubes of one sample up to several pieces of the staging copy (8 MiB, filled in blocks of
+    512 KiB), whole rows or pol 0 alone, give the bits of the same cube on the device."""
+    print(f"staged pieces: {n_ant} antennas, {T} t, {C} ch, {P} pols, {np.dtype(dtype).name}", flush=True)
+    s = leap.SynthMS(n_antennas=n_ant, n_timesteps=T, n_channels=C, n_pols=P, nan_fraction=0.002, seed=C)
+    s.fill_host(dtype)
+    ms = s.host_dict()
+    vis = np.ascontiguousarray(ms["vis"])
+    host_view = leap.view_from_arrays(ms)
+    md = ctx.metadata(host_view)
+    vis_p, uvw_p = ctx.malloc(vis.nbytes), ctx.malloc(ms["uvw"].nbytes)
+    try:
+        ctx.h2d(vis_p, vis)
+        ctx.h2d(uvw_p, np.ascontiguousarray(ms["uvw"]))
+        dev_view = leap.view_from_arrays(ms, vis_device=vis_p, uvw_device=uvw_p,
+                                         vis_dtype=leap.LEAP_VIS_C64 if dtype is np.complex64 else leap.LEAP_VIS_C128)
+        dirs = dirs_near(ms["phase_centre"], 3, C)
+        opts = leap.options(strategy=strategy, **(dict(direction_block=64, lane_directions=1) if strategy else {}))
+        got, _ = ctx.calibrate(host_view, dirs, opts=opts, md=md)
+        elem = vis.itemsize // 2
+        assert ctx.last_staged_bytes() == vis.size // P * 2 * elem * (1 if strategy else P)
+        want, _ = ctx.calibrate(dev_view, dirs, opts=opts, md=md)
+        assert np.array_equal(got, want)
+    finally:
+        ctx.free(vis_p)
+        ctx.free(uvw_p)
