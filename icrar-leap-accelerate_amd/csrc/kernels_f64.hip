@@ -351,6 +351,22 @@ __global__ void assemble_ad_kernel(const double* __restrict__ Gp, int32_t N,
 // and the kernels around it took 150.
 // ---------------------------------------------------------------------------
 
+// Antenna j's signed sum of its rows' phases, 0 for the constraint.
+__device__ inline double antenna_phase(const double* __restrict__ a_d, uint32_t nbl, uint32_t P, const PhaseRows& r,
+                                       int32_t j) {
+    double b = 0.0;
+    if (j != r.constraint)
+        for (int32_t e = r.csr_off[j]; e < r.csr_off[j + 1]; ++e) {
+            const int32_t v = r.csr_ent[e];
+            int32_t idx = r.I[v >> 1];
+            if (idx < 0) idx += int32_t(nbl);  // VectorRangeSelect wrap (math/cpu/vector.h:97-104)
+            const double* a = a_d + size_t(idx) * (2 * P);
+            const double ph = atan2(a[1], a[0]);
+            b += (v & 1) ? -ph : ph;
+        }
+    return b;
+}
+
 // cal1: one workgroup per (direction, 64 antennas), eight groups of 64 lanes taking every
 // eighth column each; every workgroup forms the direction's antenna sums for itself (one
 // arg per antenna when A1 is a star).
@@ -373,17 +389,7 @@ __global__ __launch_bounds__(64 * kCal1Groups) void cal1_kernel(const double* __
         const int32_t jn = min(kCal1Chunk, r.N - j0);
         __syncthreads();
         for (int32_t j = threadIdx.x; j < jn; j += 64 * kCal1Groups) {
-            double b = 0.0;
-            if (j0 + j != r.constraint)
-                for (int32_t e = r.csr_off[j0 + j]; e < r.csr_off[j0 + j + 1]; ++e) {
-                    const int32_t v = r.csr_ent[e];
-                    int32_t idx = r.I[v >> 1];
-                    if (idx < 0) idx += int32_t(nbl);  // VectorRangeSelect wrap (math/cpu/vector.h:97-104)
-                    const double* a = a_d + size_t(idx) * (2 * P);
-                    const double ph = atan2(a[1], a[0]);
-                    b += (v & 1) ? -ph : ph;
-                }
-            s_b[j] = b;
+            s_b[j] = antenna_phase(a_d, nbl, P, r, j0 + j);
         }
         __syncthreads();
 #pragma unroll 8
@@ -431,6 +437,61 @@ __global__ __launch_bounds__(kBlock) void cal_kernel(const double* __restrict__ 
     for (int32_t j = int32_t(lane); j < N; j += 64) acc = fma(row[j], x[j], acc);
     for (int off = 32; off > 0; off >>= 1) acc += __shfl_xor(acc, off, 64);
     if (lane == 0) cal[size_t(d) * N + a] = acc + cal1[size_t(d) * N + a];
+}
+
+// The three kernels above for one direction a workgroup, where a direction's rows and antennas fit one:
+// each thread forms one row's delta, each wave sums the antennas' rows from LDS.  Sums in the same
+// order, so the same bits.  Six stations, one direction: a call 36 us with the three launches, 32 with
+// one; 45 antennas (990 rows), 512 directions 342 and 333.
+constexpr int32_t kSmallWaves = 16, kSmallRows = 64 * kSmallWaves, kSmallAntennas = 64;
+
+__global__ __launch_bounds__(kSmallRows) void inversion_small_kernel(const double* __restrict__ avg, uint32_t nbl,
+                                                                     uint32_t P, const PhaseRows r1, const PhaseRows r,
+                                                                     double* __restrict__ cal,
+                                                                     uint64_t* __restrict__ started) {
+#pragma clang fp contract(off)
+    dev::stamp(started);
+    __shared__ double s_b[kSmallAntennas], s_cal1[kSmallAntennas], s_sums[kSmallAntennas];
+    __shared__ double s_part[kCal1Groups][64];
+    __shared__ double s_delta[kSmallRows];
+    const uint32_t d = blockIdx.x;
+    const int32_t lane = threadIdx.x % 64, wave = threadIdx.x / 64;
+    const double* a_d = avg + size_t(d) * nbl * (2 * P);
+    if (int32_t(threadIdx.x) < r1.N) s_b[threadIdx.x] = antenna_phase(a_d, nbl, P, r1, threadIdx.x);
+    __syncthreads();
+    if (wave < kCal1Groups) {
+        double acc = 0.0;
+        const int32_t ic = min(lane, r1.N - 1);
+        for (int32_t j = wave; j < r1.N; j += kCal1Groups) acc = fma(r1.Gx[size_t(j) * r1.N + ic], s_b[j], acc);
+        s_part[wave][lane] = acc;
+    }
+    __syncthreads();
+    if (wave == 0 && lane < r1.N) {
+        double acc = s_part[0][lane];
+        for (int g = 1; g < kCal1Groups; ++g) acc += s_part[g][lane];
+        s_cal1[lane] = acc;
+    }
+    __syncthreads();
+    const int32_t n = int32_t(threadIdx.x);
+    if (n < r.K - 1) s_delta[n] = dev::delta_phase(avg, nbl, P, r.pairs, r.K, 0, s_cal1, d, n);
+    __syncthreads();
+    for (int32_t a = wave; a < r.N; a += kSmallWaves) {
+        double acc = 0.0;
+        if (a != r.constraint)
+            for (int32_t e = r.csr_off[a] + lane; e < r.csr_off[a + 1]; e += 64) {
+                const int32_t v = r.csr_ent[e];
+                const double t = s_delta[v >> 1];
+                acc += (v & 1) ? -t : t;
+            }
+        for (int off = 32; off > 0; off >>= 1) acc += __shfl_xor(acc, off, 64);
+        if (lane == 0) s_sums[a] = acc;
+    }
+    __syncthreads();
+    for (int32_t a = wave; a < r.N; a += kSmallWaves) {
+        double acc = lane < r.N ? fma(r.Gx[size_t(a) * r.N + lane], s_sums[lane], 0.0) : 0.0;
+        for (int off = 32; off > 0; off >>= 1) acc += __shfl_xor(acc, off, 64);
+        if (lane == 0) cal[size_t(d) * r.N + a] = acc + s_cal1[a];
+    }
 }
 
 // ---------------------------------------------------------------------------
@@ -707,8 +768,13 @@ void launch_cal1(hipStream_t s, const leap_metadata& md, const double* avg, uint
 void launch_inversion_f64(hipStream_t s, const leap_metadata& md, const double* avg, uint32_t avg_pols, uint32_t D,
                           double* cal1, double* sums, double* cal, uint64_t* started) {
     if (D == 0) return;
-    launch_cal1(s, md, avg, avg_pols, D, cal1, started);
     const PhaseRows r = md.rows_of_A();
+    if (r.N <= kSmallAntennas && r.K - 1 <= kSmallRows) {
+        inversion_small_kernel<<<D, kSmallRows, 0, s>>>(avg, md.nbl, avg_pols, md.rows_of_A1(), r, cal, started);
+        LEAP_HIP(hipGetLastError());
+        return;
+    }
+    launch_cal1(s, md, avg, avg_pols, D, cal1, started);
     const dim3 grid(D, uint32_t(r.N + kBlock / 64 - 1) / (kBlock / 64));
     delta_sum_kernel<<<grid, kBlock, 0, s>>>(avg, md.nbl, avg_pols, r, cal1, sums);
     LEAP_HIP(hipGetLastError());

@@ -113,3 +113,19 @@ def test_calibrations_and_times_of_small_and_large_results(leap, ctx, opts_kw):
     finally:
         ctx.free(vp)
         ctx.free(up)
+
+
+@pytest.mark.parametrize("n_ant,autos,D", [(2, 1, 1), (3, 1, 5), (45, 0, 3), (46, 0, 3), (46, 1, 2), (64, 0, 2)])
+def test_inversion_of_few_antennas(leap, ctx, oracle, n_ant, autos, D):
+    """Calibrations by the one-launch inversion (up to 64 antennas and 1,024 rows: 990 rows of 45 antennas)
+    and, past it (1,035 rows of 46), by the three launches, with flagged baselines and NaNs, within
+    1e-9 rad of the oracle (the bar of test_gpu_parity.py)."""
+    print(f"inversion: {n_ant} antennas, autocorrelations {autos}, {D} directions", flush=True)
+    s = leap.SynthMS(n_antennas=n_ant, autocorrelations=autos, n_timesteps=2, n_channels=3, nan_fraction=0.01,
+                     flag_fraction=0.05 if n_ant > 10 else 0.0, seed=n_ant)
+    s.fill_host(np.complex64)
+    ms = s.host_dict()
+    dirs = np.asarray(ms["phase_centre"]) + np.random.default_rng(D).uniform(-0.02, 0.02, (D, 2))
+    got, _ = ctx.calibrate(leap.view_from_arrays(ms), dirs)
+    want, _ = oracle.calibrate(ms, dirs)
+    assert np.abs(npr.wrap(got - want)).max() < 1e-9
