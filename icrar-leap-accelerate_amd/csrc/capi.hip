@@ -1711,7 +1711,12 @@ int leap_hip_metadata_create(leap_ctx* ctx, const leap_ms_view* ms, int32_t ref_
     return guarded(ctx, [&] {
         require(ctx && ms && out, LEAP_ERR_INVALID_ARGUMENT, "null argument");
         DeviceScope scope(ctx->device);
-        *out = create_metadata(ctx, *ms, ref_ant, thr, use_cache);
+        std::unique_ptr<leap_metadata> md(create_metadata(ctx, *ms, ref_ant, thr, use_cache));
+        md->need_ad(ctx->stream);
+        if (nufft_supported(md->channels))
+            for (int32_t cs : {LEAP_CHANNEL_SUM_NUFFT, LEAP_CHANNEL_SUM_NUFFT_FP32, LEAP_CHANNEL_SUM_NUFFT_W16})
+                md->need_nufft(ctx->stream, cs);
+        *out = md.release();
     });
 }
 

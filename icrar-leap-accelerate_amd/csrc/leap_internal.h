@@ -195,8 +195,8 @@ struct leap_metadata {
         return {A1.rows, A1.cols, A1.constraint, d_I1.as<int32_t>(), d_pairs1.as<int2>(), d_csr1_off.as<int32_t>(),
                 d_csr1_ent.as<int32_t>(), gram(3)};
     }
-    // Made by the first call that needs them (need_ad, need_nufft): a metadata may be shared by contexts
-    // and threads.
+    // Made with a metadata that is kept; where a call makes its own, only what its options read
+    // (need_ad, need_nufft).  A metadata may be shared by contexts and threads.
     mutable std::mutex making;
     mutable leap::DeviceBuffer d_AdT;         // K x N row-major == Ad column-major (N x K) transposed
     mutable leap::DeviceBuffer d_Ad1T;        // K1 x N

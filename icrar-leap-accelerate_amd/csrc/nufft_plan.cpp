@@ -121,12 +121,14 @@ NufftPlan make_nufft_plan(uint32_t C, bool fp32, bool w16) {
     gauss_legendre(kNufftQuadratureNodes, gx, gw);
     const double half = p.W * M_PI / N;
     p.scale.resize(C);
-    std::vector<double> phi(gx.size());
-    for (size_t q = 0; q < gx.size(); ++q) phi[q] = gw[q] * es_kernel(gx[q], p.beta);
+    // The nodes lie in pairs +-z, where the integrand is even.
+    static_assert(kNufftQuadratureNodes % 2 == 0, "no node at 0");
+    std::vector<double> phi(gx.size() / 2);
+    for (size_t q = 0; q < phi.size(); ++q) phi[q] = 2.0 * gw[q] * es_kernel(gx[q], p.beta);
     for (uint32_t c = 0; c < C; ++c) {
         const double k = double(int64_t(c) - int64_t(p.h));
         double acc = 0.0;
-        for (size_t q = 0; q < gx.size(); ++q) acc += phi[q] * std::cos(k * gx[q] * half);
+        for (size_t q = 0; q < phi.size(); ++q) acc += phi[q] * std::cos(k * gx[q] * half);
         p.scale[c] = (2.0 * M_PI / N) / (half * acc);
     }
     // P_j(s) for j < W/2: Chebyshev interpolation in x = 2 s on [-1, 1], then monomials in s.
