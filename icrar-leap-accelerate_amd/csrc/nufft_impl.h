@@ -564,6 +564,18 @@ __device__ inline void turn_phasor_n(const Z* table, const double* dl, double sc
     }
 }
 
+// Whether N values are all finite: the largest magnitude by v_maximum3_f32, which keeps a NaN, two
+// values an instruction where a class test takes one each.  With the selection made before the
+// values are widened 30 of a row's 1,170 vector instructions less (256 stations, 32 t, 384 channels of
+// complex64: 256 directions 1% less, 64 directions 2 to 3%).
+template <int N>
+__device__ inline bool all_finite(const float* x) {
+    float m = __builtin_fabsf(x[0]);
+#pragma unroll
+    for (int k = 1; k < N; ++k) m = __builtin_elementwise_maximum(m, __builtin_fabsf(x[k]));
+    return m < __builtin_inff();
+}
+
 // Row sources.  The lane owns channels c = lane + 64 i, i < CPL (C <= 64 CPL
 // <= N / 2); load() fetches them for one row (channels past C read channel
 // C - 1 and are zeroed by freq()), freq() returns the precorrected pol-0
@@ -617,10 +629,9 @@ struct Source {
     __device__ void freq(C2<F>* x, uint32_t, uint32_t) const {
 #pragma unroll
         for (int i = 0; i < CPL; ++i) {
-            bool finite = true;
-#pragma unroll
-            for (int k = 0; k < 2 * P; ++k) finite = finite && __builtin_isfinite(raw[i][k]);
-            const float re = finite ? raw[i][0] : 0.0f, im = finite ? raw[i][1] : 0.0f;
+            const bool finite = all_finite<2 * P>(raw[i]);
+            float re = finite ? raw[i][0] : 0.0f, im = finite ? raw[i][1] : 0.0f;
+            asm volatile("" : "+v"(re), "+v"(im));  // selected before they are widened
             x[i] = to_transform<F>(double(re) * sc[i], double(im) * sc[i]);
         }
     }
