@@ -676,17 +676,16 @@ def run_adjoint(args):
     ctx.free(uvw_ptr)
     ctx.close()
     # Roofline of the dominant kernel, the forward pass with row sums (HBM): it reads the cube and
-    # uvw, writes avgData and each row's sums (e0 P, e0 z P', 32 bytes per row and direction); it
-    # also runs 16 flop per (row, channel, direction) (the P and P' Horner chains), reported
-    # against the FP64 vector peak.  The adjoint kernel reads the row sums, uvw and abar and writes
-    # the uvw gradient and the per-baseline dz partials.  Kernel times from HIP events on the
-    # library's stream.
+    # uvw, writes avgData and each row's sums (e0 P, e0 z P', 32 bytes per row and direction); P and
+    # P' by Horner's rule would be 16 flop per (row, channel, direction), reported against the FP64
+    # vector peak.  The adjoint kernel reads the row sums, uvw and abar and writes
+    # the uvw gradient and the per-baseline dz partials.  Kernel times from the device's clock.
     a_ms, f_ms = float(np.median(adj_k)), float(np.median(fwd_k))
     q_bytes = R * D * 32
     fwd_bytes = R * C * P * 8 + R * 24 + D * nbl * P * 16 + q_bytes
     fwd_flops = 16 * R * C * D
     adj_bytes = q_bytes + R * 24 + D * nbl * 16 + R * 24 + nbl * D * 24
-    roofline = {"kernel": "rotate_average_horner64_q (16-direction tile, row sums kept)", "bound": "hbm",
+    roofline = {"kernel": "horner_wave_kernel (row sums kept)", "bound": "hbm",
                 "achieved": round(fwd_bytes / (f_ms * 1e-3) / 1e9, 1), "peak": HBM_PEAK_GBS, "unit": "GB/s",
                 "frac": round(fwd_bytes / (f_ms * 1e-3) / 1e9 / HBM_PEAK_GBS, 4), "traffic": None,
                 "kernel_ms": round(f_ms, 4), "algorithmic_bytes_per_launch": fwd_bytes,

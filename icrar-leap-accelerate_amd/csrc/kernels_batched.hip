@@ -809,17 +809,6 @@ void launch_db(hipStream_t s, int tile, const void* vis, const double* uvw, cons
         launch_one<VT, A, DB_, ND_, NP>(s, vis, uvw, dd, D, T, nbl, nbl_grid, C, P, kappa0, dkappa, avg); \
         return;
     if constexpr (sizeof(A) == 8) {
-        if constexpr (NP == 1) {
-            // 16 directions per workgroup (internal: the residual-loss forward pass)
-            if (tile == 161) {
-                launch_one<VT, A, 16, 1, NP>(s, vis, uvw, dd, D, T, nbl, nbl_grid, C, P, kappa0, dkappa, avg);
-                return;
-            }
-            if (tile == 162) {
-                launch_one<VT, A, 16, 2, NP>(s, vis, uvw, dd, D, T, nbl, nbl_grid, C, P, kappa0, dkappa, avg);
-                return;
-            }
-        }
         switch (tile) {
             LEAP_TILE(32, 1)
             LEAP_TILE(64, 1)

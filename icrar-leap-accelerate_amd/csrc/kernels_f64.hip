@@ -3,13 +3,13 @@
 //   dd_kernel               MetaData::GenerateDDMatrix (model/cpu/MetaData.cc:166-203)
 //   rotate_average_f64      CpuLeapCalibrator::RotateVisibilities (CpuLeapCalibrator.cc:181-217)
 //   assemble_ad_kernel      pinv(A) = G+ A^T from the Gram pseudo-inverse
-//   phase_i1 / cal1 / delta / gemv kernels
+//   cal1, delta_sum, cal and inversion_small kernels
 //                           the inversion of CpuLeapCalibrator::PhaseRotate (:159-178)
+//   gram_* kernels          G+ = pinv(A^T A) (MetaData.cc:111, :123)
 //
 // Layouts in HBM: visibilities MS-native [row][channel][pol] complex (c128 or
 // c64); uvw [row][3] f64; avgData [direction][baseline][pol] complex128;
-// Ad stored transposed as AdT [K][N] (row k = column k of Ad) so the GEMV
-// reads whole rows; cal [direction][N].
+// Ad stored transposed as AdT [K][N] (row k = column k of Ad); cal [direction][N].
 #include "batched_common.h"
 #include "inversion_common.h"
 #include "leap_internal.h"

@@ -108,18 +108,21 @@ typedef enum leap_precision {
 } leap_precision;
 
 typedef enum leap_strategy {
-    /* One pass over the visibilities per direction (the reference's schedule). */
+    /* Every sample rotated by its own phase, as the reference; up to eight directions per
+     * pass over the visibilities. */
     LEAP_STRATEGY_PER_DIRECTION = 0,
-    /* One pass over the visibilities for a block of directions; the
-     * pseudo-inverse products become one GEMM per block. */
+    /* One pass over the visibilities for a block of directions. */
     LEAP_STRATEGY_BATCHED = 1
 } leap_strategy;
 
 typedef enum leap_channel_sum {
     /* Pol 0, 96..512 channels and at least 16 directions: the NUFFT in mixed precision,
-     * the width-16 NUFFT in FP64 precision; otherwise Horner. */
+     * the width-16 NUFFT in FP64 precision; otherwise Horner.  FP64 calls on a device cube that
+     * name no tile take Horner up to 32 directions on 2,048 rows or more and up to 48 on 16,384,
+     * where its folded kernel is the faster. */
     LEAP_CHANNEL_SUM_AUTO = 0,
-    /* FP64 Horner: four FMAs per channel and direction (rounding error n eps of sum |v|). */
+    /* FP64 Horner sums (rounding error at most n eps of sum |v|): on a device cube with no tile
+     * named by folded blocks of eight channels, 2.5 FMAs per channel and direction; else four. */
     LEAP_CHANNEL_SUM_HORNER = 1,
     /* Type-2 non-uniform FFT per row (one inverse FFT of 256..1024 points, then W = 10 or 12
      * grid points per direction); mixed precision, pol 0, 1..512 channels.  A device-resident
@@ -163,12 +166,12 @@ typedef struct leap_options {
                                  context and replayed by later calls with the same shapes,
                                  options and device addresses; results reach the callback
                                  after the whole graph.  Needs vis_on_device and uvw_device. */
-    int32_t direct_cube;      /* batched pol 0: 1 = run the Horner kernel straight from the cube
-                                 through LDS; 0 = automatic: a tuned call on a device cube packs
+    int32_t direct_cube;      /* batched pol 0: 1 = run the Horner kernel straight from the cube;
+                                 0 = automatic: a tuned call on a device cube packs
                                  pol 0 first (FP64, non-finite (row, channel)s zeroed; 16 B per
                                  row and channel of device memory; the Horner kernel then reads
-                                 it with scalar loads) only where a cost model of measured rates
-                                 expects the pack to pay (from about 800 directions on complex64,
+                                 it with scalar loads) only above a number of directions set by
+                                 measured rates (from about 800 directions on complex64,
                                  480 on complex128); host cubes and packed tiles always pack */
     int32_t pack_timesteps;   /* packed path: timesteps per pack chunk; chunks are packed on a
                                  second stream while the Horner kernel runs the previous one.
@@ -233,7 +236,7 @@ int leap_hip_calibrate_md(leap_ctx* ctx, const leap_metadata* md, const leap_ms_
  * memory (code under HIP graph capture, tight serving loops, harnesses that
  * forbid hipMalloc): leap_hip_calibrate_md on its FP64 per-direction route,
  * allocating nothing.  The direction table, dd matrices, one direction's
- * avgData and the inversion's phases, cal1, dphi and GEMV partial sums live in
+ * avgData and the inversion's cal1 and antenna sums live in
  * a fixed device array of LEAP_NOALLOC_SCRATCH_BYTES per GPU; the results are
  * bit-identical to leap_hip_calibrate_md with opts NULL.
  *   ms         visibilities and uvw device-resident (vis_on_device = 1,
@@ -243,7 +246,8 @@ int leap_hip_calibrate_md(leap_ctx* ctx, const leap_metadata* md, const leap_ms_
  *   epochs_out host memory, [n_solutions][2] (start, end), or NULL
  * Returns LEAP_ERR_RANGE when one solution's working set (16 B per direction
  * and 72 B of dd, 16 B per baseline and pol, 8 B per row of A and A1 and per
- * antenna, plus the GEMV partials) exceeds the scratch.  Every call on a GPU
+ * antenna, plus 8 B per antenna and 64 of those rows) exceeds the scratch (more than the
+ * sums above take; the bound is part of the interface).  Every call on a GPU
  * shares that GPU's scratch: calls that overlap on one GPU (other threads,
  * other contexts on the device) race.  Synchronous on return. */
 int leap_hip_calibrate_md_noalloc(leap_ctx* ctx, const leap_metadata* md, const leap_ms_view* ms,
@@ -269,15 +273,17 @@ typedef int (*leap_batch_cb)(void* user, uint32_t set, const leap_solution* solu
 /* Calibrate of several measurement sets with uneven antenna, baseline, channel
  * and timestep counts: each set gets the solutions leap_hip_calibrate_md would
  * give it with the same options.  Solution interval s of all sets, all
- * directions, is rotated and averaged in ONE persistent launch: a device
- * descriptor per set and (set, baseline, direction block) work items
+ * directions, is rotated and averaged in ONE persistent launch where a tile is named, and
+ * for the sets that do not fill the GPU by themselves (fewer than 8,192 rows; a set that does
+ * takes the launch of a single-set call): a device descriptor per set and (set, baseline, direction block) work items
  * statically load-balanced over the grid on the host (longest processing time
  * first), so the result does not depend on scheduling.  In mixed precision the
  * sets that qualify for the NUFFT channel sums (channel_sum automatic: 96..512
  * channels, 16 or more directions; or channel_sum = LEAP_CHANNEL_SUM_NUFFT)
  * and hold complex64 cubes with 1, 2 or 4 pols take them instead, one launch
  * per group of sets that share a grid and kernel width, with their
- * (set, baseline, direction block) items in decreasing rows per item; each
+ * (set, baseline, direction block) items in decreasing rows per item (the single-set launch
+ * for a group of one set); each
  * item's sums are those of the single-set NUFFT kernel.  Needs the batched
  * strategy, all_pols = 0, fp32_blocks = 0 and channel_sum other than
  * LEAP_CHANNEL_SUM_NUFFT_FP32.  No reference counterpart: the
