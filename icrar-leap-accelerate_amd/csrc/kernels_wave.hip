@@ -25,10 +25,10 @@
 // p' = sum_s s ((v+ - v-) cos(s theta) + i (v+ + v-) sin(s theta)), beside H <- w H + p.
 //
 // With up to 32 directions it runs at the cube's bytes (256 stations, 32 t, 384 channels of
-// complex64: 8 directions 2.27 ms, 32 directions 2.36 ms, 5.5 TB/s; 64 directions 3.51 ms, where the
-// VALU is never idle; Horner's rule over the channels took 2.41 ms and 5.35 ms).  128 antennas, 14 t, 48
+// complex64: 8 directions 2.27 ms, 32 directions 2.36 ms, 5.5 TB/s; 64 directions 3.56 ms, where its
+// instructions cost more than the cube; Horner's rule over the channels took 2.41 ms and 5.35 ms).  128 antennas, 14 t, 48
 // channels of complex128, 64 directions: 93 us, three quarters of it issued FP64 instructions.
-// Row sums of 16 directions (128 stations, 64 t, 192 channels of complex64) 706 us against 840.
+// Row sums of 16 directions (128 stations, 64 t, 192 channels of complex64) 714 us against 849.
 #include "batched_common.h"
 
 #include <algorithm>
