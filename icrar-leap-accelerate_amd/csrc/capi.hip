@@ -870,13 +870,21 @@ void key_common(std::vector<uint64_t>& k, const leap_ctx* ctx, const leap_option
                        key_ptr(ctx->d_cal.ptr), key_ptr(ctx->d_partial.ptr), key_ptr(ctx->d_a_planes.ptr)});
 }
 
+// A phase matrix, which the inversion's kernels take by value.
+void key_rows(std::vector<uint64_t>& k, const PhaseRows& r) {
+    k.insert(k.end(), {uint64_t(r.K), uint64_t(r.N), uint64_t(uint32_t(r.constraint)), key_ptr(r.I), key_ptr(r.pairs),
+                       key_ptr(r.csr_off), key_ptr(r.csr_ent), key_ptr(r.Gx)});
+}
+
+// A set with its metadata and the channel sums it takes.  A metadata may have gone and another be at
+// its addresses, with what it holds: whatever of it the kernels take is here, by value or by address.
 void key_set(std::vector<uint64_t>& k, const leap_metadata& md, const leap_ms_view& ms, uint32_t D,
-             int32_t solutions, uint32_t interval) {
-    k.insert(k.end(), {key_ptr(&md), uint64_t(md.A.rows), uint64_t(md.A.cols), uint64_t(md.A1.rows), md.nbl,
-                       md.channels, md.pols, key_bits(md.freq_start_hz), key_bits(md.freq_inc_hz),
-                       key_ptr(md.d_Gp.ptr), key_ptr(md.d_csr_ent.ptr), key_ptr(md.d_csr1_ent.ptr), key_ptr(md.d_I1.ptr),
-                       key_ptr(md.d_pairs.ptr),
-                       key_ptr(md.d_lambda.ptr), key_ptr(md.d_AdT_planes.ptr), key_ptr(ms.vis),
+             int32_t solutions, uint32_t interval, int32_t channel_sum) {
+    key_rows(k, md.rows_of_A());
+    key_rows(k, md.rows_of_A1());
+    k.insert(k.end(), {md.nbl, md.channels, md.pols, key_bits(md.freq_start_hz), key_bits(md.freq_inc_hz),
+                       key_ptr(md.d_lambda.ptr), key_ptr(md.d_AdT_planes.ptr), uint64_t(channel_sum),
+                       key_ptr(is_nufft(channel_sum) ? md.nufft_tables(channel_sum) : nullptr), key_ptr(ms.vis),
                        key_ptr(ms.uvw_device), uint64_t(ms.vis_dtype), ms.num_rows, D, uint64_t(solutions),
                        interval});
 }
@@ -929,7 +937,7 @@ void calibrate_loop_graph(leap_ctx* ctx, const leap_metadata& md, const leap_ms_
         }
         std::vector<uint64_t> key{uint64_t(uint32_t(tile))};
         key_common(key, ctx, opts);
-        key_set(key, md, ms, D, solutions, interval);
+        key_set(key, md, ms, D, solutions, interval, opts.channel_sum);
         if (!ctx->seq_single || ctx->seq_single->key != key) {
             ctx->seq_single = std::make_unique<CapturedSequence>();
             seq = ctx->seq_single.get();
@@ -1508,7 +1516,7 @@ void calibrate_batch(leap_ctx* ctx, const leap_batch_set* sets, uint32_t n_sets,
         key_common(key, ctx, opts);
         for (uint32_t i = 0; i < n_sets; ++i) {
             const BatchState& b = st[i];
-            key_set(key, *b.md, *b.ms, b.D, b.solutions, b.interval);
+            key_set(key, *b.md, *b.ms, b.D, b.solutions, b.interval, b.nufft);
             key.insert(key.end(), {key_ptr(ctx->batch_sets[i]->d_dd.ptr), key_ptr(ctx->batch_sets[i]->d_avg.ptr)});
         }
         CapturedSequence* seq = ctx->seq_batch.get();

@@ -182,3 +182,52 @@ def test_multi_set_graph_replays_equal_eager(leap, ctx):
     finally:
         for st in sets:
             st.free()
+
+
+@pytest.mark.parametrize("precision,strategy,cs", [(0, 0, 0), (0, 1, 1), (1, 1, 1), (0, 1, 4), (1, 1, 2)],
+                         ids=["fp64-per-dir", "fp64-horner", "mixed-horner", "fp64-nufft", "mixed-nufft"])
+def test_graph_follows_the_metadata_of_each_call(leap, precision, strategy, cs):
+    """Captured calls that make their own metadata, one after the other with other reference antennas:
+    a call's metadata can lie where the last one's did, and its graph must not be replayed with what
+    the kernels took of that one by value.  Each equals its eager call."""
+    c2 = leap.Context(0)
+    a = DeviceSet(leap, c2, np.complex64, n_antennas=20, n_timesteps=4, n_channels=50, flag_fraction=0.0, seed=90)
+    try:
+        dirs = dirs_near(a.ms["phase_centre"], 17, 9)
+        seen = []
+        for ref in (0, 3, 7, 3, None, 0):
+            print(f"reference antenna {ref}", flush=True)
+            got, _ = c2.calibrate(a.view, dirs, (0, 2, -1), ref_ant=ref,
+                                  opts=leap.options(precision, strategy, graph=1, channel_sum=cs))
+            want, _ = c2.calibrate(a.view, dirs, (0, 2, -1), ref_ant=ref,
+                                   opts=leap.options(precision, strategy, channel_sum=cs))
+            assert np.array_equal(got, want), ref
+            seen.append(want)
+        assert not np.array_equal(seen[0], seen[1]) and np.array_equal(seen[0], seen[-1])
+    finally:
+        a.free()
+        c2.close()
+
+
+@pytest.mark.parametrize("precision", [0, 1])
+def test_multi_set_graph_follows_new_metadata(leap, precision):
+    """The same for multi-set calls with metadata made anew between them."""
+    c3 = leap.Context(0)
+    sets = [DeviceSet(leap, c3, np.complex64, n_antennas=20, n_timesteps=2, n_channels=40, flag_fraction=0.0, seed=91),
+            DeviceSet(leap, c3, np.complex64, n_antennas=11, n_timesteps=3, n_channels=130, flag_fraction=0.0, seed=92)]
+    try:
+        for st in sets:
+            st.md = None
+        for ref in (0, 3, 7, 0):
+            print(f"reference antenna {ref}", flush=True)
+            arg = [(c3.metadata(st.view, ref_ant=ref), st.view, dirs_near(st.ms["phase_centre"], 17, 3), (0, -1, -1))
+                   for st in sets]
+            got = c3.calibrate_batch(arg, leap.options(precision, 1, graph=1))
+            want = c3.calibrate_batch(arg, leap.options(precision, 1))
+            del arg
+            for (gc, _), (wc, _) in zip(got, want):
+                assert np.array_equal(gc, wc), ref
+    finally:
+        for st in sets:
+            st.free()
+        c3.close()
