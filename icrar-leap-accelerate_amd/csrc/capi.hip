@@ -622,17 +622,21 @@ void invert_directions(leap_ctx* ctx, const leap_metadata& md, uint32_t D, const
                        ctx->d_a_planes.ptr, ctx->d_cal1.as<double>(), static_cast<float*>(ctx->d_partial.ptr), cal);
 }
 
-// The inversion of several solution intervals' averages [interval][direction]: all at once in
-// FP64; in mixed precision as many as the GEMM takes in one K-split of its whole output, whose
-// sums do not depend on how many directions it is given.
+// Solution intervals of one inversion out of the given number: all at once in FP64; in mixed precision
+// as many as the GEMM takes in one K-split of its whole output, whose sums do not depend on how many
+// directions it is given.
+uint32_t inversion_step(int32_t N, uint32_t D, uint32_t intervals, const leap_options& opts) {
+    if (opts.precision != LEAP_PRECISION_MIXED) return intervals;
+    uint32_t step = 1;
+    while (step < intervals && mfma_full_output(D, N) && mfma_full_output((step + 1) * D, N)) ++step;
+    return step;
+}
+
+// The inversion of several solution intervals' averages [interval][direction].
 void invert_intervals(leap_ctx* ctx, const leap_metadata& md, uint32_t D, uint32_t intervals, const leap_options& opts,
                       uint32_t avg_pols, double* cal = nullptr) {
     const int32_t N = md.A.cols;
-    uint32_t step = intervals;
-    if (opts.precision == LEAP_PRECISION_MIXED) {
-        step = 1;
-        while (step < intervals && mfma_full_output(D, N) && mfma_full_output((step + 1) * D, N)) ++step;
-    }
+    const uint32_t step = inversion_step(N, D, intervals, opts);
     if (cal == nullptr) {
         ctx->d_cal.reserve(size_t(N) * D * intervals * sizeof(double));
         cal = ctx->d_cal.as<double>();
@@ -837,14 +841,15 @@ void reserve_solution(leap_ctx* ctx, const leap_metadata& md, uint32_t D, uint32
     }
     if (opts.strategy == LEAP_STRATEGY_BATCHED)
         ctx->d_nufft_tail.reserve(nufft_tail_bytes(D));  // the NUFFT route's chunked last round
-    D *= intervals;  // the inversion takes every interval's directions alike
-    ctx->d_cal1.reserve(size_t(N) * D * sizeof(double));
-    ctx->d_cal.reserve(size_t(N) * D * sizeof(double));
+    // the directions of the largest inversion; a last one of fewer intervals takes no more
+    const uint32_t most = D * inversion_step(N, D, intervals, opts);
+    ctx->d_cal1.reserve(size_t(N) * most * sizeof(double));
+    ctx->d_cal.reserve(size_t(N) * D * intervals * sizeof(double));
     if (opts.precision == LEAP_PRECISION_MIXED) {
-        ctx->d_a_planes.reserve(bf16_planes_bytes((D + 63) / 64 * 64, K));
-        ctx->d_partial.reserve(mfma_partial_floats(K, D, N) * sizeof(float));
+        ctx->d_a_planes.reserve(bf16_planes_bytes((most + 63) / 64 * 64, K));
+        ctx->d_partial.reserve(mfma_partial_floats(K, most, N) * sizeof(float));
     } else {
-        ctx->d_sums.reserve(size_t(N) * D * sizeof(double));
+        ctx->d_sums.reserve(size_t(N) * most * sizeof(double));
     }
 }
 

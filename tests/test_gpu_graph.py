@@ -231,3 +231,26 @@ def test_multi_set_graph_follows_new_metadata(leap, precision):
         for st in sets:
             st.free()
         c3.close()
+
+
+@pytest.mark.parametrize("solutions,D", [(17, 16), (31, 16), (5, 100), (3, 300)])
+def test_mixed_graph_of_many_intervals_first_on_a_fresh_context(leap, solutions, D):
+    """A captured mixed-precision call of grouped solution intervals as a context's first: what the
+    inversions of 16 (of 17 and 31), 2 (of 5) and 1 interval at a time need is there before the capture,
+    although the GEMM's workspace does not grow with the number of directions.  Equal to the eager call,
+    also replayed."""
+    c4 = leap.Context(0)
+    a = DeviceSet(leap, c4, np.complex64, n_antennas=128, autocorrelations=0, n_timesteps=solutions, n_channels=3,
+                  n_pols=1, seed=93)
+    try:
+        print(f"{solutions} solutions of {D} directions", flush=True)
+        dirs = dirs_near(a.ms["phase_centre"], D, 6)
+        got = []
+        for _ in range(2):
+            got.append(c4.calibrate(a.view, dirs, (0, 1, -1), opts=leap.options(1, 1, graph=1), md=a.md)[0])
+        assert c4.last_graph() == 2
+        want, _ = c4.calibrate(a.view, dirs, (0, 1, -1), opts=leap.options(1, 1), md=a.md)
+        assert np.array_equal(got[0], want) and np.array_equal(got[1], want)
+    finally:
+        a.free()
+        c4.close()
