@@ -1808,9 +1808,15 @@ int leap_hip_rotate_visibilities(leap_ctx* ctx, const leap_metadata* md, const l
         if (D > 0) need_metadata(ctx, *md, o, o.channel_sum);
         begin_timing(ctx);
         const DeviceRows rows = stage_rows(ctx, *ms, row_start, row_start + n_rows, !packed_route(o, 0));
+        const size_t n = size_t(md->nbl) * md->pols * 2 * D;
+        if (n_rows == 0 && (names_no_tile(o) || packed_route(o, 0))) {  // sums over nothing; other tiles write them
+            std::fill_n(avg_out, n, 0.0);
+            finish_stream(ctx);
+            end_timing(ctx);
+            return;
+        }
         upload_directions(ctx, *md, dirs, D);
         rotate_directions(ctx, *md, *ms, rows, n_rows / ms->num_baselines, D, o);
-        const size_t n = size_t(md->nbl) * md->pols * 2 * D;
         if (n) LEAP_HIP(hipMemcpyAsync(avg_out, ctx->d_avg.ptr, n * sizeof(double), hipMemcpyDeviceToHost, ctx->stream));
         finish_stream(ctx);
         end_timing(ctx);

@@ -270,3 +270,38 @@ def test_device_pseudo_inverse_matches_host_gram_routine(leap, ctx, case):
     assert err < 1e-13
     assert np.abs(got["Ad"] - np.linalg.pinv(A)).max() < 1e-11
     assert np.abs(got["Ad1"] - np.linalg.pinv(A1)).max() < 1e-11
+
+
+NO_ROWS = {
+    "direct-cube": dict(strategy=1, channel_sum=1, direct_cube=1),
+    "per-direction": dict(),
+    "automatic": dict(strategy=1),
+    "nufft": dict(strategy=1, channel_sum=4),
+    "packed-tile": dict(strategy=1, direction_block=64),
+    "cube-tile": dict(strategy=1, direction_block=64, direct_cube=1),
+    "all-pols": dict(strategy=1, all_pols=1),
+    "mixed": dict(strategy=1, precision=1),
+}
+
+
+@pytest.mark.parametrize("where", ["device", "host"])
+@pytest.mark.parametrize("route", list(NO_ROWS))
+def test_rotate_over_no_rows_is_zero(leap, ctx, route, where):
+    """Sums over no rows are zero whatever an earlier call left in the context's buffers."""
+    print(f"no rows: {route}, {where}", flush=True)
+    s = leap.SynthMS(n_antennas=9, n_timesteps=2, n_channels=20, seed=61)
+    vis = s.fill_host()
+    p = ctx.malloc(vis.nbytes)
+    try:
+        ctx.h2d(p, vis)
+        view = leap.view_from_arrays(s.host_dict(), **(dict(vis_device=p, vis_dtype=leap.LEAP_VIS_C128)
+                                                       if where == "device" else {}))
+        md = ctx.metadata(view)
+        dirs = np.asarray(s.host_dict()["phase_centre"]) + [[0.01, 0.0], [0.0, 0.01], [0.02, -0.01]]
+        opts = leap.options(**NO_ROWS[route])
+        assert md.rotate(view, dirs, opts=opts).any()
+        assert not md.rotate(view, dirs, row_start=0, n_rows=0, opts=opts).any()
+        with pytest.raises(leap.LeapError):
+            md.rotate(view, dirs, row_start=view.num_rows + 1, n_rows=0, opts=opts)
+    finally:
+        ctx.free(p)
