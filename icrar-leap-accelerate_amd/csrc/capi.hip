@@ -1572,6 +1572,7 @@ void calibrate_batch(leap_ctx* ctx, const leap_batch_set* sets, uint32_t n_sets,
         return;
     }
     ctx->last_graph = 0;
+    bool waited = false;
     for (int32_t r = 0; r < rounds; ++r) {
         std::vector<MultiSetDesc> descs;
         std::vector<MultiShape> shapes;
@@ -1599,6 +1600,7 @@ void calibrate_batch(leap_ctx* ctx, const leap_batch_set* sets, uint32_t n_sets,
             LEAP_HIP(hipMemcpyAsync(ctx->h_cal.ptr, ctx->d_cal.ptr, total * sizeof(double), hipMemcpyDeviceToHost,
                                     ctx->stream));
             finish_stream(ctx);
+            waited = true;
             const double* from = ctx->h_cal.as<double>();
             for (uint32_t i : active) {
                 std::copy(from, from + st[i].h_cal.size(), st[i].h_cal.begin());
@@ -1607,7 +1609,7 @@ void calibrate_batch(leap_ctx* ctx, const leap_batch_set* sets, uint32_t n_sets,
         }
         deliver(r, [&](uint32_t i) -> const double* { return st[i].h_cal.data(); });
     }
-    if (n_dirs == 0 || rounds == 0) finish_stream(ctx);
+    if (!waited) finish_stream(ctx);  // no set had both directions and a solution
     end_timing(ctx);
 }
 

@@ -287,3 +287,26 @@ def test_uneven_batch_full_size(leap, ctx, oracle, precision):
     finally:
         for p in ptrs:
             ctx.free(p)
+
+
+@pytest.mark.parametrize("before", [0, 1], ids=["first-call", "after-another"])
+def test_batch_of_sets_without_work(leap, before):
+    """A set with directions whose slice holds no whole solution interval beside one with solutions but
+    no directions: nothing to compute, and the empty solutions are delivered."""
+    c = leap.Context(0)
+    try:
+        views = []
+        for n_ant, seed in ((8, 62), (9, 63)):
+            s = leap.SynthMS(n_antennas=n_ant, n_timesteps=2, n_channels=5, seed=seed)
+            s.fill_host()
+            views.append(leap.view_from_arrays(s.host_dict()))
+        mds = [c.metadata(v) for v in views]
+        if before:
+            c.calibrate(views[0], [(0.5, -0.47)], md=mds[0])
+        some, none = np.array([[0.5, -0.47], [0.51, -0.47]]), np.zeros((0, 2))
+        for _ in range(2):
+            got = c.calibrate_batch([(mds[0], views[0], some, (0, 9, -1)), (mds[1], views[1], none, (0, 1, -1))])
+            assert got[0][0].shape[0] == 0 and got[1][0].shape == (2, 0, 9)
+            assert c.last_kernel_times()[1] == 0
+    finally:
+        c.close()
