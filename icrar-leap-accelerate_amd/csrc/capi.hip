@@ -1017,13 +1017,17 @@ void calibrate_loop(leap_ctx* ctx, const leap_metadata& md, const leap_ms_view& 
     double* h_cal = ctx->h_cal.as<double>();
     const bool direct = per_sol * group <= kDirectResults;
     begin_stamps(ctx);
+    const uint32_t whole = std::min(uint32_t(T) / interval, uint32_t(std::max(solutions, 0)));  // with all of their rows
+    uint32_t first = 0, end = 0;  // of the group at hand
     for (int32_t s = 0; s < solutions; ++s) {  // :104
-        const uint32_t at = uint32_t(s) % group;
-        if (D > 0 && at == 0) {
-            // :113-119 — rows [s * interval * nbl, +interval * nbl); the slice start is not added.
-            const uint32_t n = std::min(group, uint32_t(solutions - s));
-            const DeviceRows rows = stage_rows(ctx, ms, uint32_t(size_t(s) * interval * nbl),
-                                               uint32_t(size_t(s + n) * interval * nbl), !packed_route(opts, 0));
+        if (D > 0 && uint32_t(s) == end) {
+            // :113-119 — rows [s * interval * nbl, +interval * nbl); the slice start is not added.  A slice
+            // may go past the last row: the first solution that does is refused once those before it are out.
+            first = end;
+            const uint32_t n = first < whole ? std::min(group, whole - first) : 1;
+            end = first + n;
+            const DeviceRows rows = stage_rows(ctx, ms, uint32_t(size_t(first) * interval * nbl),
+                                               uint32_t(size_t(end) * interval * nbl), !packed_route(opts, 0));
             const uint32_t ap = rotate_directions(ctx, md, ms, rows, interval, D, opts, 0, true, n);
             invert_intervals(ctx, md, D, n, opts, ap, direct ? h_cal : nullptr);
             if (!direct)
@@ -1038,7 +1042,7 @@ void calibrate_loop(leap_ctx* ctx, const leap_metadata& md, const leap_ms_view& 
         sol.n_directions = D;
         sol.directions = dirs;
         sol.n_antennas = uint32_t(N);
-        sol.calibrations = h_cal + per_sol * at;
+        sol.calibrations = h_cal + per_sol * (uint32_t(s) - first);
         if (cb && cb(user, &sol) != 0) throw Error(LEAP_ERR_CALLBACK, "output callback requested a stop");
     }
     if (D == 0 || solutions <= 0) finish_stream(ctx);

@@ -86,3 +86,29 @@ def test_callback_stops_between_grouped_intervals(leap, ctx):
     rc = leap.lib().leap_hip_calibrate_md(ctx.h, md.h, ctypes.byref(view), d.ctypes.data_as(leap._dp), len(d), 0, 1, -1,
                                           ctypes.byref(leap.options()), leap.SOLUTION_CB(cb), None)
     assert rc == -6 and seen == [0, 1]
+
+
+@pytest.mark.parametrize("route", ["plain", "wave", "mixed-wave", "nufft-w16"])
+def test_slice_past_the_last_row_delivers_its_whole_intervals(leap, ctx, route):
+    """Eleven timesteps in intervals of three to an end of 30: three solutions, then the range error,
+    whatever the intervals are grouped into; and four of a slice that ends inside a group."""
+    kw, C, D = ROUTES[route]
+    ms, dirs = _set(leap, C, D, 7)
+    view = leap.view_from_arrays(ms)
+    md = ctx.metadata(view)
+    want, _ = ctx.calibrate(view, dirs, (0, 3, -1), opts=leap.options(**kw), md=md)
+    seen = []
+
+    def cb(_user, sol):
+        n = sol.contents.n_directions * sol.contents.n_antennas
+        seen.append(np.ctypeslib.as_array(sol.contents.calibrations, shape=(n,)).copy())
+        return 0
+
+    d = np.ascontiguousarray(dirs)
+    rc = leap.lib().leap_hip_calibrate_md(ctx.h, md.h, ctypes.byref(view), d.ctypes.data_as(leap._dp), len(d), 0, 3, 30,
+                                          ctypes.byref(leap.options(**kw)), leap.SOLUTION_CB(cb), None)
+    assert rc == -2 and len(seen) == len(want) == 3
+    assert np.abs(npr.wrap(np.array(seen).reshape(want.shape) - want)).max() < 1e-9
+    part, _ = ctx.calibrate(view, dirs, (0, 1, 4), opts=leap.options(**kw), md=md)
+    every, _ = ctx.calibrate(view, dirs, (0, 1, -1), opts=leap.options(**kw), md=md)
+    assert len(part) == 4 and np.abs(npr.wrap(part - every[:4])).max() < (1e-7 if kw.get("precision") else 1e-10)
