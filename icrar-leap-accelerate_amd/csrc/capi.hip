@@ -1113,8 +1113,7 @@ struct NufftGroup {
 // complex128 for the width-16 kernel, with 1, 2 or 4 pols), by the single-set
 // automatic rule (96..512 channels, 16 or more directions) unless the NUFFT is
 // asked for.
-int32_t set_nufft_route(const leap_options& opts, const leap_metadata& md, const leap_ms_view& ms, uint32_t D,
-                        uint32_t interval) {
+int32_t set_nufft_route(const leap_options& opts, const leap_metadata& md, const leap_ms_view& ms, uint32_t D) {
     if (D == 0) return 0;
     int32_t cs = opts.channel_sum;
     if (cs == LEAP_CHANNEL_SUM_AUTO)
@@ -1129,18 +1128,27 @@ int32_t set_nufft_route(const leap_options& opts, const leap_metadata& md, const
                     "pols at an aligned address");
         return cs;
     }
-    if (opts.precision == LEAP_PRECISION_FP64 && names_no_tile(opts) && folded_beats_nufft(interval * md.nbl, D))
-        return 0;
     return cube_ok && md.channels >= kNufftMinChannels && D >= kNufftMinDirections ? cs : 0;
+}
+
+// Whether the kinds of launch are left to the multi-set call: no tile or grid named.
+bool names_no_launch(const leap_options& opts) { return names_no_tile(opts) && opts.workgroups_per_cu == 0; }
+
+// Whether a set that the rule above gives the width-16 NUFFT takes the folded kernel instead, as a
+// call of the set's own does; in a launch of its own, since the shared Horner tiles are another
+// kernel, which would also have to be tuned for the call's shapes first (64 antennas, 3 t, 128
+// channels, 24 directions beside two smaller sets: a context's first call 0.87 ms, 3.9 with the set
+// among the tiles; later ones 161 us against 317).
+bool set_takes_folded(const leap_options& opts, int32_t nufft, uint32_t rows, uint32_t D) {
+    return nufft && opts.channel_sum == LEAP_CHANNEL_SUM_AUTO && opts.precision == LEAP_PRECISION_FP64 &&
+           names_no_launch(opts) && folded_beats_nufft(rows, D);
 }
 
 // Whether a Horner set of a multi-set call gets a launch of the folded kernel of its own instead of a
 // place in the shared launch of Horner tiles: where no tile is named and the set's rows give the chip
 // two waves per SIMD.  128 antennas, 14 t, 48 channels of complex64, 64 directions: 81 us against 151,
 // and the host plans no schedule of the set's 8,256 work items (0.4 ms).
-bool own_launch(const leap_options& opts, uint32_t rows) {
-    return names_no_tile(opts) && opts.workgroups_per_cu == 0 && rows >= 8192;
-}
+bool own_launch(const leap_options& opts, uint32_t rows) { return names_no_launch(opts) && rows >= 8192; }
 
 // NUFFT tile of a multi-set launch: the caller's when it is a NUFFT tile,
 // otherwise 64, 128 or 256 directions per workgroup, the fewest that hold the
@@ -1399,8 +1407,11 @@ void calibrate_batch(leap_ctx* ctx, const leap_batch_set* sets, uint32_t n_sets,
         evaluate_slice(in.slice_start, in.slice_interval, in.slice_end, T, range);
         st[i] = BatchState{in.metadata, in.ms, in.directions, in.n_directions,
                            (range[2] - range[0]) / range[1], uint32_t(range[1]), {},
-                           set_nufft_route(opts, *in.metadata, *in.ms, in.n_directions, uint32_t(range[1]))};
-        st[i].own = !st[i].nufft && own_launch(opts, uint32_t(range[1]) * in.metadata->nbl);
+                           set_nufft_route(opts, *in.metadata, *in.ms, in.n_directions)};
+        const uint32_t rows = uint32_t(range[1]) * in.metadata->nbl;
+        const bool folded = set_takes_folded(opts, st[i].nufft, rows, in.n_directions);
+        if (folded) st[i].nufft = 0;
+        st[i].own = folded || (!st[i].nufft && own_launch(opts, rows));
         rounds = std::max(rounds, st[i].solutions);
     }
     while (ctx->batch_sets.size() < n_sets) ctx->batch_sets.push_back(std::make_unique<SetBuffers>());

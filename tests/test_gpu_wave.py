@@ -144,3 +144,33 @@ def test_multi_set_launches_of_their_own(leap, ctx, on_device, precision):
         again = ctx.calibrate_batch(sets, leap.options(graph=1, **opts))
         for (got, _), (want, _) in zip(again, eager):
             assert np.array_equal(got, want)
+
+
+@pytest.mark.parametrize("graph", [0, 1])
+def test_multi_set_calls_take_the_folded_kernel_or_the_nufft(leap, on_device, graph):
+    """An FP64 set of 2,080 rows that the automatic rule gives the folded sums gets a launch of that kernel
+    (its own call's bits), not a place among the shared Horner tiles, which would be tuned first; with a
+    grid named it keeps the width-16 NUFFT, and so does one of 1,953 rows."""
+    c = leap.Context(0)
+    try:
+        sets = []
+        for n_ant in (64, 62):
+            s = leap.SynthMS(n_antennas=n_ant, n_timesteps=1, n_channels=128, nan_fraction=0.003, seed=n_ant)
+            s.fill_host(np.complex64)
+            ms = s.host_dict()
+            view = on_device(ms)
+            dirs = np.asarray(ms["phase_centre"]) + np.random.default_rng(n_ant).uniform(-0.02, 0.02, (24, 2))
+            sets.append((c.metadata(view), view, dirs, (0, -1, -1)))
+        opts = dict(strategy=1, graph=graph)
+        for case, route in (([sets[0]], 1), (sets, 4), ([sets[1]], 4)):
+            got = c.calibrate_batch(case, leap.options(**opts))
+            assert c.last_route()[0] == route and c.last_direction_block() == 0
+            for (md, view, dirs, slice_), (cal, _) in zip(case, got):
+                want, _ = c.calibrate(view, dirs, slice_, opts=leap.options(strategy=1), md=md)
+                assert np.abs(np.angle(np.exp(1j * (cal - want)))).max() <= (0 if md is sets[0][0] else 1e-9)
+        named = c.calibrate_batch(sets, leap.options(workgroups_per_cu=4, **opts))
+        assert c.last_route()[0] == 4 and c.last_direction_block() == 0
+        for (cal, _), (want, _) in zip(named, c.calibrate_batch(sets, leap.options(**opts))):
+            assert np.abs(np.angle(np.exp(1j * (cal - want)))).max() <= 1e-9
+    finally:
+        c.close()
