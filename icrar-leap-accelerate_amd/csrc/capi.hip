@@ -2305,17 +2305,19 @@ extern "C" int leap_hip_residual_loss_grad(leap_ctx* ctx, const leap_metadata* m
         // adjoint of rotate -> average on the device
         DeviceBuffer &d_guvw = ctx->d_adj_guvw, &d_gdzp = ctx->d_adj_gdzp;
         d_guvw.reserve(size_t(R) * 3 * sizeof(double));
-        d_gdzp.reserve(size_t(nbl) * D * 3 * sizeof(double));
+        const uint32_t parts = row_sums ? adjoint_q_parts(D, T, nbl) : 1;
+        d_gdzp.reserve(size_t(nbl) * parts * D * 3 * sizeof(double));
         if (row_sums)
             launch_adjoint_q(s, ctx->d_adj_q.as<double>(), uvw, ctx->d_dd.as<double>(), ia.avg, ia.g_arg, D, T, nbl,
-                             md->freq_start_hz, md->freq_inc_hz, d_guvw.as<double>(), d_gdzp.as<double>(), stamps + 2);
+                             parts, md->freq_start_hz, md->freq_inc_hz, d_guvw.as<double>(), d_gdzp.as<double>(),
+                             stamps + 2);
         else
             launch_rotate_adjoint(s, rows.vis, ms->vis_dtype, uvw, ctx->d_dd.as<double>(), ia.avg, ia.g_arg, D, T, nbl,
                                   md->channels, md->pols, md->freq_start_hz, md->freq_inc_hz, d_guvw.as<double>(),
                                   d_gdzp.as<double>(), stamps + 2);
         // dL/d(dz row of dd) reduced over baselines and mapped to dL/d(ra, dec) (MetaData.cc:166-203
         // differentiated) on the device
-        launch_reduce_gdz_offsets(s, d_gdzp.as<double>(), nbl, D, md->phase_centre_ra, md->phase_centre_dec,
+        launch_reduce_gdz_offsets(s, d_gdzp.as<double>(), nbl * parts, D, md->phase_centre_ra, md->phase_centre_dec,
                                   ctx->h_dirs.as<double>(), h_out + D, stamps + 3);
         if (grad_antenna)
             launch_antenna_grad(s, d_guvw.as<double>(), d_M.as<double>(), ctx->d_adj_off.as<int32_t>(),

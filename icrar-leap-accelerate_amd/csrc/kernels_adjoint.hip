@@ -238,7 +238,10 @@ __global__ __launch_bounds__(kThreads) void rotate_adjoint_kernel(
 // baselines side by side, whose rows lie side by side in q, uvw and g_uvw, and the workgroup's four
 // waves their timesteps in turn.  Bound by reading q: 128 stations, 64 t, 16 directions
 // (266 MB) 69 us (4.2 TB/s with the gradients written) against 81 with a
-// baseline a workgroup and the sums in LDS behind two barriers a row.
+// baseline a workgroup and the sums in LDS behind two barriers a row.  Sets of few baselines would
+// leave most CUs idle for a long chain of rows, so there the timesteps go over several workgroups too
+// (blockIdx.y), each with partial sums of its own (15 baselines, 4,096 t, 16 directions: 10 us, 623 with
+// four workgroups).
 template <int DL, int ND>
 __global__ __launch_bounds__(kThreads) void adjoint_q_kernel(const double* __restrict__ q,
                                                              const double* __restrict__ uvw,
@@ -272,7 +275,7 @@ __global__ __launch_bounds__(kThreads) void adjoint_q_kernel(const double* __res
         if (dir_ok[j]) ab[j] = abar_of(avg, g_arg, size_t(dc) * nbl + bl);
         gdz[j][0] = gdz[j][1] = gdz[j][2] = 0.0;
     }
-    for (uint32_t t = wave; t < T; t += kW) {
+    for (uint32_t t = blockIdx.y * kW + wave; t < T; t += gridDim.y * kW) {
         const size_t row = size_t(t) * nbl + bl;
         const double u = uvw[3 * row], v = uvw[3 * row + 1], w = uvw[3 * row + 2];
         double g[3] = {0.0, 0.0, 0.0};
@@ -307,7 +310,7 @@ __global__ __launch_bounds__(kThreads) void adjoint_q_kernel(const double* __res
         if (blockIdx.x * BB + b >= nbl) continue;
         double s = 0.0;
         for (int w = 0; w < kW; ++w) s += s_g[w][b][o / 3][o % 3];
-        g_dz_partial[size_t(o) * nbl + blockIdx.x * BB + b] = s;
+        g_dz_partial[(size_t(o) * gridDim.y + blockIdx.y) * nbl + blockIdx.x * BB + b] = s;
     }
 }
 
@@ -348,7 +351,8 @@ __global__ __launch_bounds__(64 * kReduceWaves) void reduce_gdz_kernel(const dou
 }
 
 // One workgroup per antenna: sum over its baselines (sign +1 as antenna2, -1 as
-// antenna1) and timesteps of M_t^T g_uvw(t, b); a wave takes whole timesteps.
+// antenna1) and timesteps of M_t^T g_uvw(t, b); a wave takes whole timesteps, several at once where an
+// antenna has fewer than 33 baselines (the same set: 35 us, 212 with a timestep a wave).
 __global__ __launch_bounds__(64 * kReduceWaves) void antenna_grad_kernel(const double* __restrict__ g_uvw,
                                                                         const double* __restrict__ M,
                                                                         const int32_t* __restrict__ csr_off,
@@ -360,12 +364,15 @@ __global__ __launch_bounds__(64 * kReduceWaves) void antenna_grad_kernel(const d
     const int32_t a = blockIdx.x;
     const int32_t j0 = csr_off[a], j1 = csr_off[a + 1];
     const uint32_t lane = threadIdx.x % 64, wave = threadIdx.x / 64;
+    uint32_t per = 64;  // lanes of a timestep, a baseline each
+    while (per > 1 && int32_t(per / 2) >= j1 - j0) per /= 2;
+    const uint32_t at_once = 64 / per;  // timesteps of a wave
     double acc[3] = {0.0, 0.0, 0.0};
-    for (int32_t j = j0 + int32_t(lane); j < j1; j += 64) {
+    for (int32_t j = j0 + int32_t(lane % per); j < j1; j += int32_t(per)) {
         const double sgn = double(csr_sign[j]);
         const double* g_b = g_uvw + 3 * size_t(csr_bl[j]);
 #pragma unroll 4
-        for (uint32_t t = wave; t < T; t += kReduceWaves) {
+        for (uint32_t t = wave * at_once + lane / per; t < T; t += kReduceWaves * at_once) {
             const double* m = M + 9 * size_t(t);
             const double* g = g_b + 3 * size_t(t) * nbl;
             for (int k = 0; k < 3; ++k) acc[k] += sgn * (m[k] * g[0] + m[3 + k] * g[1] + m[6 + k] * g[2]);
@@ -603,13 +610,19 @@ void launch_rotate_adjoint(hipStream_t s, const void* vis, int32_t vis_dtype, co
     LEAP_HIP(hipGetLastError());
 }
 
+// Two workgroups a CU, of at least four rows a wave, where the baselines alone do not give them.
+uint32_t adjoint_q_parts(uint32_t D, uint32_t T, uint32_t nbl) {
+    const uint32_t side = D <= 16 ? 4 : D <= 32 ? 2 : 1;  // baselines of a wave
+    return std::max(1u, std::min(512 / ((nbl + side - 1) / side), T / (4 * (kThreads / 64))));
+}
+
 void launch_adjoint_q(hipStream_t s, const double* q, const double* uvw, const double* dd, const double* avg,
-                      const double* g_arg, uint32_t D, uint32_t T, uint32_t nbl, double f0, double df, double* g_uvw,
-                      double* g_dz_partial, uint64_t* started) {
+                      const double* g_arg, uint32_t D, uint32_t T, uint32_t nbl, uint32_t parts, double f0, double df,
+                      double* g_uvw, double* g_dz_partial, uint64_t* started) {
     const double kappa0 = f0 / kSpeedOfLight, dkappa = df / kSpeedOfLight;
     require(D >= 1 && D <= 256, LEAP_ERR_NOT_IMPLEMENTED, "the adjoint handles 1 to 256 directions per call");
 #define LEAP_ADJ(DL_, ND_)                                                                                           \
-    adjoint_q_kernel<DL_, ND_><<<(nbl + 64 / DL_ - 1) / (64 / DL_), kThreads, 0, s>>>(                               \
+    adjoint_q_kernel<DL_, ND_><<<dim3((nbl + 64 / DL_ - 1) / (64 / DL_), parts), kThreads, 0, s>>>(                  \
         q, uvw, dd, avg, g_arg, D, T, nbl, kappa0, dkappa, g_uvw, g_dz_partial, started)
     if (D <= 16)
         LEAP_ADJ(16, 1);

@@ -519,10 +519,12 @@ void launch_rotate_adjoint(hipStream_t s, const void* vis, int32_t vis_dtype, co
                            const double* avg, const double* g_arg, uint32_t D, uint32_t T, uint32_t nbl, uint32_t C,
                            uint32_t P, double f0, double df, double* g_uvw, double* g_dz_partial,
                            uint64_t* started = nullptr);
-// launch_rotate_adjoint's outputs from the row sums of HornerWave::q (no pass over the cube).
+// launch_rotate_adjoint's outputs from the row sums of HornerWave::q (no pass over the cube), with each
+// baseline's timesteps in adjoint_q_parts partial sums: g_dz_partial[3 D][parts nbl].
+uint32_t adjoint_q_parts(uint32_t D, uint32_t T, uint32_t nbl);
 void launch_adjoint_q(hipStream_t s, const double* q, const double* uvw, const double* dd, const double* avg,
-                      const double* g_arg, uint32_t D, uint32_t T, uint32_t nbl, double f0, double df, double* g_uvw,
-                      double* g_dz_partial, uint64_t* started = nullptr);
+                      const double* g_arg, uint32_t D, uint32_t T, uint32_t nbl, uint32_t parts, double f0, double df,
+                      double* g_uvw, double* g_dz_partial, uint64_t* started = nullptr);
 // dL/d(ra, dec) of each direction (2 D doubles at out) from g_dz_partial; dirs = the directions (ra, dec).
 void launch_reduce_gdz_offsets(hipStream_t s, const double* part, uint32_t nbl, uint32_t D, double ra0, double dec0,
                                const double* dirs, double* out, uint64_t* started = nullptr);

@@ -193,3 +193,22 @@ def test_adjoint_from_row_sums_equals_recomputed(leap, ctx, adjoint_mode, n_ant,
         got.append(md.loss_grad(view, dirs, s.enu_to_uvw, off, dp))
     for a, b in zip(*got):
         assert np.abs(a - b).max() <= 1e-9 * max(np.abs(a).max(), 1e-300)
+
+
+@pytest.mark.parametrize("mode", [1, 2], ids=["recompute", "row-sums"])
+@pytest.mark.parametrize("n_ant,T,D", [(2, 15, 1), (2, 70, 3), (3, 201, 16), (6, 513, 17), (5, 130, 64), (4, 99, 70), (34, 17, 2)])
+def test_adjoint_of_few_baselines_and_many_timesteps(leap, ctx, oracle, adjoint_mode, n_ant, T, D, mode):
+    """Timesteps over several workgroups of the row-sum adjoint (one to 256 of them, the last ones with
+    fewer or no rows) and several timesteps of a wave in the antenna gradient (1 to 33 baselines an
+    antenna), against the oracle at the bars above."""
+    print(f"few baselines: {n_ant} antennas, {T} t, {D} directions, mode {mode}", flush=True)
+    # two antennas need their autocorrelations: a reference antenna past the baselines is refused
+    s, ms, dirs, off, dp = problem(leap, n_ant, T, 3, D, 51 + D, autos=1 if n_ant == 2 else 0)
+    view = leap.view_from_arrays(ms)
+    md = ctx.metadata(view)
+    adjoint_mode(mode)
+    L, g_off, g_ant = md.loss_grad(view, dirs, s.enu_to_uvw, off, dp)
+    Lo, go_off, go_ant = oracle.loss_grad(ms, dirs, s.enu_to_uvw, off, dp)
+    assert abs(L - Lo) <= 1e-11 * max(abs(Lo), 1e-300)
+    assert np.abs(g_off - go_off).max() <= 1e-7 * max(np.abs(go_off).max(), 1e-300)
+    assert np.abs(g_ant - go_ant).max() <= 1e-7 * max(np.abs(go_ant).max(), 1e-300)
