@@ -97,6 +97,18 @@ void join_copy_stream(leap_ctx* ctx) {
     LEAP_HIP(hipStreamWaitEvent(ctx->stream, ctx->ev_copy_join, 0));
 }
 
+// A staging call that ends early leaves no copy in flight: its pieces' event is recorded after the last
+// one only, and the next call fills the same pinned buffers.
+struct EndsEarly {
+    leap_ctx* ctx;
+    bool done = false;
+    ~EndsEarly() {
+        if (done) return;
+        (void)hipStreamSynchronize(ctx->copy_stream);
+        ctx->h2d_pending[0] = ctx->h2d_pending[1] = false;
+    }
+};
+
 // The pinned buffer b is free once its previous copy has completed.
 void acquire(leap_ctx* ctx, int b) {
     if (ctx->h2d_pending[b]) {
@@ -131,6 +143,7 @@ void pack_pol0_host(const VT* src, uint32_t P, size_t begin, size_t end, VT* out
 void stage_copy(leap_ctx* ctx, const void* host_src, size_t bytes, void* device_dst) {
     if (bytes == 0) return;
     ensure_staging(ctx);
+    EndsEarly call{ctx};
     fork_copy_stream(ctx);
     const char* src = static_cast<const char*>(host_src);
     char* dst = static_cast<char*>(device_dst);
@@ -145,6 +158,7 @@ void stage_copy(leap_ctx* ctx, const void* host_src, size_t bytes, void* device_
         sent(ctx, b);
     }
     join_copy_stream(ctx);
+    call.done = true;
 }
 
 void stage_pol0(leap_ctx* ctx, const void* host_vis, int32_t vis_dtype, uint32_t P, size_t n, double* device_dst) {
@@ -155,6 +169,7 @@ void stage_pol0(leap_ctx* ctx, const void* host_vis, int32_t vis_dtype, uint32_t
     const size_t per_chunk = kChunkBytes / out_elem;
     if (c64)
         for (int b = 0; b < 2; ++b) ctx->d_widen[b].reserve(kChunkBytes);
+    EndsEarly call{ctx};
     fork_copy_stream(ctx);
     int b = 0;
     for (size_t e0 = 0; e0 < n; e0 += per_chunk, b ^= 1) {
@@ -187,6 +202,7 @@ void stage_pol0(leap_ctx* ctx, const void* host_vis, int32_t vis_dtype, uint32_t
         }
     }
     join_copy_stream(ctx);
+    call.done = true;
 }
 
 }  // namespace leap
