@@ -779,14 +779,15 @@ leap_metadata* create_metadata(leap_ctx* ctx, const leap_ms_view& ms, int32_t re
     table(d_mats, mats);
     table(d_status, status);
     const size_t up = l.bytes;
-    const size_t at_gp = l.add(4 * nn * sizeof(double)), at_scratch = l.add(2 * nn * sizeof(double) * mats.size());
+    const size_t at_gp = l.add(4 * nn * sizeof(double));
     md->d_all.reserve(l.bytes);
     char* base = md->d_all.as<char>();
     for (const Part& p : parts) p.part->ptr = base + p.at;
     md->d_Gp.ptr = base + at_gp;
     double* gp = md->d_Gp.as<double>();
     double* g1p = gp + 2 * nn;
-    double* scratch = reinterpret_cast<double*>(base + at_scratch);
+    ctx->d_gram.reserve(2 * nn * sizeof(double) * mats.size());  // the context's: a metadata keeps what calls read
+    double* scratch = ctx->d_gram.as<double>();
     auto gram = [&](size_t i, const PhaseMatrix& pm, const DevicePart& csr_off, const DevicePart& csr_ent,
                     const DevicePart& ant_pairs, double* out) {
         double* buf = scratch + 2 * nn * i;

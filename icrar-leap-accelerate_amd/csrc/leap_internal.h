@@ -325,6 +325,7 @@ struct leap_ctx {
     std::vector<double> h_avg;
     // calibrations of the last group of solution intervals (pinned: written by a kernel or a direct DMA)
     leap::PinnedBuffer h_cal;
+    leap::DeviceBuffer d_gram;  // a metadata's matrices while they are inverted (GramPinv::buf)
     // a metadata's tables on their way up (pinned); in use until the stream is waited for
     leap::PinnedBuffer h_md;
     bool md_in_use = false;

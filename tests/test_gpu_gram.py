@@ -5,6 +5,8 @@ exact integer matrix.  Both invert a diagonally dominant matrix and add the exac
 of the constraint's component, with N rounded steps per entry each: the tolerance is
 16 N eps of the largest entry.
 """
+import ctypes
+
 import numpy as np
 import pytest
 
@@ -74,3 +76,28 @@ def test_inversion_through_antenna_sums(leap, ctx, n_ant, graph, n_dirs):
     for cached in (False, True, True):
         md = ctx.metadata(view, ref_ant=0, use_cache=cached)
         assert np.abs(npr.wrap(md.apply_inversion(avg) - want)).max() < 1e-9
+
+
+def test_a_metadata_keeps_no_scratch(leap, ctx):
+    """Device memory of kept metadata with few baselines, where the antennas' square counts: what calls
+    read (G+ with and without the ones for A and A1, Ad, Ad1 and Ad's BF16 planes) and a tenth, without the
+    two more matrices each that the inversion works in."""
+    hip = ctypes.CDLL("libamdhip64.so.7")  # the runtime that the library has loaded
+
+    def free_bytes():
+        free, total = ctypes.c_size_t(), ctypes.c_size_t()
+        assert hip.hipMemGetInfo(ctypes.byref(free), ctypes.byref(total)) == 0
+        return free.value
+
+    n, count = 1024, 5
+    a1 = np.concatenate([np.arange(n - 1), [0]]).astype(np.int32)
+    a2 = np.concatenate([np.arange(1, n), [n - 1]]).astype(np.int32)
+    view = leap.view_from_arrays(_ms(a1, a2, np.zeros(n, dtype=np.uint8)))
+    kept = [ctx.metadata(view, ref_ant=0)]  # the context's own buffers are there after the first
+    K, K1 = kept[0].K, kept[0].K1
+    before = free_bytes()
+    kept += [ctx.metadata(view, ref_ant=0) for _ in range(count)]
+    used = (before - free_bytes()) / count
+    need = 8 * (4 * n * n + (K + K1) * n) + 6 * (K + 31) // 32 * 32 * n
+    print(f"{used / 2**20:.1f} MiB a metadata, {need / 2**20:.1f} read by calls", flush=True)
+    assert used <= 1.1 * need + 4 * 2**20
