@@ -645,8 +645,10 @@ __global__ __launch_bounds__(kThreads) void widen_c64_kernel(const C2<float>* __
 // SGPRs and feed the FMAs directly (no LDS traffic, no VGPRs for them); each
 // lane carries ND directions, a workgroup 64 * ND directions of one baseline
 // over 4 rows in flight.  Same operation order as rotate_average_horner64
-// with 64 lanes per row, hence the same results.
-template <int ND>
+// with 64 lanes per row, hence the same results.  MANY: blockIdx.z is the solution
+// interval; a kernel of its own, since the row loop has no scalar register left for
+// it (256 directions a workgroup: 2.61 ms, 2.83 with the interval's terms in it).
+template <int ND, bool MANY>
 __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(ND == 4 ? 4 : 1, 8))) void rotate_average_packed(
     const C2<double>* __restrict__ w, const double* __restrict__ uvw, const double* __restrict__ dd, uint32_t D,
     uint32_t T, uint32_t nbl, uint32_t C, uint32_t P, double kappa0, double dkappa, double* __restrict__ avg,
@@ -663,7 +665,7 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(ND == 
     __shared__ double s_red[RP][L][ND][2];
     const uint32_t lane = threadIdx.x % L;
     const uint32_t wave = __builtin_amdgcn_readfirstlane(threadIdx.x / L);
-    const uint32_t bl = blockIdx.x;
+    const uint32_t bl = blockIdx.x, z_interval = MANY ? blockIdx.z : 0;
     if (wave == 0) {
 #pragma unroll
         for (int j = 0; j < ND; ++j) {
@@ -684,7 +686,7 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(ND == 
     volatile double* vacc = &s_red[wave][lane][0][0];
     const uint32_t npairs = C / 2;
     for (uint32_t t = wave; t < T; t += RP) {
-        const size_t row = size_t(blockIdx.z) * T * nbl + size_t(t) * nbl + bl;  // z: solution interval
+        const size_t row = size_t(z_interval) * T * nbl + size_t(t) * nbl + bl;
         const double u = uvw[3 * row], v = uvw[3 * row + 1], ww = uvw[3 * row + 2];
         const C2<double>* wr = w + row * C;
         double sf[ND];
@@ -767,7 +769,7 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(ND == 
                 re += s_red[r][lane][j][0];
                 im += s_red[r][lane][j][1];
             }
-            double* o = avg + ((size_t(blockIdx.z) * D + dj) * nbl + bl) * P * 2;
+            double* o = avg + ((size_t(z_interval) * D + dj) * nbl + bl) * P * 2;
             if (accumulate) {
                 o[0] += re;
                 o[1] += im;
@@ -908,10 +910,14 @@ void launch_rotate_packed(hipStream_t s, int32_t tile, const double* w, const do
     const C2<double>* wp = reinterpret_cast<const C2<double>*>(w);
     const uint32_t db = uint32_t(tile / 10);
     const dim3 grid(nbl_grid, (D + db - 1) / db, intervals);
+    auto launch = [&](auto* kernel) {
+        kernel<<<grid, kThreads, 0, s>>>(wp, uvw, dd, D, T, nbl, C, P, kappa0, dkappa, avg, accumulate);
+    };
+    const bool many = intervals > 1;
     switch (tile) {
-        case 641: rotate_average_packed<1><<<grid, kThreads, 0, s>>>(wp, uvw, dd, D, T, nbl, C, P, kappa0, dkappa, avg, accumulate); break;
-        case 1282: rotate_average_packed<2><<<grid, kThreads, 0, s>>>(wp, uvw, dd, D, T, nbl, C, P, kappa0, dkappa, avg, accumulate); break;
-        case 2564: rotate_average_packed<4><<<grid, kThreads, 0, s>>>(wp, uvw, dd, D, T, nbl, C, P, kappa0, dkappa, avg, accumulate); break;
+        case 641: launch(many ? rotate_average_packed<1, true> : rotate_average_packed<1, false>); break;
+        case 1282: launch(many ? rotate_average_packed<2, true> : rotate_average_packed<2, false>); break;
+        case 2564: launch(many ? rotate_average_packed<4, true> : rotate_average_packed<4, false>); break;
         default: throw Error(LEAP_ERR_INVALID_ARGUMENT, "unsupported packed tile " + std::to_string(tile));
     }
     LEAP_HIP(hipGetLastError());

@@ -112,3 +112,20 @@ def test_slice_past_the_last_row_delivers_its_whole_intervals(leap, ctx, route):
     part, _ = ctx.calibrate(view, dirs, (0, 1, 4), opts=leap.options(**kw), md=md)
     every, _ = ctx.calibrate(view, dirs, (0, 1, -1), opts=leap.options(**kw), md=md)
     assert len(part) == 4 and np.abs(npr.wrap(part - every[:4])).max() < (1e-7 if kw.get("precision") else 1e-10)
+
+
+@pytest.mark.parametrize("tile,D", [((64, 1), 5), ((128, 2), 70), ((256, 4), 130)])
+def test_grouped_intervals_of_packed_tiles(leap, ctx, oracle, tile, D):
+    """Every packed tile over several intervals at once and over one, against the oracle and each other."""
+    print(f"packed tile {tile}, {D} directions", flush=True)
+    ms, dirs = _set(leap, 21, D, D)
+    view = leap.view_from_arrays(ms)
+    md = ctx.metadata(view)
+    opts = leap.options(strategy=1, channel_sum=1, direction_block=tile[0], lane_directions=tile[1])
+    got, _ = ctx.calibrate(view, dirs, (0, 2, -1), opts=opts, md=md)
+    want, _ = oracle.calibrate(ms, dirs[:: max(1, D // 5)], (0, 2, -1))
+    assert np.abs(npr.wrap(got[:, :: max(1, D // 5)] - want)).max() < 1e-9
+    rows = slice(0, 2 * ms["num_baselines"])
+    one = dict(ms, vis=ms["vis"][rows], uvw=ms["uvw"][rows], time=ms["time"][rows], num_rows=rows.stop)
+    alone, _ = ctx.calibrate(leap.view_from_arrays(one), dirs, (0, 2, -1), opts=opts, md=md)
+    assert np.abs(npr.wrap(got[0] - alone[0])).max() < 1e-10
