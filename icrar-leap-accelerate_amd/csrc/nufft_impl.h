@@ -956,8 +956,11 @@ __global__ __launch_bounds__(kWave) void rotate_average_nufft(const void* __rest
     const LEAP_GLOBAL double* uvr = uvw + row0 * 3;
     LEAP_GLOBAL double* out = mode == kNufftPartial ? avg + size_t(item) * D * 2
                                                     : avg + (size_t(blockIdx.z) * D * nbl + bl) * Pout * 2;
-    // Opaque, so that the row loop keeps the resolved pointers instead of their parts.
-    asm volatile("" : "+s"(wr), "+s"(uvr), "+s"(out));
+    // Opaque, so that the row loop keeps the resolved pointers instead of their parts (1 to 4% less time from
+    // complex64).  Not for several complex128 pols, whose loads hold the registers that this takes: with it
+    // 300 channels of 4 pols leave one wave a SIMD instead of two (64 directions of 128 antennas, 6 t: 245 us
+    // against 210; 384 channels 267 against 253).
+    if constexpr (SP <= 17) asm volatile("" : "+s"(wr), "+s"(uvr), "+s"(out));
     const uint32_t dstride = mode == kNufftPartial ? 2u : nbl * Pout * 2;  // doubles between directions
     nufft_rows<N, W, NDL, SP, CPL, F>(wr, scale, uvr, dd, D, t_count, nbl, bl, C, args, blockIdx.y * (kWave * NDL),
                                       out, dstride, mode, Pout, s_g, s_turn, lane);
