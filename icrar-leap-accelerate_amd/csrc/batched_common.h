@@ -67,9 +67,9 @@ __device__ inline C2<double> phasor_f64(double theta) {
 
 // exp(i th) by reduction modulo pi / 32 with a two-part constant through FMAs, a 64-entry
 // table in LDS and the series to r^8 (cos) and r^7 (sin) on |r| <= pi / 64, whose next terms
-// are below 2.5e-20 and 4.6e-18: 17 instructions.  The multiple k of pi / 32 is rounded by
-// adding 1.5 2^52, which leaves k mod 2^32 in the low word.  Accurate for |th| < 2^40, NaN for
-// a th that is not finite.
+// are below 2.5e-20 and 4.6e-18: 17 FP64 instructions, two for the table's address and an LDS
+// read.  The multiple k of pi / 32 is rounded by adding 1.5 2^52, which leaves k mod 2^32 in the
+// low word.  Accurate for |th| < 2^40, NaN for a th that is not finite.
 constexpr int kPhasorTable = 64;
 
 // By every thread of the workgroup; a barrier orders it before the first use.

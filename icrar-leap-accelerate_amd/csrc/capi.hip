@@ -267,13 +267,14 @@ bool folded_beats_nufft(uint32_t rows, uint32_t D) {
 bool names_no_tile(const leap_options& opts) { return opts.direction_block == 0 && opts.lane_directions == 0; }
 
 // The route of a batched call.  Horner calls on a device-resident cube that name no tile are routed by
-// the rates measured before the folded kernel: pack 5.2 TB/s; packed Horner 32 / 50 / 55 TFLOP/s with 1
+// the rates of the kernels before the folded one: pack 5.2 TB/s; packed Horner 32 / 50 / 55 TFLOP/s with 1
 // / 2 / 4 directions per lane (up to 64, 128, more directions); from the cube 5.7 TB/s and 50 TFLOP/s
-// (complex64) or 47 (complex128), both less by the phasors of a row (20 channels' worth).  So the
-// pack takes over from about 800 directions on complex64 and 480 on complex128, where callers that
-// look at the pack's times expect it.  (The folded kernel would be the faster there too: 128 antennas,
-// 14 t, 48 channels, 1,024 directions 0.88 ms against 1.17 packed.)  Host-resident cubes always take
-// the packed route (pol 0 only crosses the bus).
+// (complex64) or 47 (complex128), both less by the phasors of a row (20 channels' worth).  So with 4
+// pols the pack takes over above about 600 directions of 384 channels and 440 of 48.  The folded kernel,
+// which calls below that take, is the faster one there too (128 antennas, 14 t, 48 channels of complex64:
+// 448 directions 0.41 ms against 0.56 and 0.04 for the pack, 1,024 0.89 against 1.13 and 0.04; 600
+// channels, 640 directions 0.74 against 1.03 and 0.08), so the line can move.  Host-resident cubes always
+// take the packed route (pol 0 only crosses the bus).
 leap_options routed(const leap_options& o, const leap_ms_view& ms, uint32_t T, uint32_t D) {
     leap_options r = o;
     if (r.channel_sum == LEAP_CHANNEL_SUM_AUTO) {

@@ -66,9 +66,7 @@ __global__ void dd_kernel(double ra0, double dec0, const double* __restrict__ di
 // A wave owns its samples of one baseline and holds ND sums per pol in registers:
 //  - shift is the correctly rounded quotient: q = sf * r, r = RN(1 / lambda), then
 //    fma(fma(-q, lambda, sf), r, q) (Markstein 1990), 3 instructions against a division's 11
-//  - exp(i shift) by reduction modulo pi / 32 with a two-part constant through FMAs,
-//    a 64-entry table in LDS and the series to r^8 (cos) and r^7 (sin) on |r| <= pi / 64,
-//    whose next terms are below 2.5e-20 and 4.6e-18: 18 instructions
+//  - exp(i shift) from the 64-entry table in LDS (phasor_table)
 //  - the rotated sample goes into the sums as four FMAs
 // Samples that are not finite, a baseline's chunk of rows where a shift is not below 2^25 rad
 // (looked at once a row and direction) and channels without a finite wavelength take the plain

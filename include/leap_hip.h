@@ -171,8 +171,8 @@ typedef struct leap_options {
                                  pol 0 first (FP64, non-finite (row, channel)s zeroed; 16 B per
                                  row and channel of device memory; the Horner kernel then reads
                                  it with scalar loads) only above a number of directions set by
-                                 measured rates (from about 800 directions on complex64,
-                                 480 on complex128); host cubes and packed tiles always pack */
+                                 measured rates (with 4 pols about 600 of 384 channels, 440
+                                 of 48); host cubes and packed tiles always pack */
     int32_t pack_timesteps;   /* packed path: timesteps per pack chunk; chunks are packed on a
                                  second stream while the Horner kernel runs the previous one.
                                  0 = automatic; >= the interval's timesteps = one chunk */
@@ -274,8 +274,9 @@ typedef int (*leap_batch_cb)(void* user, uint32_t set, const leap_solution* solu
  * and timestep counts: each set gets the solutions leap_hip_calibrate_md would
  * give it with the same options.  Solution interval s of all sets, all
  * directions, is rotated and averaged in ONE persistent launch where a tile is named, and
- * for the sets that do not fill the GPU by themselves (fewer than 8,192 rows; a set that does
- * takes the launch of a single-set call): a device descriptor per set and (set, baseline, direction block) work items
+ * for the sets that do not fill the GPU by themselves (fewer than 8,192 rows, and not given the
+ * folded kernel by the automatic rule; the others take the launch of a single-set call): a device
+ * descriptor per set and (set, baseline, direction block) work items
  * statically load-balanced over the grid on the host (longest processing time
  * first), so the result does not depend on scheduling.  In mixed precision the
  * sets that qualify for the NUFFT channel sums (channel_sum automatic: 96..512
